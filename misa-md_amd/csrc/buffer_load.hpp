@@ -71,6 +71,7 @@ __device__ __forceinline__ void ldRec(Rsrc r, uint32_t o, T (&out)[N]) {
 
 typedef unsigned int u32x3 __attribute__((ext_vector_type(3)));
 typedef float f32x3 __attribute__((ext_vector_type(3)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Three floats (12 bytes) at byte offset `o`: a load whose destination
 // registers are all used, so none of them is reused while it is in flight.

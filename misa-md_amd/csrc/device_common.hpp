@@ -188,16 +188,22 @@ __device__ __forceinline__ bool wideTarget(int8_t ti, int8_t tj) { return !(tj <
 __device__ __forceinline__ int species(int8_t t) { return t & 3; }
 __device__ __forceinline__ int pairIdx(int a, int b) { return a >= b ? a * (a + 1) / 2 + b : b * (b + 1) / 2 + a; }
 
-// Knot search of the mixed-precision passes for r below the cutoff: knot
-// floor(r/dr) (at most n-2) and the local coordinate r/dr - knot (at most 1).
-// The same knot and coordinate as knotOf in exact arithmetic, without the
-// one-based detour.
+// Knot search of the site passes for r >= 0: t = r/dr, at most the last knot,
+// its whole part m and its fraction q.  The same segment and coordinate as
+// knotOf in exact arithmetic, without the one-based detour; a pair at or
+// beyond the last knot takes that knot with q = 0, whose value and slope are
+// those of the last segment's end.
 __device__ __forceinline__ int knotM(float r, float rdr, int n, float& q) {
 #pragma clang fp contract(off)
-  const float t = r * rdr;
-  const int m = min(static_cast<int>(t), n - 2);
-  q = fminf(t - static_cast<float>(m), 1.0f);
-  return m;
+  const float t = fminf(r * rdr, static_cast<float>(n - 1));
+  q = __builtin_amdgcn_fractf(t);
+  return static_cast<int>(t);
+}
+__device__ __forceinline__ int knotM(double r, double rdr, int n, double& q) {
+#pragma clang fp contract(off)
+  const double t = fmin(r * rdr, static_cast<double>(n - 1));
+  q = __builtin_amdgcn_fract(t);
+  return static_cast<int>(t);
 }
 
 // Knot search of the eam/alloy convention: p = x/delta + 1 (one-based knot),
@@ -250,16 +256,12 @@ __device__ __forceinline__ T embed(const Tables<T>& tb, int e, T rho) {
   return v;
 }
 
+// x^-1/2 to FP64 rounding: the hardware's estimate (relative error e/2 near
+// 2^-24) and one step of third order, y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2.
 __device__ __forceinline__ double rsqrtRefined(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  // two Newton steps on y = x^-1/2: y <- y (3 - x y^2) / 2
-  double h = x * y;
-  double e = fma(-h, y, 1.0);
-  y = fma(0.5 * y, e, y);
-  h = x * y;
-  e = fma(-h, y, 1.0);
-  y = fma(0.5 * y, e, y);
-  return y;
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
 // Pair force factor (pot eam::toForce): fpair = -(F'_i rho'_j + F'_j rho'_i +
@@ -299,6 +301,27 @@ __device__ __forceinline__ float pairForce(const Tables<float>& tb, int ei, int 
   const float phi = z2 * rinv;
   const float phip = z2p * rinv - phi * rinv;
   const float psip = dfi * rhojp + dfj * rhoip + phip;
+  return -psip * rinv;
+}
+
+// fpair of one pair (pot eam::toForce) in FP64 from its value cubics: r*phi
+// {c3, c4, c5, c6}, the neighbour's density and the centre's {c3, c4, c5}, per
+// knot spacing; the slopes from the same chains as the values
+// (a = c3 q + c4, b = a q + c5, slope = (c3 q + a) q + b).  One fixed rounding
+// for every pass.
+__device__ __forceinline__ double pairFpD(double q, double rinv, double z3, double z4, double z5, double z6,
+                                          double j3, double j4, double j5, double i3, double i4, double i5,
+                                          double dfi, double dfj, double rdr) {
+#pragma clang fp contract(off)
+  const double a = fma(z3, q, z4), b = fma(a, q, z5);
+  const double z2 = fma(b, q, z6);
+  const double z2p = fma(fma(z3, q, a), q, b) * rdr;
+  const double ja = fma(j3, q, j4), ia = fma(i3, q, i4);
+  const double rhojp = fma(fma(j3, q, ja), q, fma(ja, q, j5)) * rdr;
+  const double rhoip = fma(fma(i3, q, ia), q, fma(ia, q, i5)) * rdr;
+  const double phi = z2 * rinv;
+  const double phip = (z2p - phi) * rinv;
+  const double psip = fma(dfi, rhojp, fma(dfj, rhoip, phip));
   return -psip * rinv;
 }
 

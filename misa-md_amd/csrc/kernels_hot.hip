@@ -68,6 +68,15 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
   return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
+// The lane's record address, or for a lane without an atom that of the
+// wavefront's first atom (same parity), from where every offset is readable.
+// Called by whole wavefronts.
+__device__ __forceinline__ uint32_t addressOfLives(uint32_t o16, bool live, uint64_t lives) {
+  const uint32_t first = static_cast<uint32_t>(
+      __builtin_amdgcn_readlane(static_cast<int>(o16), __builtin_ctzll(lives)));
+  return live ? o16 : first;
+}
+
 // Calls visit(ks, nv) for the set bits of (b0, b1) in increasing order, U at
 // a time, then one at a time (nv = U or 1; ks holds the offsets).
 template <int U, typename Visit>
@@ -362,111 +371,63 @@ __device__ __forceinline__ void pairSegD(Rsrc rtab, Rsrc rtabR, const double* kn
   }
 }
 
-// One site of the FP64 force pass: thread tl of block b (also a virtual
-// block of the persistent launch).  With LDS, knD holds the segments of the
-// Fe-Fe pairs from knot mlo on, 7 doubles a knot: the r*phi value cubic
-// c3..c6 and the Fe density cubic c3..c5 (its c6 enters no force); a pair
-// of Fe atoms at such a knot reads them there, every other pair from the
-// tables in global memory.  Both give the same values, so the same bits.
-template <typename T, int ACC, int MODE, int U, bool LDS>
-__device__ __forceinline__ void forceSiteD(const Geom& G, const LatOffsets& O, const Tables<T>& tb, CXPtr x, XPtr xn,
-                                           const int8_t* __restrict__ type, const T* __restrict__ df,
-                                           const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
-                                           const uint64_t* __restrict__ id, const VerletParams& vp,
-                                           const StageArgs& st, Ctl* ctl, const InterView& iv, const Rec64& r64,
-                                           const Rec64& rn64, const T* knD, int mlo, uint32_t b, uint32_t tl,
-                                           unsigned long long& vb, unsigned long long& db) {
-  int64_t s;
-  int p, cx, cy, cz;
-  if (!siteOfBlock(G, b, tl, s, p, cx, cy, cz)) return;
-  const int8_t ti = type[s];
-  const double xi0 = x.c[0][s], xi1 = x.c[1][s], xi2 = x.c[2][s];
-  if (isVacant(ti)) {  // vacancy: keeps its stale position (atom.cpp:43-47)
-    if (MODE != 1) {   // clearForce left 0 there and latForce skips it (atom.cpp:86-100, 311-358)
-      f.c[0][s] = 0.0;
-      f.c[1][s] = 0.0;
-      f.c[2][s] = 0.0;
-    } else {
-      xn.c[0][s] = xi0;
-      xn.c[1][s] = xi1;
-      xn.c[2][s] = xi2;
-      putRec64(rn64, s, ti, xi0, xi1, xi2);
-      forEachImage(G, p, cx, cy, cz, [&](int64_t q, int sx, int sy, int sz) {
-        xn.c[0][q] = xi0 + sx * G.L0;
-        xn.c[1][q] = xi1 + sy * G.L1;
-        xn.c[2][q] = xi2 + sz * G.L2;
-        putRec64(rn64, q, ti, xn.c[0][q], xn.c[1][q], xn.c[2][q]);
-      });
-    }
+// The sums of the FP64 force passes run over four ranges of 32 offsets (the
+// 32-bit words of the wavefront's mask): in each range the pairs that the LDS
+// pass holds segments for and the others apart (heldPair), each in offset
+// order, and the ranges' sums one after the other.
+__device__ __forceinline__ uint32_t maskWord(uint64_t m0, uint64_t m1, int r) {
+  return static_cast<uint32_t>((r < 2 ? m0 : m1) >> (32 * (r & 1)));
+}
+
+struct Force3 {
+  double x = 0, y = 0, z = 0;
+  __device__ __forceinline__ void add(double d0, double d1, double d2, double fp) {
+    x = __fma_rn(d0, fp, x);
+    y = __fma_rn(d1, fp, y);
+    z = __fma_rn(d2, fp, z);
+  }
+  __device__ __forceinline__ void add(const Force3& o) {
+    x += o.x;
+    y += o.y;
+    z += o.z;
+  }
+};
+
+// A vacancy in the FP64 force pass: f = 0 (clearForce, and latForce skips it),
+// or in the fused pass its stale position into the next buffers.
+template <int MODE>
+__device__ __forceinline__ void vacancyForceD(const Geom& G, int64_t s, int p, int cx, int cy, int cz, int8_t ti,
+                                              CXPtr x, XPtr xn, XPtr f, const Rec64& rn64) {
+  if (MODE != 1) {  // clearForce left 0 there and latForce skips it (atom.cpp:86-100, 311-358)
+    f.c[0][s] = 0.0;
+    f.c[1][s] = 0.0;
+    f.c[2][s] = 0.0;
     return;
   }
-  const int ei = species(ti);
-  const T dfi = df[s];
-  // neighbours from the FP64 site records: position and, in w, F' with the
-  // species (a vacancy sits far out, so the distance test drops it)
-  const Rsrc rxy = rsrcBelow(r64.xy, O.lo), rzw = rsrcBelow(r64.zw, O.lo);
-  const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.pairF));
-  const Rsrc rtabR = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoV));
-  const uint32_t o16 = static_cast<uint32_t>(s) * 16u;
-  const uint32_t pairBase = static_cast<uint32_t>(ei * 3) * static_cast<uint32_t>(tb.nr);
-  const uint32_t* sh = O.sh[p];
-  Sum3<ACC> acc;
-  auto group = [&](auto UC, const int* ks) {
-    constexpr int V = decltype(UC)::value;
-    double d0[V], d1[V], d2[V], wj[V];
-#pragma unroll
-    for (int u = 0; u < V; ++u) {
-      const uint32_t so = sh[ks[u]] * 16u;
-      const double2 xy = ldRec64(rxy, o16, so), zw = ldRec64(rzw, o16, so);
-      d0[u] = xy.x;
-      d1[u] = xy.y;
-      d2[u] = zw.x;
-      wj[u] = zw.y;
-    }
-    bool in[V];
-    T pp[V], ri[V], dfj[V];
-    T rec[V][kPairRec], reci[V][kRhoRec];
-#pragma unroll
-    for (int u = 0; u < V; ++u) {
-      d0[u] = xi0 - d0[u];
-      d1[u] = xi1 - d1[u];
-      d2[u] = xi2 - d2[u];
-      const double r2 = dist2D(d0[u], d1[u], d2[u]);
-      in[u] = r2 < G.rc2;
-      if (in[u]) {
-        const T q2 = static_cast<T>(r2);
-        ri[u] = rsqT(q2);
-        const int m = knotOf(q2 * ri[u], tb.rdr, tb.nr, false, pp[u]);
-        pairSegD<LDS>(rtab, rtabR, knD, mlo, pairBase, tb.nr, ei, recSpecies64(wj[u]), m, rec[u], reci[u]);
-        dfj[u] = static_cast<T>(wj[u]);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < V; ++u) {
-      if (in[u]) {
-        // value cubics c3..c6 in the knot-local coordinate q; derivatives
-        // (3 c3 q + 2 c4) q + c5 per knot spacing, times 1/dr
-        const T q = pp[u], rinv = ri[u];
-        const T* z = rec[u];
-        const T* rj = rec[u] + 4;
-        const T* rI = reci[u];
-        const T z2 = ((z[0] * q + z[1]) * q + z[2]) * q + z[3];
-        const T z2p = ((T(3) * z[0] * q + T(2) * z[1]) * q + z[2]) * tb.rdr;
-        const T rhojp = ((T(3) * rj[0] * q + T(2) * rj[1]) * q + rj[2]) * tb.rdr;
-        const T rhoip = ((T(3) * rI[0] * q + T(2) * rI[1]) * q + rI[2]) * tb.rdr;
-        const T phi = z2 * rinv;
-        const T phip = z2p * rinv - phi * rinv;
-        const T psip = dfi * rhojp + dfj[u] * rhoip + phip;
-        acc.add(d0[u], d1[u], d2[u], -psip * rinv);
-      }
-    }
-  };
-  // the offsets the density pass found in range for some lane of this wavefront
-  const uint32_t wv = b * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tl >> 6);
-  forMaskGroups<U>(uniform64(wmask[2 * wv]), uniform64(wmask[2 * wv + 1]), [&](const int* ks, int nv) {
-    if (nv == U) group(std::integral_constant<int, U>{}, ks);
-    else group(std::integral_constant<int, 1>{}, ks);
+  const double xi0 = x.c[0][s], xi1 = x.c[1][s], xi2 = x.c[2][s];
+  xn.c[0][s] = xi0;
+  xn.c[1][s] = xi1;
+  xn.c[2][s] = xi2;
+  putRec64(rn64, s, ti, xi0, xi1, xi2);
+  forEachImage(G, p, cx, cy, cz, [&](int64_t q, int sx, int sy, int sz) {
+    xn.c[0][q] = xi0 + sx * G.L0;
+    xn.c[1][q] = xi1 + sy * G.L1;
+    xn.c[2][q] = xi2 + sz * G.L2;
+    putRec64(rn64, q, ti, xn.c[0][q], xn.c[1][q], xn.c[2][q]);
   });
+}
+
+// After the lattice sum of an occupied site: the inter atoms, the full-list
+// remainder near far lattice atoms, then the Verlet step.
+template <int MODE>
+__device__ __forceinline__ void forceTailD(const Geom& G, int64_t s, int p, int cx, int cy, int cz, int8_t ti,
+                                           int ei, double dfi, const Force3& lat, double xi0, double xi1, double xi2,
+                                           const Tables<double>& tb, CXPtr x, XPtr xn,
+                                           const int8_t* __restrict__ type, const double* __restrict__ df, XPtr v,
+                                           XPtr f, const uint64_t* __restrict__ id, const VerletParams& vp,
+                                           const StageArgs& st, Ctl* ctl, const InterView& iv, const Rec64& rn64,
+                                           unsigned long long& vb, unsigned long long& db) {
+  Force3 acc = lat;
   if (ti & kNearInter) {  // forces from inter atoms on lattice neighbours (atom.cpp:397-422)
     const int ne = static_cast<int>(iv.ctl->n_inter + iv.ctl->n_ghost);
     const FullPlaneOffsets& full = *iv.full;
@@ -474,7 +435,7 @@ __device__ __forceinline__ void forceSiteD(const Geom& G, const LatOffsets& O, c
       const int src = iv.e_src[e];
       const double d0 = xi0 - iv.e_x[0][e], d1 = xi1 - iv.e_x[1][e], d2 = xi2 - iv.e_x[2][e];
       const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-      if (r2 < G.rc2) acc.add(d0, d1, d2, pairForce(tb, ei, species(iv.type[src]), r2, dfi, dfOf<T>(iv, src)));
+      if (r2 < G.rc2) acc.add(d0, d1, d2, pairForce(tb, ei, species(iv.type[src]), r2, dfi, iv.df64[src]));
     });
   }
   if (ti & kWide) {  // full-list offsets beyond the pruned list, near a far lattice atom
@@ -484,22 +445,317 @@ __device__ __forceinline__ void forceSiteD(const Geom& G, const LatOffsets& O, c
       if (r2 < G.rc2) acc.add(e0, e1, e2, pairForce(tb, ei, species(tj), r2, dfi, df[j]));
     });
   }
-  double f0, f1, f2;
-  sum3Value<ACC>(acc, f0, f1, f2);
-  checkFinite(ctl, f0, f1, f2);
-  verletTail<MODE>(G, s, p, cx, cy, cz, ti, ei, xi0, xi1, xi2, f0, f1, f2, xn, v, f, id, vp, st, ctl, rn64, vb, db);
+  checkFinite(ctl, acc.x, acc.y, acc.z);
+  verletTail<MODE>(G, s, p, cx, cy, cz, ti, ei, xi0, xi1, xi2, acc.x, acc.y, acc.z, xn, v, f, id, vp, st, ctl, rn64,
+                   vb, db);
 }
 
-template <typename T, int ACC, int MODE, int U>
-__global__ __launch_bounds__(kBlock) void kForce(Geom G, LatOffsets O, Tables<T> tb, CXPtr x, XPtr xn,
-                                                 const int8_t* __restrict__ type, const T* __restrict__ df,
+// One site of the FP64 force pass, the segments from the tables in global
+// memory.
+template <int MODE, int U>
+__device__ __forceinline__ void forceSiteD(const Geom& G, const LatOffsets& O, const Tables<double>& tb, CXPtr x,
+                                           XPtr xn, const int8_t* __restrict__ type, const double* __restrict__ df,
+                                           const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
+                                           const uint64_t* __restrict__ id, const VerletParams& vp,
+                                           const StageArgs& st, Ctl* ctl, const InterView& iv, const Rec64& r64,
+                                           const Rec64& rn64, int mlo, uint32_t b, uint32_t tl,
+                                           unsigned long long& vb, unsigned long long& db) {
+  int64_t s;
+  int p, cx, cy, cz;
+  if (!siteOfBlock(G, b, tl, s, p, cx, cy, cz)) return;
+  const int8_t ti = type[s];
+  if (isVacant(ti)) {  // vacancy: keeps its stale position (atom.cpp:43-47)
+    vacancyForceD<MODE>(G, s, p, cx, cy, cz, ti, x, xn, f, rn64);
+    return;
+  }
+  const double xi0 = x.c[0][s], xi1 = x.c[1][s], xi2 = x.c[2][s];
+  const int ei = species(ti);
+  const double dfi = df[s];
+  // neighbours from the FP64 site records: position and, in w, F' with the
+  // species (a vacancy sits far out, so the distance test drops it)
+  const Rsrc rxy = rsrcBelow(r64.xy, O.lo), rzw = rsrcBelow(r64.zw, O.lo);
+  const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.pairF));
+  const Rsrc rtabR = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoV));
+  const uint32_t o16 = static_cast<uint32_t>(s) * 16u;
+  const uint32_t pairBase = static_cast<uint32_t>(ei * 3) * static_cast<uint32_t>(tb.nr);
+  const uint32_t* sh = O.sh[p];
+  Force3 tot, otot;
+  // the offsets the density pass found in range for some lane of this wavefront
+  const uint32_t wv = b * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tl >> 6);
+  const uint64_t m0 = uniform64(wmask[2 * wv]), m1 = uniform64(wmask[2 * wv + 1]);
+  for (int rg = 0; rg < 4; ++rg) {
+    Force3 part, opart;
+    auto group = [&](auto UC, const int* ks) {
+      constexpr int V = decltype(UC)::value;
+      double d0[V], d1[V], d2[V], wj[V];
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        const uint32_t so = sh[ks[u]] * 16u;
+        const double2 xy = ldRec64(rxy, o16, so), zw = ldRec64(rzw, o16, so);
+        d0[u] = xy.x;
+        d1[u] = xy.y;
+        d2[u] = zw.x;
+        wj[u] = zw.y;
+      }
+      bool in[V], held[V];
+      double pp[V], ri[V], rec[V][kPairRec], reci[V][kRhoRec];
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        d0[u] = xi0 - d0[u];
+        d1[u] = xi1 - d1[u];
+        d2[u] = xi2 - d2[u];
+        const double r2 = dist2D(d0[u], d1[u], d2[u]);
+        in[u] = r2 < G.rc2;
+        if (in[u]) {
+          ri[u] = rsqT(r2);
+          const int m = knotM(r2 * ri[u], tb.rdr, tb.nr, pp[u]);
+          const int ej = recSpecies64(wj[u]);
+          held[u] = heldPair(ei, static_cast<uint32_t>(ej), m, mlo);
+          pairSegD<false>(rtab, rtabR, nullptr, 0, pairBase, tb.nr, ei, ej, m, rec[u], reci[u]);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        if (!in[u]) continue;
+        const double* z = rec[u];
+        const double fp = pairFpD(pp[u], ri[u], z[0], z[1], z[2], z[3], z[4], z[5], z[6], reci[u][0], reci[u][1],
+                                  reci[u][2], dfi, wj[u], tb.rdr);
+        if (held[u]) part.add(d0[u], d1[u], d2[u], fp);
+        else opart.add(d0[u], d1[u], d2[u], fp);
+      }
+    };
+    forMaskGroups<U>(static_cast<uint64_t>(maskWord(m0, m1, rg)), 0ull, [&](const int* k32, int nv) {
+      int ks[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) ks[u] = k32[u] + 32 * rg;
+      if (nv == U) group(std::integral_constant<int, U>{}, ks);
+      else group(std::integral_constant<int, 1>{}, ks);
+    });
+    tot.add(part);
+    otot.add(opart);
+  }
+  tot.add(otot);
+  forceTailD<MODE>(G, s, p, cx, cy, cz, ti, ei, dfi, tot, xi0, xi1, xi2, tb, x, xn, type, df, v, f, id, vp, st, ctl,
+                   iv, rn64, vb, db);
+}
+
+// The Fe-Fe segments of the FP64 LDS pass from knot mlo on, 40 bytes a knot:
+// {slope of r*phi, slope of rho} and {value of r*phi, its step to the next
+// knot} in 16-byte halves, and the density's step.  The cubics' two other
+// coefficients come from the knot and its successor, with the operations and
+// roundings that the tables were built with, so the segments are the tables'.
+struct KnotsD {
+  const double2* s;   // {s_z, s_rho} of knot m at s[m] (the arrays start at knot mlo)
+  const double2* yd;  // {y_z, y_z(m+1) - y_z(m)}
+  const double* dr;   // y_rho(m+1) - y_rho(m)
+};
+__device__ __forceinline__ double hermite4(double dy, double s0, double s1) {  // 3 dy - 2 s0 - s1
+  return __dsub_rn(__fma_rn(-2.0, s0, __dmul_rn(3.0, dy)), s1);
+}
+__device__ __forceinline__ double hermite3(double dy, double s0, double s1) {  // s0 + s1 - 2 dy
+  return __fma_rn(-2.0, dy, __dadd_rn(s0, s1));
+}
+
+// Works off the first n (at most 64) noted pairs, one a lane, as
+// drainQueueM does; the pairs of one rank are added before those of the next,
+// so every site's pairs join its sum in offset order.
+__device__ __forceinline__ void drainQueueD(const uint16_t* q, int n, int rg, double xi0, double xi1, double xi2,
+                                            int ei, double dfi, uint32_t o16, Rsrc rxy, Rsrc rzw, Rsrc rtab, Rsrc rtabR,
+                                            const Tables<double>& tb, const uint32_t* __restrict__ sh, WaveSums& ws) {
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+  const bool on = lane < n;
+  const uint32_t e = q[on ? lane : 0];
+  const int owner = static_cast<int>(e & 63u);
+  const uint32_t rank = e >> 11;
+  const uint32_t oo = static_cast<uint32_t>(laneGet(static_cast<int>(o16), owner)) + sh[32 * rg + ((e >> 6) & 31u)] * 16u;
+  const double2 xy = ldRec64(rxy, oo, 0), zw = ldRec64(rzw, oo, 0);
+  const double d0 = laneGet(xi0, owner) - xy.x, d1 = laneGet(xi1, owner) - xy.y, d2 = laneGet(xi2, owner) - zw.x;
+  const int ti = laneGet(ei, owner), tj = recSpecies64(zw.y);
+  const double r2 = dist2D(d0, d1, d2);
+  const double ri = rsqT(r2);
+  double pp, rec[kPairRec], reci[kRhoRec];
+  const int m = knotM(r2 * ri, tb.rdr, tb.nr, pp);
+  pairSegD<false>(rtab, rtabR, nullptr, 0, static_cast<uint32_t>(ti * 3) * static_cast<uint32_t>(tb.nr), tb.nr, ti,
+                  tj, m, rec, reci);
+  const double fp = pairFpD(pp, ri, rec[0], rec[1], rec[2], rec[3], rec[4], rec[5], rec[6], reci[0], reci[1],
+                            reci[2], laneGet(dfi, owner), zw.y, tb.rdr);
+  bool wait = on;
+  for (uint32_t r = 0; __ballot(wait); ++r) {
+    if (wait && rank == r) {
+      ws.s[0][owner] = __fma_rn(d0, fp, ws.s[0][owner]);
+      ws.s[1][owner] = __fma_rn(d1, fp, ws.s[1][owner]);
+      ws.s[2][owner] = __fma_rn(d2, fp, ws.s[2][owner]);
+      wait = false;
+    }
+    waveLdsFence();  // another lane's pair of this site reads what was just written
+  }
+}
+
+// One virtual block of the FP64 LDS force pass: per site the same pairs and
+// sums as kForce (forceSiteD), the segments of the held pairs from LDS and
+// the other pairs worked off by the whole wavefront at the end of each range.
+template <int MODE, int U>
+__device__ __forceinline__ void forceVBlockD(const Geom& G, const LatOffsets& O, const Tables<double>& tb, CXPtr x,
+                                             XPtr xn, const int8_t* __restrict__ type,
+                                             const double* __restrict__ df, const uint64_t* __restrict__ wmask,
+                                             XPtr v, XPtr f, const uint64_t* __restrict__ id, const VerletParams& vp,
+                                             const StageArgs& st, Ctl* ctl, const InterView& iv, const Rec64& r64,
+                                             const Rec64& rn64, const KnotsD& kn, int mlo, WaveQueueD<U>& wq,
+                                             WaveSums& ws, uint32_t b, uint32_t tl, unsigned long long& vb,
+                                             unsigned long long& db) {
+  int64_t s = 0;
+  int p = 0, cx = 0, cy = 0, cz = 0;
+  const bool site = siteOfBlock(G, b, tl, s, p, cx, cy, cz);
+  int8_t ti = kVacant;
+  if (site) {
+    ti = type[s];
+    if (isVacant(ti)) vacancyForceD<MODE>(G, s, p, cx, cy, cz, ti, x, xn, f, rn64);
+  }
+  const bool live = !isVacant(ti);
+  const uint64_t lives = __ballot(live);
+  if (!lives) return;
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+  const int ei = live ? species(ti) : 0;
+  double xi0 = kNoAtom, xi1 = kNoAtom, xi2 = kNoAtom, dfi = 0.0;
+  if (live) {
+    xi0 = x.c[0][s];
+    xi1 = x.c[1][s];
+    xi2 = x.c[2][s];
+    dfi = df[s];
+  }
+  const Rsrc rxy = rsrcBelow(r64.xy, O.lo), rzw = rsrcBelow(r64.zw, O.lo);
+  const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.pairF));
+  const Rsrc rtabR = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoV));
+  const uint32_t o16 = addressOfLives(static_cast<uint32_t>(s) * 16u, live, lives);
+  const uint32_t* sh = O.sh[__builtin_amdgcn_readfirstlane((b >> 3) & 1u)];
+  const uint32_t wv = b * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tl >> 6);
+  const uint64_t m0 = uniform64(wmask[2 * wv]), m1 = uniform64(wmask[2 * wv + 1]);
+  Force3 tot, otot;
+  // The next U offsets of a range and their records' loads; an entry past the
+  // range's last offset reads the site's own record and counts for no lane,
+  // and so does a group past the last range (rg 4).
+  struct Group {
+    int rg;
+    int ks[U];
+    bool act[U];
+    double2 xy[U], zw[U];
+  } g, h;
+  uint32_t w = maskWord(m0, m1, 0);
+  int next = 0;  // the range w belongs to
+  auto fetch = [&](Group& q) {
+    while (w == 0 && next < 3) w = maskWord(m0, m1, ++next);
+    q.rg = w ? next : 4;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      q.act[u] = w != 0;
+      q.ks[u] = w ? 32 * next + __builtin_ctz(w) : kPadOffset;
+      w &= w - 1;
+      const uint32_t so = sh[q.ks[u]] * 16u;
+      q.xy[u] = ldRec64(rxy, o16, so);
+      q.zw[u] = ldRec64(rzw, o16, so);
+    }
+  };
+  int rg = 0, qn = 0;  // the range being summed, the pairs noted in it
+  uint32_t rank = 0;
+  bool sums = false;
+  Force3 part;
+  auto pairs = [&](const Group& q) {
+    bool held[U];
+    uint64_t other[U];
+    double d0[U], d1[U], d2[U], fp[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      d0[u] = xi0 - q.xy[u].x;
+      d1[u] = xi1 - q.xy[u].y;
+      d2[u] = xi2 - q.zw[u].x;
+      const double r2 = dist2D(d0[u], d1[u], d2[u]);
+      const double ri = rsqT(r2);
+      double pp;
+      const int m = knotM(r2 * ri, tb.rdr, tb.nr, pp);
+      const uint64_t in = q.act[u] ? __ballot(r2 < G.rc2) : 0;
+      const uint64_t hm =
+          in & __ballot((static_cast<uint32_t>(ei) | static_cast<uint32_t>(recSpecies64(q.zw[u].y))) == 0u) &
+          __ballot(m >= mlo);
+      other[u] = in & ~hm;
+      held[u] = __builtin_amdgcn_inverse_ballot_w64(hm);
+      const int k = max(m, mlo);
+      const double2 s0 = kn.s[k], s1 = kn.s[k + 1], yd = kn.yd[k];
+      const double dr = kn.dr[k];
+      const double z3 = hermite3(yd.y, s0.x, s1.x), z4 = hermite4(yd.y, s0.x, s1.x);
+      const double j3 = hermite3(dr, s0.y, s1.y), j4 = hermite4(dr, s0.y, s1.y);
+      fp[u] = pairFpD(pp, ri, z3, z4, s0.x, yd.x, j3, j4, s0.y, j3, j4, s0.y, dfi, q.zw[u].y, tb.rdr);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (other[u]) {
+        if (__builtin_amdgcn_inverse_ballot_w64(other[u]))
+          wq.q[qn + laneRank(other[u])] =
+              static_cast<uint16_t>((rank++ << 11) | ((static_cast<uint32_t>(q.ks[u]) & 31u) << 6) |
+                                    static_cast<uint32_t>(lane));
+        qn += __builtin_popcountll(other[u]);
+      }
+      if (held[u]) part.add(d0[u], d1[u], d2[u], fp[u]);
+    }
+  };
+  // Before a group of range `to`: works off full wavefronts of noted pairs
+  // and, where a range ends, all of them, and closes its sums.
+  auto settle = [&](int to) {
+    while (qn >= (to != rg ? 1 : 64)) {
+      if (!sums) {
+        sums = true;
+        for (int c = 0; c < 3; ++c) ws.s[c][lane] = 0.0;
+      }
+      waveLdsFence();
+      const int n = qn < 64 ? qn : 64;
+      drainQueueD(wq.q, n, rg, xi0, xi1, xi2, ei, dfi, o16, rxy, rzw, rtab, rtabR, tb, sh, ws);
+      qn -= n;
+      waveLdsFence();
+      if (qn > 0) shiftQueueD(wq, lane);
+    }
+    if (to == rg) return;
+    rg = to;
+    rank = 0;
+    tot.add(part);
+    part = Force3();
+    if (sums) {
+      Force3 o;
+      o.x = ws.s[0][lane];
+      o.y = ws.s[1][lane];
+      o.z = ws.s[2][lane];
+      otot.add(o);
+      sums = false;
+    }
+  };
+  fetch(g);
+  while (g.rg < 4) {
+    fetch(h);
+    if (g.rg != rg || qn >= 64) settle(g.rg);
+    pairs(g);
+    if (h.rg == 4) break;
+    fetch(g);
+    if (h.rg != rg || qn >= 64) settle(h.rg);
+    pairs(h);
+  }
+  settle(4);
+  if (!live) return;
+  tot.add(otot);
+  unsigned long long vbs = 0, dbs = 0;
+  forceTailD<MODE>(G, s, p, cx, cy, cz, ti, ei, dfi, tot, xi0, xi1, xi2, tb, x, xn, type, df, v, f, id, vp, st, ctl,
+                   iv, rn64, vbs, dbs);
+  vb = vbs > vb ? vbs : vb;
+  db = dbs > db ? dbs : db;
+}
+
+template <int MODE, int U>
+__global__ __launch_bounds__(kBlock) void kForce(Geom G, LatOffsets O, Tables<double> tb, CXPtr x, XPtr xn,
+                                                 const int8_t* __restrict__ type, const double* __restrict__ df,
                                                  const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                                  const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
-                                                 Ctl* ctl, InterView iv, Rec64 r64, Rec64 rn64) {
+                                                 Ctl* ctl, InterView iv, Rec64 r64, Rec64 rn64, int mlo) {
   unsigned long long vb = 0;  // |v|^2 bits after the secondstep (MODE 0)
   unsigned long long db = 0;  // |dx|^2 bits of the drift (MODE 1)
-  forceSiteD<T, ACC, MODE, U, false>(G, O, tb, x, xn, type, df, wmask, v, f, id, vp, st, ctl, iv, r64, rn64, nullptr,
-                                     0, blockIdx.x, threadIdx.x, vb, db);
+  forceSiteD<MODE, U>(G, O, tb, x, xn, type, df, wmask, v, f, id, vp, st, ctl, iv, r64, rn64, mlo, blockIdx.x,
+                      threadIdx.x, vb, db);
   if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
   if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
 }
@@ -511,7 +767,7 @@ __global__ __launch_bounds__(kBlock) void kForce(Geom G, LatOffsets O, Tables<T>
 // wavefront's skin mask (within the cutoff plus the skin of every pair at the
 // last full density scan, so a superset of the pairs within the cutoff), or
 // all pruned offsets when all is set (no skin).  With LDS the Fe-Fe segments
-// come from knD as in forceSiteD.  Near a far lattice atom the rest of the
+// come from knD, 7 doubles a knot (pairSegD).  Near a far lattice atom the rest of the
 // full list follows from x and df.
 template <bool LDS>
 __device__ __forceinline__ void energySiteD(const Geom& G, const LatOffsets& O, const FullPlaneOffsets* full,
@@ -669,28 +925,38 @@ __global__ __launch_bounds__(kBlockP) void kEnergyDL(Geom G, LatOffsets O, const
 }
 
 // The FP64 force pass in persistent blocks, one per compute unit, with the
-// Fe-Fe segments from knot mlo on in LDS (forceSiteD): per site the same
-// pairs, in the same order and with the same values, as kForce.
+// Fe-Fe segments from knot mlo on in LDS (forceVBlockD).  2M atoms with the
+// fused half steps: 546 us, against 657 with 7 doubles a knot, the other pairs
+// re-read under a mask and one group in flight.  Its four wavefronts per SIMD
+// still wait a third of their time; VALU issue takes 59 % of the slots.
 template <int MODE, int U>
 __global__ __launch_bounds__(kBlockP) void kForceDL(Geom G, LatOffsets O, Tables<double> tb, CXPtr x, XPtr xn,
                                                     const int8_t* __restrict__ type, const double* __restrict__ df,
                                                     const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                                     const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
                                                     Ctl* ctl, InterView iv, Rec64 r64, Rec64 rn64, int mlo, int nkn) {
-  extern __shared__ double knD[];
+  __shared__ WaveQueueD<U> queues[kBlockP / 64];
+  __shared__ WaveSums sums[kBlockP / 64];
+  extern __shared__ double2 knS[];  // nkn {s_z, s_rho}, nkn {y_z, dy_z}, nkn dy_rho
+  double2* ks = knS;  // one knot more: the last one starts no segment, but a pair there reads two
+  double2* kyd = knS + nkn + 1;
+  double* kdr = reinterpret_cast<double*>(knS + 2 * nkn + 1);
   const double* z = tb.pairF + static_cast<size_t>(mlo) * kPairRec;  // row (Fe, Fe) is the first
-  for (int i = threadIdx.x; i < 7 * nkn; i += kBlockP) {
-    const int k = i / 7, q = i - 7 * k;
-    knD[i] = z[static_cast<size_t>(k) * kPairRec + q];
+  for (int i = threadIdx.x; i < nkn; i += kBlockP) {
+    const double* c = z + static_cast<size_t>(i) * kPairRec;       // r*phi c3..c6, rho c3..c6
+    const double* n = i + 1 < nkn ? c + kPairRec : c;              // the last knot starts no segment
+    ks[i] = make_double2(c[2], c[6]);
+    if (i + 1 == nkn) ks[nkn] = ks[i];
+    kyd[i] = make_double2(c[3], __dsub_rn(n[3], c[3]));
+    kdr[i] = __dsub_rn(n[7], c[7]);
   }
   __syncthreads();
+  const KnotsD kn{ks - mlo, kyd - mlo, kdr - mlo};
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   unsigned long long vb = 0, db = 0;
   forVirtualBlocks(G, [&](uint32_t b, uint32_t tl) {
-    unsigned long long vbs = 0, dbs = 0;
-    forceSiteD<double, 0, MODE, U, true>(G, O, tb, x, xn, type, df, wmask, v, f, id, vp, st, ctl, iv, r64, rn64, knD,
-                                         mlo, b, tl, vbs, dbs);
-    vb = vbs > vb ? vbs : vb;
-    db = dbs > db ? dbs : db;
+    forceVBlockD<MODE, U>(G, O, tb, x, xn, type, df, wmask, v, f, id, vp, st, ctl, iv, r64, rn64, kn, mlo,
+                          queues[wave], sums[wave], b, tl, vb, db);
   });
   if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
   if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
@@ -815,7 +1081,7 @@ __global__ __launch_bounds__(kBlock) void kForceM(Geom G, LatOffsets O, Tables<f
                                                   float4* __restrict__ recn, const float4* __restrict__ dl,
                                                   const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                                   const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
-                                                  Ctl* ctl, InterView iv) {
+                                                  Ctl* ctl, InterView iv, int mlo) {
   unsigned long long vb = 0;  // |v|^2 bits after the secondstep (MODE 0)
   unsigned long long db = 0;  // |dx|^2 bits of the drift (MODE 1)
   [&] {
@@ -839,6 +1105,7 @@ __global__ __launch_bounds__(kBlock) void kForceM(Geom G, LatOffsets O, Tables<f
   const float4* D = dl + p * kMaxLatOffsets;
   const float rc2 = static_cast<float>(G.rc2);
   Sum3<ACC> acc;
+  OtherM oth;
   // the offsets the density pass found in range for some lane of this wavefront
   const uint32_t wv = waveId();
   // a group's entries past the mask's last offset get a lattice vector out
@@ -851,9 +1118,10 @@ __global__ __launch_bounds__(kBlock) void kForceM(Geom G, LatOffsets O, Tables<f
       nb[u] = ldRec4(rr, o16, sh[k] * 16u);
       d[u] = D[k];
     }
-    forceGroupM<ACC, U>(me, dfi, ei, pairBase, nb, d, rc2, rtab, rtabD, tb, ks, acc);
+    forceGroupM<ACC, U>(me, dfi, ei, pairBase, nb, d, rc2, rtab, rtabD, tb, mlo, ks, acc, oth);
   });
   flushChunk3(acc);
+  addOther3(acc, oth);
   forceTailM<ACC, MODE>(G, s, p, cx, cy, cz, ti, ei, dfi, acc, x, xn, type, rec, recn, v, f, id, vp, st, ctl, tb,
                         iv, vb, db);
   }();
@@ -861,50 +1129,130 @@ __global__ __launch_bounds__(kBlock) void kForceM(Geom G, LatOffsets O, Tables<f
   if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
 }
 
+// The byte shift of a neighbour's record from the w of its offset's table
+// entry: the shift itself, or a packed delta that a box turns into its own
+// shift (scalar arithmetic where the entry was read by a scalar load).
+struct RecShift {
+  __device__ __forceinline__ uint32_t operator()(float w) const { return __float_as_uint(w); }
+};
+struct PackedShift {
+  int32_t plane, NX, NY, lo;
+  __device__ __forceinline__ uint32_t operator()(float w) const {
+    const uint32_t u = __float_as_uint(w);
+    const int32_t dp = static_cast<int8_t>(u & 0xffu), dz = static_cast<int8_t>((u >> 8) & 0xffu);
+    const int32_t dy = static_cast<int8_t>((u >> 16) & 0xffu), dcx = static_cast<int8_t>(u >> 24);
+    return static_cast<uint32_t>(dp * plane + (dz * NY + dy) * NX + dcx - lo) * 16u;
+  }
+};
+
 // One virtual block of the LDS force pass (block b of a box): per site the
-// same pairs, in the same order and with the same rounding, as kForceM.
-// offT holds, per pruned offset of the centre's parity, the lattice vector
-// and in w what shift(w) turns into the byte shift of the neighbour's record.
+// same pairs and sums as kForceM.  dl holds, per pruned offset of either
+// parity, the lattice vector and in w what shift(w) turns into the byte shift
+// of the neighbour's record (RecShift, PackedShift), for scalar loads, and
+// offT the same in LDS, for the lanes that work off noted pairs.  The next
+// group's records are on their way while a group is computed: four
+// wavefronts per SIMD do not cover their round trip.  Every lane of a wavefront with an
+// atom stays to the end of the loop, since the noted pairs are worked off by
+// the whole wavefront: a lane without an atom sits out of every cutoff.
 template <int ACC, int MODE, int U, typename Shift>
 __device__ __forceinline__ void forceVBlockL(const Geom& G, const LatOffsets& O, const Tables<float>& tb, CXPtr x,
                                              XPtr xn, const int8_t* __restrict__ type,
                                              const float4* __restrict__ rec, float4* __restrict__ recn,
                                              const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                              const uint64_t* __restrict__ id, const VerletParams& vp,
-                                             const StageArgs& st, Ctl* ctl, const InterView& iv, const float4* offT,
-                                             const float4* knT, int mlo, uint32_t b, uint32_t tl, Shift shift,
-                                             unsigned long long& vb, unsigned long long& db) {
-  int64_t s;
-  int p, cx, cy, cz;
-  if (!siteOfBlock(G, b, tl, s, p, cx, cy, cz)) return;
-  const int8_t ti = type[s];
-  if (isVacant(ti)) {  // vacancy: keeps its stale position (atom.cpp:43-47)
-    vacancyForceM<MODE>(G, s, p, cx, cy, cz, x, xn, recn, f);
-    return;
+                                             const StageArgs& st, Ctl* ctl, const InterView& iv, const float4* dl,
+                                             const float4* offT, const float4* knT, int mlo, WaveQueueM& wq, WaveSums& ws, uint32_t b,
+                                             uint32_t tl, Shift shift, unsigned long long& vb,
+                                             unsigned long long& db) {
+  int64_t s = 0;
+  int p = 0, cx = 0, cy = 0, cz = 0;
+  const bool site = siteOfBlock(G, b, tl, s, p, cx, cy, cz);
+  int8_t ti = kVacant;
+  if (site) {
+    ti = type[s];
+    if (isVacant(ti)) vacancyForceM<MODE>(G, s, p, cx, cy, cz, x, xn, recn, f);  // keeps its stale position
   }
+  const bool live = !isVacant(ti);
+  const uint64_t lives = __ballot(live);
+  if (!lives) return;
   const Rsrc rr = rsrcBelow(rec, O.lo);
   const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.pairZ));
   const Rsrc rtabD = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoD));
   const float rc2 = static_cast<float>(G.rc2);
-  const int ei = species(ti);
-  const float4 me = rec[s];
+  const int ei = live ? species(ti) : 0;
+  float4 me = make_float4(kNoAtom, kNoAtom, kNoAtom, 0.0f);
+  if (live) me = rec[s];
+  const uint32_t o16 = addressOfLives(static_cast<uint32_t>(s) * 16u, live, lives);
   const float dfi = me.w;
-  const uint32_t o16 = static_cast<uint32_t>(s) * 16u;
-  const uint32_t pairBase = static_cast<uint32_t>(ei * 3) * static_cast<uint32_t>(tb.nr);
-  const float4* T = offT + p * kMaxLatOffsets;
+  const uint32_t pu = __builtin_amdgcn_readfirstlane((b >> 3) & 1u) * kMaxLatOffsets;
+  const float4* T = offT + pu;
+  const f32x4* dlp = reinterpret_cast<const f32x4*>(dl) + pu;
   Sum3<ACC> acc;
   const uint32_t wv = b * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tl >> 6);
-  // a group's entries past the mask's last offset get a lattice vector out
-  // of range: beyond the cutoff, they add nothing
-  forMaskGroupsFull<U>(uniform64(wmask[2 * wv]), uniform64(wmask[2 * wv + 1]), [&](const int* ks, const bool* act) {
-    float4 nb[U], d[U];
+  uint64_t b0 = uniform64(wmask[2 * wv]), b1 = uniform64(wmask[2 * wv + 1]);
+  int left = __builtin_popcountll(b0) + __builtin_popcountll(b1), base = 0;
+  int groups = (left + U - 1) / U;
+  int qn = 0;
+  bool sums = false;
+  // The next U offsets and their records' loads.  Entries past the mask's
+  // last offset get a lattice vector out of range: beyond the cutoff, they
+  // add nothing.
+  struct Group {
+    int ks[U];
+    f32x4 d[U];
+    float4 nb[U];
+  } g, h;
+  int k = 0;
+  auto fetch = [&](Group& q) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) d[u] = T[act[u] ? ks[u] : kPadOffset];
+    for (int u = 0; u < U; ++u) {
+      if (b0 == 0) {  // on to the mask's second word
+        b0 = b1;
+        b1 = 0;
+        base = 64;
+      }
+      const bool act = u < left;
+      const int t = __builtin_ctzll(b0 | (1ull << 63));
+      b0 &= ~(1ull << t);
+      k = act ? base + t : k;
+      q.ks[u] = k;
+      q.d[u] = scalarRead(dlp + (act ? k : kPadOffset));
+    }
+    left -= U;
 #pragma unroll
-    for (int u = 0; u < U; ++u) nb[u] = ldRec4(rr, o16 + shift(d[u].w), 0);
-    forceGroupL<ACC, U>(me, dfi, ei, pairBase, nb, d, rc2, rtab, rtabD, tb, knT, mlo, ks, acc);
-  });
+    for (int u = 0; u < U; ++u) q.nb[u] = ldRec4(rr, o16, shift(q.d[u].w));
+  };
+  auto drain = [&](int least) {
+    while (qn >= least) {
+      if (!sums) {
+        sums = true;
+        for (int c = 0; c < 3; ++c) ws.s[c][threadIdx.x & 63u] = 0.0;
+      }
+      waveLdsFence();
+      const int n = qn < 64 ? qn : 64;
+      drainQueueM(wq.q + (qn - n), n, me, o16, rr, rtab, rtabD, tb, T, shift, ws);
+      qn -= n;
+    }
+  };
+  fetch(g);  // also past the last group: the loads of the site's own record
+  while (groups > 0) {
+    fetch(h);
+    forceGroupL<ACC, U>(me, dfi, ei, g.nb, g.d, rc2, tb, knT, mlo, g.ks, acc, wq, qn);
+    fetch(g);
+    if (groups > 1) forceGroupL<ACC, U>(me, dfi, ei, h.nb, h.d, rc2, tb, knT, mlo, h.ks, acc, wq, qn);
+    groups -= 2;
+    drain(groups > 0 ? 64 : 1);
+  }
   flushChunk3(acc);
+  OtherM oth;
+  if (sums) {
+    waveLdsFence();
+    oth.x = ws.s[0][threadIdx.x & 63u];
+    oth.y = ws.s[1][threadIdx.x & 63u];
+    oth.z = ws.s[2][threadIdx.x & 63u];
+  }
+  if (!live) return;
+  addOther3(acc, oth);
   unsigned long long vbs = 0, dbs = 0;
   forceTailM<ACC, MODE>(G, s, p, cx, cy, cz, ti, ei, dfi, acc, x, xn, type, rec, recn, v, f, id, vp, st, ctl, tb,
                         iv, vbs, dbs);
@@ -912,14 +1260,14 @@ __device__ __forceinline__ void forceVBlockL(const Geom& G, const LatOffsets& O,
   db = dbs > db ? dbs : db;
 }
 
-// The LDS knots of the force pass, per knot the Fe-Fe r*phi cubic and the Fe
-// density slope cubic side by side, from knot mlo on (one block fills them).
+// The LDS knots of the force pass, the Fe-Fe r*phi cubics from knot mlo on and
+// kKnotsM entries further the Fe density slope cubics (one block fills them).
 __device__ __forceinline__ void fillKnots(const Tables<float>& tb, float4* knT, int mlo, int nkn) {
   const float4* z4 = reinterpret_cast<const float4*>(tb.pairZ);  // row (Fe, Fe) is the first
   const float4* s4 = reinterpret_cast<const float4*>(tb.rhoD);   // row Fe is the first
   for (int i = threadIdx.x; i < nkn; i += kBlockP) {
-    knT[2 * i] = z4[mlo + i];
-    knT[2 * i + 1] = s4[mlo + i];
+    knT[i] = z4[mlo + i];
+    knT[kKnotsM + i] = s4[mlo + i];
   }
 }
 
@@ -928,6 +1276,10 @@ __device__ __forceinline__ void fillKnots(const Tables<float>& tb, float4* knT, 
 // one broadcast per offset), the Fe-Fe r*phi cubics and the Fe density slope
 // cubics from knot mlo on (one block fills them once).  Per site the same
 // pairs, in the same order and with the same rounding, as kForceM.
+// 16M-atom cascade 2.44 -> 2.24 ms against segments re-read under a mask, one
+// group in flight and the two cubics side by side in LDS; 2M atoms with the
+// fused half steps 309 -> 280 us.  Its VALU issue (71 % of the slots, 3,800
+// instructions per 64 sites) and its LDS reads (44 %) bound it.
 template <int ACC, int MODE, int U>
 __global__ __launch_bounds__(kBlockP) void kForceL(Geom G, LatOffsets O, Tables<float> tb, CXPtr x, XPtr xn,
                                                    const int8_t* __restrict__ type, const float4* __restrict__ rec,
@@ -937,22 +1289,20 @@ __global__ __launch_bounds__(kBlockP) void kForceL(Geom G, LatOffsets O, Tables<
                                                    Ctl* ctl, InterView iv, int mlo, int nkn,
                                                    unsigned long long* zwork) {
   __shared__ float4 offT[2 * kMaxLatOffsets];  // {lattice vector, record shift * 16}
-  extern __shared__ float4 knT[];              // per knot: Fe-Fe r*phi cubic, Fe density slope cubic
-  for (int i = threadIdx.x; i < 2 * kMaxLatOffsets; i += kBlockP) {
-    const int q = i / kMaxLatOffsets, k = i - q * kMaxLatOffsets;
-    float4 d = dl[i];
-    d.w = __uint_as_float(O.sh[q][k] * 16u);
-    offT[i] = d;
-  }
+  __shared__ WaveQueueM queues[kBlockP / 64];
+  __shared__ WaveSums sums[kBlockP / 64];
+  extern __shared__ float4 knT[];  // Fe-Fe r*phi cubics, Fe density slope cubics (fillKnots)
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int i = threadIdx.x; i < 2 * kMaxLatOffsets; i += kBlockP) offT[i] = dl[2 * kMaxLatOffsets + i];
   fillKnots(tb, knT, mlo, nkn);
   __syncthreads();
   unsigned long long vb = 0;  // |v|^2 bits after the secondstep (MODE 0), largest over the lane's sites
   unsigned long long db = 0;  // |dx|^2 bits of the drift (MODE 1), likewise
-  auto shift = [](float w) { return __float_as_uint(w); };
+  const RecShift shift;
   forVirtualBlocks(G, [&](uint32_t b, uint32_t tl) {
     const long long t0 = zwork ? clock64() : 0;
-    forceVBlockL<ACC, MODE, U>(G, O, tb, x, xn, type, rec, recn, wmask, v, f, id, vp, st, ctl, iv, offT, knT, mlo, b,
-                               tl, shift, vb, db);
+    forceVBlockL<ACC, MODE, U>(G, O, tb, x, xn, type, rec, recn, wmask, v, f, id, vp, st, ctl, iv, dl + 2 * kMaxLatOffsets,
+                               offT, knT, mlo, queues[wave], sums[wave], b, tl, shift, vb, db);
     if (zwork) addPlaneWork(G, zwork, b, tl, t0);
   });
   if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
@@ -970,7 +1320,10 @@ __global__ __launch_bounds__(kBlockP) void kForceLB(const BatchBox* __restrict__
                                                     int nbox, int flip, const float4* __restrict__ dlp, int mlo,
                                                     int nkn) {
   __shared__ float4 offT[2 * kMaxLatOffsets];
+  __shared__ WaveQueueM queues[kBlockP / 64];
+  __shared__ WaveSums sums[kBlockP / 64];
   extern __shared__ float4 knT[];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   for (int i = threadIdx.x; i < 2 * kMaxLatOffsets; i += kBlockP) offT[i] = dlp[i];
   fillKnots(boxes[0].t32, knT, mlo, nkn);
   __syncthreads();
@@ -994,15 +1347,10 @@ __global__ __launch_bounds__(kBlockP) void kForceLB(const BatchBox* __restrict__
     }
     const int cb = B.cur ^ flip;
     const int32_t plane = static_cast<int32_t>(B.G.plane), NX = B.G.NX, NY = B.G.NY, lo = B.O.lo;
-    auto shift = [&](float w) {
-      const uint32_t u = __builtin_amdgcn_readfirstlane(__float_as_uint(w));
-      const int32_t dp = static_cast<int8_t>(u & 0xffu), dz = static_cast<int8_t>((u >> 8) & 0xffu);
-      const int32_t dy = static_cast<int8_t>((u >> 16) & 0xffu), dcx = static_cast<int8_t>(u >> 24);
-      return static_cast<uint32_t>(dp * plane + (dz * NY + dy) * NX + dcx - lo) * 16u;
-    };
+    const PackedShift shift{plane, NX, NY, lo};
     forceVBlockL<ACC, MODE, U>(B.G, B.O, B.t32, cxp(B.x[cb]), xp(B.x[1 - cb]), B.type, B.rec[cb], B.rec[1 - cb],
-                               B.wmask, xp(B.v), xp(B.f), B.id, B.vp, B.st, B.ctl, B.iv, offT, knT, mlo,
-                               c + 8u * (k - vstart[bi]), tl, shift, vb, db);
+                               B.wmask, xp(B.v), xp(B.f), B.id, B.vp, B.st, B.ctl, B.iv, dlp, offT, knT, mlo,
+                               queues[wave], sums[wave], c + 8u * (k - vstart[bi]), tl, shift, vb, db);
   }
   if (lastBox >= 0) {
     if (MODE == 0 && boxes[lastBox].vp.vmax) waveMaxTo(vb, boxes[lastBox].vp.vmax);
@@ -1010,34 +1358,41 @@ __global__ __launch_bounds__(kBlockP) void kForceLB(const BatchBox* __restrict__
   }
 }
 
-// LDS knots of the force pass: the Fe-Fe r*phi and Fe slope cubics (32 bytes
-// a knot) from knot mlo to the last, within one block per compute unit
-// (160 KB of LDS) beside the kernel's static LDS (the offset table, 3.5 KB;
-// 64 bytes are kept beyond it).
-constexpr int kForceLdsBytes = 160 * 1024 - 2 * kMaxLatOffsets * 16 - 64;
+// Offsets a group in the FP64 force passes.
+constexpr int kUDouble = 2;
+
+// LDS of the mixed force pass: kKnotsM knots (mixed_site.hpp) beside the
+// kernel's static LDS (the offset table, 4 KB, the queues, 18 KB, and the sums
+// of the pairs set aside, 24 KB) in the 160 KB of a compute unit.
+constexpr int kForceLdsBytes = 32 * kKnotsM;
+static_assert(kForceLdsBytes + 2 * kMaxLatOffsets * 16 +
+                      static_cast<int>(kBlockP / 64 * (sizeof(WaveQueueM) + sizeof(WaveSums))) <=
+                  160 * 1024,
+              "the LDS of one block per compute unit");
 struct LdsKnots {
   int mlo, nkn;
   size_t bytes;
 };
 LdsKnots ldsKnotsForce(int nr) {
   LdsKnots k;
-  k.nkn = std::min(nr, kForceLdsBytes / 32);
+  k.nkn = std::min(nr, kKnotsM);
   k.mlo = nr - k.nkn;
-  k.bytes = static_cast<size_t>(32) * static_cast<size_t>(k.nkn);
+  k.bytes = kForceLdsBytes;
   return k;
 }
-// The FP64 pass's LDS knots: 7 doubles (56 bytes) a knot, from knot mlo to
-// the last, in one block per compute unit (the kernel has no static LDS;
-// 64 bytes are kept).
-constexpr int kForceLdsBytesD = 160 * 1024 - 64;
+// The FP64 pass's LDS knots, 40 bytes each (KnotsD), from knot mlo to the
+// last, beside its queues (6 KB) and sums (24 KB): 3325 knots, from 1.88 A on
+// where the table has 5000 over 5.6 A.
+constexpr int kForceLdsBytesD =
+    160 * 1024 - static_cast<int>(kBlockP / 64 * (sizeof(WaveQueueD<kUDouble>) + sizeof(WaveSums))) - 64;
 LdsKnots ldsKnotsForceD(int nr) {
   LdsKnots k;
-  k.nkn = std::min(nr, kForceLdsBytesD / 56);
+  k.nkn = std::min(nr, (kForceLdsBytesD - 16) / 40);
   k.mlo = nr - k.nkn;
-  k.bytes = static_cast<size_t>(56) * static_cast<size_t>(k.nkn);
+  k.bytes = static_cast<size_t>(40) * static_cast<size_t>(k.nkn) + 16;
   return k;
 }
-// The energy pass's LDS knots: as the FP64 force pass's, beside its static
+// The energy pass's LDS knots: 7 doubles (56 bytes) a knot beside its static
 // LDS (the block sums; 512 bytes are kept).
 constexpr int kEnergyLdsBytes = 160 * 1024 - 512;
 LdsKnots ldsKnotsEnergy(int nr) {
@@ -1061,8 +1416,6 @@ bool useLds(const DevState& s) {
   const int64_t perXcd = static_cast<int64_t>(persistentGrid(s) / 8) * (kBlockP / kBlock);
   return 2 * s.G.W.bpx >= 4 * perXcd;
 }
-
-constexpr int kUDouble = 2;
 
 }  // namespace
 
@@ -1118,9 +1471,8 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
           s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv, r64, rn64,   \
           lkd.mlo, lkd.nkn);                                                                                  \
     } else {                                                                                                  \
-      kForce<double, 0, M, kUDouble><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, xn, s.type, s.df64, s.wmask,    \
-                                                             xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv, r64, \
-                                                             rn64);                                          \
+      kForce<M, kUDouble><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v),      \
+                                                   xp(s.f), s.id, vp, sa, s.ctl, iv, r64, rn64, lkd.mlo);     \
     }                                                                                                         \
   } while (0)
 #define MISA_FORCE_MU(A, M, U)                                                                                \
@@ -1134,7 +1486,8 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
           sa, s.ctl, iv, lk.mlo, lk.nkn, s.zmeasure ? s.zwork : nullptr);                                     \
     } else {                                                                                                  \
       kForceM<A, M, U><<<grid, kBlock, 0, st>>>(s.G, o, t32, x, xn, s.type, s.rec[s.cur], s.rec[1 - s.cur],    \
-                                                s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv);    \
+                                                s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv,      \
+                                                lk.mlo);                                                        \
     }                                                                                                         \
   } while (0)
 #define MISA_FORCE_M(A, M)            \

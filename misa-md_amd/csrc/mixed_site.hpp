@@ -14,6 +14,7 @@
 #include "buffer_load.hpp"
 #include "device_common.hpp"
 #include "inter_common.hpp"
+#include "pair_queue.hpp"
 #include "resident.hpp"
 #include "site_common.hpp"
 
@@ -22,7 +23,8 @@ namespace site {
 
 // x_i - x_j and |x_i - x_j|^2 of a neighbour, rounded the same way in every
 // pass, so that the density and force passes see the same pair set.
-__device__ __forceinline__ float dist2M(const float4& me, const float4& nb, const float4& d, float& d0, float& d1,
+template <typename V4>  // the lattice vector: a float4, or four floats in scalar registers
+__device__ __forceinline__ float dist2M(const float4& me, const float4& nb, const V4& d, float& d0, float& d1,
                                         float& d2) {
   d0 = __fsub_rn(__fsub_rn(me.x, nb.x), d.x);
   d1 = __fsub_rn(__fsub_rn(me.y, nb.y), d.y);
@@ -92,14 +94,28 @@ __device__ __forceinline__ float pairFpM(float q, float rinv, const float4& z, c
   return -psip * rinv;
 }
 
+// Knots the mixed LDS force pass holds, from the last one down (1.55 A on where
+// the table has 5000 over 5.6 A).  The two cubics of a knot sit in arrays of
+// their own, so that the lanes' 16-byte reads spread over all banks (side by
+// side, either read met only every second group of four banks), at a distance
+// that fits the read's immediate offset.
+constexpr int kKnotsM = 3616;
+
+// Whether a pair is one that the LDS force passes hold segments for: two Fe
+// atoms at a knot from mlo on.  The others are summed apart (pair_queue.hpp).
+__device__ __forceinline__ bool heldPair(int ei, uint32_t ej, int m, int mlo) {
+  return (static_cast<uint32_t>(ei) | ej) == 0u && m >= mlo;
+}
+
 // f_i += sum over the group of (x_i - x_j) fpair_ij, the segments gathered
 // from the tables in global memory (16-byte knots).
 template <int ACC, int V>
 __device__ __forceinline__ void forceGroupM(const float4& me, float dfi, int ei, uint32_t pairBase,
                                             const float4 (&nb)[V], const float4 (&d)[V], float rc2, Rsrc rtab,
-                                            Rsrc rtabD, const Tables<float>& tb, const int* ks, Sum3<ACC>& acc) {
+                                            Rsrc rtabD, const Tables<float>& tb, int mlo, const int* ks,
+                                            Sum3<ACC>& acc, OtherM& oth) {
 #pragma clang fp contract(off)
-  bool in[V], like[V];
+  bool in[V], held[V], like[V];
   float d0[V], d1[V], d2[V], pp[V], ri[V];
   float4 zc[V];
   f32x3 sj[V], si[V];
@@ -107,6 +123,7 @@ __device__ __forceinline__ void forceGroupM(const float4& me, float dfi, int ei,
   for (int u = 0; u < V; ++u) {
     const float r2 = dist2M(me, nb[u], d[u], d0[u], d1[u], d2[u]);
     in[u] = r2 < rc2;
+    held[u] = false;
     if (in[u]) {
       ri[u] = __builtin_amdgcn_rsqf(r2);
       const int m = knotM(r2 * ri[u], tb.rdr, tb.nr, pp[u]);
@@ -114,6 +131,7 @@ __device__ __forceinline__ void forceGroupM(const float4& me, float dfi, int ei,
       const uint32_t rowj = __umul24(ej, static_cast<uint32_t>(tb.nr)) + static_cast<uint32_t>(m);
       zc[u] = ldRec4(rtab, (pairBase + rowj) * 16u, 0);
       sj[u] = ld3(rtabD, rowj * 16u);
+      held[u] = heldPair(ei, ej, m, mlo);
       like[u] = ej == static_cast<uint32_t>(ei);
       si[u] = f32x3{0.0f, 0.0f, 0.0f};
       if (!like[u])  // rho_ei differs from rho_ej only for unlike pairs
@@ -126,66 +144,114 @@ __device__ __forceinline__ void forceGroupM(const float4& me, float dfi, int ei,
   for (int u = 0; u < V; ++u) {
     fp[u] = 0.0f;  // the segments of a neighbour beyond the cutoff are not read
     if (in[u]) fp[u] = pairFpM(pp[u], ri[u], zc[u], sj[u], si[u], like[u], dfi, nb[u].w, tb.rdr);
+    if (in[u] && !held[u]) {
+      oth.add(d0[u], d1[u], d2[u], fp[u]);
+      fp[u] = 0.0f;
+    }
   }
-  addGroup3<ACC, V>(acc, ks, in, d0, d1, d2, fp);
+  addGroup3<ACC, V>(acc, ks, held, d0, d1, d2, fp);
 }
 
 // forceGroupM with the Fe-Fe r*phi cubics and the Fe density slope cubics
-// from knot mlo on in LDS (knT, the two of a knot side by side): every lane
-// reads its segments there,
-// at a clamped knot; a lane whose pair involves another species, or lies
-// below knot mlo, then re-reads what it needs from global memory, in a
-// branch that only a wavefront with such a lane enters (after the LDS reads,
-// so that no global load waits in front of them).
+// from knot mlo on in LDS (knT, kKnotsM entries apart): the held pairs of the
+// group, the same terms in the same order.  The other pairs
+// within the cutoff go to the wavefront's queue; qn counts it.  The pass is
+// bound by its VALU instructions (80 % of the issue slots), so the tests are
+// combined as wavefront masks in scalar registers.
 template <int ACC, int V>
-__device__ __forceinline__ void forceGroupL(const float4& me, float dfi, int ei, uint32_t pairBase,
-                                            const float4 (&nb)[V], const float4 (&d)[V], float rc2, Rsrc rtab,
-                                            Rsrc rtabD, const Tables<float>& tb, const float4* knT, int mlo,
-                                            const int* ks, Sum3<ACC>& acc) {
+__device__ __forceinline__ void forceGroupL(const float4& me, float dfi, int ei, const float4 (&nb)[V],
+                                            const f32x4 (&d)[V], float rc2, const Tables<float>& tb,
+                                            const float4* knT, int mlo, const int* ks, Sum3<ACC>& acc,
+                                            WaveQueueM& wq, int& qn) {
 #pragma clang fp contract(off)
-  bool in[V], like[V], fz[V];
-  float d0[V], d1[V], d2[V], pp[V], ri[V];
-  int mm[V];
-  uint32_t ejv[V];
-  float4 zc[V];
-  f32x3 sj[V], si[V];
-  bool any = false;
+  bool held[V];
+  uint64_t other[V];
+  float d0[V], d1[V], d2[V], fp[V];
 #pragma unroll
   for (int u = 0; u < V; ++u) {
     const float r2 = dist2M(me, nb[u], d[u], d0[u], d1[u], d2[u]);
-    in[u] = r2 < rc2;
-    ri[u] = __builtin_amdgcn_rsqf(r2);
-    mm[u] = knotM(r2 * ri[u], tb.rdr, tb.nr, pp[u]);
-    ejv[u] = static_cast<uint32_t>(recSpecies(nb[u].x));
-    like[u] = ejv[u] == static_cast<uint32_t>(ei);
-    const float4* k2 = knT + 2 * max(mm[u] - mlo, 0);  // {r*phi cubic, density slope cubic} of the knot
-    zc[u] = k2[0];
-    const float4 s4 = k2[1];
-    sj[u] = f32x3{s4.x, s4.y, s4.z};
-    si[u] = sj[u];
-    fz[u] = in[u] && ((static_cast<uint32_t>(ei) | ejv[u]) != 0u || mm[u] < mlo);
-    any |= fz[u];
+    const float ri = __builtin_amdgcn_rsqf(r2);
+    float pp;
+    const int m = knotM(r2 * ri, tb.rdr, tb.nr, pp);
+    const uint64_t in = __ballot(r2 < rc2);
+    const uint64_t h = in & __ballot((static_cast<uint32_t>(ei) | static_cast<uint32_t>(recSpecies(nb[u].x))) == 0u) &
+                       __ballot(m >= mlo);
+    other[u] = in & ~h;
+    held[u] = __builtin_amdgcn_inverse_ballot_w64(h);
+    const float4* kn = knT + (max(m, mlo) - mlo);
+    const float4 zc = kn[0];
+    const float4 s4 = kn[kKnotsM];
+    const f32x3 sj{s4.x, s4.y, s4.z};
+    const float f = pairFpM(pp, ri, zc, sj, sj, true, dfi, nb[u].w, tb.rdr);
+    fp[u] = held[u] ? f : 0.0f;
   }
-  if (__ballot(any)) {  // the pair needs r*phi from memory; the slopes as their species or knot say
 #pragma unroll
-    for (int u = 0; u < V; ++u) {
-      if (!fz[u]) continue;
-      const bool low = mm[u] < mlo;
-      const uint32_t rowj = __umul24(ejv[u], static_cast<uint32_t>(tb.nr)) + static_cast<uint32_t>(mm[u]);
-      zc[u] = ldRec4(rtab, (pairBase + rowj) * 16u, 0);
-      if (ejv[u] != 0u || low) sj[u] = ld3(rtabD, rowj * 16u);
-      if (!like[u] && (ei != 0 || low))
-        si[u] = ld3(rtabD, (__umul24(static_cast<uint32_t>(ei), static_cast<uint32_t>(tb.nr)) +
-                            static_cast<uint32_t>(mm[u])) * 16u);
+  for (int u = 0; u < V; ++u)
+    if (other[u]) {
+      if (__builtin_amdgcn_inverse_ballot_w64(other[u]))
+        wq.q[qn + laneRank(other[u])] = static_cast<uint16_t>((ks[u] << 6) | (threadIdx.x & 63u));
+      qn += __builtin_popcountll(other[u]);
     }
+  addGroup3<ACC, V>(acc, ks, held, d0, d1, d2, fp);
+}
+
+// Works off n (at most 64) noted pairs q[0 .. n), one a lane: the owner's
+// record and address from its lane, the neighbour's record and the segments
+// from global memory, the terms into the owner's sums.  shift(w) turns the w
+// of an offset's table entry into the byte shift of the neighbour's record.
+template <typename Shift>
+__device__ __forceinline__ void drainQueueM(const uint16_t* q, int n, const float4& me, uint32_t o16, Rsrc rr,
+                                            Rsrc rtab, Rsrc rtabD, const Tables<float>& tb, const float4* T,
+                                            Shift shift, WaveSums& ws) {
+#pragma clang fp contract(off)
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+  const bool on = lane < n;
+  const uint32_t e = q[on ? lane : 0];
+  const int owner = static_cast<int>(e & 63u);
+  const float4 d = T[e >> 6];
+  float4 own;
+  own.x = laneGet(me.x, owner);
+  own.y = laneGet(me.y, owner);
+  own.z = laneGet(me.z, owner);
+  own.w = laneGet(me.w, owner);
+  const uint32_t oo = static_cast<uint32_t>(laneGet(static_cast<int>(o16), owner));
+  const float4 nb = ldRec4(rr, oo + shift(d.w), 0);
+  float d0, d1, d2;
+  const float r2 = dist2M(own, nb, d, d0, d1, d2);
+  const float ri = __builtin_amdgcn_rsqf(r2);
+  float pp;
+  const uint32_t m = static_cast<uint32_t>(knotM(r2 * ri, tb.rdr, tb.nr, pp));
+  const uint32_t ei = static_cast<uint32_t>(recSpecies(own.x)), ej = static_cast<uint32_t>(recSpecies(nb.x));
+  const uint32_t nr = static_cast<uint32_t>(tb.nr);
+  const uint32_t rowj = __umul24(ej, nr) + m;
+  const float4 zc = ldRec4(rtab, (__umul24(3u * ei, nr) + rowj) * 16u, 0);
+  const f32x3 sj = ld3(rtabD, rowj * 16u);
+  const f32x3 si = ld3(rtabD, (__umul24(ei, nr) + m) * 16u);
+  const float fp = pairFpM(pp, ri, zc, sj, si, ej == ei, own.w, nb.w, tb.rdr);
+  if (on) {
+    ldsAdd(&ws.s[0][owner], gridTerm(d0, fp));
+    ldsAdd(&ws.s[1][owner], gridTerm(d1, fp));
+    ldsAdd(&ws.s[2][owner], gridTerm(d2, fp));
   }
-  float fp[V];
-#pragma unroll
-  for (int u = 0; u < V; ++u) {
-    fp[u] = 0.0f;  // the segments of a neighbour beyond the cutoff are not read
-    if (in[u]) fp[u] = pairFpM(pp[u], ri[u], zc[u], sj[u], si[u], like[u], dfi, nb[u].w, tb.rdr);
+}
+
+// The sum of the pairs set aside joins the site's force, as one term a
+// component (where it is not zero: a site without such pairs keeps its bits).
+template <int ACC>
+__device__ __forceinline__ void addOther3(Sum3<ACC>& acc, const OtherM& o) {
+  if constexpr (ACC == 0) {
+    acc.f0 += o.x;
+    acc.f1 += o.y;
+    acc.f2 += o.z;
+  } else if constexpr (ACC == 1) {
+    if (o.x != 0.0) acc.a.add(static_cast<float>(o.x));
+    if (o.y != 0.0) acc.b.add(static_cast<float>(o.y));
+    if (o.z != 0.0) acc.c.add(static_cast<float>(o.z));
+  } else {
+    acc.f0 += static_cast<float>(o.x);
+    acc.f1 += static_cast<float>(o.y);
+    acc.f2 += static_cast<float>(o.z);
   }
-  addGroup3<ACC, V>(acc, ks, in, d0, d1, d2, fp);
 }
 
 // After the lattice sum of site s: the inter atoms and, near a far lattice

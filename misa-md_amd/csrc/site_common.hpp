@@ -167,6 +167,11 @@ __device__ __forceinline__ float4 packRec(double u0, double u1, double u2, int s
   return make_float4(__uint_as_float(bx), static_cast<float>(u1), static_cast<float>(u2), w);
 }
 constexpr float kVacantDisp = 1.0e4f;
+// Displacement of a lane without an atom in the passes whose wavefronts stay
+// whole: -2^60 A, so that every neighbour and the offset tables' padding entry
+// (a lattice vector of +1e18 A) lie farther out still, the square stays finite
+// and the species bits are those of Fe.
+constexpr float kNoAtom = -1152921504606846976.0f;
 __device__ __forceinline__ float4 vacantRec() { return make_float4(kVacantDisp, kVacantDisp, kVacantDisp, 0.0f); }
 __device__ __forceinline__ int recSpecies(float ux) { return static_cast<int>(__float_as_uint(ux) & 3u); }
 // Record of the atom at x on site (p, cx, cy, cz) of species sp.
