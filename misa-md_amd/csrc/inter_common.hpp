@@ -17,7 +17,7 @@ namespace misa {
 // The site kernels read the offsets eight at a time (one scalar load of 32
 // bytes): the arrays come first, 32-byte aligned, and the entries from n
 // (nw) on are 0, the site itself.
-static_assert(kMaxFullOffsets % 8 == 0, "offset rows are read eight at a time");
+static_assert(kMaxFullOffsets % 32 == 0, "offset rows are searched 32 entries at a time");
 struct FullPlaneOffsets {
   alignas(32) int32_t off[2][kMaxFullOffsets];
   // the full-list offsets missing from the pruned lattice list (kWide sites)
@@ -156,12 +156,14 @@ __device__ __forceinline__ T scalarRead(const T* p) {
   return *p;  // the host pass only parses device code
 #endif
 }
-struct alignas(32) Offsets8 {
-  int32_t o[8];
+template <int B>
+struct alignas(4 * B) OffsetGroup {
+  int32_t o[B];
 };
-// Entries q0 .. q0 + 7 of an offset row (q0 a multiple of 8).
-__device__ __forceinline__ Offsets8 offsets8(const int32_t* row, int q0) {
-  return scalarRead(reinterpret_cast<const Offsets8*>(row + q0));
+// Entries q0 .. q0 + B - 1 of an offset row (q0 a multiple of B).
+template <int B>
+__device__ __forceinline__ OffsetGroup<B> offsetGroup(const int32_t* row, int q0) {
+  return scalarRead(reinterpret_cast<const OffsetGroup<B>*>(row + q0));
 }
 
 // Visits the entries of bucket `slot` in insertion order, from its head h.
@@ -174,48 +176,123 @@ __device__ __forceinline__ void followBucket(const InterView& iv, int64_t slot, 
   }
 }
 
+// Bit u: the bucket of full-list neighbour q0 + u of site s (q0 a multiple of
+// 32) has entries.  The heads are read B at a time, since nearly all are empty:
+// their reads then overlap instead of queueing one round trip behind the other.
+template <int B>
+__device__ __forceinline__ uint32_t nearHits(const InterView& iv, const FullPlaneOffsets& full, int p, int64_t s,
+                                             int q0) {
+  const int n = scalarRead(&full.n[p]) - q0;
+  uint32_t hits = 0;
+#pragma unroll 1
+  for (int b = 0; b < 32 && b < n; b += B) {
+    int32_t h[B];
+#pragma unroll
+    for (int c = 0; c < B; c += 8) {
+      const OffsetGroup<8> o = offsetGroup<8>(full.off[p], q0 + b + c);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) h[c + u] = iv.head[s + o.o[u]];
+    }
+    uint32_t w = 0;
+#pragma unroll
+    for (int u = 0; u < B; ++u) w |= (h[u] >= 0 ? 1u : 0u) << u;
+    hits |= w << b;
+  }
+  return n < 32 ? hits & ((1u << n) - 1) : hits;
+}
+
+// Bit u: entry q0 + u of the full-list offsets beyond the pruned list (q0 a
+// multiple of 32) is, for site s at (x0, x1, x2), a target that may hold a
+// pair within the cutoff, with a rounding allowance on the distance.  Types
+// and positions are read B at a time (8 or 4).
+template <int B>
+__device__ __forceinline__ uint32_t wideHits(const FullPlaneOffsets& full, const double* const (&x)[3],
+                                             const int8_t* __restrict__ type, double rc2, int p, int64_t s, int8_t ti,
+                                             double x0, double x1, double x2, int q0) {
+  const int n = scalarRead(&full.nw[p]) - q0;
+  const double lim = rc2 * (1.0 + 1e-12);
+  uint32_t hits = 0;
+#pragma unroll 1
+  for (int b = 0; b < 32 && b < n; b += B) {
+    int8_t t[B];
+    double r2[B];
+    const OffsetGroup<B> o = offsetGroup<B>(full.woff[p], q0 + b);
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int64_t j = s + o.o[u];
+      const double d0 = x0 - x[0][j], d1 = x1 - x[1][j], d2 = x2 - x[2][j];
+      t[u] = type[j];
+      r2[u] = d0 * d0 + d1 * d1 + d2 * d2;
+    }
+    uint32_t w = 0;
+#pragma unroll
+    for (int u = 0; u < B; ++u) w |= (wideTarget(ti, t[u]) && r2[u] < lim ? 1u : 0u) << u;
+    hits |= w << b;
+  }
+  return n < 32 ? hits & ((1u << n) - 1) : hits;
+}
+
+// The hits of 64 sites (one a lane), where the wavefronts that share the sites
+// find them together: word w of either list by wavefront w % 4.  A serial
+// chain of round trips bounds the end of a pass over few sites, not the work:
+// one wavefront alone took 30 us over both lists (2 000 sites, 17 us for all
+// the rest of the pass), four of them and the wider reads take 5.
+struct TailHits {
+  static constexpr int kWords = kMaxFullOffsets / 32;
+  uint32_t near[kWords][64], wide[kWords][64];
+};
+__device__ __forceinline__ void findTailHits(TailHits& hits, int wave, const InterView& iv,
+                                             const double* const (&x)[3], const int8_t* __restrict__ type, double rc2,
+                                             int p, int64_t s, int8_t ti) {
+  if (isVacant(ti) || !(ti & (kNearInter | kWide))) return;
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+  const FullPlaneOffsets& full = *iv.full;
+  if (ti & kNearInter)
+    for (int w = wave; 32 * w < scalarRead(&full.n[p]); w += 4)
+      hits.near[w][lane] = nearHits<32>(iv, full, p, s, 32 * w);
+  if (ti & kWide) {
+    const double x0 = x[0][s], x1 = x[1][s], x2 = x[2][s];
+    for (int w = wave; 32 * w < scalarRead(&full.nw[p]); w += 4)
+      hits.wide[w][lane] = wideHits<8>(full, x, type, rc2, p, s, ti, x0, x1, x2, 32 * w);
+  }
+}
+
 // Visits, in full-list order (the site itself first), the entries of the
 // buckets of site s (parity p, the same over the wavefront) and of its
-// full-list neighbours.  The bucket heads are read eight at a time before
-// any bucket is followed: nearly all are empty, and the reads then overlap
-// instead of queueing one round trip behind the other.
+// full-list neighbours; hits: as found before, or null.
 template <typename Fn>
 __device__ __forceinline__ void forNearBuckets(const InterView& iv, const FullPlaneOffsets& full, int p, int64_t s,
-                                               int ne, Fn fn) {
+                                               int ne, const TailHits* hits, Fn fn) {
   const int n = scalarRead(&full.n[p]);
-  const int32_t* off = full.off[p];
   {
     const int h0 = iv.head[s];
     if (h0 >= 0) followBucket(iv, s, h0, ne, fn);
   }
-  for (int q0 = 0; q0 < n; q0 += 8) {
-    const Offsets8 o = offsets8(off, q0);
-    int32_t h[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) h[u] = iv.head[s + o.o[u]];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (q0 + u < n && h[u] >= 0) followBucket(iv, s + o.o[u], h[u], ne, fn);
+  for (int q0 = 0; q0 < n; q0 += 32) {
+    uint32_t m = hits ? hits->near[q0 / 32][threadIdx.x & 63u] : nearHits<8>(iv, full, p, s, q0);
+    for (; m; m &= m - 1) {
+      const int64_t j = s + full.off[p][q0 + __builtin_ctz(m)];
+      followBucket(iv, j, iv.head[j], ne, fn);
+    }
   }
 }
 
 // Visits, in order, the full-list offsets of site s beyond the pruned list
-// that hold a pair possibly within the cutoff (the site or the target a far
-// lattice atom), calling fn(slot, type) for each; the target types are read
-// eight at a time.
+// that may hold a pair within the cutoff (the site or the target a far
+// lattice atom), calling fn(slot, type) for each; hits as above.
 template <typename Fn>
-__device__ __forceinline__ void forWideTargets(const FullPlaneOffsets& full, const int8_t* __restrict__ type, int p,
-                                               int64_t s, int8_t ti, Fn fn) {
+__device__ __forceinline__ void forWideTargets(const FullPlaneOffsets& full, const double* const (&x)[3],
+                                               const int8_t* __restrict__ type, double rc2, int p, int64_t s,
+                                               int8_t ti, double x0, double x1, double x2, const TailHits* hits,
+                                               Fn fn) {
   const int n = scalarRead(&full.nw[p]);
-  const int32_t* woff = full.woff[p];
-  for (int q0 = 0; q0 < n; q0 += 8) {
-    const Offsets8 o = offsets8(woff, q0);
-    int8_t t[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) t[u] = type[s + o.o[u]];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (q0 + u < n && wideTarget(ti, t[u])) fn(s + o.o[u], t[u]);
+  for (int q0 = 0; q0 < n; q0 += 32) {
+    uint32_t m = hits ? hits->wide[q0 / 32][threadIdx.x & 63u]
+                      : wideHits<4>(full, x, type, rc2, p, s, ti, x0, x1, x2, q0);
+    for (; m; m &= m - 1) {
+      const int64_t j = s + full.woff[p][q0 + __builtin_ctz(m)];
+      fn(j, type[j]);
+    }
   }
 }
 

@@ -164,9 +164,121 @@ __device__ __forceinline__ void writeMasks(bool gathers, uint32_t wv, uint64_t w
 // (Ctl::skin_mode) the density pass visits only those: the same pairs in the
 // same order, so the sums do not change.
 // ---------------------------------------------------------------------------
-template <typename T, int ACC, int U>
-__global__ __launch_bounds__(kBlock) void kRhoDf(Geom G, LatOffsets O, Tables<T> tb, CXPtr x,
-                                                 const int8_t* __restrict__ type, T* __restrict__ df,
+// What a lane's site needs for the FP64 density sum.
+struct RhoSiteD {
+  double x0, x1, x2;
+  Rsrc rxy, rzw, rtab;  // neighbours' FP64 site records (a vacancy sits far out); the density cubics
+  uint32_t o16;
+  const uint32_t* sh;
+  double rc2, rcs2;
+};
+__device__ __forceinline__ RhoSiteD rhoSiteD(const Geom& G, const LatOffsets& O, const Tables<double>& tb, CXPtr x,
+                                             const Rec64& r64, double rcs2, int64_t s, int p) {
+  return RhoSiteD{x.c[0][s], x.c[1][s], x.c[2][s], rsrcBelow(r64.xy, O.lo), rsrcBelow(r64.zw, O.lo),
+                  rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoV)), static_cast<uint32_t>(s) * 16u, O.sh[p], G.rc2, rcs2};
+}
+// The densities of V neighbours at offsets ks; sets the bits of the offsets
+// within the cutoff for some lane (w) and, on a full scan, within cutoff +
+// skin (s).
+template <int V>
+__device__ __forceinline__ void rhoGroupD(const RhoSiteD& c, const Tables<double>& tb, const int* ks, bool skin,
+                                          RangeSum<0>& acc, uint64_t& w0, uint64_t& w1, uint64_t& s0, uint64_t& s1) {
+  double2 xy[V], zw[V];
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    const uint32_t so = c.sh[ks[u]] * 16u;
+    xy[u] = ldRec64(c.rxy, c.o16, so);
+    zw[u] = ldRec64(c.rzw, c.o16, so);
+  }
+  bool in[V];
+  double pp[V], rec[V][kRhoRec];
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    const double r2 = dist2D(c.x0 - xy[u].x, c.x1 - xy[u].y, c.x2 - zw[u].x);
+    in[u] = r2 < c.rc2;
+    if (!skin && __ballot(r2 < c.rcs2)) setBit(s0, s1, ks[u]);
+    if (__ballot(in[u])) setBit(w0, w1, ks[u]);
+    if (in[u]) {
+      const int m = knotM(r2 * rsqT(r2), tb.rdr, tb.nr, pp[u]);
+      ldRec<double, kRhoRec>(c.rtab, static_cast<uint32_t>(recSpecies64(zw[u].y) * tb.nr + m) * (kRhoRec * 8u),
+                             rec[u]);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    acc.at(ks[u]);
+    if (in[u]) acc.part.add(__fma_rn(__fma_rn(__fma_rn(rec[u][0], pp[u], rec[u][1]), pp[u], rec[u][2]), pp[u], rec[u][3]));
+  }
+}
+// Calls group(ks, V) over the offsets [k0, k1), or over the set bits of
+// (b0, b1) when skin is set, U at a time and then one at a time.
+template <int U, typename Group>
+__device__ __forceinline__ void forRhoGroups(bool skin, int k0, int k1, uint64_t b0, uint64_t b1, Group group) {
+  if (!skin) {
+    int ks[U];
+    int k = k0;
+    for (; k + U <= k1; k += U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) ks[u] = k + u;
+      group(std::integral_constant<int, U>{}, ks);
+    }
+    for (; k < k1; ++k) {
+      ks[0] = k;
+      group(std::integral_constant<int, 1>{}, ks);
+    }
+  } else {
+    forMaskGroups<U>(b0, b1, [&](const int* ks, int nv) {
+      if (nv == U) group(std::integral_constant<int, U>{}, ks);
+      else group(std::integral_constant<int, 1>{}, ks);
+    });
+  }
+}
+// After the lattice sum: the inter atoms and, near a far lattice atom, the
+// rest of the full list; then F'(rho), into df and the w of the site's record
+// (and of its images' records).
+__device__ __forceinline__ void rhoTailD(const Geom& G, int64_t s, int p, int cx, int cy, int cz, int8_t ti,
+                                         Sum1<0>& acc, CXPtr x, const int8_t* __restrict__ type,
+                                         const Tables<double>& tb, double* __restrict__ df,
+                                         double* __restrict__ rho_out, const InterView& iv, const Rec64& r64,
+                                         const TailHits* hits = nullptr) {
+  double dfi = 0.0, rho = 0.0;
+  if (!isVacant(ti)) {
+    const double xi0 = x.c[0][s], xi1 = x.c[1][s], xi2 = x.c[2][s];
+    if (ti & kNearInter) {  // inter atoms whose nearest site is within the full list (atom.cpp:224-240)
+      const int ne = static_cast<int>(iv.ctl->n_inter + iv.ctl->n_ghost);
+      const FullPlaneOffsets& full = *iv.full;
+      forNearBuckets(iv, full, p, s, ne, hits, [&](int e) {
+        const double d0 = xi0 - iv.e_x[0][e], d1 = xi1 - iv.e_x[1][e], d2 = xi2 - iv.e_x[2][e];
+        const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
+        if (r2 < G.rc2) acc.add(rhoPair(tb, species(iv.type[iv.e_src[e]]), r2));
+      });
+    }
+    if (ti & kWide) {  // full-list offsets beyond the pruned list, near a far lattice atom
+      forWideTargets(*iv.full, x.c, type, G.rc2, p, s, ti, xi0, xi1, xi2, hits, [&](int64_t j, int8_t tj) {
+        const double d0 = xi0 - x.c[0][j], d1 = xi1 - x.c[1][j], d2 = xi2 - x.c[2][j];
+        const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
+        if (r2 < G.rc2) acc.add(rhoPair(tb, species(tj), r2));
+      });
+    }
+    rho = acc.value();
+    checkRho(iv.ctl, rho, tb.rhomax);
+    dfi = dEmbed(tb, species(ti), rho);
+  }
+  df[s] = dfi;
+  double* w64 = reinterpret_cast<double*>(r64.zw) + 1;
+  const double wi = packW64(dfi, species(ti));
+  if (!isVacant(ti)) w64[2 * s] = wi;
+  if (rho_out) rho_out[s] = rho;
+  forEachImage(G, p, cx, cy, cz, [&](int64_t q, int, int, int) {
+    df[q] = dfi;
+    if (rho_out) rho_out[q] = rho;
+    if (!isVacant(ti)) w64[2 * q] = wi;
+  });
+}
+
+template <int U>
+__global__ __launch_bounds__(kBlock, 7) void kRhoDf(Geom G, LatOffsets O, Tables<double> tb, CXPtr x,
+                                                 const int8_t* __restrict__ type, double* __restrict__ df,
                                                  double* __restrict__ rho_out, uint64_t* __restrict__ wmask,
                                                  uint64_t* __restrict__ smask, double rcs2, InterView iv,
                                                  Rec64 r64) {
@@ -178,106 +290,132 @@ __global__ __launch_bounds__(kBlock) void kRhoDf(Geom G, LatOffsets O, Tables<T>
   const bool skin =
       __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(!isVacant(ti) && (ti & kWide));
   const uint32_t wv = waveId();
-  T dfi = T(0);
-  double rho = 0.0;
+  RangeSum<0> acc;
   uint64_t w0 = 0, w1 = 0, s0 = 0, s1 = 0;
   if (!isVacant(ti)) {
-    const double xi0 = x.c[0][s], xi1 = x.c[1][s], xi2 = x.c[2][s];
-    // neighbours from the FP64 site records (a vacancy sits far out, so every
-    // distance test against it fails as the type test did)
-    const Rsrc rxy = rsrcBelow(r64.xy, O.lo), rzw = rsrcBelow(r64.zw, O.lo);
-    const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoV));
-    const uint32_t o16 = static_cast<uint32_t>(s) * 16u;
-    const uint32_t* sh = O.sh[p];
-    const int nk = O.n[p];
-    Sum1<ACC> acc;
-    auto group = [&](auto UC, const int* ks) {
-      constexpr int V = decltype(UC)::value;
-      double2 xy[V], zw[V];
-#pragma unroll
-      for (int u = 0; u < V; ++u) {
-        const uint32_t so = sh[ks[u]] * 16u;
-        xy[u] = ldRec64(rxy, o16, so);
-        zw[u] = ldRec64(rzw, o16, so);
-      }
-      bool in[V];
-      T pp[V];
-      T rec[V][kRhoRec];
-#pragma unroll
-      for (int u = 0; u < V; ++u) {
-        const double r2 = dist2D(xi0 - xy[u].x, xi1 - xy[u].y, xi2 - zw[u].x);
-        in[u] = r2 < G.rc2;
-        if (!skin && __ballot(r2 < rcs2)) setBit(s0, s1, ks[u]);
-        if (__ballot(in[u])) setBit(w0, w1, ks[u]);
-        if (in[u]) {
-          const T q2 = static_cast<T>(r2);
-          const int m = knotOf(q2 * rsqT(q2), tb.rdr, tb.nr, false, pp[u]);
-          const uint32_t off = (static_cast<uint32_t>(recSpecies64(zw[u].y) * tb.nr + m)) *
-                               static_cast<uint32_t>(kRhoRec * sizeof(T));
-          ldRec<T, kRhoRec>(rtab, off, rec[u]);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < V; ++u)
-        if (in[u]) acc.add(((rec[u][0] * pp[u] + rec[u][1]) * pp[u] + rec[u][2]) * pp[u] + rec[u][3]);
-    };
-    if (!skin) {
-      int ks[U];
-      int k = 0;
-      for (; k + U <= nk; k += U) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) ks[u] = k + u;
-        group(std::integral_constant<int, U>{}, ks);
-      }
-      for (; k < nk; ++k) {
-        ks[0] = k;
-        group(std::integral_constant<int, 1>{}, ks);
-      }
-    } else {
-      forMaskGroups<U>(uniform64(smask[2 * wv]), uniform64(smask[2 * wv + 1]), [&](const int* ks, int nv) {
-        if (nv == U) group(std::integral_constant<int, U>{}, ks);
-        else group(std::integral_constant<int, 1>{}, ks);
-      });
-    }
-    if (ti & kNearInter) {  // inter atoms whose nearest site is within the full list (atom.cpp:224-240)
-      const int ne = static_cast<int>(iv.ctl->n_inter + iv.ctl->n_ghost);
-      const FullPlaneOffsets& full = *iv.full;
-      forNearBuckets(iv, full, p, s, ne, [&](int e) {
-        const double d0 = xi0 - iv.e_x[0][e], d1 = xi1 - iv.e_x[1][e], d2 = xi2 - iv.e_x[2][e];
-        const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-        if (r2 < G.rc2) acc.add(rhoPair(tb, species(iv.type[iv.e_src[e]]), r2));
-      });
-    }
-    if (ti & kWide) {  // full-list offsets beyond the pruned list, near a far lattice atom
-      forWideTargets(*iv.full, type, p, s, ti, [&](int64_t j, int8_t tj) {
-        const double d0 = xi0 - x.c[0][j], d1 = xi1 - x.c[1][j], d2 = xi2 - x.c[2][j];
-        const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-        if (r2 < G.rc2) acc.add(rhoPair(tb, species(tj), r2));
-      });
-    }
-    rho = acc.value();
-    checkRho(iv.ctl, rho, static_cast<double>(tb.rhomax));
-    dfi = dEmbed(tb, species(ti), static_cast<T>(rho));
+    const RhoSiteD c = rhoSiteD(G, O, tb, x, r64, rcs2, s, p);
+    forRhoGroups<U>(skin, 0, O.n[p], skin ? uniform64(smask[2 * wv]) : 0, skin ? uniform64(smask[2 * wv + 1]) : 0,
+                    [&](auto UC, const int* ks) {
+                      rhoGroupD<decltype(UC)::value>(c, tb, ks, skin, acc, w0, w1, s0, s1);
+                    });
   }
+  acc.close();
   writeMasks(!isVacant(ti), wv, w0, w1, wmask, !skin, s0, s1, smask);
-  df[s] = dfi;
-  // F' into the w of the site's record (and of its images' records)
-  double* w64 = reinterpret_cast<double*>(r64.zw) + 1;
-  const double wi = packW64(static_cast<double>(dfi), species(ti));
-  if (!isVacant(ti)) w64[2 * s] = wi;
-  if (rho_out) {
-    rho_out[s] = rho;
-    forEachImage(G, p, cx, cy, cz, [&](int64_t q, int, int, int) {
-      df[q] = dfi;
-      rho_out[q] = rho;
-      if (!isVacant(ti)) w64[2 * q] = wi;
-    });
-  } else {
-    forEachImage(G, p, cx, cy, cz, [&](int64_t q, int, int, int) {
-      df[q] = dfi;
-      if (!isVacant(ti)) w64[2 * q] = wi;
+  rhoTailD(G, s, p, cx, cy, cz, ti, acc.tot, x, type, tb, df, rho_out, iv, r64);
+}
+
+// ---------------------------------------------------------------------------
+// Boxes with few sites.  One wavefront's walk over its offsets is a chain of
+// some sixteen to thirty groups, each a round trip to the records and one to
+// the tables, about 1.5 us a group; when the sites fill only a few wavefronts
+// per SIMD nothing hides it (2,000 atoms: kRhoDf 28 us and kForce 40-50 us,
+// the same as at 16,000).  There the four wavefronts of a block share 64
+// sites, each takes one range of 32 offsets (one word of the mask), and the
+// first of them joins the four sums in the order the one-wavefront passes use
+// and does what follows the lattice sum.  Same bits, a quarter of the chain.
+// ---------------------------------------------------------------------------
+
+// The offsets of range rg of a list of n: [32 rg, min(32 rg + 32, n)), and the
+// mask bits of that range.
+struct Range {
+  int k0, k1;
+};
+__device__ __forceinline__ Range rangeOf(int rg, int n) { return Range{32 * rg, min(32 * rg + 32, n)}; }
+__device__ __forceinline__ void rangeBits(const uint64_t* mask, uint32_t wv, int rg, uint64_t& b0, uint64_t& b1) {
+  const uint32_t w = __builtin_amdgcn_readfirstlane(reinterpret_cast<const uint32_t*>(mask)[4 * wv + rg]);
+  const uint64_t b = static_cast<uint64_t>(w) << (32 * (rg & 1));
+  b0 = rg < 2 ? b : 0;
+  b1 = rg < 2 ? 0 : b;
+}
+// writeMasks for one word of the masks.
+__device__ __forceinline__ void writeMaskWord(bool gathers, uint32_t wv, int rg, uint64_t w0, uint64_t w1,
+                                              uint64_t* wmask, bool full, uint64_t s0, uint64_t s1,
+                                              uint64_t* smask) {
+  const uint64_t gathered = __ballot(gathers);
+  if (!gathered) return;
+  const int leader = __builtin_ctzll(gathered);
+  if (static_cast<int>(threadIdx.x & 63) == leader) {
+    reinterpret_cast<uint32_t*>(wmask)[4 * wv + rg] = static_cast<uint32_t>((rg < 2 ? w0 : w1) >> (32 * (rg & 1)));
+    if (full)
+      reinterpret_cast<uint32_t*>(smask)[4 * wv + rg] = static_cast<uint32_t>((rg < 2 ? s0 : s1) >> (32 * (rg & 1)));
+  }
+}
+
+// The shared site of this thread's wavefront (four wavefronts, the same site a
+// lane): block b of a siteGrid launch, thread tl of it.  False without a site;
+// ti is then a vacancy's type.
+struct SharedSite {
+  int64_t s = 0;
+  int p = 0, cx = 0, cy = 0, cz = 0;
+  uint32_t wv = 0;  // index of the masks
+  int rg = 0;       // this wavefront's range
+  int8_t ti = kVacant;
+  bool site = false;
+};
+__device__ __forceinline__ SharedSite sharedSite(const Geom& G, const int8_t* __restrict__ type, uint32_t id) {
+  SharedSite q;
+  uint32_t b, sub;
+  sharedUnit(id, b, sub);
+  q.rg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  q.wv = b * (kBlock / 64) + sub;
+  q.p = static_cast<int>((b >> 3) & 1u);
+  q.site = siteOfBlock(G, b, sub * 64u + (threadIdx.x & 63u), q.s, q.p, q.cx, q.cy, q.cz);
+  if (q.site) q.ti = type[q.s];
+  return q;
+}
+
+// Sums of the four ranges in LDS: what the later three wavefronts hand over.
+struct RangeParts {
+  double v[3][2][64];
+};
+template <int ACC>
+__device__ __forceinline__ void putPart(RangeParts& r, int rg, const Sum1<ACC>& a) {
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+  r.v[rg - 1][0][lane] = static_cast<double>(a.s);
+  if constexpr (ACC == 1) r.v[rg - 1][1][lane] = static_cast<double>(a.c);
+}
+template <int ACC>
+__device__ __forceinline__ void joinParts(const RangeParts& r, Sum1<ACC>& tot) {
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+#pragma unroll
+  for (int rg = 1; rg < 4; ++rg) {
+    Sum1<ACC> a;
+    a.s = static_cast<decltype(a.s)>(r.v[rg - 1][0][lane]);
+    if constexpr (ACC == 1) a.c = static_cast<float>(r.v[rg - 1][1][lane]);
+    tot.join(a);
+  }
+}
+
+template <int U>
+__global__ __launch_bounds__(kBlock) void kRhoDfP(Geom G, LatOffsets O, Tables<double> tb, CXPtr x,
+                                                  const int8_t* __restrict__ type, double* __restrict__ df,
+                                                  double* __restrict__ rho_out, uint64_t* __restrict__ wmask,
+                                                  uint64_t* __restrict__ smask, double rcs2, InterView iv,
+                                                  Rec64 r64) {
+  __shared__ RangeParts parts;
+  __shared__ TailHits hits;
+  const SharedSite q = sharedSite(G, type, blockIdx.x);
+  const bool live = !isVacant(q.ti);
+  const bool skin = __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(live && (q.ti & kWide));
+  RangeSum<0> acc;
+  acc.range = q.rg;
+  uint64_t w0 = 0, w1 = 0, s0 = 0, s1 = 0, b0 = 0, b1 = 0;
+  if (live) {
+    const RhoSiteD c = rhoSiteD(G, O, tb, x, r64, rcs2, q.s, q.p);
+    const Range r = rangeOf(q.rg, O.n[q.p]);
+    if (skin) rangeBits(smask, q.wv, q.rg, b0, b1);
+    forRhoGroups<U>(skin, r.k0, r.k1, b0, b1, [&](auto UC, const int* ks) {
+      rhoGroupD<decltype(UC)::value>(c, tb, ks, skin, acc, w0, w1, s0, s1);
     });
   }
+  writeMaskWord(live, q.wv, q.rg, w0, w1, wmask, !skin, s0, s1, smask);
+  if (q.rg > 0) putPart(parts, q.rg, acc.part);
+  findTailHits(hits, q.rg, iv, x.c, type, G.rc2, q.p, q.s, q.ti);
+  __syncthreads();
+  if (q.rg > 0 || !q.site) return;
+  acc.close();
+  joinParts(parts, acc.tot);
+  rhoTailD(G, q.s, q.p, q.cx, q.cy, q.cz, q.ti, acc.tot, x, type, tb, df, rho_out, iv, r64, &hits);
 }
 
 // secondstep (and, fused, the next firststep and decide) of a lattice atom,
@@ -328,7 +466,7 @@ __device__ __forceinline__ void verletTail(const Geom& G, int64_t s, int p, int 
   xn.c[1][s] = y1;
   xn.c[2][s] = y2;
   putRec64(rn64, s, ti, y0, y1, y2);
-  forEachImage(G, p, cx, cy, cz, [&](int64_t q, int sx, int sy, int sz) {
+  forEachImageLoop(G, p, cx, cy, cz, [&](int64_t q, int sx, int sy, int sz) {
     const double q0 = y0 + sx * G.L0, q1 = y1 + sy * G.L1, q2 = y2 + sz * G.L2;
     xn.c[0][q] = q0;
     xn.c[1][q] = q1;
@@ -426,12 +564,13 @@ __device__ __forceinline__ void forceTailD(const Geom& G, int64_t s, int p, int 
                                            const int8_t* __restrict__ type, const double* __restrict__ df, XPtr v,
                                            XPtr f, const uint64_t* __restrict__ id, const VerletParams& vp,
                                            const StageArgs& st, Ctl* ctl, const InterView& iv, const Rec64& rn64,
-                                           unsigned long long& vb, unsigned long long& db) {
+                                           unsigned long long& vb, unsigned long long& db,
+                                           const TailHits* hits = nullptr) {
   Force3 acc = lat;
   if (ti & kNearInter) {  // forces from inter atoms on lattice neighbours (atom.cpp:397-422)
     const int ne = static_cast<int>(iv.ctl->n_inter + iv.ctl->n_ghost);
     const FullPlaneOffsets& full = *iv.full;
-    forNearBuckets(iv, full, p, s, ne, [&](int e) {
+    forNearBuckets(iv, full, p, s, ne, hits, [&](int e) {
       const int src = iv.e_src[e];
       const double d0 = xi0 - iv.e_x[0][e], d1 = xi1 - iv.e_x[1][e], d2 = xi2 - iv.e_x[2][e];
       const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
@@ -439,7 +578,7 @@ __device__ __forceinline__ void forceTailD(const Geom& G, int64_t s, int p, int 
     });
   }
   if (ti & kWide) {  // full-list offsets beyond the pruned list, near a far lattice atom
-    forWideTargets(*iv.full, type, p, s, ti, [&](int64_t j, int8_t tj) {
+    forWideTargets(*iv.full, x.c, type, G.rc2, p, s, ti, xi0, xi1, xi2, hits, [&](int64_t j, int8_t tj) {
       const double e0 = xi0 - x.c[0][j], e1 = xi1 - x.c[1][j], e2 = xi2 - x.c[2][j];
       const double r2 = e0 * e0 + e1 * e1 + e2 * e2;
       if (r2 < G.rc2) acc.add(e0, e1, e2, pairForce(tb, ei, species(tj), r2, dfi, df[j]));
@@ -450,8 +589,92 @@ __device__ __forceinline__ void forceTailD(const Geom& G, int64_t s, int p, int 
                    vb, db);
 }
 
-// One site of the FP64 force pass, the segments from the tables in global
-// memory.
+// What a lane's site needs for the FP64 force sum with the segments from the
+// tables in global memory.
+struct ForceSiteD {
+  double x0, x1, x2, dfi;
+  int ei;
+  Rsrc rxy, rzw, rtab, rtabR;
+  uint32_t o16, pairBase;
+  const uint32_t* sh;
+  double rc2;
+  int mlo;
+};
+__device__ __forceinline__ ForceSiteD forceSiteOf(const Geom& G, const LatOffsets& O, const Tables<double>& tb,
+                                                  CXPtr x, const double* __restrict__ df, const Rec64& r64, int mlo,
+                                                  int64_t s, int p, int8_t ti) {
+  const int ei = species(ti);
+  // neighbours from the FP64 site records: position and, in w, F' with the
+  // species (a vacancy sits far out, so the distance test drops it)
+  return ForceSiteD{x.c[0][s],
+                    x.c[1][s],
+                    x.c[2][s],
+                    df[s],
+                    ei,
+                    rsrcBelow(r64.xy, O.lo),
+                    rsrcBelow(r64.zw, O.lo),
+                    rsrcAt(reinterpret_cast<uintptr_t>(tb.pairF)),
+                    rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoV)),
+                    static_cast<uint32_t>(s) * 16u,
+                    static_cast<uint32_t>(ei * 3) * static_cast<uint32_t>(tb.nr),
+                    O.sh[p],
+                    G.rc2,
+                    mlo};
+}
+// The pairs of range rg (mask word w) of a site: the held ones into part, the
+// others into opart, in offset order.
+template <int U>
+__device__ __forceinline__ void forceRangeD(const ForceSiteD& c, const Tables<double>& tb, uint32_t w, int rg,
+                                            Force3& part, Force3& opart) {
+  auto group = [&](auto UC, const int* ks) {
+    constexpr int V = decltype(UC)::value;
+    double d0[V], d1[V], d2[V], wj[V];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      const uint32_t so = c.sh[ks[u]] * 16u;
+      const double2 xy = ldRec64(c.rxy, c.o16, so), zw = ldRec64(c.rzw, c.o16, so);
+      d0[u] = xy.x;
+      d1[u] = xy.y;
+      d2[u] = zw.x;
+      wj[u] = zw.y;
+    }
+    bool in[V], held[V];
+    double pp[V], ri[V], rec[V][kPairRec], reci[V][kRhoRec];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      d0[u] = c.x0 - d0[u];
+      d1[u] = c.x1 - d1[u];
+      d2[u] = c.x2 - d2[u];
+      const double r2 = dist2D(d0[u], d1[u], d2[u]);
+      in[u] = r2 < c.rc2;
+      if (in[u]) {
+        ri[u] = rsqT(r2);
+        const int m = knotM(r2 * ri[u], tb.rdr, tb.nr, pp[u]);
+        const int ej = recSpecies64(wj[u]);
+        held[u] = heldPair(c.ei, static_cast<uint32_t>(ej), m, c.mlo);
+        pairSegD<false>(c.rtab, c.rtabR, nullptr, 0, c.pairBase, tb.nr, c.ei, ej, m, rec[u], reci[u]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      if (!in[u]) continue;
+      const double* z = rec[u];
+      const double fp = pairFpD(pp[u], ri[u], z[0], z[1], z[2], z[3], z[4], z[5], z[6], reci[u][0], reci[u][1],
+                                reci[u][2], c.dfi, wj[u], tb.rdr);
+      if (held[u]) part.add(d0[u], d1[u], d2[u], fp);
+      else opart.add(d0[u], d1[u], d2[u], fp);
+    }
+  };
+  forMaskGroups<U>(static_cast<uint64_t>(w), 0ull, [&](const int* k32, int nv) {
+    int ks[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) ks[u] = k32[u] + 32 * rg;
+    if (nv == U) group(std::integral_constant<int, U>{}, ks);
+    else group(std::integral_constant<int, 1>{}, ks);
+  });
+}
+
+// One site of the FP64 force pass, one wavefront over all its offsets.
 template <int MODE, int U>
 __device__ __forceinline__ void forceSiteD(const Geom& G, const LatOffsets& O, const Tables<double>& tb, CXPtr x,
                                            XPtr xn, const int8_t* __restrict__ type, const double* __restrict__ df,
@@ -468,75 +691,78 @@ __device__ __forceinline__ void forceSiteD(const Geom& G, const LatOffsets& O, c
     vacancyForceD<MODE>(G, s, p, cx, cy, cz, ti, x, xn, f, rn64);
     return;
   }
-  const double xi0 = x.c[0][s], xi1 = x.c[1][s], xi2 = x.c[2][s];
-  const int ei = species(ti);
-  const double dfi = df[s];
-  // neighbours from the FP64 site records: position and, in w, F' with the
-  // species (a vacancy sits far out, so the distance test drops it)
-  const Rsrc rxy = rsrcBelow(r64.xy, O.lo), rzw = rsrcBelow(r64.zw, O.lo);
-  const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.pairF));
-  const Rsrc rtabR = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoV));
-  const uint32_t o16 = static_cast<uint32_t>(s) * 16u;
-  const uint32_t pairBase = static_cast<uint32_t>(ei * 3) * static_cast<uint32_t>(tb.nr);
-  const uint32_t* sh = O.sh[p];
+  const ForceSiteD c = forceSiteOf(G, O, tb, x, df, r64, mlo, s, p, ti);
   Force3 tot, otot;
   // the offsets the density pass found in range for some lane of this wavefront
   const uint32_t wv = b * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tl >> 6);
   const uint64_t m0 = uniform64(wmask[2 * wv]), m1 = uniform64(wmask[2 * wv + 1]);
   for (int rg = 0; rg < 4; ++rg) {
     Force3 part, opart;
-    auto group = [&](auto UC, const int* ks) {
-      constexpr int V = decltype(UC)::value;
-      double d0[V], d1[V], d2[V], wj[V];
-#pragma unroll
-      for (int u = 0; u < V; ++u) {
-        const uint32_t so = sh[ks[u]] * 16u;
-        const double2 xy = ldRec64(rxy, o16, so), zw = ldRec64(rzw, o16, so);
-        d0[u] = xy.x;
-        d1[u] = xy.y;
-        d2[u] = zw.x;
-        wj[u] = zw.y;
-      }
-      bool in[V], held[V];
-      double pp[V], ri[V], rec[V][kPairRec], reci[V][kRhoRec];
-#pragma unroll
-      for (int u = 0; u < V; ++u) {
-        d0[u] = xi0 - d0[u];
-        d1[u] = xi1 - d1[u];
-        d2[u] = xi2 - d2[u];
-        const double r2 = dist2D(d0[u], d1[u], d2[u]);
-        in[u] = r2 < G.rc2;
-        if (in[u]) {
-          ri[u] = rsqT(r2);
-          const int m = knotM(r2 * ri[u], tb.rdr, tb.nr, pp[u]);
-          const int ej = recSpecies64(wj[u]);
-          held[u] = heldPair(ei, static_cast<uint32_t>(ej), m, mlo);
-          pairSegD<false>(rtab, rtabR, nullptr, 0, pairBase, tb.nr, ei, ej, m, rec[u], reci[u]);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < V; ++u) {
-        if (!in[u]) continue;
-        const double* z = rec[u];
-        const double fp = pairFpD(pp[u], ri[u], z[0], z[1], z[2], z[3], z[4], z[5], z[6], reci[u][0], reci[u][1],
-                                  reci[u][2], dfi, wj[u], tb.rdr);
-        if (held[u]) part.add(d0[u], d1[u], d2[u], fp);
-        else opart.add(d0[u], d1[u], d2[u], fp);
-      }
-    };
-    forMaskGroups<U>(static_cast<uint64_t>(maskWord(m0, m1, rg)), 0ull, [&](const int* k32, int nv) {
-      int ks[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) ks[u] = k32[u] + 32 * rg;
-      if (nv == U) group(std::integral_constant<int, U>{}, ks);
-      else group(std::integral_constant<int, 1>{}, ks);
-    });
+    forceRangeD<U>(c, tb, maskWord(m0, m1, rg), rg, part, opart);
     tot.add(part);
     otot.add(opart);
   }
   tot.add(otot);
-  forceTailD<MODE>(G, s, p, cx, cy, cz, ti, ei, dfi, tot, xi0, xi1, xi2, tb, x, xn, type, df, v, f, id, vp, st, ctl,
-                   iv, rn64, vb, db);
+  forceTailD<MODE>(G, s, p, cx, cy, cz, ti, c.ei, c.dfi, tot, c.x0, c.x1, c.x2, tb, x, xn, type, df, v, f, id, vp,
+                   st, ctl, iv, rn64, vb, db);
+}
+
+// The FP64 force pass with four wavefronts to 64 sites (boxes with few sites).
+template <int MODE, int U>
+__global__ __launch_bounds__(kBlock) void kForceP(Geom G, LatOffsets O, Tables<double> tb, CXPtr x, XPtr xn,
+                                                  const int8_t* __restrict__ type, const double* __restrict__ df,
+                                                  const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
+                                                  const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
+                                                  Ctl* ctl, InterView iv, Rec64 r64, Rec64 rn64, int mlo) {
+  __shared__ double parts[3][6][64];
+  __shared__ TailHits hits;
+  const SharedSite q = sharedSite(G, type, blockIdx.x);
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+  ForceSiteD c{};
+  Force3 part, opart;
+  if (!isVacant(q.ti)) {
+    c = forceSiteOf(G, O, tb, x, df, r64, mlo, q.s, q.p, q.ti);
+    const uint32_t w =
+        __builtin_amdgcn_readfirstlane(reinterpret_cast<const uint32_t*>(wmask)[4 * q.wv + q.rg]);
+    forceRangeD<U>(c, tb, w, q.rg, part, opart);
+  }
+  if (q.rg > 0) {
+    double(&o)[6][64] = parts[q.rg - 1];
+    o[0][lane] = part.x;
+    o[1][lane] = part.y;
+    o[2][lane] = part.z;
+    o[3][lane] = opart.x;
+    o[4][lane] = opart.y;
+    o[5][lane] = opart.z;
+  }
+  findTailHits(hits, q.rg, iv, x.c, type, G.rc2, q.p, q.s, q.ti);
+  __syncthreads();
+  if (q.rg > 0) return;
+  unsigned long long vb = 0, db = 0;
+  if (q.site && isVacant(q.ti)) {
+    vacancyForceD<MODE>(G, q.s, q.p, q.cx, q.cy, q.cz, q.ti, x, xn, f, rn64);
+  } else if (q.site) {
+    Force3 tot, otot;
+    tot.add(part);
+    otot.add(opart);
+#pragma unroll
+    for (int rg = 1; rg < 4; ++rg) {
+      const double(&o)[6][64] = parts[rg - 1];
+      part.x = o[0][lane];
+      part.y = o[1][lane];
+      part.z = o[2][lane];
+      opart.x = o[3][lane];
+      opart.y = o[4][lane];
+      opart.z = o[5][lane];
+      tot.add(part);
+      otot.add(opart);
+    }
+    tot.add(otot);
+    forceTailD<MODE>(G, q.s, q.p, q.cx, q.cy, q.cz, q.ti, c.ei, c.dfi, tot, c.x0, c.x1, c.x2, tb, x, xn, type, df, v,
+                     f, id, vp, st, ctl, iv, rn64, vb, db, &hits);
+  }
+  if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
+  if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
 }
 
 // The Fe-Fe segments of the FP64 LDS pass from knot mlo on, 40 bytes a knot:
@@ -855,7 +1081,7 @@ __device__ __forceinline__ void energySiteD(const Geom& G, const LatOffsets& O, 
     });
   }
   if (ti & kWide) {  // full-list offsets beyond the pruned list, near a far lattice atom
-    forWideTargets(*full, type, p, s, ti, [&](int64_t j, int8_t tj) {
+    forWideTargets(*full, x.c, type, G.rc2, p, s, ti, xi0, xi1, xi2, nullptr, [&](int64_t j, int8_t tj) {
       const double e0 = xi0 - x.c[0][j], e1 = xi1 - x.c[1][j], e2 = xi2 - x.c[2][j];
       const double q2 = e0 * e0 + e1 * e1 + e2 * e2;
       if (q2 < G.rc2) {
@@ -973,6 +1199,66 @@ __global__ __launch_bounds__(kBlockP) void kForceDL(Geom G, LatOffsets O, Tables
 // ---------------------------------------------------------------------------
 // The masks of pass 1 work as in FP64: both passes see the same records and
 // round the distances the same way (dist2M), so a skipped offset has no pair.
+// Per lane: the density sum of site s over the offsets [k0, k1), or with skin
+// set over the bits of (b0, b1) of the last full scan's mask, U at a time; the
+// entries past the last repeat its offset with the padding entry's lattice
+// vector: they add nothing.  Sets the mask bits as rhoGroupD does.
+template <int ACC, int U>
+__device__ __forceinline__ void rhoSumM(const LatOffsets& O, const Tables<float>& tb, const float4* rec,
+                                        const float4* __restrict__ dl, float rc2, float rcs2, int64_t s, int p,
+                                        bool skin, int k0, int k1, uint64_t b0, uint64_t b1, RangeSum<ACC>& acc,
+                                        uint64_t& w0, uint64_t& w1, uint64_t& s0, uint64_t& s1) {
+  const float4 me = rec[s];
+  const Rsrc rr = rsrcBelow(rec, O.lo);
+  const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoH));
+  const uint32_t o16 = static_cast<uint32_t>(s) * 16u;
+  // per pruned offset: the lattice vector and, in w, the record shift * 16
+  const float4* D = dl + (2 + p) * kMaxLatOffsets;
+  auto group = [&](const int (&ks)[U], const bool (&act)[U]) {
+    float4 nb[U], d[U];
+    bool in[U], sk[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) d[u] = D[act[u] ? ks[u] : kPadOffset];
+#pragma unroll
+    for (int u = 0; u < U; ++u) nb[u] = ldRec4(rr, o16, __float_as_uint(d[u].w));
+    rhoGroupM<ACC, U>(me, nb, d, rc2, rcs2, rtab, tb, ks, acc, in, sk);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (__ballot(in[u])) setBit(w0, w1, ks[u]);
+      if (!skin && __ballot(sk[u])) setBit(s0, s1, ks[u]);
+    }
+  };
+  int ks[U];
+  bool act[U];
+  if (!skin) {
+    for (int k = k0; k < k1; k += U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        act[u] = k + u < k1;
+        ks[u] = act[u] ? k + u : k1 - 1;
+      }
+      group(ks, act);
+    }
+  } else {
+    int k = 0;
+    while (b0 | b1) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        act[u] = (b0 | b1) != 0;
+        if (b0) {
+          k = __builtin_ctzll(b0);
+          b0 &= b0 - 1;
+        } else if (b1) {
+          k = 64 + __builtin_ctzll(b1);
+          b1 &= b1 - 1;
+        }
+        ks[u] = k;
+      }
+      group(ks, act);
+    }
+  }
+}
+
 // The density pass of block `blk` of one box (the kernel's own block, or a
 // block of one box of a batch).
 template <int ACC, int U>
@@ -989,72 +1275,56 @@ __device__ __forceinline__ void rhoPassM(const Geom& G, const LatOffsets& O, con
   const bool skin =
       __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(!isVacant(ti) && (ti & kWide));
   const uint32_t wv = blk * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  Sum1<ACC> acc;
+  RangeSum<ACC> acc;
   uint64_t w0 = 0, w1 = 0;  // offsets in range for some lane (uniform among the lanes that gather)
   uint64_t s0 = 0, s1 = 0;  // offsets within cutoff + skin for some lane (full scan)
   if (!isVacant(ti)) {
-    const float4 me = rec[s];
-    const Rsrc rr = rsrcBelow(rec, O.lo);
-    const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoH));
-    const uint32_t o16 = static_cast<uint32_t>(s) * 16u;
-    // per pruned offset: the lattice vector and, in w, the record shift * 16
-    const float4* D = dl + (2 + p) * kMaxLatOffsets;
-    const float rc2 = static_cast<float>(G.rc2);
-    const int nk = O.n[p];
-    // U offsets at a time; the entries past the last repeat the group's first
-    // offset, with the padding entry's lattice vector: they add nothing
-    auto group = [&](const int (&ks)[U], const bool (&act)[U]) {
-      float4 nb[U], d[U];
-      bool in[U], sk[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) d[u] = D[act[u] ? ks[u] : kPadOffset];
-#pragma unroll
-      for (int u = 0; u < U; ++u) nb[u] = ldRec4(rr, o16, __float_as_uint(d[u].w));
-      rhoGroupM<ACC, U>(me, nb, d, rc2, rcs2, rtab, tb, acc, in, sk);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (__ballot(in[u])) setBit(w0, w1, ks[u]);
-        if (!skin && __ballot(sk[u])) setBit(s0, s1, ks[u]);
-      }
-    };
-    int ks[U];
-    bool act[U];
-    if (!skin) {
-      for (int k = 0; k < nk; k += U) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          act[u] = k + u < nk;
-          ks[u] = act[u] ? k + u : k;
-        }
-        group(ks, act);
-      }
-    } else {
-      // the offsets of the last full scan's skin mask, in ascending order
-      uint64_t b0 = uniform64(smask[2 * wv]), b1 = uniform64(smask[2 * wv + 1]);
-      while (b0 | b1) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          act[u] = (b0 | b1) != 0;
-          int k;
-          if (b0) {
-            k = __builtin_ctzll(b0);
-            b0 &= b0 - 1;
-          } else {
-            k = b1 ? 64 + __builtin_ctzll(b1) : 0;
-            b1 &= b1 - 1;
-          }
-          ks[u] = act[u] ? k : ks[0];
-        }
-        group(ks, act);
-      }
+    uint64_t b0 = 0, b1 = 0;
+    if (skin) {  // the offsets of the last full scan's skin mask, in ascending order
+      b0 = uniform64(smask[2 * wv]);
+      b1 = uniform64(smask[2 * wv + 1]);
     }
+    rhoSumM<ACC, U>(O, tb, rec, dl, static_cast<float>(G.rc2), rcs2, s, p, skin, 0, O.n[p], b0, b1, acc, w0, w1, s0,
+                    s1);
   }
+  acc.close();
   writeMasks(!isVacant(ti), wv, w0, w1, wmask, !skin, s0, s1, smask);
-  rhoTailM<ACC>(G, s, p, cx, cy, cz, ti, acc, x, type, tb, iv, rec, rho_out);
+  rhoTailM<ACC>(G, s, p, cx, cy, cz, ti, acc.tot, x, type, tb, iv, rec, rho_out);
+}
+
+// The mixed density pass with four wavefronts to 64 sites (boxes with few sites).
+template <int ACC, int U>
+__global__ __launch_bounds__(kBlock) void kRhoDfMP(Geom G, LatOffsets O, Tables<float> tb, CXPtr x,
+                                                   const int8_t* __restrict__ type, float4* rec,
+                                                   const float4* __restrict__ dl, double* __restrict__ rho_out,
+                                                   uint64_t* __restrict__ wmask, uint64_t* __restrict__ smask,
+                                                   float rcs2, InterView iv) {
+  __shared__ RangeParts parts;
+  __shared__ TailHits hits;
+  const SharedSite q = sharedSite(G, type, blockIdx.x);
+  const bool live = !isVacant(q.ti);
+  const bool skin = __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(live && (q.ti & kWide));
+  RangeSum<ACC> acc;
+  acc.range = q.rg;
+  uint64_t w0 = 0, w1 = 0, s0 = 0, s1 = 0, b0 = 0, b1 = 0;
+  if (live) {
+    const Range r = rangeOf(q.rg, O.n[q.p]);
+    if (skin) rangeBits(smask, q.wv, q.rg, b0, b1);
+    rhoSumM<ACC, U>(O, tb, rec, dl, static_cast<float>(G.rc2), rcs2, q.s, q.p, skin, r.k0, r.k1, b0, b1, acc, w0, w1,
+                    s0, s1);
+  }
+  writeMaskWord(live, q.wv, q.rg, w0, w1, wmask, !skin, s0, s1, smask);
+  if (q.rg > 0) putPart(parts, q.rg, acc.part);
+  findTailHits(hits, q.rg, iv, x.c, type, G.rc2, q.p, q.s, q.ti);
+  __syncthreads();
+  if (q.rg > 0 || !q.site) return;
+  acc.close();
+  joinParts(parts, acc.tot);
+  rhoTailM<ACC>(G, q.s, q.p, q.cx, q.cy, q.cz, q.ti, acc.tot, x, type, tb, iv, rec, rho_out, &hits);
 }
 
 template <int ACC, int U>
-__global__ __launch_bounds__(kBlock) void kRhoDfM(Geom G, LatOffsets O, Tables<float> tb, CXPtr x,
+__global__ __launch_bounds__(kBlock, U == 4 ? 8 : 6) void kRhoDfM(Geom G, LatOffsets O, Tables<float> tb, CXPtr x,
                                                   const int8_t* __restrict__ type, float4* rec,
                                                   const float4* __restrict__ dl, double* __restrict__ rho_out,
                                                   uint64_t* __restrict__ wmask, uint64_t* __restrict__ smask,
@@ -1075,6 +1345,35 @@ __global__ __launch_bounds__(kBlock) void kRhoDfMB(const BatchBox* __restrict__ 
                    blockIdx.x - start[b]);
 }
 
+// Per lane: the force sum of the atom on site s (record me) over the offsets
+// of the mask (b0, b1), the segments from the tables in global memory: the
+// held pairs into acc, the others into oth.
+template <int U, typename Acc>
+__device__ __forceinline__ void forceSumM(const LatOffsets& O, const Tables<float>& tb, const float4* rec,
+                                          const float4* __restrict__ dl, float rc2, int mlo, int64_t s, int p, int ei,
+                                          const float4& me, uint64_t b0, uint64_t b1, Acc& acc, OtherM& oth) {
+  const Rsrc rr = rsrcBelow(rec, O.lo);
+  const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.pairZ));
+  const Rsrc rtabD = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoD));
+  const uint32_t o16 = static_cast<uint32_t>(s) * 16u;
+  const uint32_t pairBase = static_cast<uint32_t>(ei * 3) * static_cast<uint32_t>(tb.nr);
+  const uint32_t* sh = O.sh[p];
+  const float4* D = dl + p * kMaxLatOffsets;
+  // a group's entries past the mask's last offset get a lattice vector out
+  // of range: beyond the cutoff, they add nothing
+  forMaskGroupsFull<U>(b0, b1, [&](const int* ks, const bool* act) {
+    float4 nb[U], d[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = act[u] ? ks[u] : kPadOffset;
+      nb[u] = ldRec4(rr, o16, sh[k] * 16u);
+      d[u] = D[k];
+    }
+    forceGroupM(me, me.w, ei, pairBase, nb, d, rc2, rtab, rtabD, tb, mlo, ks, acc, oth);
+  });
+  flushChunk3(acc);
+}
+
 template <int ACC, int MODE, int U>
 __global__ __launch_bounds__(kBlock) void kForceM(Geom G, LatOffsets O, Tables<float> tb, CXPtr x, XPtr xn,
                                                   const int8_t* __restrict__ type, const float4* __restrict__ rec,
@@ -1085,46 +1384,91 @@ __global__ __launch_bounds__(kBlock) void kForceM(Geom G, LatOffsets O, Tables<f
   unsigned long long vb = 0;  // |v|^2 bits after the secondstep (MODE 0)
   unsigned long long db = 0;  // |dx|^2 bits of the drift (MODE 1)
   [&] {
-  int64_t s;
-  int p, cx, cy, cz;
-  if (!siteOfThread(G, s, p, cx, cy, cz)) return;
-  const int8_t ti = type[s];
-  if (isVacant(ti)) {  // vacancy: keeps its stale position (atom.cpp:43-47)
-    vacancyForceM<MODE>(G, s, p, cx, cy, cz, x, xn, recn, f);
-    return;
-  }
-  const int ei = species(ti);
-  const float4 me = rec[s];
-  const float dfi = me.w;
-  const Rsrc rr = rsrcBelow(rec, O.lo);
-  const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.pairZ));
-  const Rsrc rtabD = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoD));
-  const uint32_t o16 = static_cast<uint32_t>(s) * 16u;
-  const uint32_t pairBase = static_cast<uint32_t>(ei * 3) * static_cast<uint32_t>(tb.nr);
-  const uint32_t* sh = O.sh[p];
-  const float4* D = dl + p * kMaxLatOffsets;
-  const float rc2 = static_cast<float>(G.rc2);
-  Sum3<ACC> acc;
-  OtherM oth;
-  // the offsets the density pass found in range for some lane of this wavefront
-  const uint32_t wv = waveId();
-  // a group's entries past the mask's last offset get a lattice vector out
-  // of range: beyond the cutoff, they add nothing
-  forMaskGroupsFull<U>(uniform64(wmask[2 * wv]), uniform64(wmask[2 * wv + 1]), [&](const int* ks, const bool* act) {
-    float4 nb[U], d[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = act[u] ? ks[u] : kPadOffset;
-      nb[u] = ldRec4(rr, o16, sh[k] * 16u);
-      d[u] = D[k];
+    int64_t s;
+    int p, cx, cy, cz;
+    if (!siteOfThread(G, s, p, cx, cy, cz)) return;
+    const int8_t ti = type[s];
+    if (isVacant(ti)) {  // vacancy: keeps its stale position (atom.cpp:43-47)
+      vacancyForceM<MODE>(G, s, p, cx, cy, cz, x, xn, recn, f);
+      return;
     }
-    forceGroupM<ACC, U>(me, dfi, ei, pairBase, nb, d, rc2, rtab, rtabD, tb, mlo, ks, acc, oth);
-  });
-  flushChunk3(acc);
-  addOther3(acc, oth);
-  forceTailM<ACC, MODE>(G, s, p, cx, cy, cz, ti, ei, dfi, acc, x, xn, type, rec, recn, v, f, id, vp, st, ctl, tb,
-                        iv, vb, db);
+    const int ei = species(ti);
+    const float4 me = rec[s];
+    Sum3<ACC> acc;
+    OtherM oth;
+    // the offsets the density pass found in range for some lane of this wavefront
+    const uint32_t wv = waveId();
+    forceSumM<U>(O, tb, rec, dl, static_cast<float>(G.rc2), mlo, s, p, ei, me, uniform64(wmask[2 * wv]),
+                 uniform64(wmask[2 * wv + 1]), acc, oth);
+    addOther3(acc, oth);
+    forceTailM<ACC, MODE>(G, s, p, cx, cy, cz, ti, ei, me.w, acc, x, xn, type, rec, recn, v, f, id, vp, st, ctl, tb,
+                          iv, vb, db);
   }();
+  if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
+  if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
+}
+
+// The mixed force pass with four wavefronts to 64 sites (boxes with few
+// sites): the chunk sums of a site meet in LDS, and the first wavefront takes
+// them in order.
+template <int ACC, int MODE, int U>
+__global__ __launch_bounds__(kBlock) void kForceMP(Geom G, LatOffsets O, Tables<float> tb, CXPtr x, XPtr xn,
+                                                   const int8_t* __restrict__ type, const float4* __restrict__ rec,
+                                                   float4* __restrict__ recn, const float4* __restrict__ dl,
+                                                   const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
+                                                   const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
+                                                   Ctl* ctl, InterView iv, int mlo) {
+  using Term = typename Sum3<ACC>::Term;
+  __shared__ Term chunks[kChunks][3][64];
+  __shared__ double others[3][3][64];
+  __shared__ TailHits hits;
+  const SharedSite q = sharedSite(G, type, blockIdx.x);
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+  const int ei = species(q.ti);
+  float4 me = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  OtherM oth;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) chunks[4 * q.rg + t][k][lane] = 0;
+  if (!isVacant(q.ti)) {
+    me = rec[q.s];
+    ChunkSums<ACC> sums;
+    sums.chunk = 4 * q.rg;
+    sums.out = chunks;
+    uint64_t b0, b1;
+    rangeBits(wmask, q.wv, q.rg, b0, b1);
+    forceSumM<U>(O, tb, rec, dl, static_cast<float>(G.rc2), mlo, q.s, q.p, ei, me, b0, b1, sums, oth);
+  }
+  if (q.rg > 0) {
+    others[q.rg - 1][0][lane] = oth.x;
+    others[q.rg - 1][1][lane] = oth.y;
+    others[q.rg - 1][2][lane] = oth.z;
+  }
+  findTailHits(hits, q.rg, iv, x.c, type, G.rc2, q.p, q.s, q.ti);
+  __syncthreads();
+  if (q.rg > 0) return;
+  unsigned long long vb = 0, db = 0;
+  if (q.site && isVacant(q.ti)) {
+    vacancyForceM<MODE>(G, q.s, q.p, q.cx, q.cy, q.cz, x, xn, recn, f);
+  } else if (q.site) {
+    Sum3<ACC> acc;
+    for (int t = 0; t < kChunks; ++t) {
+      acc.g0 = chunks[t][0][lane];
+      acc.g1 = chunks[t][1][lane];
+      acc.g2 = chunks[t][2][lane];
+      acc.flush();
+    }
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      oth.x += others[r][0][lane];
+      oth.y += others[r][1][lane];
+      oth.z += others[r][2][lane];
+    }
+    addOther3(acc, oth);
+    forceTailM<ACC, MODE>(G, q.s, q.p, q.cx, q.cy, q.cz, q.ti, ei, me.w, acc, x, xn, type, rec, recn, v, f, id, vp,
+                          st, ctl, tb, iv, vb, db, &hits);
+  }
   if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
   if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
 }
@@ -1407,14 +1751,23 @@ bool setLdsBytes(const void* fn, int bytes) {
 }
 // One persistent block per compute unit, a whole number per XCD.
 unsigned persistentGrid(const DevState& s) { return static_cast<unsigned>(s.ncu / 8 * 8); }
-// The LDS-table force pass: on request, or by default when every persistent
-// block walks at least four virtual blocks per sub-block (a block's fill of
-// its tables then costs little beside its share of the pass).
+// The LDS-table passes: on request, or by default where the sites fill the
+// wavefronts of the persistent launch, 16 a compute unit, at least once.
+// Force pass against the one from global memory (its form for few sites up to
+// 4096 wavefronts): at 60^3 cells FP64 156 against 216 us, mixed 83 against
+// 108; at 50^3 148 against 163 and 81 against 80; at 40^3, half the
+// wavefronts idle, 83 against 73 and 46 against 43.
 bool useLds(const DevState& s) {
   if (s.ncu < 8 || s.lds == kLdsOff) return false;
   if (s.lds == kLdsOn) return true;
-  const int64_t perXcd = static_cast<int64_t>(persistentGrid(s) / 8) * (kBlockP / kBlock);
-  return 2 * s.G.W.bpx >= 4 * perXcd;
+  return static_cast<int64_t>(siteGrid(s.G)) * kBlock >= static_cast<int64_t>(persistentGrid(s)) * kBlockP;
+}
+
+// Boxes whose sites fill at most this many wavefronts (64 sites each) take the
+// passes that share 64 sites among four wavefronts.
+constexpr int64_t kSharedWaves = 4096;
+bool useShared(const DevState& s) {
+  return static_cast<int64_t>(siteGrid(s.G)) * (kBlock / 64) <= kSharedWaves;
 }
 
 }  // namespace
@@ -1426,10 +1779,24 @@ void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t
   const InterView iv = interView(s, mixed);
   const CXPtr x = cxp(s.x[s.cur]);
   const double rcs = std::sqrt(s.G.rc2) + s.skin;
-  if (!mixed)
-    kRhoDf<double, 0, 4><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs,
-                                                   iv, Rec64{s.pxy[s.cur], s.pzw[s.cur]});
-  else {
+  const bool shared = useShared(s);
+  if (!mixed) {
+    const Rec64 r64{s.pxy[s.cur], s.pzw[s.cur]};
+    if (shared)
+      kRhoDfP<4><<<4 * grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs, iv,
+                                              r64);
+    else
+      kRhoDf<4><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs, iv, r64);
+  } else if (shared) {
+    const float rcs2 = static_cast<float>(rcs * rcs);
+#define MISA_RHO_MP(A)                                                                                          \
+  kRhoDfMP<A, 4><<<4 * grid, kBlock, 0, st>>>(s.G, o, t32, x, s.type, s.rec[s.cur], s.dl, rho, s.wmask, s.smask, \
+                                              rcs2, iv)
+    if (acc == 0) MISA_RHO_MP(0);
+    else if (acc == 1) MISA_RHO_MP(1);
+    else MISA_RHO_MP(2);
+#undef MISA_RHO_MP
+  } else {
     const float rcs2 = static_cast<float>(rcs * rcs);
 #define MISA_RHO_M(A, U)                                                                                   \
   kRhoDfM<A, U><<<grid, kBlock, 0, st>>>(s.G, o, t32, x, s.type, s.rec[s.cur], s.dl, rho, s.wmask, s.smask, \
@@ -1457,7 +1824,7 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
   const XPtr xn = xp(s.x[1 - s.cur]);
   const StageArgs sa = stageOf(s);
   const InterView iv = interView(s, mixed);
-  const bool lds = useLds(s);
+  const bool lds = useLds(s), shared = useShared(s);
   const LdsKnots lk = ldsKnotsForce(t32.nr);
   const LdsKnots lkd = ldsKnotsForceD(t64.nr);
 #define MISA_FORCE(M)                                                                                         \
@@ -1470,6 +1837,9 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
       kForceDL<M, kUDouble><<<persistentGrid(s), kBlockP, lkd.bytes, st>>>(                                   \
           s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv, r64, rn64,   \
           lkd.mlo, lkd.nkn);                                                                                  \
+    } else if (shared) {                                                                                      \
+      kForceP<M, kUDouble><<<4 * grid, kBlock, 0, st>>>(s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v), \
+                                                        xp(s.f), s.id, vp, sa, s.ctl, iv, r64, rn64, lkd.mlo); \
     } else {                                                                                                  \
       kForce<M, kUDouble><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v),      \
                                                    xp(s.f), s.id, vp, sa, s.ctl, iv, r64, rn64, lkd.mlo);     \
@@ -1484,6 +1854,10 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
       kForceL<A, M, U><<<persistentGrid(s), kBlockP, lk.bytes, st>>>(                                         \
           s.G, o, t32, x, xn, s.type, s.rec[s.cur], s.rec[1 - s.cur], s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, \
           sa, s.ctl, iv, lk.mlo, lk.nkn, s.zmeasure ? s.zwork : nullptr);                                     \
+    } else if (shared) {                                                                                      \
+      kForceMP<A, M, U><<<4 * grid, kBlock, 0, st>>>(s.G, o, t32, x, xn, s.type, s.rec[s.cur],                \
+                                                     s.rec[1 - s.cur], s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, \
+                                                     sa, s.ctl, iv, lk.mlo);                                  \
     } else {                                                                                                  \
       kForceM<A, M, U><<<grid, kBlock, 0, st>>>(s.G, o, t32, x, xn, s.type, s.rec[s.cur], s.rec[1 - s.cur],    \
                                                 s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv,      \

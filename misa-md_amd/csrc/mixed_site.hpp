@@ -45,13 +45,14 @@ __device__ __forceinline__ float hermiteValue(const float4& k, float q) {
   return fmaf(fmaf(fmaf(c3, q, c4), q, k.y), q, k.x);
 }
 
-// rho_i += sum over the group of rho_{t_j}(r_ij) (pot eam::chargeDensity);
+// rho_i += sum over the group of rho_{t_j}(r_ij) (pot eam::chargeDensity); ks
+// holds the group's offsets, ascending over a site's groups;
 // in[u] tells whether neighbour u is within the cutoff, sk[u] whether it is
 // within the cutoff plus the neighbour skin (r^2 < rcs2).
 template <int ACC, int V>
 __device__ __forceinline__ void rhoGroupM(const float4& me, const float4 (&nb)[V], const float4 (&d)[V], float rc2,
-                                          float rcs2, Rsrc rtab, const Tables<float>& tb, Sum1<ACC>& acc,
-                                          bool (&in)[V], bool (&sk)[V]) {
+                                          float rcs2, Rsrc rtab, const Tables<float>& tb, const int (&ks)[V],
+                                          RangeSum<ACC>& acc, bool (&in)[V], bool (&sk)[V]) {
 #pragma clang fp contract(off)  // explicit FMAs only: every instantiation rounds alike
   float pp[V];
   float4 cr[V];
@@ -68,8 +69,10 @@ __device__ __forceinline__ void rhoGroupM(const float4& me, const float4 (&nb)[V
     }
   }
 #pragma unroll
-  for (int u = 0; u < V; ++u)
-    if (in[u]) acc.add(hermiteValue(cr[u], pp[u]));
+  for (int u = 0; u < V; ++u) {
+    acc.at(ks[u]);
+    if (in[u]) acc.part.add(hermiteValue(cr[u], pp[u]));
+  }
 }
 
 // fpair of one pair (pot eam::toForce) from its segments: the value cubic
@@ -109,11 +112,11 @@ __device__ __forceinline__ bool heldPair(int ei, uint32_t ej, int m, int mlo) {
 
 // f_i += sum over the group of (x_i - x_j) fpair_ij, the segments gathered
 // from the tables in global memory (16-byte knots).
-template <int ACC, int V>
+template <typename Acc, int V>
 __device__ __forceinline__ void forceGroupM(const float4& me, float dfi, int ei, uint32_t pairBase,
                                             const float4 (&nb)[V], const float4 (&d)[V], float rc2, Rsrc rtab,
-                                            Rsrc rtabD, const Tables<float>& tb, int mlo, const int* ks,
-                                            Sum3<ACC>& acc, OtherM& oth) {
+                                            Rsrc rtabD, const Tables<float>& tb, int mlo, const int* ks, Acc& acc,
+                                            OtherM& oth) {
 #pragma clang fp contract(off)
   bool in[V], held[V], like[V];
   float d0[V], d1[V], d2[V], pp[V], ri[V];
@@ -149,7 +152,7 @@ __device__ __forceinline__ void forceGroupM(const float4& me, float dfi, int ei,
       fp[u] = 0.0f;
     }
   }
-  addGroup3<ACC, V>(acc, ks, held, d0, d1, d2, fp);
+  addGroup3(acc, ks, d0, d1, d2, fp);
 }
 
 // forceGroupM with the Fe-Fe r*phi cubics and the Fe density slope cubics
@@ -192,7 +195,7 @@ __device__ __forceinline__ void forceGroupL(const float4& me, float dfi, int ei,
         wq.q[qn + laneRank(other[u])] = static_cast<uint16_t>((ks[u] << 6) | (threadIdx.x & 63u));
       qn += __builtin_popcountll(other[u]);
     }
-  addGroup3<ACC, V>(acc, ks, held, d0, d1, d2, fp);
+  addGroup3(acc, ks, d0, d1, d2, fp);
 }
 
 // Works off n (at most 64) noted pairs q[0 .. n), one a lane: the owner's
@@ -261,7 +264,7 @@ template <int ACC>
 __device__ __forceinline__ void rhoTailM(const Geom& G, int64_t s, int p, int cx, int cy, int cz, int8_t ti,
                                          Sum1<ACC>& acc, CXPtr x, const int8_t* __restrict__ type,
                                          const Tables<float>& tb, const InterView& iv, float4* rec,
-                                         double* __restrict__ rho_out) {
+                                         double* __restrict__ rho_out, const TailHits* hits = nullptr) {
   float dfi = 0.0f;
   double rho = 0.0;
   if (!isVacant(ti)) {
@@ -270,14 +273,14 @@ __device__ __forceinline__ void rhoTailM(const Geom& G, int64_t s, int p, int cx
       const FullPlaneOffsets& full = *iv.full;
       if (ti & kNearInter) {  // inter atoms whose nearest site is within the full list (atom.cpp:224-240)
         const int ne = static_cast<int>(iv.ctl->n_inter + iv.ctl->n_ghost);
-        forNearBuckets(iv, full, p, s, ne, [&](int e) {
+        forNearBuckets(iv, full, p, s, ne, hits, [&](int e) {
           const double d0 = xi0 - iv.e_x[0][e], d1 = xi1 - iv.e_x[1][e], d2 = xi2 - iv.e_x[2][e];
           const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
           if (r2 < G.rc2) acc.add(rhoPair(tb, species(iv.type[iv.e_src[e]]), r2));
         });
       }
       if (ti & kWide) {  // full-list offsets beyond the pruned list, near a far lattice atom
-        forWideTargets(full, type, p, s, ti, [&](int64_t j, int8_t tj) {
+        forWideTargets(full, x.c, type, G.rc2, p, s, ti, xi0, xi1, xi2, hits, [&](int64_t j, int8_t tj) {
           const double d0 = xi0 - x.c[0][j], d1 = xi1 - x.c[1][j], d2 = xi2 - x.c[2][j];
           const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
           if (r2 < G.rc2) acc.add(rhoPair(tb, species(tj), r2));
@@ -333,14 +336,15 @@ __device__ __forceinline__ void forceTailM(const Geom& G, int64_t s, int p, int 
                                            float4* __restrict__ recn, XPtr v, XPtr f,
                                            const uint64_t* __restrict__ id, const VerletParams& vp,
                                            const StageArgs& st, Ctl* ctl, const Tables<float>& tb,
-                                           const InterView& iv, unsigned long long& vb, unsigned long long& db) {
+                                           const InterView& iv, unsigned long long& vb, unsigned long long& db,
+                                           const TailHits* hits = nullptr) {
 #pragma clang fp contract(off)  // the half kicks and drift round as newton_motion.cpp does
   const double xi0 = x.c[0][s], xi1 = x.c[1][s], xi2 = x.c[2][s];
   if (ti & (kNearInter | kWide)) {
     const FullPlaneOffsets& full = *iv.full;
     if (ti & kNearInter) {  // forces from inter atoms on lattice neighbours (atom.cpp:397-422)
       const int ne = static_cast<int>(iv.ctl->n_inter + iv.ctl->n_ghost);
-      forNearBuckets(iv, full, p, s, ne, [&](int e) {
+      forNearBuckets(iv, full, p, s, ne, hits, [&](int e) {
         const int src = iv.e_src[e];
         const double e0 = xi0 - iv.e_x[0][e], e1 = xi1 - iv.e_x[1][e], e2 = xi2 - iv.e_x[2][e];
         const double r2 = e0 * e0 + e1 * e1 + e2 * e2;
@@ -348,7 +352,7 @@ __device__ __forceinline__ void forceTailM(const Geom& G, int64_t s, int p, int 
       });
     }
     if (ti & kWide) {  // full-list offsets beyond the pruned list, near a far lattice atom
-      forWideTargets(full, type, p, s, ti, [&](int64_t j, int8_t tj) {
+      forWideTargets(full, x.c, type, G.rc2, p, s, ti, xi0, xi1, xi2, hits, [&](int64_t j, int8_t tj) {
         const double e0 = xi0 - x.c[0][j], e1 = xi1 - x.c[1][j], e2 = xi2 - x.c[2][j];
         const double r2 = e0 * e0 + e1 * e1 + e2 * e2;
         if (r2 < G.rc2) acc.add(e0, e1, e2, pairForce(tb, ei, species(tj), r2, dfi, rec[j].w));
@@ -394,7 +398,7 @@ __device__ __forceinline__ void forceTailM(const Geom& G, int64_t s, int p, int 
   xn.c[2][s] = y2;
   const float4 r = siteRec(G, p, cx, cy, cz, y0, y1, y2, ei);
   recn[s] = r;
-  forEachImage(G, p, cx, cy, cz, [&](int64_t q, int sx, int sy, int sz) {
+  forEachImage26(G, p, cx, cy, cz, [&](int64_t q, int sx, int sy, int sz) {
     xn.c[0][q] = y0 + sx * G.L0;
     xn.c[1][q] = y1 + sy * G.L1;
     xn.c[2][q] = y2 + sz * G.L2;

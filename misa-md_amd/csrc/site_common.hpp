@@ -80,6 +80,14 @@ __device__ __forceinline__ void forVirtualBlocks(const Geom& G, Body body) {
   for (uint32_t k = q * V + sub; k < nvb; k += Q * V) body(c + 8u * k, tl);
 }
 
+// Launches in which the four wavefronts of a block share 64 sites: block id
+// takes wavefront `sub` of block b of a siteGrid launch, on b's XCD.
+__device__ __forceinline__ void sharedUnit(uint32_t id, uint32_t& b, uint32_t& sub) {
+  const uint32_t j = id >> 3;
+  b = (id & 7u) + 8u * (j >> 2);
+  sub = j & 3u;
+}
+
 inline unsigned siteGrid(const Geom& G) { return static_cast<unsigned>(16 * G.W.bpx); }
 // Grid of a pass that strides over the siteGrid virtual blocks: up to 8
 // blocks per compute unit, a whole number per XCD.
@@ -110,7 +118,7 @@ __device__ __forceinline__ bool nearFace(const Geom& G, int cx, int cy, int cz) 
 // image shift in box lengths (exchangeAtom: x_ghost = x + offset,
 // lat_particle_packer.cpp:22-32,163-194).
 template <typename Fn>
-__device__ __forceinline__ void forEachImage(const Geom& G, int p, int cx, int cy, int cz, Fn fn) {
+__device__ __forceinline__ void forEachImage26(const Geom& G, int p, int cx, int cy, int cz, Fn fn) {
   if (!nearFace(G, cx, cy, cz)) return;
 #pragma unroll
   for (int dz = -1; dz <= 1; dz++) {
@@ -128,6 +136,59 @@ __device__ __forceinline__ void forEachImage(const Geom& G, int p, int cx, int c
         fn(slotOf(G, p, ix, iy, iz), dx, dy, dz);
       }
     }
+  }
+}
+
+// The same in any box, one copy of fn's code in a loop over the 26 shifts.
+template <typename Fn>
+__device__ __forceinline__ void forEachImageLoop(const Geom& G, int p, int cx, int cy, int cz, Fn fn) {
+  if (!nearFace(G, cx, cy, cz)) return;
+  // a cell near at most one face of each dimension has the 7 combinations of its own shifts
+  const bool wide = G.n0 >= 2 * G.g && G.n1 >= 2 * G.g && G.n2 >= 2 * G.g;
+  const int sx = cx < G.g ? 1 : (cx >= G.n0 - G.g ? -1 : 0);
+  const int sy = cy < G.g ? 1 : (cy >= G.n1 - G.g ? -1 : 0);
+  const int sz = cz < G.g ? 1 : (cz >= G.n2 - G.g ? -1 : 0);
+  const int last = wide ? 8 : 27;
+#pragma unroll 1
+  for (int c = 1; c < last; c++) {
+    int dx, dy, dz;
+    if (wide) {
+      if (((c & 1) && sx == 0) || ((c & 2) && sy == 0) || ((c & 4) && sz == 0)) continue;
+      dx = (c & 1) ? sx : 0;
+      dy = (c & 2) ? sy : 0;
+      dz = (c & 4) ? sz : 0;
+    } else {
+      dx = c % 3 == 2 ? -1 : c % 3;
+      dy = c / 3 % 3 == 2 ? -1 : c / 3 % 3;
+      dz = c / 9 == 2 ? -1 : c / 9;
+      const int ix = cx + dx * G.n0, iy = cy + dy * G.n1, iz = cz + dz * G.n2;
+      if (ix < -G.g || ix >= G.n0 + G.g || iy < -G.g || iy >= G.n1 + G.g || iz < -G.g || iz >= G.n2 + G.g) continue;
+    }
+    fn(slotOf(G, p, cx + dx * G.n0, cy + dy * G.n1, cz + dz * G.n2), dx, dy, dz);
+  }
+}
+
+// In a box of at least 2g cells a side a cell lies near at most one face of
+// each dimension, and its images are the 7 combinations of its own shifts.
+// Three forms, by what the registers of the kernels around them bear (one box,
+// one state): the 7 unrolled, for most; one copy in a loop in the FP64 force
+// tail, whose fused form spills (536 against 557 us unrolled, 2M atoms); all
+// 26 unrolled in the mixed force tail (274 against 282 us).
+template <typename Fn>
+__device__ __forceinline__ void forEachImage(const Geom& G, int p, int cx, int cy, int cz, Fn fn) {
+  if (G.n0 < 2 * G.g || G.n1 < 2 * G.g || G.n2 < 2 * G.g) {
+    forEachImageLoop(G, p, cx, cy, cz, fn);
+    return;
+  }
+  if (!nearFace(G, cx, cy, cz)) return;
+  const int sx = cx < G.g ? 1 : (cx >= G.n0 - G.g ? -1 : 0);
+  const int sy = cy < G.g ? 1 : (cy >= G.n1 - G.g ? -1 : 0);
+  const int sz = cz < G.g ? 1 : (cz >= G.n2 - G.g ? -1 : 0);
+#pragma unroll
+  for (int c = 1; c < 8; c++) {
+    if (((c & 1) && sx == 0) || ((c & 2) && sy == 0) || ((c & 4) && sz == 0)) continue;
+    const int dx = (c & 1) ? sx : 0, dy = (c & 2) ? sy : 0, dz = (c & 4) ? sz : 0;
+    fn(slotOf(G, p, cx + dx * G.n0, cy + dy * G.n1, cz + dz * G.n2), dx, dy, dz);
   }
 }
 
@@ -308,6 +369,7 @@ template <>
 struct Sum1<0> {
   double s = 0;
   __device__ __forceinline__ void add(double v) { s += v; }
+  __device__ __forceinline__ void join(const Sum1<0>& o) { s += o.s; }
   __device__ __forceinline__ double value() const { return s; }
 };
 template <>
@@ -320,6 +382,11 @@ struct Sum1<1> {
     c = (t - s) - y;
     s = t;
   }
+  // another sum and what its compensation still holds back (an empty one changes nothing)
+  __device__ __forceinline__ void join(const Sum1<1>& o) {
+    if (o.s != 0.0f) add(o.s);
+    if (o.c != 0.0f) add(-o.c);
+  }
   __device__ __forceinline__ double value() const { return static_cast<double>(s); }
 };
 
@@ -328,14 +395,44 @@ template <>
 struct Sum1<2> {
   float s = 0;
   __device__ __forceinline__ void add(float v) { s += v; }
+  __device__ __forceinline__ void join(const Sum1<2>& o) { s += o.s; }
   __device__ __forceinline__ double value() const { return static_cast<double>(s); }
 };
 
+// The sum of a density pass: over the four ranges of 32 offsets (the 32-bit
+// words of a wavefront's mask) one after the other, each summed by itself, so
+// that the ranges of a site may be summed by one wavefront or by four.
+template <int ACC>
+struct RangeSum {
+  Sum1<ACC> tot, part;
+  int range = 0;
+  __device__ __forceinline__ void close() {
+    tot.join(part);
+    part = Sum1<ACC>();
+  }
+  __device__ __forceinline__ void at(int k) {  // offset k (the same in every lane) comes next
+    if ((k >> 5) != range) {
+      close();
+      range = k >> 5;
+    }
+  }
+};
+
+// Force sums.  The terms of the lattice offsets 8t .. 8t+7 are summed by fused
+// multiply-adds in an open chunk g (FP64 for ACC 0, else FP32), and that
+// chunk's sum joins the site's sum as one term when the offsets move past it
+// (addGroup3) and once more at the end (flushChunk3).  The chunks hang on the
+// offsets alone, not on how they are grouped for the gathers, nor on which
+// wavefront sums them, nor on which other sites share the wavefront, so every
+// launch shape gives the same bits.
 template <int ACC>
 struct Sum3;
 template <>
 struct Sum3<0> {
+  using Term = double;
   double f0 = 0, f1 = 0, f2 = 0;
+  double g0 = 0, g1 = 0, g2 = 0;
+  int chunk = 0;
   template <typename T>
   __device__ __forceinline__ void add(double d0, double d1, double d2, T fp) {
     const double q = static_cast<double>(fp);
@@ -343,12 +440,19 @@ struct Sum3<0> {
     f1 = fma(d1, q, f1);
     f2 = fma(d2, q, f2);
   }
+  __device__ __forceinline__ void flush() {
+    f0 += g0;
+    f1 += g1;
+    f2 += g2;
+    g0 = g1 = g2 = 0.0;
+  }
 };
 template <>
 struct Sum3<1> {
+  using Term = float;
   Sum1<1> a, b, c;
-  float g0 = 0, g1 = 0, g2 = 0;  // the open chunk of lattice terms (addGroup3)
-  int chunk = 0;                 // its offsets: 8 chunk .. 8 chunk + 7
+  float g0 = 0, g1 = 0, g2 = 0;
+  int chunk = 0;
   __device__ __forceinline__ void add(double d0, double d1, double d2, float fp) {
 #pragma clang fp contract(off)
     a.add(static_cast<float>(d0) * fp);
@@ -365,49 +469,64 @@ struct Sum3<1> {
 };
 template <>
 struct Sum3<2> {
+  using Term = float;
   float f0 = 0, f1 = 0, f2 = 0;
+  float g0 = 0, g1 = 0, g2 = 0;
+  int chunk = 0;
   __device__ __forceinline__ void add(float d0, float d1, float d2, float fp) {
     f0 = fmaf(d0, fp, f0);
     f1 = fmaf(d1, fp, f1);
     f2 = fmaf(d2, fp, f2);
   }
+  __device__ __forceinline__ void flush() {
+    f0 += g0;
+    f1 += g1;
+    f2 += g2;
+    g0 = g1 = g2 = 0.0f;
+  }
 };
-// The force terms of a group of lattice neighbours (in[u]: neighbour u
-// counts; ks[u]: its offset, ascending over a site's groups).  With
-// compensated sums (ACC 1) the terms of the offsets 8t .. 8t+7 are summed in
-// FP32 (fused multiply-adds) and that chunk's sum joins the compensated sum
-// as one term, when the offsets move past the chunk and once more at the end
-// (flushChunk3); a lane adds no empty chunk.  The chunks hang on the offsets
-// alone, not on how they are grouped for the gathers nor on which other
-// sites share the wavefront, so every launch shape gives the same bits.
-// Otherwise term by term.
-template <int ACC, int V>
-__device__ __forceinline__ void addGroup3(Sum3<ACC>& acc, const int* ks, const bool (&in)[V], const float (&d0)[V],
-                                          const float (&d1)[V], const float (&d2)[V], const float (&fp)[V]) {
+constexpr int kChunks = 16;  // chunks of eight offsets of a wavefront's 128-bit mask
+// The chunk sums of one lane written out instead (a wavefront that sums only
+// part of its sites' offsets): out[chunk][component][lane], zeroed before.
+template <int ACC>
+struct ChunkSums {
+  using Term = typename Sum3<ACC>::Term;
+  Term g0 = 0, g1 = 0, g2 = 0;
+  int chunk;
+  Term (*out)[3][64];
+  __device__ __forceinline__ void flush() {
+    const int lane = static_cast<int>(threadIdx.x & 63u);
+    out[chunk][0][lane] = g0;
+    out[chunk][1][lane] = g1;
+    out[chunk][2][lane] = g2;
+    g0 = g1 = g2 = 0;
+  }
+};
+// The force terms of a group of lattice neighbours (ks[u]: its offset, the
+// same in every lane, ascending over a site's groups).  fp is 0 for a
+// neighbour that does not count and the displacements are finite (a
+// vacancy's too), so such a term adds an exact zero.
+template <typename Acc, int V>
+__device__ __forceinline__ void addGroup3(Acc& acc, const int* ks, const float (&d0)[V], const float (&d1)[V],
+                                          const float (&d2)[V], const float (&fp)[V]) {
 #pragma clang fp contract(off)
-  if constexpr (ACC == 1) {
+  using T = typename Acc::Term;
 #pragma unroll
-    for (int u = 0; u < V; ++u) {
-      const int t = ks[u] >> 3;  // the same in every lane
-      if (t != acc.chunk) {
-        acc.flush();
-        acc.chunk = t;
-      }
-      // fp is 0 beyond the cutoff and the displacements are finite (a
-      // vacancy's too), so those terms add an exact zero
-      acc.g0 = fmaf(d0[u], fp[u], acc.g0);
-      acc.g1 = fmaf(d1[u], fp[u], acc.g1);
-      acc.g2 = fmaf(d2[u], fp[u], acc.g2);
+  for (int u = 0; u < V; ++u) {
+    const int t = ks[u] >> 3;
+    if (t != acc.chunk) {
+      acc.flush();
+      acc.chunk = t;
     }
-  } else {
-#pragma unroll
-    for (int u = 0; u < V; ++u)
-      if (in[u]) acc.add(d0[u], d1[u], d2[u], fp[u]);
+    const T f = static_cast<T>(fp[u]);
+    acc.g0 = __builtin_elementwise_fma(static_cast<T>(d0[u]), f, acc.g0);
+    acc.g1 = __builtin_elementwise_fma(static_cast<T>(d1[u]), f, acc.g1);
+    acc.g2 = __builtin_elementwise_fma(static_cast<T>(d2[u]), f, acc.g2);
   }
 }
-template <int ACC>
-__device__ __forceinline__ void flushChunk3(Sum3<ACC>& acc) {
-  if constexpr (ACC == 1) acc.flush();
+template <typename Acc>
+__device__ __forceinline__ void flushChunk3(Acc& acc) {
+  acc.flush();
 }
 
 template <int ACC>
