@@ -61,6 +61,7 @@ struct misa_handle {
   int force_pass = -1;       // MISA_FORCE_PASS_* of the last force pass launched
   bool range_check = false;  // a density beyond the F(rho) table fails the call
   int64_t flags_seen = 0;    // the device flags at the last check
+  bool few_listed = false;   // at the last look the decide's lists were short (kFewListed)
   // XCD slabs cut by measured work (misa_set_xcd_balance); virtual blocks
   // per parity per XCD the wave-mask and partial-sum arrays are sized for
   bool balance = true;
@@ -233,11 +234,21 @@ void makeWalk(Geom& G) {
   evenSlabs(G);
 }
 
+// A box of up to kDecideAllSites sites takes its decide in one workgroup
+// while at most kFewListed inter atoms, images and far atoms are listed: five
+// launches, some 2 us each, become one (16 000 cells FP64 at rest: 48 -> 41 us
+// a step).  A list of thousands wants the grid (the same box with 10 000 far
+// atoms: 86 us a step with it, 300 us without).
+constexpr int64_t kFewListed = 64;
+constexpr int64_t kLookSteps = 128;  // steps between two looks at the lists
+bool fewListed(const Ctl& c) { return c.n_prev + c.n_far_prev <= kFewListed; }
+
 int syncAndCheck(misa_handle* h) {
   HIPCHECK(h, hipStreamSynchronize(h->stream));
   Ctl c;
   HIPCHECK(h, hipMemcpy(&c, h->s.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
   h->flags_seen = c.err_flags;
+  h->few_listed = fewListed(c);
   if (c.err_flags & kErrInterCap) return fail(h, MISA_E_CAPACITY, "inter-atom list capacity exceeded");
   if (c.err_flags & kErrGhostCap) return fail(h, MISA_E_CAPACITY, "ghost inter-atom capacity exceeded");
   if (c.err_flags & kErrNonFinite) return fail(h, MISA_E_DEVICE, "non-finite force or electron density");
@@ -918,24 +929,16 @@ int misa_set_inter_capacity(misa_handle* h, int64_t cap) {
 
 // clearForce + computeEam (atom.cpp:86-149) on the resident state, after the
 // inter-atom migration, ghost images and index (mode 1 of the decide kernel).
-static void forcePass(misa_handle* h, int lattice_mode, int inter_mode, bool store_rho, const VerletParams& vp) {
+static void forcePass(misa_handle* h, int mode, bool store_rho, const VerletParams& vp) {
   const bool mixed = h->precision == MISA_PREC_MIXED;
-  {
-    Timer t(h, 2);
-    launchInterRho(h->s, h->t64, h->t32, mixed, h->stream);
-  }
   {
     Timer t(h, 0);
     launchRhoDf(h->s, h->lat, h->t64, h->t32, mixed, h->acc, store_rho, h->stream);
     h->mask_gen = h->gen;
   }
   {
-    Timer t(h, 2);
-    launchInterForce(h->s, h->t64, h->t32, mixed, inter_mode, vp, h->stream);
-  }
-  {
     Timer t(h, 1);
-    h->force_pass = launchForce(h->s, h->lat, h->t64, h->t32, mixed, h->acc, lattice_mode, vp, h->stream);
+    h->force_pass = launchForce(h->s, h->lat, h->t64, h->t32, mixed, h->acc, mode, vp, h->stream);
   }
 }
 
@@ -950,8 +953,8 @@ int misa_compute_forces(misa_handle* h) {
   const bool mixed = h->precision == MISA_PREC_MIXED;
   launchPackRec(h->s, h->s.cur, !mixed, h->stream);
   launchFarScan(h->s, h->stream);
-  launchDecide(h->s, 1, mixed, h->stream);
-  forcePass(h, 2, 2, true, vp);
+  launchDecide(h->s, 1, mixed, false, h->stream);
+  forcePass(h, 2, true, vp);
   h->profile = prof;
   HIPCHECK(h, hipGetLastError());
   const int rc = syncAndCheck(h);
@@ -972,6 +975,7 @@ namespace {
 //             step) and its decide
 struct StepPlan {
   bool adaptive, mixed;
+  bool few = false;  // the decide in one workgroup
   VerletParams vp;
 };
 
@@ -995,14 +999,16 @@ void enqRescanIfChanged(misa_handle* h) {
 void enqFirstAndDecide(misa_handle* h, const StepPlan& p, bool lattice, bool vmax_done = false) {
   {
     Timer t(h, 2);
-    if (p.adaptive) launchAdaptiveDt(h->s, h->dt_max, h->max_disp, !vmax_done, h->stream);
+    // the inter atoms' first half step comes with the step length, or else in
+    // the fused force pass, or else here
+    if (p.adaptive) launchAdaptiveDt(h->s, h->dt_max, h->max_disp, !vmax_done, p.vp, h->stream);
     if (lattice) launchFirst(h->s, p.mixed, p.vp, h->stream);
-    launchInterFirst(h->s, p.vp, h->stream);
+    if (lattice && !p.adaptive) launchInterFirst(h->s, p.vp, h->stream);
   }
   h->s.cur = 1 - h->s.cur;
   {
     Timer t(h, 2);
-    launchDecide(h->s, 0, p.mixed, h->stream);
+    launchDecide(h->s, 0, p.mixed, p.few, h->stream);
   }
 }
 
@@ -1011,7 +1017,7 @@ void enqBody(misa_handle* h, const StepPlan& p, bool last) {
   VerletParams vp = p.vp;
   // adaptive: the secondstep pass reduces the lattice sites' max |v|^2 itself
   if (p.adaptive && !last) vp.vmax = &h->s.ctl->vmax2;
-  forcePass(h, fuse ? 1 : 0, 0, last, vp);
+  forcePass(h, fuse ? 1 : 0, last, vp);
   if (!last) enqFirstAndDecide(h, p, !fuse, p.adaptive);
 }
 
@@ -1095,7 +1101,9 @@ int misa_step(misa_handle* h, int64_t nsteps) {
   if (!h->forces_ready) return fail(h, MISA_E_ARG, "misa_compute_forces must run before misa_step");
   if (nsteps == 0) return MISA_OK;
   HIPCHECK(h, hipSetDevice(h->device));
-  const StepPlan p = planOf(h);
+  StepPlan p = planOf(h);
+  const bool look = decideBySize(h->s) == DecideForm::byLists;
+  p.few = look && h->few_listed;
   clearEvents(h);
   hipEvent_t e0, e1;
   HIPCHECK(h, hipEventCreate(&e0));
@@ -1112,6 +1120,12 @@ int misa_step(misa_handle* h, int64_t nsteps) {
     }
     enqBody(h, p, i == nsteps - 1);
     h->s.zmeasure = false;
+    if (look && (i + 1) % kLookSteps == 0) {
+      Ctl c;
+      HIPCHECK(h, hipStreamSynchronize(h->stream));
+      HIPCHECK(h, hipMemcpy(&c, h->s.ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+      p.few = fewListed(c);
+    }
   }
   HIPCHECK(h, hipGetLastError());
   HIPCHECK(h, hipEventRecord(e1, h->stream));
@@ -1394,8 +1408,8 @@ int buildFused(misa_batch* b) {
 
 // Two loop bodies of every box of a fused batch as one launch per pass:
 // the inter atoms' density, the lattice density pass, the inter atoms'
-// forces, the LDS force pass with the next half step and decide staging,
-// the inter atoms' first half step and the decide (on the other buffer).
+// forces and next half step, the LDS force pass with the next half step and
+// decide staging, and the decide (on the other buffer).
 int captureFused(misa_batch* b) {
   if (b->exec) {
     (void)hipGraphExecDestroy(b->exec);
@@ -1410,8 +1424,7 @@ int captureFused(misa_batch* b) {
     launchRhoDfBatch(b->boxes, b->rhoStart, n, b->rhoBlocks, h0->acc, f, b->origin);
     launchInterBatch(1, b->boxes, n, f, nullptr, b->origin);
     lds = lds && launchForceBatch(b->boxes, b->vstart, n, h0->s.dl, h0->t32.nr, h0->s.ncu, h0->acc, f, b->origin);
-    launchInterBatch(2, b->boxes, n, f, nullptr, b->origin);
-    launchInterBatch(3, b->boxes, n, f ^ 1, b->decideArgs, b->origin);
+    launchInterBatch(2, b->boxes, n, f ^ 1, b->decideArgs, b->origin);
   }
   const hipError_t e0 = hipGetLastError();
   hipGraph_t g = nullptr;

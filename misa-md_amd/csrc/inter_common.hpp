@@ -107,11 +107,12 @@ __device__ __forceinline__ int64_t nearSubBoxSlot(const Geom& G, double x0, doub
 
 __device__ __forceinline__ void decodeSlot(const Geom& G, int64_t slot, int& p, int& cx, int& cy, int& cz) {
   p = slot >= G.plane ? 1 : 0;
-  int64_t r = slot - p * G.plane;
-  cx = static_cast<int>(r % G.NX) - G.g;
-  r /= G.NX;
-  cy = static_cast<int>(r % G.NY) - G.g;
-  cz = static_cast<int>(r / G.NY) - G.g;
+  // 32-bit divisions: a plane of 2^32 slots would not fit in memory
+  const uint32_t r = static_cast<uint32_t>(slot - p * G.plane), NX = static_cast<uint32_t>(G.NX);
+  const uint32_t row = r / NX, NY = static_cast<uint32_t>(G.NY), z = row / NY;
+  cx = static_cast<int>(r - row * NX) - G.g;
+  cy = static_cast<int>(row - z * NY) - G.g;
+  cz = static_cast<int>(z) - G.g;
 }
 
 __device__ __forceinline__ bool isSubBoxSlot(const Geom& G, int64_t slot) {

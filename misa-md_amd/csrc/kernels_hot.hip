@@ -37,6 +37,7 @@
 
 #include "device_common.hpp"
 #include "inter_common.hpp"
+#include "inter_step.hpp"
 #include "resident.hpp"
 #include "site_common.hpp"
 #include "buffer_load.hpp"
@@ -56,11 +57,21 @@ __device__ __forceinline__ double dist2D(double d0, double d1, double d2) {
   return __fma_rn(d2, d2, __fma_rn(d1, d1, __dmul_rn(d0, d0)));
 }
 
-// Index of the wavefront in the grid, in a scalar register (threadIdx.x >> 6
-// is the same in every lane of a wavefront).
-__device__ __forceinline__ uint32_t waveId() {
-  return blockIdx.x * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+// Index of the wavefront among those of block b and its predecessors, in a
+// scalar register (threadIdx.x >> 6 is the same in every lane of a wavefront).
+__device__ __forceinline__ uint32_t waveId(uint32_t b) {
+  return b * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
+
+// The site passes carry the inter atoms' work of the same pass along, in their
+// first kFrontBlocks blocks (a multiple of 8, so that the others keep their
+// XCD): neither part reads what the other writes, and a launch of its own for
+// a list that is mostly empty costs 2 to 5 us.
+constexpr uint32_t kFrontBlocks = 64;
+__device__ __forceinline__ int frontWave() {
+  return static_cast<int>(blockIdx.x * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+}
+constexpr int kFrontWaves = static_cast<int>(kFrontBlocks) * (kBlock / 64);
 // A wavefront-uniform 64-bit value moved to scalar registers.
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
@@ -281,15 +292,20 @@ __global__ __launch_bounds__(kBlock, 7) void kRhoDf(Geom G, LatOffsets O, Tables
                                                  const int8_t* __restrict__ type, double* __restrict__ df,
                                                  double* __restrict__ rho_out, uint64_t* __restrict__ wmask,
                                                  uint64_t* __restrict__ smask, double rcs2, InterView iv,
-                                                 Rec64 r64) {
+                                                 InterDev in, Rec64 r64) {
+  if (blockIdx.x < kFrontBlocks) {
+    interRhoBody<double>(G, tb, iv, x, type, in, frontWave(), kFrontWaves);
+    return;
+  }
+  const uint32_t b = blockIdx.x - kFrontBlocks;
   int64_t s;
   int p, cx, cy, cz;
-  if (!siteOfThread(G, s, p, cx, cy, cz)) return;
+  if (!siteOfBlock(G, b, threadIdx.x, s, p, cx, cy, cz)) return;
   const int8_t ti = type[s];
   // a wavefront next to a far lattice atom (kWide) scans in full and records its masks afresh
   const bool skin =
       __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(!isVacant(ti) && (ti & kWide));
-  const uint32_t wv = waveId();
+  const uint32_t wv = waveId(b);
   RangeSum<0> acc;
   uint64_t w0 = 0, w1 = 0, s0 = 0, s1 = 0;
   if (!isVacant(ti)) {
@@ -391,10 +407,14 @@ __global__ __launch_bounds__(kBlock) void kRhoDfP(Geom G, LatOffsets O, Tables<d
                                                   const int8_t* __restrict__ type, double* __restrict__ df,
                                                   double* __restrict__ rho_out, uint64_t* __restrict__ wmask,
                                                   uint64_t* __restrict__ smask, double rcs2, InterView iv,
-                                                  Rec64 r64) {
+                                                  InterDev in, Rec64 r64) {
   __shared__ RangeParts parts;
   __shared__ TailHits hits;
-  const SharedSite q = sharedSite(G, type, blockIdx.x);
+  if (blockIdx.x < kFrontBlocks) {
+    interRhoBody<double>(G, tb, iv, x, type, in, frontWave(), kFrontWaves);
+    return;
+  }
+  const SharedSite q = sharedSite(G, type, blockIdx.x - kFrontBlocks);
   const bool live = !isVacant(q.ti);
   const bool skin = __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(live && (q.ti & kWide));
   RangeSum<0> acc;
@@ -713,10 +733,15 @@ __global__ __launch_bounds__(kBlock) void kForceP(Geom G, LatOffsets O, Tables<d
                                                   const int8_t* __restrict__ type, const double* __restrict__ df,
                                                   const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                                   const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
-                                                  Ctl* ctl, InterView iv, Rec64 r64, Rec64 rn64, int mlo) {
+                                                  Ctl* ctl, InterView iv, InterDev in, Rec64 r64, Rec64 rn64,
+                                                  int mlo) {
   __shared__ double parts[3][6][64];
   __shared__ TailHits hits;
-  const SharedSite q = sharedSite(G, type, blockIdx.x);
+  if (blockIdx.x < kFrontBlocks) {
+    interForceBody<double, MODE>(G, tb, iv, x, type, df, 1, in, vp, frontWave(), kFrontWaves);
+    return;
+  }
+  const SharedSite q = sharedSite(G, type, blockIdx.x - kFrontBlocks);
   const int lane = static_cast<int>(threadIdx.x & 63u);
   ForceSiteD c{};
   Force3 part, opart;
@@ -977,11 +1002,16 @@ __global__ __launch_bounds__(kBlock) void kForce(Geom G, LatOffsets O, Tables<do
                                                  const int8_t* __restrict__ type, const double* __restrict__ df,
                                                  const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                                  const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
-                                                 Ctl* ctl, InterView iv, Rec64 r64, Rec64 rn64, int mlo) {
+                                                 Ctl* ctl, InterView iv, InterDev in, Rec64 r64, Rec64 rn64,
+                                                 int mlo) {
   unsigned long long vb = 0;  // |v|^2 bits after the secondstep (MODE 0)
   unsigned long long db = 0;  // |dx|^2 bits of the drift (MODE 1)
-  forceSiteD<MODE, U>(G, O, tb, x, xn, type, df, wmask, v, f, id, vp, st, ctl, iv, r64, rn64, mlo, blockIdx.x,
-                      threadIdx.x, vb, db);
+  if (blockIdx.x < kFrontBlocks) {
+    interForceBody<double, MODE>(G, tb, iv, x, type, df, 1, in, vp, frontWave(), kFrontWaves);
+    return;
+  }
+  forceSiteD<MODE, U>(G, O, tb, x, xn, type, df, wmask, v, f, id, vp, st, ctl, iv, r64, rn64, mlo,
+                      blockIdx.x - kFrontBlocks, threadIdx.x, vb, db);
   if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
   if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
 }
@@ -1160,7 +1190,8 @@ __global__ __launch_bounds__(kBlockP) void kForceDL(Geom G, LatOffsets O, Tables
                                                     const int8_t* __restrict__ type, const double* __restrict__ df,
                                                     const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                                     const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
-                                                    Ctl* ctl, InterView iv, Rec64 r64, Rec64 rn64, int mlo, int nkn) {
+                                                    Ctl* ctl, InterView iv, InterDev in, Rec64 r64, Rec64 rn64,
+                                                    int mlo, int nkn) {
   __shared__ WaveQueueD<U> queues[kBlockP / 64];
   __shared__ WaveSums sums[kBlockP / 64];
   extern __shared__ double2 knS[];  // nkn {s_z, s_rho}, nkn {y_z, dy_z}, nkn dy_rho
@@ -1179,6 +1210,8 @@ __global__ __launch_bounds__(kBlockP) void kForceDL(Geom G, LatOffsets O, Tables
   __syncthreads();
   const KnotsD kn{ks - mlo, kyd - mlo, kdr - mlo};
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  interForceBody<double, MODE>(G, tb, iv, x, type, df, 1, in, vp, static_cast<int>(wave * gridDim.x + blockIdx.x),
+                               static_cast<int>(gridDim.x) * (kBlockP / 64));
   unsigned long long vb = 0, db = 0;
   forVirtualBlocks(G, [&](uint32_t b, uint32_t tl) {
     forceVBlockD<MODE, U>(G, O, tb, x, xn, type, df, wmask, v, f, id, vp, st, ctl, iv, r64, rn64, kn, mlo,
@@ -1298,10 +1331,14 @@ __global__ __launch_bounds__(kBlock) void kRhoDfMP(Geom G, LatOffsets O, Tables<
                                                    const int8_t* __restrict__ type, float4* rec,
                                                    const float4* __restrict__ dl, double* __restrict__ rho_out,
                                                    uint64_t* __restrict__ wmask, uint64_t* __restrict__ smask,
-                                                   float rcs2, InterView iv) {
+                                                   float rcs2, InterView iv, InterDev in) {
   __shared__ RangeParts parts;
   __shared__ TailHits hits;
-  const SharedSite q = sharedSite(G, type, blockIdx.x);
+  if (blockIdx.x < kFrontBlocks) {
+    interRhoBody<float>(G, tb, iv, x, type, in, frontWave(), kFrontWaves);
+    return;
+  }
+  const SharedSite q = sharedSite(G, type, blockIdx.x - kFrontBlocks);
   const bool live = !isVacant(q.ti);
   const bool skin = __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(live && (q.ti & kWide));
   RangeSum<ACC> acc;
@@ -1328,8 +1365,12 @@ __global__ __launch_bounds__(kBlock, U == 4 ? 8 : 6) void kRhoDfM(Geom G, LatOff
                                                   const int8_t* __restrict__ type, float4* rec,
                                                   const float4* __restrict__ dl, double* __restrict__ rho_out,
                                                   uint64_t* __restrict__ wmask, uint64_t* __restrict__ smask,
-                                                  float rcs2, InterView iv) {
-  rhoPassM<ACC, U>(G, O, tb, x, type, rec, dl, rho_out, wmask, smask, rcs2, iv, blockIdx.x);
+                                                  float rcs2, InterView iv, InterDev in) {
+  if (blockIdx.x < kFrontBlocks) {
+    interRhoBody<float>(G, tb, iv, x, type, in, frontWave(), kFrontWaves);
+    return;
+  }
+  rhoPassM<ACC, U>(G, O, tb, x, type, rec, dl, rho_out, wmask, smask, rcs2, iv, blockIdx.x - kFrontBlocks);
 }
 
 // The density pass of every box of a batch in one launch: the blocks of box
@@ -1380,13 +1421,19 @@ __global__ __launch_bounds__(kBlock) void kForceM(Geom G, LatOffsets O, Tables<f
                                                   float4* __restrict__ recn, const float4* __restrict__ dl,
                                                   const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                                   const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
-                                                  Ctl* ctl, InterView iv, int mlo) {
+                                                  Ctl* ctl, InterView iv, InterDev in, int mlo) {
   unsigned long long vb = 0;  // |v|^2 bits after the secondstep (MODE 0)
   unsigned long long db = 0;  // |dx|^2 bits of the drift (MODE 1)
+  if (blockIdx.x < kFrontBlocks) {
+    interForceBody<float, MODE>(G, tb, iv, x, type, reinterpret_cast<const float*>(rec) + 3, 4, in, vp, frontWave(),
+                                kFrontWaves);
+    return;
+  }
+  const uint32_t b = blockIdx.x - kFrontBlocks;
   [&] {
     int64_t s;
     int p, cx, cy, cz;
-    if (!siteOfThread(G, s, p, cx, cy, cz)) return;
+    if (!siteOfBlock(G, b, threadIdx.x, s, p, cx, cy, cz)) return;
     const int8_t ti = type[s];
     if (isVacant(ti)) {  // vacancy: keeps its stale position (atom.cpp:43-47)
       vacancyForceM<MODE>(G, s, p, cx, cy, cz, x, xn, recn, f);
@@ -1397,7 +1444,7 @@ __global__ __launch_bounds__(kBlock) void kForceM(Geom G, LatOffsets O, Tables<f
     Sum3<ACC> acc;
     OtherM oth;
     // the offsets the density pass found in range for some lane of this wavefront
-    const uint32_t wv = waveId();
+    const uint32_t wv = waveId(b);
     forceSumM<U>(O, tb, rec, dl, static_cast<float>(G.rc2), mlo, s, p, ei, me, uniform64(wmask[2 * wv]),
                  uniform64(wmask[2 * wv + 1]), acc, oth);
     addOther3(acc, oth);
@@ -1417,12 +1464,17 @@ __global__ __launch_bounds__(kBlock) void kForceMP(Geom G, LatOffsets O, Tables<
                                                    float4* __restrict__ recn, const float4* __restrict__ dl,
                                                    const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                                    const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
-                                                   Ctl* ctl, InterView iv, int mlo) {
+                                                   Ctl* ctl, InterView iv, InterDev in, int mlo) {
   using Term = typename Sum3<ACC>::Term;
   __shared__ Term chunks[kChunks][3][64];
   __shared__ double others[3][3][64];
   __shared__ TailHits hits;
-  const SharedSite q = sharedSite(G, type, blockIdx.x);
+  if (blockIdx.x < kFrontBlocks) {
+    interForceBody<float, MODE>(G, tb, iv, x, type, reinterpret_cast<const float*>(rec) + 3, 4, in, vp, frontWave(),
+                                kFrontWaves);
+    return;
+  }
+  const SharedSite q = sharedSite(G, type, blockIdx.x - kFrontBlocks);
   const int lane = static_cast<int>(threadIdx.x & 63u);
   const int ei = species(q.ti);
   float4 me = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -1630,7 +1682,7 @@ __global__ __launch_bounds__(kBlockP) void kForceL(Geom G, LatOffsets O, Tables<
                                                    float4* __restrict__ recn, const float4* __restrict__ dl,
                                                    const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                                    const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
-                                                   Ctl* ctl, InterView iv, int mlo, int nkn,
+                                                   Ctl* ctl, InterView iv, InterDev in, int mlo, int nkn,
                                                    unsigned long long* zwork) {
   __shared__ float4 offT[2 * kMaxLatOffsets];  // {lattice vector, record shift * 16}
   __shared__ WaveQueueM queues[kBlockP / 64];
@@ -1643,6 +1695,9 @@ __global__ __launch_bounds__(kBlockP) void kForceL(Geom G, LatOffsets O, Tables<
   unsigned long long vb = 0;  // |v|^2 bits after the secondstep (MODE 0), largest over the lane's sites
   unsigned long long db = 0;  // |dx|^2 bits of the drift (MODE 1), likewise
   const RecShift shift;
+  interForceBody<float, MODE>(G, tb, iv, x, type, reinterpret_cast<const float*>(rec) + 3, 4, in, vp,
+                              static_cast<int>(wave * gridDim.x + blockIdx.x),
+                              static_cast<int>(gridDim.x) * (kBlockP / 64));
   forVirtualBlocks(G, [&](uint32_t b, uint32_t tl) {
     const long long t0 = zwork ? clock64() : 0;
     forceVBlockL<ACC, MODE, U>(G, O, tb, x, xn, type, rec, recn, wmask, v, f, id, vp, st, ctl, iv, dl + 2 * kMaxLatOffsets,
@@ -1775,23 +1830,24 @@ bool useShared(const DevState& s) {
 void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
                  bool mixed, int acc, bool store_rho, hipStream_t st) {
   double* rho = store_rho ? s.rho : nullptr;
-  const unsigned grid = siteGrid(s.G);
+  const bool shared = useShared(s);
+  const unsigned grid = kFrontBlocks + (shared ? 4 : 1) * siteGrid(s.G);
   const InterView iv = interView(s, mixed);
   const CXPtr x = cxp(s.x[s.cur]);
   const double rcs = std::sqrt(s.G.rc2) + s.skin;
-  const bool shared = useShared(s);
   if (!mixed) {
     const Rec64 r64{s.pxy[s.cur], s.pzw[s.cur]};
     if (shared)
-      kRhoDfP<4><<<4 * grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs, iv,
-                                              r64);
+      kRhoDfP<4><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs, iv,
+                                              s.in, r64);
     else
-      kRhoDf<4><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs, iv, r64);
+      kRhoDf<4><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs, iv, s.in,
+                                         r64);
   } else if (shared) {
     const float rcs2 = static_cast<float>(rcs * rcs);
 #define MISA_RHO_MP(A)                                                                                          \
-  kRhoDfMP<A, 4><<<4 * grid, kBlock, 0, st>>>(s.G, o, t32, x, s.type, s.rec[s.cur], s.dl, rho, s.wmask, s.smask, \
-                                              rcs2, iv)
+  kRhoDfMP<A, 4><<<grid, kBlock, 0, st>>>(s.G, o, t32, x, s.type, s.rec[s.cur], s.dl, rho, s.wmask, s.smask, \
+                                              rcs2, iv, s.in)
     if (acc == 0) MISA_RHO_MP(0);
     else if (acc == 1) MISA_RHO_MP(1);
     else MISA_RHO_MP(2);
@@ -1800,7 +1856,7 @@ void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t
     const float rcs2 = static_cast<float>(rcs * rcs);
 #define MISA_RHO_M(A, U)                                                                                   \
   kRhoDfM<A, U><<<grid, kBlock, 0, st>>>(s.G, o, t32, x, s.type, s.rec[s.cur], s.dl, rho, s.wmask, s.smask, \
-                                        rcs2, iv)
+                                        rcs2, iv, s.in)
     const bool u8 = s.uRho == 8;
     if (acc == 0) {
       if (u8) MISA_RHO_M(0, 8);
@@ -1819,12 +1875,13 @@ void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t
 int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
                 bool mixed, int acc, int mode, const VerletParams& vp, hipStream_t st) {
   int kind = mixed ? 1 : 0;
-  const unsigned grid = siteGrid(s.G);
+  const bool shared = useShared(s);
+  const unsigned grid = kFrontBlocks + (shared ? 4 : 1) * siteGrid(s.G);
   const CXPtr x = cxp(s.x[s.cur]);
   const XPtr xn = xp(s.x[1 - s.cur]);
   const StageArgs sa = stageOf(s);
   const InterView iv = interView(s, mixed);
-  const bool lds = useLds(s), shared = useShared(s);
+  const bool lds = useLds(s);
   const LdsKnots lk = ldsKnotsForce(t32.nr);
   const LdsKnots lkd = ldsKnotsForceD(t64.nr);
 #define MISA_FORCE(M)                                                                                         \
@@ -1835,14 +1892,16 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
     if (lds && ldsReady) {                                                                                    \
       kind = 3;                                                                                               \
       kForceDL<M, kUDouble><<<persistentGrid(s), kBlockP, lkd.bytes, st>>>(                                   \
-          s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv, r64, rn64,   \
-          lkd.mlo, lkd.nkn);                                                                                  \
+          s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv, s.in, r64,   \
+          rn64, lkd.mlo, lkd.nkn);                                                                            \
     } else if (shared) {                                                                                      \
-      kForceP<M, kUDouble><<<4 * grid, kBlock, 0, st>>>(s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v), \
-                                                        xp(s.f), s.id, vp, sa, s.ctl, iv, r64, rn64, lkd.mlo); \
+      kForceP<M, kUDouble><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v), \
+                                                    xp(s.f), s.id, vp, sa, s.ctl, iv, s.in, r64, rn64,    \
+                                                    lkd.mlo);                                             \
     } else {                                                                                                  \
       kForce<M, kUDouble><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v),      \
-                                                   xp(s.f), s.id, vp, sa, s.ctl, iv, r64, rn64, lkd.mlo);     \
+                                                   xp(s.f), s.id, vp, sa, s.ctl, iv, s.in, r64, rn64,         \
+                                                   lkd.mlo);                                                  \
     }                                                                                                         \
   } while (0)
 #define MISA_FORCE_MU(A, M, U)                                                                                \
@@ -1853,14 +1912,14 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
       kind = 2;                                                                                               \
       kForceL<A, M, U><<<persistentGrid(s), kBlockP, lk.bytes, st>>>(                                         \
           s.G, o, t32, x, xn, s.type, s.rec[s.cur], s.rec[1 - s.cur], s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, \
-          sa, s.ctl, iv, lk.mlo, lk.nkn, s.zmeasure ? s.zwork : nullptr);                                     \
+          sa, s.ctl, iv, s.in, lk.mlo, lk.nkn, s.zmeasure ? s.zwork : nullptr);                                     \
     } else if (shared) {                                                                                      \
-      kForceMP<A, M, U><<<4 * grid, kBlock, 0, st>>>(s.G, o, t32, x, xn, s.type, s.rec[s.cur],                \
+      kForceMP<A, M, U><<<grid, kBlock, 0, st>>>(s.G, o, t32, x, xn, s.type, s.rec[s.cur],                \
                                                      s.rec[1 - s.cur], s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, \
-                                                     sa, s.ctl, iv, lk.mlo);                                  \
+                                                     sa, s.ctl, iv, s.in, lk.mlo);                                  \
     } else {                                                                                                  \
       kForceM<A, M, U><<<grid, kBlock, 0, st>>>(s.G, o, t32, x, xn, s.type, s.rec[s.cur], s.rec[1 - s.cur],    \
-                                                s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv,      \
+                                                s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv, s.in, \
                                                 lk.mlo);                                                        \
     }                                                                                                         \
   } while (0)

@@ -27,6 +27,7 @@
 
 #include "device_common.hpp"
 #include "inter_common.hpp"
+#include "inter_step.hpp"
 #include "resident.hpp"
 #include "site_common.hpp"
 
@@ -84,6 +85,14 @@ __device__ int blockScan(int v, int& total) {
   total = wsum[kDT / 64 - 1];
   __syncthreads();
   return before + x - v;
+}
+
+// Reads past the compute unit's cache, for words that other threads of the
+// launch change with atomics (those act on the L2 and leave a cached copy
+// stale).
+template <typename T>
+__device__ __forceinline__ T fresh(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ void setFlag(unsigned long long* f, unsigned long long bit) { atomicOr(f, bit); }
@@ -224,28 +233,25 @@ __device__ __forceinline__ void typeBitsAnd(int8_t* t, int64_t i, int8_t keep) {
   atomicAnd(reinterpret_cast<unsigned*>(a & ~uintptr_t(3)), m);
 }
 
-// Calls fn(t) for neighbour k (-1: the slot itself) of `slot` in the full
-// list when that neighbour is a sub-box site.
-template <typename Fn>
-__device__ __forceinline__ void fullNeighbour(const Geom& G, const FullPlaneOffsets& full, int64_t slot, int k,
-                                              Fn fn) {
+// Neighbour k (-1: the slot itself) of `slot` in the full list when that is a
+// sub-box site, else -1.
+__device__ __forceinline__ int64_t fullNeighbour(const Geom& G, const FullPlaneOffsets& full, int64_t slot, int k) {
   const int par = slot >= G.plane ? 1 : 0;
-  if (k >= full.n[par]) return;
+  if (k >= full.n[par]) return -1;
   const int64_t t = k < 0 ? slot : slot + full.off[par][k];
-  if (t >= 0 && t < 2 * G.plane && isSubBoxSlot(G, t)) fn(t);
+  return t >= 0 && t < 2 * G.plane && isSubBoxSlot(G, t) ? t : -1;
 }
 
-// Calls fn(t) for the sub-box site t that neighbour k (-1: the site itself) of
-// the sub-box site `slot` is, or is a periodic image of: the one sub-box site
-// that the offset reaches from the slot or from one of the slot's images.  An
-// offset is at most the ghost layer long, so every slot it names exists.
-// (Trying the slot and its seven possible images in turn, eight decodes an
-// offset, kFlag took 9.7 us at a few dozen far atoms; now 7.3.)
-template <typename Fn>
-__device__ __forceinline__ void wrappedNeighbour(const Geom& G, const FullPlaneOffsets& full, int64_t slot, int k,
-                                                 Fn fn) {
+// The sub-box site that neighbour k (-1: the site itself) of the sub-box site
+// `slot` is, or is a periodic image of: the one sub-box site that the offset
+// reaches from the slot or from one of the slot's images, or -1.  An offset is
+// at most the ghost layer long, so every slot it names exists.  (Trying the
+// slot and its seven possible images in turn, eight decodes an offset, kFlag
+// took 9.7 us at a few dozen far atoms; now 6.9.)
+__device__ __forceinline__ int64_t wrappedNeighbour(const Geom& G, const FullPlaneOffsets& full, int64_t slot,
+                                                    int k) {
   const int par = slot >= G.plane ? 1 : 0;
-  if (k >= full.n[par]) return;
+  if (k >= full.n[par]) return -1;
   int p, c[3];
   decodeSlot(G, k < 0 ? slot : slot + full.off[par][k], p, c[0], c[1], c[2]);
   const int n[3] = {G.n0, G.n1, G.n2};
@@ -253,9 +259,33 @@ __device__ __forceinline__ void wrappedNeighbour(const Geom& G, const FullPlaneO
   for (int d = 0; d < 3; ++d) {
     if (c[d] < 0) c[d] += n[d];
     else if (c[d] >= n[d]) c[d] -= n[d];
-    if (c[d] < 0 || c[d] >= n[d]) return;  // no image of the slot is that far out
+    if (c[d] < 0 || c[d] >= n[d]) return -1;  // no image of the slot is that far out
   }
-  fn(slotOf(G, p, c[0], c[1], c[2]));
+  return slotOf(G, p, c[0], c[1], c[2]);
+}
+
+// fn(t, type of t) for the sites t = site(slots[e], k) of n slots and their
+// nfull neighbours, four items a thread at a time: an item is a chain of three
+// reads, and one workgroup has few threads to hide them.
+template <typename Site, typename Fn>
+__device__ __forceinline__ void forNeighbourhoods(const int64_t* slots, int n, int nfull, const int8_t* ltype,
+                                                  int64_t t0, int64_t stride, Site site, Fn fn) {
+  const int64_t total = static_cast<int64_t>(n) * nfull;
+  for (int64_t q0 = t0; q0 < total; q0 += 4 * stride) {
+    int64_t t[4];
+    int8_t v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t q = q0 + u * stride;
+      const int64_t e = total < (int64_t(1) << 32) ? static_cast<uint32_t>(q) / static_cast<uint32_t>(nfull) : q / nfull;
+      t[u] = q < total ? site(slots[e], static_cast<int>(q - e * nfull) - 1) : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = t[u] >= 0 ? fresh(ltype + t[u]) : kVacant;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (t[u] >= 0) fn(t[u], v[u]);
+  }
 }
 
 // Far lattice atoms on an eighth of the sites or more (a small box far above
@@ -265,12 +295,13 @@ __device__ __forceinline__ void wrappedNeighbour(const Geom& G, const FullPlaneO
 // before, 10 now).  A site flagged without a far atom around sums the same pairs.
 __device__ __forceinline__ bool farEverywhere(const Geom& G, int64_t nfar) { return 4 * nfar >= G.nsub; }
 template <typename Fn>
-__device__ __forceinline__ void forSubBoxSites(const Geom& G, int64_t t0, int64_t stride, Fn fn) {
+__device__ __forceinline__ void forSubBoxSites(const Geom& G, const int8_t* ltype, int64_t t0, int64_t stride,
+                                               Fn fn) {
   for (int64_t t = t0; t < 2 * G.nsub; t += stride) {
     int64_t s;
     int p, cx, cy, cz;
     siteInOrder(G, t, s, p, cx, cy, cz);
-    fn(s);
+    fn(s, fresh(ltype + s));
   }
 }
 
@@ -289,41 +320,67 @@ __device__ __forceinline__ void unflagBody(const Geom& G, const InterDev& in, in
   const FullPlaneOffsets& full = *in.full;
   const int nfull = 1 + max(full.n[0], full.n[1]);
   for (int64_t q = t0; q < nprev; q += stride) in.head[in.prev_slot[q]] = -1;
-  for (int64_t q = t0; q < static_cast<int64_t>(nprev) * nfull; q += stride) {
-    const int e = static_cast<int>(q / nfull), k = static_cast<int>(q % nfull) - 1;
-    fullNeighbour(G, full, in.prev_slot[e], k, [&](int64_t t) {
-      if (ltype[t] & kNearInter) typeBitsAnd(ltype, t, static_cast<int8_t>(~kNearInter));
-    });
-  }
-  const auto clear = [&](int64_t t) {
-    const int8_t v = ltype[t];
+  const auto wrapped = [&](int64_t slot, int k) { return wrappedNeighbour(G, full, slot, k); };
+  forNeighbourhoods(
+      in.prev_slot, nprev, nfull, ltype, t0, stride,
+      [&](int64_t slot, int k) { return fullNeighbour(G, full, slot, k); },
+      [&](int64_t t, int8_t v) {
+        if (v & kNearInter) typeBitsAnd(ltype, t, static_cast<int8_t>(~kNearInter));
+      });
+  const auto clear = [&](int64_t t, int8_t v) {
     if (!isVacant(v) && (v & kWide)) typeBitsAnd(ltype, t, static_cast<int8_t>(~kWide));
   };
-  if (farEverywhere(G, nfarPrev)) {
-    forSubBoxSites(G, t0, stride, clear);
-  } else {
-    for (int64_t q = t0; q < static_cast<int64_t>(nfarPrev) * nfull; q += stride) {
-      const int e = static_cast<int>(q / nfull), k = static_cast<int>(q % nfull) - 1;
-      wrappedNeighbour(G, full, in.far_prev[e], k, clear);
-    }
-  }
+  if (farEverywhere(G, nfarPrev)) forSubBoxSites(G, ltype, t0, stride, clear);
+  else forNeighbourhoods(in.far_prev, nfarPrev, nfull, ltype, t0, stride, wrapped, clear);
   for (int64_t q = t0; q < nfarPrev; q += stride)
     forSlotAndImages(G, in.far_prev[q], [&](int64_t slot) {
-      const int8_t v = ltype[slot];
+      const int8_t v = fresh(ltype + slot);
       if (!isVacant(v) && (v & kFar)) typeBitsAnd(ltype, slot, static_cast<int8_t>(~kFar));
     });
 }
-__global__ __launch_bounds__(kBlock) void kUnflag(Geom G, InterDev in, int8_t* ltype, const Ctl* ctl) {
-  unflagBody(G, in, ltype, ctl, static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x,
-             static_cast<int64_t>(gridDim.x) * kBlock);
-}
-
 // Priority of a staged atom's claim on a vacated site (above every list
 // index, ordered by the reference index of the site it left), and the stage
-// key of an entry that kQuickRefill has put back.
+// key of an entry that quickRefill has put back.
 constexpr int32_t kStagedPri = 1 << 30;
 constexpr int64_t kQuickDone = (int64_t(1) << 42) - 1;
 constexpr int kQuickBlocks = 128;
+// Boxes of at most so many sites always take the whole decide in one workgroup
+// (their lists are short whatever happens), those up to kDecideAllSites while
+// the lists are short.
+constexpr int64_t kOneGroupSites = 10000;
+constexpr int64_t kDecideAllSites = 100000;
+
+// The counters and the neighbour skin's state at the end of a decide that
+// leaves nl local atoms, ne entries and nfar far lattice atoms.
+__device__ __forceinline__ void finishDecide(const DecideArgs& A, int nl, int ne, int nfar, int staged, int refills,
+                                             int near) {
+  A.ctl->n_inter = nl;
+  A.ctl->n_ghost = ne - nl;
+  A.ctl->n_stage = 0;
+  A.ctl->n_quick = 0;
+  A.ctl->n_prev = ne;
+  A.ctl->n_far_prev = nfar;
+  A.ctl->n_far = 0;
+  A.ctl->staged_total += staged;
+  A.ctl->refill_total += refills;
+  A.ctl->far_total += A.mode == 0 ? nfar : 0;
+  // Neighbour skin of the density pass (both precisions).  Since the last full scan no
+  // lattice atom has moved farther than disp_acc, so no pair has come closer
+  // by more than 2 disp_acc: an offset beyond cutoff + skin for every lane
+  // then is beyond the cutoff now while disp_acc < skin / 2.  A refill puts
+  // a new atom on a site: when it lands farther than 0.2a from the site, its
+  // whole neighbourhood carries kWide, and the wavefronts holding such
+  // sites scan in full and record their masks afresh; any other refill, and
+  // the first force pass after an upload (mode 1), need a full scan of all.
+  Ctl* c = A.ctl;
+  const double acc = c->disp_acc + sqrt(__longlong_as_double(static_cast<long long>(c->dispmax2)));
+  const bool full = A.mode != 0 || !(A.skin > 0.0) || c->rescan != 0 || near > 0 ||
+                    acc >= 0.5 * A.skin - kSkinMargin;
+  c->skin_mode = full ? 0 : 1;
+  c->disp_acc = full ? 0.0 : acc;
+  c->dispmax2 = 0ull;
+  c->rescan = 0;
+}
 
 // Decide, step 2: the list work in one workgroup (the lists hold the
 // interstitials and the atoms that moved more than 0.2a this step: hundreds
@@ -337,21 +394,28 @@ __device__ __forceinline__ void decideBody(const DecideArgs& A) {
   __shared__ int sNear;  // refilled atoms within 0.2a of their site
   __shared__ uint64_t sKeys[kSortLds];
   if (tid == 0) {
-    sFar = static_cast<int>(min(A.ctl->n_far, in.cap));
+    sFar = static_cast<int>(min(fresh(&A.ctl->n_far), in.cap));
     sNear = 0;
   }
   __syncthreads();
   unsigned long long* err = reinterpret_cast<unsigned long long*>(&A.ctl->err_flags);
   int refills = 0, staged = 0;
+  // no inter atom, and every staged atom put back already: the lists stay empty
+  const int64_t quick = A.mode == 0 ? fresh(&A.ctl->n_quick) : 0;
+  if (nl == 0 && (A.mode != 0 || A.ctl->n_stage == quick)) {
+    const int back = static_cast<int>(quick);
+    if (tid == 0) finishDecide(A, 0, 0, min(sFar, static_cast<int>(in.cap)), back, back, 0);
+    return;
+  }
 
   if (A.mode == 0) {
     // P1: append the new inter atoms in the order of the sites they left
     // (atom.cpp:28-53 walks the sub-box z -> y -> x and appends): sort the
     // staged atoms by the reference linear index of their site.  Entries
-    // that kQuickRefill already put back (key kQuickDone) are left out.
+    // that quickRefill already put back (key kQuickDone) are left out.
     const int nsAll = static_cast<int>(min(A.ctl->n_stage, in.cap));
     staged = nsAll;
-    refills = static_cast<int>(A.ctl->n_quick);
+    refills = static_cast<int>(quick);
     int ns = 0;  // the entries still staged, compacted before the sort
     for (int base = 0; base < nsAll; base += kDT) {
       const int i = base + tid;
@@ -398,7 +462,7 @@ __device__ __forceinline__ void decideBody(const DecideArgs& A) {
     __syncthreads();
     for (int i = tid; i < nl; i += kDT) {
       const int t = in.tmp[i];
-      if (t >= 0 && in.site_claim[t] == i) {
+      if (t >= 0 && fresh(&in.site_claim[t]) == i) {
         A.lid[t] = in.id[i];
         A.ltype[t] = in.type[i];
         for (int k = 0; k < 3; k++) {
@@ -531,34 +595,7 @@ __device__ __forceinline__ void decideBody(const DecideArgs& A) {
     in.prev_slot[q] = slot;
   }
   __syncthreads();
-  if (tid == 0) {
-    A.ctl->n_inter = nl;
-    A.ctl->n_ghost = ne - nl;
-    A.ctl->n_stage = 0;
-    A.ctl->n_quick = 0;
-    A.ctl->n_prev = ne;
-    A.ctl->n_far_prev = nfar;
-    A.ctl->n_far = 0;
-    A.ctl->staged_total += staged;
-    A.ctl->refill_total += refills;
-    A.ctl->far_total += A.mode == 0 ? nfar : 0;
-    // Neighbour skin of the density pass (both precisions).  Since the last full scan no
-    // lattice atom has moved farther than disp_acc, so no pair has come closer
-    // by more than 2 disp_acc: an offset beyond cutoff + skin for every lane
-    // then is beyond the cutoff now while disp_acc < skin / 2.  A refill puts
-    // a new atom on a site: when it lands farther than 0.2a from the site, its
-    // whole neighbourhood carries kWide, and the wavefronts holding such
-    // sites scan in full and record their masks afresh; any other refill, and
-    // the first force pass after an upload (mode 1), need a full scan of all.
-    Ctl* c = A.ctl;
-    const double acc = c->disp_acc + sqrt(__longlong_as_double(static_cast<long long>(c->dispmax2)));
-    const bool full = A.mode != 0 || !(A.skin > 0.0) || c->rescan != 0 || sNear > 0 ||
-                      acc >= 0.5 * A.skin - kSkinMargin;
-    c->skin_mode = full ? 0 : 1;
-    c->disp_acc = full ? 0.0 : acc;
-    c->dispmax2 = 0ull;
-    c->rescan = 0;
-  }
+  if (tid == 0) finishDecide(A, nl, ne, nfar, staged, refills, sNear);
 }
 __global__ __launch_bounds__(kDT) void kDecide(DecideArgs A) { decideBody(A); }
 
@@ -575,14 +612,14 @@ __global__ __launch_bounds__(kDT) void kDecide(DecideArgs A) { decideBody(A); }
 // back here with everything decide writes for it (type, id, position,
 // velocity, images, record, the far list); decide skips its stage entry,
 // and its list work, list order and claims come out as before.
-//   kQuickClaim:   a staged atom whose nearest site is its own, with its
-//                  position in the box, opens a claim on that site with its
-//                  priority (kStagedPri + site index);
-//   kQuickCompete: every other entry whose nearest site carries a claim
-//                  lowers it to its own priority (old inter atoms: their
-//                  list index);
-//   kQuickRefill:  a staged atom still holding its site's claim is put back;
-//                  every opened claim is released.
+//   quickClaim:   a staged atom whose nearest site is its own, with its
+//                 position in the box, opens a claim on that site with its
+//                 priority (kStagedPri + site index);
+//   quickCompete: every other entry whose nearest site carries a claim
+//                 lowers it to its own priority (old inter atoms: their
+//                 list index);
+//   quickRefill:  a staged atom still holding its site's claim is put back;
+//                 every opened claim is released.
 
 __device__ __forceinline__ int quickStaged(const InterDev& in, const Ctl* ctl) {
   return static_cast<int>(min(ctl->n_stage, in.cap));
@@ -592,16 +629,16 @@ __device__ __forceinline__ bool ownSiteNearest(const Geom& G, const InterDev& in
   return nearSubBoxSlot(G, y0, y1, y2) == in.stage_slot[i] && outBoxFlags(G, y0, y1, y2) == 0u;
 }
 
-__global__ __launch_bounds__(kBlock) void kQuickClaim(Geom G, InterDev in, const Ctl* ctl) {
+__device__ __forceinline__ void quickClaim(const Geom& G, const InterDev& in, const Ctl* ctl, int t0, int stride) {
   const int ns = quickStaged(in, ctl);
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < ns; i += gridDim.x * kBlock)
+  for (int i = t0; i < ns; i += stride)
     if (ownSiteNearest(G, in, i))
       in.site_claim[in.stage_slot[i]] = kStagedPri + static_cast<int32_t>(in.stage_key[i]);
 }
 
-__global__ __launch_bounds__(kBlock) void kQuickCompete(Geom G, InterDev in, const Ctl* ctl) {
+__device__ __forceinline__ void quickCompete(const Geom& G, const InterDev& in, const Ctl* ctl, int t0, int stride) {
   const int nl = static_cast<int>(ctl->n_inter), ns = quickStaged(in, ctl);
-  for (int q = blockIdx.x * kBlock + threadIdx.x; q < nl + ns; q += gridDim.x * kBlock) {
+  for (int q = t0; q < nl + ns; q += stride) {
     double y0, y1, y2;
     int32_t pri;
     int64_t own = -1;
@@ -619,17 +656,17 @@ __global__ __launch_bounds__(kBlock) void kQuickCompete(Geom G, InterDev in, con
       own = in.stage_slot[i];
     }
     const int64_t t = nearSubBoxSlot(G, y0, y1, y2);
-    if (t >= 0 && t != own && in.site_claim[t] != INT_MAX) atomicMin(&in.site_claim[t], pri);
+    if (t >= 0 && t != own && fresh(&in.site_claim[t]) != INT_MAX) atomicMin(&in.site_claim[t], pri);
   }
 }
 
-__global__ __launch_bounds__(kBlock) void kQuickRefill(DecideArgs A) {
-  InterDev& in = A.in;
+__device__ __forceinline__ void quickRefill(const DecideArgs& A, int t0, int stride) {
+  const InterDev& in = A.in;
   const int ns = quickStaged(in, A.ctl);
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < ns; i += gridDim.x * kBlock) {
+  for (int i = t0; i < ns; i += stride) {
     if (!ownSiteNearest(A.G, in, i)) continue;
     const int64_t t = in.stage_slot[i];
-    if (in.site_claim[t] == kStagedPri + static_cast<int32_t>(in.stage_key[i])) {
+    if (fresh(&in.site_claim[t]) == kStagedPri + static_cast<int32_t>(in.stage_key[i])) {
       const int8_t ty = static_cast<int8_t>(species(in.stage_type[i]));
       A.lid[t] = in.stage_id[i];
       A.ltype[t] = ty;
@@ -649,6 +686,20 @@ __global__ __launch_bounds__(kBlock) void kQuickRefill(DecideArgs A) {
   }
 }
 
+__device__ __forceinline__ int gridThread() { return static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); }
+__device__ __forceinline__ int gridThreads() { return static_cast<int>(gridDim.x * blockDim.x); }
+// The previous index is cleared while the claims are opened: neither reads
+// what the other writes.
+__global__ __launch_bounds__(kBlock) void kUnflagClaim(Geom G, InterDev in, int8_t* ltype, const Ctl* ctl,
+                                                       int quick) {
+  unflagBody(G, in, ltype, ctl, gridThread(), gridThreads());
+  if (quick) quickClaim(G, in, ctl, gridThread(), gridThreads());
+}
+__global__ __launch_bounds__(kBlock) void kQuickCompete(Geom G, InterDev in, const Ctl* ctl) {
+  quickCompete(G, in, ctl, gridThread(), gridThreads());
+}
+__global__ __launch_bounds__(kBlock) void kQuickRefill(DecideArgs A) { quickRefill(A, gridThread(), gridThreads()); }
+
 // Decide, step 3: flag the sub-box sites within the full neighbour list of
 // every entry (kNearInter: their sums visit the inter atoms), and those
 // within the full neighbourhood of every lattice atom farther than 0.2a from
@@ -660,27 +711,21 @@ __device__ __forceinline__ void flagBody(const Geom& G, const InterDev& in, int8
   const int nfar = static_cast<int>(ctl->n_far_prev);
   const FullPlaneOffsets& full = *in.full;
   const int nfull = 1 + max(full.n[0], full.n[1]);
-  for (int64_t q = t0; q < static_cast<int64_t>(ne) * nfull; q += stride) {
-    const int e = static_cast<int>(q / nfull), k = static_cast<int>(q % nfull) - 1;
-    fullNeighbour(G, full, in.e_slot[e], k, [&](int64_t t) {
-      if (!(ltype[t] & kNearInter)) typeBitsOr(ltype, t, kNearInter);
-    });
-  }
-  const auto set = [&](int64_t t) {
-    const int8_t v = ltype[t];
+  const auto wrapped = [&](int64_t slot, int k) { return wrappedNeighbour(G, full, slot, k); };
+  forNeighbourhoods(
+      in.e_slot, ne, nfull, ltype, t0, stride,
+      [&](int64_t slot, int k) { return fullNeighbour(G, full, slot, k); },
+      [&](int64_t t, int8_t v) {
+        if (!(v & kNearInter)) typeBitsOr(ltype, t, kNearInter);
+      });
+  const auto set = [&](int64_t t, int8_t v) {
     if (!isVacant(v) && !(v & kWide)) typeBitsOr(ltype, t, kWide);
   };
-  if (farEverywhere(G, nfar)) {
-    forSubBoxSites(G, t0, stride, set);
-  } else {
-    for (int64_t q = t0; q < static_cast<int64_t>(nfar) * nfull; q += stride) {
-      const int e = static_cast<int>(q / nfull), k = static_cast<int>(q % nfull) - 1;
-      wrappedNeighbour(G, full, in.far_new[e], k, set);
-    }
-  }
+  if (farEverywhere(G, nfar)) forSubBoxSites(G, ltype, t0, stride, set);
+  else forNeighbourhoods(in.far_new, nfar, nfull, ltype, t0, stride, wrapped, set);
   for (int64_t q = t0; q < nfar; q += stride) {
     forSlotAndImages(G, in.far_new[q], [&](int64_t slot) {
-      const int8_t v = ltype[slot];
+      const int8_t v = fresh(ltype + slot);
       if (!isVacant(v) && !(v & kFar)) typeBitsOr(ltype, slot, kFar);
     });
     in.far_prev[q] = in.far_new[q];
@@ -689,6 +734,28 @@ __device__ __forceinline__ void flagBody(const Geom& G, const InterDev& in, int8
 __global__ __launch_bounds__(kBlock) void kFlag(Geom G, InterDev in, int8_t* ltype, const Ctl* ctl) {
   flagBody(G, in, ltype, ctl, static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x,
            static_cast<int64_t>(gridDim.x) * kBlock);
+}
+
+// The whole decide in one workgroup, for boxes of few sites or short lists:
+// launches bound the decide there, and five become one (2 000 cells FP64:
+// 54 -> 38 us a step at rest, 84 -> 73 with some 20 atoms staged a step).  Its
+// loops run over the counts like the grid's, with 1024 threads.
+__global__ __launch_bounds__(kDT) void kDecideAll(DecideArgs A, int quick) {
+  const int tid = threadIdx.x;
+  const bool index = A.ctl->n_prev > 0 || A.ctl->n_far_prev > 0;
+  const bool stage = quick && A.ctl->n_stage > 0;
+  if (index) unflagBody(A.G, A.in, A.ltype, A.ctl, tid, kDT);
+  if (stage) {
+    quickClaim(A.G, A.in, A.ctl, tid, kDT);
+    __syncthreads();
+    quickCompete(A.G, A.in, A.ctl, tid, kDT);
+    __syncthreads();
+    quickRefill(A, tid, kDT);
+  }
+  __syncthreads();
+  decideBody(A);
+  __syncthreads();
+  flagBody(A.G, A.in, A.ltype, A.ctl, tid, kDT);
 }
 
 __global__ void kRescan(Ctl* ctl) { ctl->rescan = 1; }
@@ -711,157 +778,6 @@ __global__ __launch_bounds__(kBlock) void kFarScan(Geom G, CXPtr x, const int8_t
 // per inter atom: rho/F', force + half kick, first half step
 // ---------------------------------------------------------------------------
 
-// Per inter atom one wavefront: lane l takes the sites of full-list items
-// l - 1, l + 63, l + 127, ... (item -1 is the nearest site itself) and the
-// inter atoms in their buckets; the lanes' partial sums then meet in a fixed
-// shuffle tree, so the result does not depend on the launch.
-constexpr int kWaveBlocks = 256;  // blocks of 4 wavefronts, grid-stride over the inter atoms
-
-__device__ __forceinline__ double waveSum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
-// atom::interRho (atom.cpp:194-284): lattice (nearest site, full list), same
-// bucket without itself, then the buckets of the full list; F' at once.
-template <typename T>
-__device__ __forceinline__ void interRhoBody(const Geom& G, const Tables<T>& tb, const InterView& iv, CXPtr lx,
-                                             const int8_t* __restrict__ ltype, const InterDev& in, int w0,
-                                             int wstride) {
-  const int nl = static_cast<int>(iv.ctl->n_inter);
-  const int ne = nl + static_cast<int>(iv.ctl->n_ghost);
-  const FullPlaneOffsets& full = *iv.full;
-  const int lane = threadIdx.x & 63;
-  for (int i = w0; i < nl; i += wstride) {
-    const int64_t n = in.e_slot[i];
-    if (!isSubBoxSlot(G, n)) continue;
-    const double xi0 = in.x[0][i], xi1 = in.x[1][i], xi2 = in.x[2][i];
-    const uint64_t myid = in.id[i];
-    const int par = n >= G.plane ? 1 : 0;
-    double rho = 0.0;
-    for (int k = lane - 1; k < full.n[par]; k += 64) {
-      const int64_t j = k < 0 ? n : n + full.off[par][k];
-      const int8_t tj = ltype[j];
-      if (!isVacant(tj)) {
-        const double d0 = xi0 - lx.c[0][j], d1 = xi1 - lx.c[1][j], d2 = xi2 - lx.c[2][j];
-        const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-        if (r2 < G.rc2) rho += rhoPair(tb, species(tj), r2);
-      }
-      forBucket(iv, j, ne, [&](int e) {
-        const int src = iv.e_src[e];
-        if (k < 0 && e < nl && iv.id[src] == myid) return;  // itself (ghost images carry no id)
-        const double d0 = xi0 - iv.e_x[0][e], d1 = xi1 - iv.e_x[1][e], d2 = xi2 - iv.e_x[2][e];
-        const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-        if (r2 < G.rc2) rho += rhoPair(tb, species(iv.type[src]), r2);
-      });
-    }
-    rho = waveSum(rho);
-    if (lane == 0) {
-      in.rho[i] = rho;
-      checkRho(iv.ctl, rho, static_cast<double>(tb.rhomax));
-      const T dfi = dEmbed(tb, species(in.type[i]), static_cast<T>(rho));
-      if constexpr (sizeof(T) == 8)
-        in.df64[i] = dfi;
-      else
-        in.df32[i] = dfi;
-    }
-  }
-}
-template <typename T>
-__global__ __launch_bounds__(kIT) void kInterRho(Geom G, Tables<T> tb, InterView iv, CXPtr lx,
-                                                 const int8_t* __restrict__ ltype, InterDev in) {
-  interRhoBody<T>(G, tb, iv, lx, ltype, in, blockIdx.x * (kIT / 64) + static_cast<int>(threadIdx.x >> 6),
-                  kWaveBlocks * (kIT / 64));
-}
-
-// atom::interForce (atom.cpp:360-473) + secondstep for the inter list.
-template <typename T, int MODE>
-__device__ __forceinline__ void interForceBody(const Geom& G, const Tables<T>& tb, const InterView& iv, CXPtr lx,
-                                               const int8_t* __restrict__ ltype, const T* __restrict__ ldf,
-                                               int ldfStride, const InterDev& in, const VerletParams& vp, int w0,
-                                               int wstride) {
-  const int nl = static_cast<int>(iv.ctl->n_inter);
-  const int ne = nl + static_cast<int>(iv.ctl->n_ghost);
-  const FullPlaneOffsets& full = *iv.full;
-  const int lane = threadIdx.x & 63;
-  for (int i = w0; i < nl; i += wstride) {
-    const int64_t n = in.e_slot[i];
-    double f0 = 0, f1 = 0, f2 = 0;
-    const int ei = species(in.type[i]);
-    if (isSubBoxSlot(G, n)) {
-      const double xi0 = in.x[0][i], xi1 = in.x[1][i], xi2 = in.x[2][i];
-      const uint64_t myid = in.id[i];
-      const T dfi = dfOf<T>(iv, i);
-      const int par = n >= G.plane ? 1 : 0;
-      for (int k = lane - 1; k < full.n[par]; k += 64) {
-        const int64_t j = k < 0 ? n : n + full.off[par][k];
-        const int8_t tj = ltype[j];
-        {
-          const double d0 = xi0 - lx.c[0][j], d1 = xi1 - lx.c[1][j], d2 = xi2 - lx.c[2][j];
-          const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-          if (r2 < G.rc2 && !isVacant(tj)) {
-            const double fp = static_cast<double>(pairForce(tb, ei, species(tj), r2, dfi, ldf[j * ldfStride]));
-            f0 += d0 * fp;
-            f1 += d1 * fp;
-            f2 += d2 * fp;
-          }
-        }
-        forBucket(iv, j, ne, [&](int e) {
-          const int src = iv.e_src[e];
-          if (k < 0 && e < nl && iv.id[src] == myid) return;
-          const double d0 = xi0 - iv.e_x[0][e], d1 = xi1 - iv.e_x[1][e], d2 = xi2 - iv.e_x[2][e];
-          const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-          if (r2 < G.rc2) {
-            const double fp =
-                static_cast<double>(pairForce(tb, ei, species(iv.type[src]), r2, dfi, dfOf<T>(iv, src)));
-            f0 += d0 * fp;
-            f1 += d1 * fp;
-            f2 += d2 * fp;
-          }
-        });
-      }
-      f0 = waveSum(f0);
-      f1 = waveSum(f1);
-      f2 = waveSum(f2);
-    }
-    if (lane == 0) {
-      checkFinite(iv.ctl, f0, f1, f2);
-      in.f[0][i] = f0;
-      in.f[1][i] = f1;
-      in.f[2][i] = f2;
-      if (MODE == 0) {  // secondstep, each product and sum rounded separately
-#pragma clang fp contract(off)
-        const double c = stepDt(vp, ei).c;
-        in.v[0][i] += c * f0;
-        in.v[1][i] += c * f1;
-        in.v[2][i] += c * f2;
-      }
-    }
-  }
-}
-template <typename T, int MODE>
-__global__ __launch_bounds__(kIT) void kInterForce(Geom G, Tables<T> tb, InterView iv, CXPtr lx,
-                                                   const int8_t* __restrict__ ltype, const T* __restrict__ ldf,
-                                                   int ldfStride, InterDev in, VerletParams vp) {
-  interForceBody<T, MODE>(G, tb, iv, lx, ltype, ldf, ldfStride, in, vp,
-                          blockIdx.x * (kIT / 64) + static_cast<int>(threadIdx.x >> 6), kWaveBlocks * (kIT / 64));
-}
-
-// NewtonMotion::firststep for the inter list (newton_motion.cpp:46-54).
-__device__ __forceinline__ void interFirstBody(const InterDev& in, const Ctl* ctl, const VerletParams& vp, int i0,
-                                               int istride) {
-#pragma clang fp contract(off)  // the half kick and drift round as newton_motion.cpp does
-  const int nl = static_cast<int>(ctl->n_inter);
-  for (int i = i0; i < nl; i += istride) {
-    const StepDt sd = stepDt(vp, species(in.type[i]));
-    const double c = sd.c;
-    for (int d = 0; d < 3; d++) {
-      const double v = in.v[d][i] + c * in.f[d][i];
-      in.v[d][i] = v;
-      in.x[d][i] += sd.dt * v;
-    }
-  }
-}
 __global__ __launch_bounds__(kIT) void kInterFirst(InterDev in, const Ctl* ctl, VerletParams vp) {
   interFirstBody(in, ctl, vp, blockIdx.x * kIT + threadIdx.x, kIT * kIB);
 }
@@ -1053,22 +969,35 @@ __global__ __launch_bounds__(kBlock) void kVmaxSites(Geom G, CXPtr v, const int8
   blockMaxToCtl<kBlock>(m, ctl);
 }
 
-__global__ __launch_bounds__(kIT) void kVmaxInter(InterDev in, Ctl* ctl) {
-  const int nl = static_cast<int>(ctl->n_inter);
+// The inter atoms' part of the maximum, the step length from it, and their
+// first half step with that length, in one workgroup: three launches of a few
+// microseconds each otherwise, for lists of a few hundred atoms.
+__global__ __launch_bounds__(kDT) void kDtInter(InterDev in, Ctl* ctl, double dt_max, double max_disp,
+                                                VerletParams vp) {
+  __shared__ unsigned long long red[kDT / 64];
+  const int nl = static_cast<int>(ctl->n_inter), tid = threadIdx.x;
   unsigned long long m = 0;
-  for (int i = blockIdx.x * kIT + threadIdx.x; i < nl; i += kIT * kIB) {
+  for (int i = tid; i < nl; i += kDT) {
     const unsigned long long b = speed2Bits(in.v[0][i], in.v[1][i], in.v[2][i]);
     m = b > m ? b : m;
   }
-  blockMaxToCtl<kIT>(m, ctl);
-}
-
-__global__ void kDtUpdate(Ctl* ctl, double dt_max, double max_disp) {
-  const double vmax = sqrt(__longlong_as_double(static_cast<long long>(ctl->vmax2)));
-  const double dt = vmax > 0.0 ? fmin(dt_max, max_disp / vmax) : dt_max;
-  ctl->dt = dt;
-  ctl->t_sim += dt;
-  ctl->vmax2 = 0ull;
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long y = __shfl_xor(m, o, 64);
+    m = y > m ? y : m;
+  }
+  if ((tid & 63) == 0) red[tid >> 6] = m;
+  __syncthreads();
+  if (tid == 0) {
+    m = ctl->vmax2;  // the lattice sites'
+    for (int k = 0; k < kDT / 64; k++) m = red[k] > m ? red[k] : m;
+    const double vmax = sqrt(__longlong_as_double(static_cast<long long>(m)));
+    const double dt = vmax > 0.0 ? fmin(dt_max, max_disp / vmax) : dt_max;
+    ctl->dt = dt;
+    ctl->t_sim += dt;
+    ctl->vmax2 = 0ull;
+  }
+  __syncthreads();
+  interFirstBody(in, ctl, vp, tid, kDT);
 }
 
 // ---------------------------------------------------------------------------
@@ -1076,16 +1005,17 @@ __global__ void kDtUpdate(Ctl* ctl, double dt_max, double max_disp) {
 // blocks per box, or one workgroup per box for the list work)
 // ---------------------------------------------------------------------------
 constexpr int kBatchBlocks = 8;
+constexpr int kBatchFlagBlocks = 32;  // of the flag kernels: a hot box has hundreds of entries with 229 sites each
 
 __global__ __launch_bounds__(kBlock) void kUnflagB(const BatchBox* __restrict__ boxes) {
-  const BatchBox& B = boxes[blockIdx.x / kBatchBlocks];
-  unflagBody(B.G, B.in, B.type, B.ctl, static_cast<int64_t>(blockIdx.x % kBatchBlocks) * kBlock + threadIdx.x,
-             static_cast<int64_t>(kBatchBlocks) * kBlock);
+  const BatchBox& B = boxes[blockIdx.x / kBatchFlagBlocks];
+  unflagBody(B.G, B.in, B.type, B.ctl, static_cast<int64_t>(blockIdx.x % kBatchFlagBlocks) * kBlock + threadIdx.x,
+             static_cast<int64_t>(kBatchFlagBlocks) * kBlock);
 }
 __global__ __launch_bounds__(kBlock) void kFlagB(const BatchBox* __restrict__ boxes) {
-  const BatchBox& B = boxes[blockIdx.x / kBatchBlocks];
-  flagBody(B.G, B.in, B.type, B.ctl, static_cast<int64_t>(blockIdx.x % kBatchBlocks) * kBlock + threadIdx.x,
-           static_cast<int64_t>(kBatchBlocks) * kBlock);
+  const BatchBox& B = boxes[blockIdx.x / kBatchFlagBlocks];
+  flagBody(B.G, B.in, B.type, B.ctl, static_cast<int64_t>(blockIdx.x % kBatchFlagBlocks) * kBlock + threadIdx.x,
+           static_cast<int64_t>(kBatchFlagBlocks) * kBlock);
 }
 // args[2 b + flip]: the decide arguments of box b for either buffer
 __global__ __launch_bounds__(kDT) void kDecideB(const DecideArgs* __restrict__ args, int flip) {
@@ -1102,17 +1032,11 @@ __global__ __launch_bounds__(kIT) void kInterForceB(const BatchBox* __restrict__
   const BatchBox& B = boxes[blockIdx.x / kBatchBlocks];
   const int c = B.cur ^ flip;
   const float* ldf = reinterpret_cast<const float*>(B.rec[c]) + 3;  // lattice F' is the w of the records
-  interForceBody<float, 0>(B.G, B.t32, B.iv, cxp(B.x[c]), B.type, ldf, 4, B.in, B.vp,
+  interForceBody<float, 1>(B.G, B.t32, B.iv, cxp(B.x[c]), B.type, ldf, 4, B.in, B.vp,
                            static_cast<int>(blockIdx.x % kBatchBlocks) * (kIT / 64) +
                                static_cast<int>(threadIdx.x >> 6),
                            kBatchBlocks * (kIT / 64));
 }
-__global__ __launch_bounds__(kIT) void kInterFirstB(const BatchBox* __restrict__ boxes) {
-  const BatchBox& B = boxes[blockIdx.x / kBatchBlocks];
-  interFirstBody(B.in, B.ctl, B.vp, static_cast<int>(blockIdx.x % kBatchBlocks) * kIT + threadIdx.x,
-                 kBatchBlocks * kIT);
-}
-
 }  // namespace
 
 size_t decideArgsBytes() { return sizeof(DecideArgs); }
@@ -1137,23 +1061,22 @@ void fillDecideArgs(const BatchBox& b, int c, void* out) {
 }
 
 void launchInterBatch(int which, const BatchBox* boxes, int nbox, int flip, const void* decideArgs, hipStream_t st) {
-  const unsigned g = static_cast<unsigned>(nbox * kBatchBlocks);
+  const unsigned g = static_cast<unsigned>(nbox * kBatchBlocks), gf = static_cast<unsigned>(nbox * kBatchFlagBlocks);
   switch (which) {
     case 0: kInterRhoB<<<g, kIT, 0, st>>>(boxes, flip); break;
     case 1: kInterForceB<<<g, kIT, 0, st>>>(boxes, flip); break;
-    case 2: kInterFirstB<<<g, kIT, 0, st>>>(boxes); break;
     default:  // the decide of every box, on buffer cur ^ flip
-      kUnflagB<<<g, kBlock, 0, st>>>(boxes);
+      kUnflagB<<<gf, kBlock, 0, st>>>(boxes);
       kDecideB<<<static_cast<unsigned>(nbox), kDT, 0, st>>>(static_cast<const DecideArgs*>(decideArgs), flip);
-      kFlagB<<<g, kBlock, 0, st>>>(boxes);
+      kFlagB<<<gf, kBlock, 0, st>>>(boxes);
       break;
   }
 }
 
-void launchAdaptiveDt(const DevState& s, double dt_max, double max_disp, bool sites, hipStream_t st) {
+void launchAdaptiveDt(const DevState& s, double dt_max, double max_disp, bool sites, const VerletParams& vp,
+                      hipStream_t st) {
   if (sites) kVmaxSites<<<kVmaxBlocks, kBlock, 0, st>>>(s.G, cxp(s.v), s.type, s.ctl);
-  kVmaxInter<<<kIB, kIT, 0, st>>>(s.in, s.ctl);
-  kDtUpdate<<<1, 1, 0, st>>>(s.ctl, dt_max, max_disp);
+  kDtInter<<<1, kDT, 0, st>>>(s.in, s.ctl, dt_max, max_disp, vp);
 }
 
 InterView interView(const DevState& s, bool mixed) {
@@ -1176,7 +1099,13 @@ void launchFarScan(const DevState& s, hipStream_t st) {
   kFarScan<<<siteGrid(s.G), kBlock, 0, st>>>(s.G, cxp(s.x[s.cur]), s.type, s.in, s.ctl);
 }
 
-void launchDecide(const DevState& s, int mode, bool mixed, hipStream_t st) {
+DecideForm decideBySize(const DevState& s) {
+  return 2 * s.G.nsub <= kOneGroupSites    ? DecideForm::oneGroup
+         : 2 * s.G.nsub <= kDecideAllSites ? DecideForm::byLists
+                                           : DecideForm::grid;
+}
+
+void launchDecide(const DevState& s, int mode, bool mixed, bool few, hipStream_t st) {
   DecideArgs A;
   A.G = s.G;
   A.mode = mode;
@@ -1192,9 +1121,14 @@ void launchDecide(const DevState& s, int mode, bool mixed, hipStream_t st) {
   A.in = s.in;
   A.ctl = s.ctl;
   A.skin = s.skin;
-  kUnflag<<<kFlagBlocks, kBlock, 0, st>>>(s.G, s.in, s.type, s.ctl);
-  if (mode == 0 && 2 * s.G.plane < kStagedPri) {  // site indices below the staged priority offset
-    kQuickClaim<<<kQuickBlocks, kBlock, 0, st>>>(s.G, s.in, s.ctl);
+  const int quick = mode == 0 && 2 * s.G.plane < kStagedPri;  // site indices below the staged priority offset
+  const DecideForm form = decideBySize(s);
+  if (form == DecideForm::oneGroup || (form == DecideForm::byLists && few)) {
+    kDecideAll<<<1, kDT, 0, st>>>(A, quick);
+    return;
+  }
+  kUnflagClaim<<<kFlagBlocks, kBlock, 0, st>>>(s.G, s.in, s.type, s.ctl, quick);
+  if (quick) {
     kQuickCompete<<<kQuickBlocks, kBlock, 0, st>>>(s.G, s.in, s.ctl);
     kQuickRefill<<<kQuickBlocks, kBlock, 0, st>>>(A);
   }
@@ -1203,33 +1137,6 @@ void launchDecide(const DevState& s, int mode, bool mixed, hipStream_t st) {
 }
 
 void launchRescan(const DevState& s, hipStream_t st) { kRescan<<<1, 1, 0, st>>>(s.ctl); }
-
-void launchInterRho(const DevState& s, const Tables<double>& t64, const Tables<float>& t32, bool mixed,
-                    hipStream_t st) {
-  const InterView iv = interView(s, mixed);
-  if (mixed)
-    kInterRho<float><<<kWaveBlocks, kIT, 0, st>>>(s.G, t32, iv, cxp(s.x[s.cur]), s.type, s.in);
-  else
-    kInterRho<double><<<kWaveBlocks, kIT, 0, st>>>(s.G, t64, iv, cxp(s.x[s.cur]), s.type, s.in);
-}
-
-void launchInterForce(const DevState& s, const Tables<double>& t64, const Tables<float>& t32, bool mixed, int mode,
-                      const VerletParams& vp, hipStream_t st) {
-  const InterView iv = interView(s, mixed);
-  const CXPtr lx = cxp(s.x[s.cur]);
-  if (mixed) {  // lattice F' is the w component of the site records
-    const float* ldf = reinterpret_cast<const float*>(s.rec[s.cur]) + 3;
-    if (mode == 0)
-      kInterForce<float, 0><<<kWaveBlocks, kIT, 0, st>>>(s.G, t32, iv, lx, s.type, ldf, 4, s.in, vp);
-    else
-      kInterForce<float, 2><<<kWaveBlocks, kIT, 0, st>>>(s.G, t32, iv, lx, s.type, ldf, 4, s.in, vp);
-  } else {
-    if (mode == 0)
-      kInterForce<double, 0><<<kWaveBlocks, kIT, 0, st>>>(s.G, t64, iv, lx, s.type, s.df64, 1, s.in, vp);
-    else
-      kInterForce<double, 2><<<kWaveBlocks, kIT, 0, st>>>(s.G, t64, iv, lx, s.type, s.df64, 1, s.in, vp);
-  }
-}
 
 void launchInterFirst(const DevState& s, const VerletParams& vp, hipStream_t st) {
   kInterFirst<<<kIB, kIT, 0, st>>>(s.in, s.ctl, vp);

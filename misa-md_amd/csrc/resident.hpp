@@ -119,6 +119,10 @@ struct VerletParams {
 void launchUpload(const DevState& s, const AtomElement* aos_dev, int64_t sx, int64_t sy, hipStream_t st);
 void launchDownload(const DevState& s, AtomElement* aos_dev, int64_t sx, int64_t sy, bool mixed, hipStream_t st);
 void launchHaloAll(const DevState& s, int buf, hipStream_t st);
+// The density pass of the inter atoms and the lattice in one launch, and the
+// force pass of both.  Force modes: 0 f stored, v += c f (secondstep); 1 and
+// the next first half step (for the lattice with the decide's staging); 2 f
+// stored only.
 void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
                  bool mixed, int acc, bool store_rho, hipStream_t st);
 // Returns the force pass launched: 0 kForce (FP64), 1 kForceM, 2 kForceL (the
@@ -143,24 +147,24 @@ void launchScaleV(const DevState& s, double factor, hipStream_t st);
 // Adaptive step: max |v|^2 over lattice and inter atoms into Ctl::vmax2, then
 // Ctl::dt = min(dt_max, max_disp / max|v|) and Ctl::t_sim += Ctl::dt; with
 // sites false the lattice sites' maximum is already in Ctl::vmax2 (reduced
-// by the secondstep pass).
-void launchAdaptiveDt(const DevState& s, double dt_max, double max_disp, bool sites, hipStream_t st);
+// by the secondstep pass); then the inter atoms' first half step.
+void launchAdaptiveDt(const DevState& s, double dt_max, double max_disp, bool sites, const VerletParams& vp,
+                      hipStream_t st);
 // Inter-atom work (kernels_inter.hip).
 // decide mode 0: the step's ownership pass (append new inter atoms, vacancy
 // recombination, migration, ghost images, index, flags); mode 1: migration,
 // ghost images, index and flags only (first force, PKA step, upload).
-void launchDecide(const DevState& s, int mode, bool mixed, hipStream_t st);
+// The small boxes' decide is one workgroup's work, the large ones' a grid's;
+// between them it depends on the lists, which the caller has seen (few).
+enum class DecideForm { oneGroup, byLists, grid };
+DecideForm decideBySize(const DevState& s);
+void launchDecide(const DevState& s, int mode, bool mixed, bool few, hipStream_t st);
 // Ask the next decide for a full scan of the mixed density pass.
 void launchRescan(const DevState& s, hipStream_t st);
 InterView interView(const DevState& s, bool mixed);
 // Lattice atoms farther than 0.2a from their site -> far list (before a
 // mode-1 decide; in a step only refilled vacancies can be far).
 void launchFarScan(const DevState& s, hipStream_t st);
-void launchInterRho(const DevState& s, const Tables<double>& t64, const Tables<float>& t32, bool mixed,
-                    hipStream_t st);
-// mode 0: f stored, v += c f (secondstep); mode 2: f stored only
-void launchInterForce(const DevState& s, const Tables<double>& t64, const Tables<float>& t32, bool mixed, int mode,
-                      const VerletParams& vp, hipStream_t st);
 void launchInterFirst(const DevState& s, const VerletParams& vp, hipStream_t st);
 void launchInterUpload(const DevState& s, const AtomElement* aos_dev, int64_t n, hipStream_t st);
 void launchInterDownload(const DevState& s, AtomElement* aos_dev, bool mixed, hipStream_t st);
@@ -176,8 +180,8 @@ void launchSetv(const DevState& s, int64_t slot, double dv0, double dv1, double 
 namespace site {
 struct BatchBox;
 }
-// Inter-atom work of every box: 0 density and F', 1 force and half kick,
-// 2 first half step, 3 the decide (clear flags, list work, set flags) on
+// Inter-atom work of every box: 0 density and F', 1 force, half kick and the
+// next first half step, 2 the decide (clear flags, list work, set flags) on
 // buffer cur ^ flip, with decideArgs holding two records per box (for
 // either buffer) of decideArgsBytes() each, filled by fillDecideArgs.
 size_t decideArgsBytes();
