@@ -11,6 +11,7 @@
 #include "../../include/misa_eam.h"
 #include "device_common.hpp"
 #include "hook.hpp"
+#include "host_copy.hpp"
 #include "host_setup.hpp"
 #include "resident.hpp"
 #include "site_common.hpp"
@@ -18,6 +19,7 @@
 using namespace misa;
 
 struct misa_handle {
+  misa::StageUser stage_user;
   std::string err;
   int device = 0;
   hipStream_t stream = nullptr;
@@ -704,8 +706,7 @@ static int hookCall(misa_handle* h, int which, void* atoms, double rc) {
   HIPCHECK(h, hipMemcpyAsync(h->aos_dev, atoms, bytes, hipMemcpyHostToDevice, h->stream));
   launchHook(which, h->box, rc, h->full, h->t64, h->aos_dev, h->stream);
   HIPCHECK(h, hipGetLastError());
-  HIPCHECK(h, hipMemcpyAsync(atoms, h->aos_dev, bytes, hipMemcpyDeviceToHost, h->stream));
-  HIPCHECK(h, hipStreamSynchronize(h->stream));
+  HIPCHECK(h, copyToHost(atoms, h->aos_dev, bytes, h->stream));
   return MISA_OK;
 }
 
@@ -791,7 +792,7 @@ int misa_download_state(misa_handle* h, void* atoms, void* inter, int64_t inter_
   if (!h->aos_dev) HIPCHECK(h, hipMalloc(&h->aos_dev, bytes));
   launchDownload(h->s, h->aos_dev, b.sx, b.sy, mixed, h->stream);
   HIPCHECK(h, hipGetLastError());
-  HIPCHECK(h, hipMemcpyAsync(atoms, h->aos_dev, bytes, hipMemcpyDeviceToHost, h->stream));
+  HIPCHECK(h, copyToHost(atoms, h->aos_dev, bytes, h->stream));
   Ctl c;
   HIPCHECK(h, hipMemcpyAsync(&c, h->s.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, h->stream));
   HIPCHECK(h, hipStreamSynchronize(h->stream));

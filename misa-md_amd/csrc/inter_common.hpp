@@ -107,7 +107,7 @@ __device__ __forceinline__ int64_t nearSubBoxSlot(const Geom& G, double x0, doub
 
 __device__ __forceinline__ void decodeSlot(const Geom& G, int64_t slot, int& p, int& cx, int& cy, int& cz) {
   p = slot >= G.plane ? 1 : 0;
-  // 32-bit divisions: a plane of 2^32 slots would not fit in memory
+  // 32-bit divisions: a handle holds fewer than 2^27 slots
   const uint32_t r = static_cast<uint32_t>(slot - p * G.plane), NX = static_cast<uint32_t>(G.NX);
   const uint32_t row = r / NX, NY = static_cast<uint32_t>(G.NY), z = row / NY;
   cx = static_cast<int>(r - row * NX) - G.g;
