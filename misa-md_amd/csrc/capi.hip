@@ -28,7 +28,6 @@ struct misa_handle {
   Offsets ref{};
   bool have_offsets = false;
   LatOffsets lat{};
-  FullOffsets full{};
   FullPlaneOffsets fullPlane{};
   float4 dlHost[2 * kMaxLatOffsets]{};  // lattice vectors of the pruned offsets (mixed records)
   void* interBlock = nullptr;  // one allocation carved into the inter-atom arrays
@@ -110,13 +109,11 @@ int buildPlaneOffsets(misa_handle* h) {
     const std::vector<int64_t>& L = p == 0 ? h->ref.even : h->ref.odd;
     if (static_cast<int>(L.size()) > kMaxFullOffsets) return fail(h, MISA_E_ARG, "offset list too long");
     int nl = 0, nw = 0;
-    h->full.n[p] = static_cast<int>(L.size());
     for (size_t k = 0; k < L.size(); k++) {
       PlaneOffset po;
       if (!decodeOffset(b, p, L[k], po)) return fail(h, MISA_E_ARG, "offset does not decode to a lattice neighbour");
       if (std::abs(po.dcx) > b.g || std::abs(po.dy) > b.g || std::abs(po.dz) > b.g)
         return fail(h, MISA_E_ARG, "offset reaches beyond the ghost layer");
-      h->full.off[p][k] = static_cast<int32_t>(L[k]);
       {
         const int64_t NX = b.n[0] + 2 * b.g, NY = b.n[1] + 2 * b.g, NZ = b.n[2] + 2 * b.g;
         h->fullPlane.off[p][k] =
@@ -697,6 +694,9 @@ int misa_get_potential_table(const misa_handle* h, int kind, int idx, double* ou
   return MISA_OK;
 }
 
+// The records of the buffer that the next step writes, as a hook's scratch.
+static site::Rec64 hookRecs(const misa_handle* h) { return site::Rec64{h->s.pxy[1 - h->s.cur], h->s.pzw[1 - h->s.cur]}; }
+
 static int hookCall(misa_handle* h, int which, void* atoms, double rc) {
   if (!h || !atoms) return MISA_E_ARG;
   if (!h->have_offsets || !h->have_pot) return fail(h, MISA_E_ARG, "offsets and potential must be set first");
@@ -704,7 +704,7 @@ static int hookCall(misa_handle* h, int which, void* atoms, double rc) {
   const size_t bytes = static_cast<size_t>(h->box.slots()) * sizeof(AtomElement);
   if (!h->aos_dev) HIPCHECK(h, hipMalloc(&h->aos_dev, bytes));
   HIPCHECK(h, hipMemcpyAsync(h->aos_dev, atoms, bytes, hipMemcpyHostToDevice, h->stream));
-  launchHook(which, h->box, rc, h->full, h->t64, h->aos_dev, h->stream);
+  launchHook(which, h->box, rc, h->s.in.full, h->t64, hookRecs(h), h->aos_dev, h->stream);
   HIPCHECK(h, hipGetLastError());
   HIPCHECK(h, copyToHost(atoms, h->aos_dev, bytes, h->stream));
   return MISA_OK;
@@ -724,7 +724,7 @@ int misa_lat_hook_noalloc(misa_handle* h, int which, void* atoms, double rc) {
   AtomElement* a = static_cast<AtomElement*>(stage);
   // the whole array is overwritten by the copy: nothing in it needs clearing
   HIPCHECK(h, hipMemcpyAsync(a, atoms, bytes, hipMemcpyHostToDevice, h->stream));
-  launchHook(which, h->box, rc, h->full, h->t64, a, h->stream);
+  launchHook(which, h->box, rc, h->s.in.full, h->t64, hookRecs(h), a, h->stream);
   HIPCHECK(h, hipGetLastError());
   HIPCHECK(h, hipMemcpyAsync(atoms, a, bytes, hipMemcpyDeviceToHost, h->stream));
   HIPCHECK(h, hipStreamSynchronize(h->stream));

@@ -1,23 +1,17 @@
-// Hook-mode launcher and the reference offset lists it walks.
+// Hook-mode launcher.
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <cstdint>
-
 #include "device_common.hpp"
 #include "host_setup.hpp"
+#include "inter_common.hpp"
+#include "site_common.hpp"
 
 namespace misa {
 
-// The reference's full lists (even x, odd x) as linear offsets into the
-// ghost-extended doubled-x array.
-struct FullOffsets {
-  int n[2];
-  int32_t off[2][kMaxFullOffsets];
-};
-
-// which: 0 rho, 1 df, 2 force
-void launchHook(int which, const Box& b, double rc, const FullOffsets& o, const Tables<double>& tb, AtomElement* a,
-                hipStream_t st);
+// which: 0 rho, 1 df, 2 force.  full: the handle's full lists on the device;
+// rec: scratch for a record per slot.
+void launchHook(int which, const Box& b, double rc, const FullPlaneOffsets* full, const Tables<double>& tb, site::Rec64 rec,
+                AtomElement* a, hipStream_t st);
 
 }  // namespace misa
