@@ -233,12 +233,13 @@ void makeWalk(Geom& G) {
   evenSlabs(G);
 }
 
-// A box of up to kDecideAllSites sites takes its decide in one workgroup
-// while at most kFewListed inter atoms, images and far atoms are listed: five
-// launches, some 2 us each, become one (16 000 cells FP64 at rest: 48 -> 41 us
-// a step).  A list of thousands wants the grid (the same box with 10 000 far
-// atoms: 86 us a step with it, 300 us without).
-constexpr int64_t kFewListed = 64;
+// A box of few sites (decideInOneGroup) takes its decide in one workgroup while
+// at most kFewListed inter atoms, images and far atoms are listed: five
+// launches, some 2 us each, become one (16 000 atoms FP64 at rest: 48 -> 41 us
+// a step).  Longer lists want the grid: level at some 50 entries, 86 us a step
+// against 146 at 2 000, 86 against 300 at 10 000.  Lists grow that long in any
+// box whose crystal drifts off its sites.
+constexpr int64_t kFewListed = 32;
 constexpr int64_t kLookSteps = 128;  // steps between two looks at the lists
 bool fewListed(const Ctl& c) { return c.n_prev + c.n_far_prev <= kFewListed; }
 
@@ -1103,7 +1104,7 @@ int misa_step(misa_handle* h, int64_t nsteps) {
   if (nsteps == 0) return MISA_OK;
   HIPCHECK(h, hipSetDevice(h->device));
   StepPlan p = planOf(h);
-  const bool look = decideBySize(h->s) == DecideForm::byLists;
+  const bool look = decideInOneGroup(h->s);
   p.few = look && h->few_listed;
   clearEvents(h);
   hipEvent_t e0, e1;

@@ -344,10 +344,8 @@ __device__ __forceinline__ void unflagBody(const Geom& G, const InterDev& in, in
 constexpr int32_t kStagedPri = 1 << 30;
 constexpr int64_t kQuickDone = (int64_t(1) << 42) - 1;
 constexpr int kQuickBlocks = 128;
-// Boxes of at most so many sites always take the whole decide in one workgroup
-// (their lists are short whatever happens), those up to kDecideAllSites while
-// the lists are short.
-constexpr int64_t kOneGroupSites = 10000;
+// Boxes of at most so many sites take the whole decide in one workgroup while
+// the lists are short; in larger ones the launches it saves are below 1 % of a step.
 constexpr int64_t kDecideAllSites = 100000;
 
 // The counters and the neighbour skin's state at the end of a decide that
@@ -736,9 +734,9 @@ __global__ __launch_bounds__(kBlock) void kFlag(Geom G, InterDev in, int8_t* lty
            static_cast<int64_t>(gridDim.x) * kBlock);
 }
 
-// The whole decide in one workgroup, for boxes of few sites or short lists:
-// launches bound the decide there, and five become one (2 000 cells FP64:
-// 54 -> 38 us a step at rest, 84 -> 73 with some 20 atoms staged a step).  Its
+// The whole decide in one workgroup, for short lists in boxes of few sites:
+// launches bound the decide there, and five become one (2 000 atoms FP64: 54 ->
+// 38 us a step at rest, 84 -> 73 with some 20 atoms staged a step).  Its
 // loops run over the counts like the grid's, with 1024 threads.
 __global__ __launch_bounds__(kDT) void kDecideAll(DecideArgs A, int quick) {
   const int tid = threadIdx.x;
@@ -1099,11 +1097,7 @@ void launchFarScan(const DevState& s, hipStream_t st) {
   kFarScan<<<siteGrid(s.G), kBlock, 0, st>>>(s.G, cxp(s.x[s.cur]), s.type, s.in, s.ctl);
 }
 
-DecideForm decideBySize(const DevState& s) {
-  return 2 * s.G.nsub <= kOneGroupSites    ? DecideForm::oneGroup
-         : 2 * s.G.nsub <= kDecideAllSites ? DecideForm::byLists
-                                           : DecideForm::grid;
-}
+bool decideInOneGroup(const DevState& s) { return 2 * s.G.nsub <= kDecideAllSites; }
 
 void launchDecide(const DevState& s, int mode, bool mixed, bool few, hipStream_t st) {
   DecideArgs A;
@@ -1122,8 +1116,7 @@ void launchDecide(const DevState& s, int mode, bool mixed, bool few, hipStream_t
   A.ctl = s.ctl;
   A.skin = s.skin;
   const int quick = mode == 0 && 2 * s.G.plane < kStagedPri;  // site indices below the staged priority offset
-  const DecideForm form = decideBySize(s);
-  if (form == DecideForm::oneGroup || (form == DecideForm::byLists && few)) {
+  if (few) {
     kDecideAll<<<1, kDT, 0, st>>>(A, quick);
     return;
   }

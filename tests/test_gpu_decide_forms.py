@@ -1,10 +1,10 @@
 """The decide in one workgroup and over a grid (needs an MI355X).
 
-A box of 10 000 to 100 000 sites takes its decide in one workgroup while its
+A box of at most 100 000 sites takes its decide in one workgroup while its
 lists are short, as seen at the last look: at the start of a call and every
 128 steps.  A call of many steps and as many calls of one step choose
 differently while the lists grow past that mark, and must end on the same
-bits; boxes on either side of the smaller limit must agree with the oracle.
+bits; and a box with inter atoms must agree with the oracle.
 """
 import numpy as np
 import pytest
