@@ -935,7 +935,7 @@ static void forcePass(misa_handle* h, int mode, bool store_rho, const VerletPara
   const bool mixed = h->precision == MISA_PREC_MIXED;
   {
     Timer t(h, 0);
-    launchRhoDf(h->s, h->lat, h->t64, h->t32, mixed, h->acc, store_rho, h->stream);
+    launchRhoDf(h->s, h->lat, h->t64, h->t32, mixed, h->acc, store_rho, mode == 2, h->stream);
     h->mask_gen = h->gen;
   }
   {

@@ -182,18 +182,23 @@ struct RhoSiteD {
   uint32_t o16;
   const uint32_t* sh;
   double rc2, rcs2;
+  int mlo;
 };
+__device__ __forceinline__ double cubicD(double c3, double c4, double c5, double c6, double q) {
+  return __fma_rn(__fma_rn(__fma_rn(c3, q, c4), q, c5), q, c6);
+}
 __device__ __forceinline__ RhoSiteD rhoSiteD(const Geom& G, const LatOffsets& O, const Tables<double>& tb, CXPtr x,
-                                             const Rec64& r64, double rcs2, int64_t s, int p) {
+                                             const Rec64& r64, double rcs2, int mlo, int64_t s, int p) {
   return RhoSiteD{x.c[0][s], x.c[1][s], x.c[2][s], rsrcBelow(r64.xy, O.lo), rsrcBelow(r64.zw, O.lo),
-                  rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoV)), static_cast<uint32_t>(s) * 16u, O.sh[p], G.rc2, rcs2};
+                  rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoV)), static_cast<uint32_t>(s) * 16u, O.sh[p], G.rc2, rcs2, mlo};
 }
 // The densities of V neighbours at offsets ks; sets the bits of the offsets
 // within the cutoff for some lane (w) and, on a full scan, within cutoff +
 // skin (s).
 template <int V>
 __device__ __forceinline__ void rhoGroupD(const RhoSiteD& c, const Tables<double>& tb, const int* ks, bool skin,
-                                          RangeSum<0>& acc, uint64_t& w0, uint64_t& w1, uint64_t& s0, uint64_t& s1) {
+                                          RangeSum<0>& acc, RangeSum<0>& oacc, uint64_t& w0, uint64_t& w1,
+                                          uint64_t& s0, uint64_t& s1) {
   double2 xy[V], zw[V];
 #pragma unroll
   for (int u = 0; u < V; ++u) {
@@ -201,7 +206,7 @@ __device__ __forceinline__ void rhoGroupD(const RhoSiteD& c, const Tables<double
     xy[u] = ldRec64(c.rxy, c.o16, so);
     zw[u] = ldRec64(c.rzw, c.o16, so);
   }
-  bool in[V];
+  bool in[V], held[V];
   double pp[V], rec[V][kRhoRec];
 #pragma unroll
   for (int u = 0; u < V; ++u) {
@@ -211,14 +216,20 @@ __device__ __forceinline__ void rhoGroupD(const RhoSiteD& c, const Tables<double
     if (__ballot(in[u])) setBit(w0, w1, ks[u]);
     if (in[u]) {
       const int m = knotM(r2 * rsqT(r2), tb.rdr, tb.nr, pp[u]);
-      ldRec<double, kRhoRec>(c.rtab, static_cast<uint32_t>(recSpecies64(zw[u].y) * tb.nr + m) * (kRhoRec * 8u),
-                             rec[u]);
+      const int ej = recSpecies64(zw[u].y);
+      held[u] = heldPair(0, static_cast<uint32_t>(ej), m, c.mlo);
+      ldRec<double, kRhoRec>(c.rtab, static_cast<uint32_t>(ej * tb.nr + m) * (kRhoRec * 8u), rec[u]);
     }
   }
 #pragma unroll
   for (int u = 0; u < V; ++u) {
     acc.at(ks[u]);
-    if (in[u]) acc.part.add(__fma_rn(__fma_rn(__fma_rn(rec[u][0], pp[u], rec[u][1]), pp[u], rec[u][2]), pp[u], rec[u][3]));
+    oacc.at(ks[u]);
+    if (in[u]) {
+      const double v = cubicD(rec[u][0], rec[u][1], rec[u][2], rec[u][3], pp[u]);
+      if (held[u]) acc.part.add(v);
+      else oacc.part.add(v);
+    }
   }
 }
 // Calls group(ks, V) over the offsets [k0, k1), or over the set bits of
@@ -292,7 +303,7 @@ __global__ __launch_bounds__(kBlock, 7) void kRhoDf(Geom G, LatOffsets O, Tables
                                                  const int8_t* __restrict__ type, double* __restrict__ df,
                                                  double* __restrict__ rho_out, uint64_t* __restrict__ wmask,
                                                  uint64_t* __restrict__ smask, double rcs2, InterView iv,
-                                                 InterDev in, Rec64 r64) {
+                                                 InterDev in, Rec64 r64, int mlo) {
   if (blockIdx.x < kFrontBlocks) {
     interRhoBody<double>(G, tb, iv, x, type, in, frontWave(), kFrontWaves);
     return;
@@ -306,16 +317,18 @@ __global__ __launch_bounds__(kBlock, 7) void kRhoDf(Geom G, LatOffsets O, Tables
   const bool skin =
       __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(!isVacant(ti) && (ti & kWide));
   const uint32_t wv = waveId(b);
-  RangeSum<0> acc;
+  RangeSum<0> acc, oacc;
   uint64_t w0 = 0, w1 = 0, s0 = 0, s1 = 0;
   if (!isVacant(ti)) {
-    const RhoSiteD c = rhoSiteD(G, O, tb, x, r64, rcs2, s, p);
+    const RhoSiteD c = rhoSiteD(G, O, tb, x, r64, rcs2, mlo, s, p);
     forRhoGroups<U>(skin, 0, O.n[p], skin ? uniform64(smask[2 * wv]) : 0, skin ? uniform64(smask[2 * wv + 1]) : 0,
                     [&](auto UC, const int* ks) {
-                      rhoGroupD<decltype(UC)::value>(c, tb, ks, skin, acc, w0, w1, s0, s1);
+                      rhoGroupD<decltype(UC)::value>(c, tb, ks, skin, acc, oacc, w0, w1, s0, s1);
                     });
   }
   acc.close();
+  oacc.close();
+  acc.tot.join(oacc.tot);
   writeMasks(!isVacant(ti), wv, w0, w1, wmask, !skin, s0, s1, smask);
   rhoTailD(G, s, p, cx, cy, cz, ti, acc.tot, x, type, tb, df, rho_out, iv, r64);
 }
@@ -407,8 +420,8 @@ __global__ __launch_bounds__(kBlock) void kRhoDfP(Geom G, LatOffsets O, Tables<d
                                                   const int8_t* __restrict__ type, double* __restrict__ df,
                                                   double* __restrict__ rho_out, uint64_t* __restrict__ wmask,
                                                   uint64_t* __restrict__ smask, double rcs2, InterView iv,
-                                                  InterDev in, Rec64 r64) {
-  __shared__ RangeParts parts;
+                                                  InterDev in, Rec64 r64, int mlo) {
+  __shared__ RangeParts parts, oparts;
   __shared__ TailHits hits;
   if (blockIdx.x < kFrontBlocks) {
     interRhoBody<double>(G, tb, iv, x, type, in, frontWave(), kFrontWaves);
@@ -417,24 +430,30 @@ __global__ __launch_bounds__(kBlock) void kRhoDfP(Geom G, LatOffsets O, Tables<d
   const SharedSite q = sharedSite(G, type, blockIdx.x - kFrontBlocks);
   const bool live = !isVacant(q.ti);
   const bool skin = __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(live && (q.ti & kWide));
-  RangeSum<0> acc;
-  acc.range = q.rg;
+  RangeSum<0> acc, oacc;
+  acc.range = oacc.range = q.rg;
   uint64_t w0 = 0, w1 = 0, s0 = 0, s1 = 0, b0 = 0, b1 = 0;
   if (live) {
-    const RhoSiteD c = rhoSiteD(G, O, tb, x, r64, rcs2, q.s, q.p);
+    const RhoSiteD c = rhoSiteD(G, O, tb, x, r64, rcs2, mlo, q.s, q.p);
     const Range r = rangeOf(q.rg, O.n[q.p]);
     if (skin) rangeBits(smask, q.wv, q.rg, b0, b1);
     forRhoGroups<U>(skin, r.k0, r.k1, b0, b1, [&](auto UC, const int* ks) {
-      rhoGroupD<decltype(UC)::value>(c, tb, ks, skin, acc, w0, w1, s0, s1);
+      rhoGroupD<decltype(UC)::value>(c, tb, ks, skin, acc, oacc, w0, w1, s0, s1);
     });
   }
   writeMaskWord(live, q.wv, q.rg, w0, w1, wmask, !skin, s0, s1, smask);
-  if (q.rg > 0) putPart(parts, q.rg, acc.part);
+  if (q.rg > 0) {
+    putPart(parts, q.rg, acc.part);
+    putPart(oparts, q.rg, oacc.part);
+  }
   findTailHits(hits, q.rg, iv, x.c, type, G.rc2, q.p, q.s, q.ti);
   __syncthreads();
   if (q.rg > 0 || !q.site) return;
   acc.close();
+  oacc.close();
   joinParts(parts, acc.tot);
+  joinParts(oparts, oacc.tot);
+  acc.tot.join(oacc.tot);
   rhoTailD(G, q.s, q.p, q.cx, q.cy, q.cz, q.ti, acc.tot, x, type, tb, df, rho_out, iv, r64, &hits);
 }
 
@@ -1014,6 +1033,224 @@ __global__ __launch_bounds__(kBlock) void kForce(Geom G, LatOffsets O, Tables<do
                       blockIdx.x - kFrontBlocks, threadIdx.x, vb, db);
   if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
   if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
+}
+
+// Sums of the neighbours set aside by the FP64 LDS density pass, per lane.
+struct WaveSum1 {
+  double s[64];
+};
+
+// drainQueueD for the density: the noted neighbours' densities, rank after rank.
+__device__ __forceinline__ void drainRhoD(const uint16_t* q, int n, int rg, double xi0, double xi1, double xi2,
+                                          uint32_t o16, Rsrc rxy, Rsrc rzw, Rsrc rtab, const Tables<double>& tb,
+                                          const uint32_t* __restrict__ sh, WaveSum1& ws) {
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+  const bool on = lane < n;
+  const uint32_t e = q[on ? lane : 0];
+  const int owner = static_cast<int>(e & 63u);
+  const uint32_t rank = e >> 11;
+  const uint32_t oo = static_cast<uint32_t>(laneGet(static_cast<int>(o16), owner)) + sh[32 * rg + ((e >> 6) & 31u)] * 16u;
+  const double2 xy = ldRec64(rxy, oo, 0), zw = ldRec64(rzw, oo, 0);
+  const double r2 = dist2D(laneGet(xi0, owner) - xy.x, laneGet(xi1, owner) - xy.y, laneGet(xi2, owner) - zw.x);
+  double pp, c[kRhoRec];
+  const int m = knotM(r2 * rsqT(r2), tb.rdr, tb.nr, pp);
+  ldRec<double, kRhoRec>(rtab, static_cast<uint32_t>(recSpecies64(zw.y) * tb.nr + m) * (kRhoRec * 8u), c);
+  const double v = cubicD(c[0], c[1], c[2], c[3], pp);
+  bool wait = on;
+  for (uint32_t r = 0; __ballot(wait); ++r) {
+    if (wait && rank == r) {
+      ws.s[owner] += v;
+      wait = false;
+    }
+    waveLdsFence();  // another lane's neighbour of this site reads what was just written
+  }
+}
+
+// The Fe density cubics of the LDS density pass, knot m's {c3, c4} at a[m] and
+// {c5, c6} at b[m], in arrays of their own: at 32 bytes a knot in one array
+// the 16-byte reads of a wavefront would meet in half the banks.
+struct KnotsRho {
+  const double2* a;
+  const double2* b;
+};
+
+// One virtual block of the FP64 LDS density pass: per site the same
+// neighbours, sums and masks as kRhoDf; an Fe neighbour's cubic at a knot from
+// mlo on from LDS, the others worked off by the whole wavefront as in
+// forceVBlockD, with the next group's records in flight during a group.
+template <int U>
+__device__ __forceinline__ void rhoVBlockD(const Geom& G, const LatOffsets& O, const Tables<double>& tb, CXPtr x,
+                                           const int8_t* __restrict__ type, double* __restrict__ df,
+                                           double* __restrict__ rho_out, uint64_t* __restrict__ wmask,
+                                           uint64_t* __restrict__ smask, double rcs2, const InterView& iv,
+                                           const Rec64& r64, const KnotsRho& kn, int mlo, WaveQueueD<U>& wq,
+                                           WaveSum1& ws, uint32_t b, uint32_t tl) {
+  int64_t s = 0;
+  int p = 0, cx = 0, cy = 0, cz = 0;
+  const bool site = siteOfBlock(G, b, tl, s, p, cx, cy, cz);
+  const int8_t ti = site ? type[s] : kVacant;
+  const bool live = !isVacant(ti);
+  const uint64_t lives = __ballot(live);
+  Sum1<0> tot, otot;
+  if (lives) {
+    const bool skin = __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(live && (ti & kWide));
+    const int lane = static_cast<int>(threadIdx.x & 63u);
+    double xi0 = kNoAtom, xi1 = kNoAtom, xi2 = kNoAtom;
+    if (live) {
+      xi0 = x.c[0][s];
+      xi1 = x.c[1][s];
+      xi2 = x.c[2][s];
+    }
+    const Rsrc rxy = rsrcBelow(r64.xy, O.lo), rzw = rsrcBelow(r64.zw, O.lo);
+    const Rsrc rtab = rsrcAt(reinterpret_cast<uintptr_t>(tb.rhoV));
+    const uint32_t o16 = addressOfLives(static_cast<uint32_t>(s) * 16u, live, lives);
+    const int pu = __builtin_amdgcn_readfirstlane((b >> 3) & 1u);
+    const uint32_t* sh = O.sh[pu];
+    const uint32_t wv = b * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tl >> 6);
+    uint64_t m0, m1;
+    if (skin) {
+      m0 = uniform64(smask[2 * wv]);
+      m1 = uniform64(smask[2 * wv + 1]);
+    } else {
+      const int nk = O.n[pu];
+      m0 = nk >= 64 ? ~0ull : (1ull << nk) - 1;
+      m1 = nk > 64 ? (1ull << (nk - 64)) - 1 : 0;  // nk < 128: kPadOffset is no offset
+    }
+    uint64_t w0 = 0, w1 = 0, s0 = 0, s1 = 0;
+    struct Group {
+      int rg;
+      int ks[U];
+      bool act[U];
+      double2 xy[U], zw[U];
+    } g, h;
+    uint32_t w = maskWord(m0, m1, 0);
+    int next = 0;  // the range w belongs to
+    auto fetch = [&](Group& q) {
+      while (w == 0 && next < 3) w = maskWord(m0, m1, ++next);
+      q.rg = w ? next : 4;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        q.act[u] = w != 0;
+        q.ks[u] = w ? 32 * next + __builtin_ctz(w) : kPadOffset;
+        w &= w - 1;
+        const uint32_t so = sh[q.ks[u]] * 16u;
+        q.xy[u] = ldRec64(rxy, o16, so);
+        q.zw[u] = ldRec64(rzw, o16, so);
+      }
+    };
+    int rg = 0, qn = 0;  // the range being summed, the neighbours noted in it
+    uint32_t rank = 0;
+    bool sums = false;
+    Sum1<0> part;
+    auto pairs = [&](const Group& q) {
+      double r2[U];
+      uint64_t in[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        r2[u] = dist2D(xi0 - q.xy[u].x, xi1 - q.xy[u].y, xi2 - q.zw[u].x);
+        in[u] = q.act[u] ? __ballot(r2[u] < G.rc2) : 0;
+        if (!skin && q.act[u] && __ballot(r2[u] < rcs2)) setBit(s0, s1, q.ks[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (!in[u]) continue;  // a third of the offsets of a full scan
+        setBit(w0, w1, q.ks[u]);
+        double pp;
+        const int m = knotM(r2[u] * rsqT(r2[u]), tb.rdr, tb.nr, pp);
+        const uint64_t hm = in[u] & __ballot(recSpecies64(q.zw[u].y) == 0) & __ballot(m >= mlo);
+        const uint64_t other = in[u] & ~hm;
+        const int k = max(m, mlo);
+        const double2 c = kn.a[k], d = kn.b[k];
+        if (other) {
+          if (__builtin_amdgcn_inverse_ballot_w64(other))
+            wq.q[qn + laneRank(other)] =
+                static_cast<uint16_t>((rank++ << 11) | ((static_cast<uint32_t>(q.ks[u]) & 31u) << 6) |
+                                      static_cast<uint32_t>(lane));
+          qn += __builtin_popcountll(other);
+        }
+        if (__builtin_amdgcn_inverse_ballot_w64(hm)) part.add(cubicD(c.x, c.y, d.x, d.y, pp));
+      }
+    };
+    // as in forceVBlockD: before a group of range `to`
+    auto settle = [&](int to) {
+      while (qn >= (to != rg ? 1 : 64)) {
+        if (!sums) {
+          sums = true;
+          ws.s[lane] = 0.0;
+        }
+        waveLdsFence();
+        const int n = qn < 64 ? qn : 64;
+        drainRhoD(wq.q, n, rg, xi0, xi1, xi2, o16, rxy, rzw, rtab, tb, sh, ws);
+        qn -= n;
+        waveLdsFence();
+        if (qn > 0) shiftQueueD(wq, lane);
+      }
+      if (to == rg) return;
+      rg = to;
+      rank = 0;
+      tot.join(part);
+      part = Sum1<0>();
+      if (sums) {
+        Sum1<0> o;
+        o.s = ws.s[lane];
+        otot.join(o);
+        sums = false;
+      }
+    };
+    fetch(g);
+    while (g.rg < 4) {
+      fetch(h);
+      if (g.rg != rg || qn >= 64) settle(g.rg);
+      pairs(g);
+      if (h.rg == 4) break;
+      fetch(g);
+      if (h.rg != rg || qn >= 64) settle(h.rg);
+      pairs(h);
+    }
+    settle(4);
+    if (lane == __builtin_ctzll(lives)) {
+      wmask[2 * wv] = w0;
+      wmask[2 * wv + 1] = w1;
+      if (!skin) {
+        smask[2 * wv] = s0;
+        smask[2 * wv + 1] = s1;
+      }
+    }
+  }
+  if (!site) return;
+  tot.join(otot);
+  rhoTailD(G, s, p, cx, cy, cz, ti, tot, x, type, tb, df, rho_out, iv, r64);
+}
+
+// The FP64 density pass in persistent blocks, one per compute unit, with the
+// Fe density cubics from knot mlo on in LDS.  Half of kRhoDf's loads are the
+// segments, scattered over 160 KB a species, and the texture units bound it;
+// from LDS two 16-byte reads take their place (2M atoms: 483 -> 372 us).  Two
+// offsets a group: four need 118 registers and leave more of a group idle at
+// the end of a range (390 us).
+template <int U>
+__global__ __launch_bounds__(kBlockP) void kRhoDL(Geom G, LatOffsets O, Tables<double> tb, CXPtr x,
+                                                  const int8_t* __restrict__ type, double* __restrict__ df,
+                                                  double* __restrict__ rho_out, uint64_t* __restrict__ wmask,
+                                                  uint64_t* __restrict__ smask, double rcs2, InterView iv, InterDev in,
+                                                  Rec64 r64, int mlo, int nkn) {
+  __shared__ WaveQueueD<U> queues[kBlockP / 64];
+  __shared__ WaveSum1 sums[kBlockP / 64];
+  extern __shared__ double2 knS[];  // nkn {c3, c4}, nkn {c5, c6}
+  const double2* z = reinterpret_cast<const double2*>(tb.rhoV) + 2 * static_cast<size_t>(mlo);  // row Fe is the first
+  for (int i = threadIdx.x; i < nkn; i += kBlockP) {
+    knS[i] = z[2 * i];
+    knS[nkn + i] = z[2 * i + 1];
+  }
+  __syncthreads();
+  const KnotsRho kn{knS - mlo, knS + nkn - mlo};
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  interRhoBody<double>(G, tb, iv, x, type, in, static_cast<int>(wave * gridDim.x + blockIdx.x),
+                       static_cast<int>(gridDim.x) * (kBlockP / 64));
+  forVirtualBlocks(G, [&](uint32_t b, uint32_t tl) {
+    rhoVBlockD<U>(G, O, tb, x, type, df, rho_out, wmask, smask, rcs2, iv, r64, kn, mlo, queues[wave], sums[wave], b,
+                  tl);
+  });
 }
 
 // Potential energy and virial of site s (FP64 tables, FP64 site records):
@@ -1791,6 +2028,18 @@ LdsKnots ldsKnotsForceD(int nr) {
   k.bytes = static_cast<size_t>(40) * static_cast<size_t>(k.nkn) + 16;
   return k;
 }
+// The FP64 density pass's LDS knots, 32 bytes each, beside its queues and
+// sums: 4542 knots, from 0.51 A on where the table has 5000 over 5.6 A.
+constexpr int kURhoD = 2;
+constexpr int kRhoLdsBytesD =
+    160 * 1024 - static_cast<int>(kBlockP / 64 * (sizeof(WaveQueueD<kURhoD>) + sizeof(WaveSum1))) - 64;
+LdsKnots ldsKnotsRhoD(int nr) {
+  LdsKnots k;
+  k.nkn = std::min(nr, kRhoLdsBytesD / 32);
+  k.mlo = nr - k.nkn;
+  k.bytes = static_cast<size_t>(32) * static_cast<size_t>(k.nkn);
+  return k;
+}
 // The energy pass's LDS knots: 7 doubles (56 bytes) a knot beside its static
 // LDS (the block sums; 512 bytes are kept).
 constexpr int kEnergyLdsBytes = 160 * 1024 - 512;
@@ -1828,7 +2077,7 @@ bool useShared(const DevState& s) {
 }  // namespace
 
 void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
-                 bool mixed, int acc, bool store_rho, hipStream_t st) {
+                 bool mixed, int acc, bool store_rho, bool scan, hipStream_t st) {
   double* rho = store_rho ? s.rho : nullptr;
   const bool shared = useShared(s);
   const unsigned grid = kFrontBlocks + (shared ? 4 : 1) * siteGrid(s.G);
@@ -1837,12 +2086,21 @@ void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t
   const double rcs = std::sqrt(s.G.rc2) + s.skin;
   if (!mixed) {
     const Rec64 r64{s.pxy[s.cur], s.pzw[s.cur]};
-    if (shared)
-      kRhoDfP<4><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs, iv,
-                                              s.in, r64);
+    const LdsKnots lk = ldsKnotsRhoD(t64.nr);
+    static const bool ldsReady = setLdsBytes(reinterpret_cast<const void*>(&kRhoDL<kURhoD>), kRhoLdsBytesD);
+    // With the skin's masks kRhoDL against kRhoDf, whole pass: 60^3 cells 101
+    // against 117 us, 100^3 372 against 483, with 6 % solutes at 900 K 60^3 123
+    // against 134, 90^3 344 against 397; where every pass scans all offsets
+    // (766 000 atoms) 257 against 238, so those stay with kRhoDf.
+    if (useLds(s) && ldsReady && !scan && s.skin > 0.0)
+      kRhoDL<kURhoD><<<persistentGrid(s), kBlockP, lk.bytes, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask,
+                                                                   s.smask, rcs * rcs, iv, s.in, r64, lk.mlo, lk.nkn);
+    else if (shared)
+      kRhoDfP<4><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs, iv, s.in,
+                                          r64, lk.mlo);
     else
       kRhoDf<4><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs, iv, s.in,
-                                         r64);
+                                         r64, lk.mlo);
   } else if (shared) {
     const float rcs2 = static_cast<float>(rcs * rcs);
 #define MISA_RHO_MP(A)                                                                                          \

@@ -123,8 +123,9 @@ void launchHaloAll(const DevState& s, int buf, hipStream_t st);
 // force pass of both.  Force modes: 0 f stored, v += c f (secondstep); 1 and
 // the next first half step (for the lattice with the decide's staging); 2 f
 // stored only.
+// scan: this density pass goes over all offsets (no skin masks yet).
 void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
-                 bool mixed, int acc, bool store_rho, hipStream_t st);
+                 bool mixed, int acc, bool store_rho, bool scan, hipStream_t st);
 // Returns the force pass launched: 0 kForce (FP64), 1 kForceM, 2 kForceL (the
 // values of MISA_FORCE_PASS_*).
 int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
@@ -154,10 +155,9 @@ void launchAdaptiveDt(const DevState& s, double dt_max, double max_disp, bool si
 // decide mode 0: the step's ownership pass (append new inter atoms, vacancy
 // recombination, migration, ghost images, index, flags); mode 1: migration,
 // ghost images, index and flags only (first force, PKA step, upload).
-// The small boxes' decide is one workgroup's work, the large ones' a grid's;
-// between them it depends on the lists, which the caller has seen (few).
-enum class DecideForm { oneGroup, byLists, grid };
-DecideForm decideBySize(const DevState& s);
+// few: the decide in one workgroup, for short lists in a box of few sites
+// (decideInOneGroup).
+bool decideInOneGroup(const DevState& s);
 void launchDecide(const DevState& s, int mode, bool mixed, bool few, hipStream_t st);
 // Ask the next decide for a full scan of the mixed density pass.
 void launchRescan(const DevState& s, hipStream_t st);
