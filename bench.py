@@ -474,7 +474,7 @@ def main():
                   "other_ms_per_step": t32["other_ms"] / args.steps, "share_of_step": shares(t32, s32)},
         "fp64": {"force_kernel": launched["fp64"], "force_ms": avg_force64,
                  "force_GBs": gbs(FORCE_BYTES["fp64"], avg_force64),
-                 "rho_kernel": "kRhoDf", "rho_ms": avg_rho64, "rho_GBs": gbs(RHO_BYTES["fp64"], avg_rho64),
+                 "rho_kernel": "kRhoDL", "rho_ms": avg_rho64, "rho_GBs": gbs(RHO_BYTES["fp64"], avg_rho64),
                  "other_ms_per_step": t64["other_ms"] / args.steps, "share_of_step": shares(t64, s64)},
     }
     res = {

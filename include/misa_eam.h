@@ -252,8 +252,9 @@ int misa_set_launch_shape(misa_handle* h, int32_t ty, int32_t gathers_rho, int32
 int misa_get_launch_shape(const misa_handle* h, int32_t* ty, int32_t* gathers_rho, int32_t* gathers_force);
 /* Force passes (mixed and FP64) in persistent blocks that hold the majority
  * species' spline knots in LDS (the mixed pass also the pruned offsets):
- * MISA_LDS_AUTO (default; boxes large enough that every block walks several
- * virtual blocks), MISA_LDS_ON, MISA_LDS_OFF.  No counterpart in the
+ * MISA_LDS_AUTO (default; boxes whose sites fill the persistent launch, some
+ * 260,000 atoms), MISA_LDS_ON, MISA_LDS_OFF.  The FP64 density and energy
+ * passes follow the same choice.  No counterpart in the
  * reference (a tuning switch of this build's kernels); the pairs, their
  * order and their rounding are the same either way, so results are
  * bit-identical. */
@@ -278,7 +279,8 @@ int misa_xcd_slabs(const misa_handle* h, int32_t zlo[9]);
  * slab leaves its XCD idle) and turn balancing off. */
 int misa_set_xcd_slabs(misa_handle* h, const int32_t zlo[9]);
 /* The force pass the last force evaluation launched (-1 before any):
- * kForce (FP64), kForceM (mixed, spline segments from global memory),
+ * kForce (FP64) or kForceM (mixed) with spline segments from global memory
+ * (kForceP and kForceMP in boxes of few sites count as these),
  * kForceL (mixed, persistent blocks with the majority species' segments in
  * LDS) or kForceDL (FP64, persistent blocks with the majority species'
  * segments in LDS).  The LDS passes run where MISA_LDS_* picks them; the

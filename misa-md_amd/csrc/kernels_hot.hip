@@ -8,6 +8,12 @@
 //            part of atom::decide and the position halo (atom::latForce,
 //            NewtonMotion, atom::decide; simulation.cpp:164-194)
 //
+// Each in three forms that give the same bits: four wavefronts to 64 sites in
+// boxes of few sites (kRhoDfP, kForceP), a wavefront each (kRhoDf, kForce), and
+// persistent blocks with the majority species' segments in LDS (kRhoDL,
+// kForceDL); the mixed ones carry an M (kForceL is the mixed LDS pass).  The
+// inter atoms' density and force ride in the same launches.
+//
 // One thread per site.  A full list (each lane owns its site's sums) replaces
 // the reference's half list with ghost partials and reverse halos: no atomics,
 // deterministic sums.  The list keeps the reference offsets whose ideal

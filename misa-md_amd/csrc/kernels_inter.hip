@@ -291,7 +291,7 @@ __device__ __forceinline__ void forNeighbourhoods(const int64_t* slots, int n, i
 // Far lattice atoms on an eighth of the sites or more (a small box far above
 // room temperature) have some 28 of their kind within every site's full list:
 // kWide goes to every site at once, one write a site instead of 229 tries per
-// far atom (32 000 sites, 10 000 far atoms: kFlag and kUnflag 46 us each
+// far atom (32 000 sites, 10 000 far atoms: kFlag and the unflagging 46 us each
 // before, 10 now).  A site flagged without a far atom around sums the same pairs.
 __device__ __forceinline__ bool farEverywhere(const Geom& G, int64_t nfar) { return 4 * nfar >= G.nsub; }
 template <typename Fn>

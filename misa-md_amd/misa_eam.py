@@ -343,7 +343,7 @@ class EamDevice:
                     "misa_set_launch_shape")
 
     def set_lds_tables(self, mode):
-        """LDS_AUTO, LDS_ON or LDS_OFF: the mixed force pass with its majority-species tables in LDS."""
+        """LDS_AUTO, LDS_ON or LDS_OFF: the passes with their majority-species tables in LDS."""
         self._check(self.lib.misa_set_lds_tables(self.h, int(mode)), "misa_set_lds_tables")
 
     def defect_counters(self):
