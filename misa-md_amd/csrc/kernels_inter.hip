@@ -95,6 +95,16 @@ __device__ __forceinline__ T fresh(const T* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A site's type in the flag bodies: fresh where one workgroup does the whole
+// decide (ONE); over a grid a stale copy at worst asks for a bit's atomic once
+// more, and reading past the cache costs more (16M-atom cascade: kFlag 68 us
+// against 58, kUnflagClaim 69 against 65).
+template <bool ONE>
+__device__ __forceinline__ int8_t typeNow(const int8_t* p) {
+  if constexpr (ONE) return fresh(p);
+  else return *p;
+}
+
 __device__ __forceinline__ void setFlag(unsigned long long* f, unsigned long long bit) { atomicOr(f, bit); }
 
 // Copy local atom src (main arrays) to scratch slot dst, shifting x[d] by sh.
@@ -267,7 +277,7 @@ __device__ __forceinline__ int64_t wrappedNeighbour(const Geom& G, const FullPla
 // fn(t, type of t) for the sites t = site(slots[e], k) of n slots and their
 // nfull neighbours, four items a thread at a time: an item is a chain of three
 // reads, and one workgroup has few threads to hide them.
-template <typename Site, typename Fn>
+template <bool ONE, typename Site, typename Fn>
 __device__ __forceinline__ void forNeighbourhoods(const int64_t* slots, int n, int nfull, const int8_t* ltype,
                                                   int64_t t0, int64_t stride, Site site, Fn fn) {
   const int64_t total = static_cast<int64_t>(n) * nfull;
@@ -281,7 +291,7 @@ __device__ __forceinline__ void forNeighbourhoods(const int64_t* slots, int n, i
       t[u] = q < total ? site(slots[e], static_cast<int>(q - e * nfull) - 1) : -1;
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = t[u] >= 0 ? fresh(ltype + t[u]) : kVacant;
+    for (int u = 0; u < 4; ++u) v[u] = t[u] >= 0 ? typeNow<ONE>(ltype + t[u]) : kVacant;
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (t[u] >= 0) fn(t[u], v[u]);
@@ -294,14 +304,14 @@ __device__ __forceinline__ void forNeighbourhoods(const int64_t* slots, int n, i
 // far atom (32 000 sites, 10 000 far atoms: kFlag and the unflagging 46 us each
 // before, 10 now).  A site flagged without a far atom around sums the same pairs.
 __device__ __forceinline__ bool farEverywhere(const Geom& G, int64_t nfar) { return 4 * nfar >= G.nsub; }
-template <typename Fn>
+template <bool ONE, typename Fn>
 __device__ __forceinline__ void forSubBoxSites(const Geom& G, const int8_t* ltype, int64_t t0, int64_t stride,
                                                Fn fn) {
   for (int64_t t = t0; t < 2 * G.nsub; t += stride) {
     int64_t s;
     int p, cx, cy, cz;
     siteInOrder(G, t, s, p, cx, cy, cz);
-    fn(s, fresh(ltype + s));
+    fn(s, typeNow<ONE>(ltype + s));
   }
 }
 
@@ -313,6 +323,7 @@ constexpr int kFlagBlocks = 1024;
 // and the flags it set, kNearInter around its entries and kWide around its
 // far lattice atoms and their images (atom.cpp:21-84 rebuilds the index each
 // step; inter_atom_list.cpp:27-45).
+template <bool ONE>
 __device__ __forceinline__ void unflagBody(const Geom& G, const InterDev& in, int8_t* ltype, const Ctl* ctl,
                                            int64_t t0, int64_t stride) {
   const int nprev = static_cast<int>(ctl->n_prev);
@@ -321,7 +332,7 @@ __device__ __forceinline__ void unflagBody(const Geom& G, const InterDev& in, in
   const int nfull = 1 + max(full.n[0], full.n[1]);
   for (int64_t q = t0; q < nprev; q += stride) in.head[in.prev_slot[q]] = -1;
   const auto wrapped = [&](int64_t slot, int k) { return wrappedNeighbour(G, full, slot, k); };
-  forNeighbourhoods(
+  forNeighbourhoods<ONE>(
       in.prev_slot, nprev, nfull, ltype, t0, stride,
       [&](int64_t slot, int k) { return fullNeighbour(G, full, slot, k); },
       [&](int64_t t, int8_t v) {
@@ -330,11 +341,11 @@ __device__ __forceinline__ void unflagBody(const Geom& G, const InterDev& in, in
   const auto clear = [&](int64_t t, int8_t v) {
     if (!isVacant(v) && (v & kWide)) typeBitsAnd(ltype, t, static_cast<int8_t>(~kWide));
   };
-  if (farEverywhere(G, nfarPrev)) forSubBoxSites(G, ltype, t0, stride, clear);
-  else forNeighbourhoods(in.far_prev, nfarPrev, nfull, ltype, t0, stride, wrapped, clear);
+  if (farEverywhere(G, nfarPrev)) forSubBoxSites<ONE>(G, ltype, t0, stride, clear);
+  else forNeighbourhoods<ONE>(in.far_prev, nfarPrev, nfull, ltype, t0, stride, wrapped, clear);
   for (int64_t q = t0; q < nfarPrev; q += stride)
     forSlotAndImages(G, in.far_prev[q], [&](int64_t slot) {
-      const int8_t v = fresh(ltype + slot);
+      const int8_t v = typeNow<ONE>(ltype + slot);
       if (!isVacant(v) && (v & kFar)) typeBitsAnd(ltype, slot, static_cast<int8_t>(~kFar));
     });
 }
@@ -690,7 +701,7 @@ __device__ __forceinline__ int gridThreads() { return static_cast<int>(gridDim.x
 // what the other writes.
 __global__ __launch_bounds__(kBlock) void kUnflagClaim(Geom G, InterDev in, int8_t* ltype, const Ctl* ctl,
                                                        int quick) {
-  unflagBody(G, in, ltype, ctl, gridThread(), gridThreads());
+  unflagBody<false>(G, in, ltype, ctl, gridThread(), gridThreads());
   if (quick) quickClaim(G, in, ctl, gridThread(), gridThreads());
 }
 __global__ __launch_bounds__(kBlock) void kQuickCompete(Geom G, InterDev in, const Ctl* ctl) {
@@ -703,6 +714,7 @@ __global__ __launch_bounds__(kBlock) void kQuickRefill(DecideArgs A) { quickRefi
 // within the full neighbourhood of every lattice atom farther than 0.2a from
 // its site and of its periodic images (kWide: their sums visit the whole full
 // list); the far list becomes the one the next decide clears.
+template <bool ONE>
 __device__ __forceinline__ void flagBody(const Geom& G, const InterDev& in, int8_t* ltype, const Ctl* ctl,
                                          int64_t t0, int64_t stride) {
   const int ne = static_cast<int>(ctl->n_prev);
@@ -710,7 +722,7 @@ __device__ __forceinline__ void flagBody(const Geom& G, const InterDev& in, int8
   const FullPlaneOffsets& full = *in.full;
   const int nfull = 1 + max(full.n[0], full.n[1]);
   const auto wrapped = [&](int64_t slot, int k) { return wrappedNeighbour(G, full, slot, k); };
-  forNeighbourhoods(
+  forNeighbourhoods<ONE>(
       in.e_slot, ne, nfull, ltype, t0, stride,
       [&](int64_t slot, int k) { return fullNeighbour(G, full, slot, k); },
       [&](int64_t t, int8_t v) {
@@ -719,18 +731,18 @@ __device__ __forceinline__ void flagBody(const Geom& G, const InterDev& in, int8
   const auto set = [&](int64_t t, int8_t v) {
     if (!isVacant(v) && !(v & kWide)) typeBitsOr(ltype, t, kWide);
   };
-  if (farEverywhere(G, nfar)) forSubBoxSites(G, ltype, t0, stride, set);
-  else forNeighbourhoods(in.far_new, nfar, nfull, ltype, t0, stride, wrapped, set);
+  if (farEverywhere(G, nfar)) forSubBoxSites<ONE>(G, ltype, t0, stride, set);
+  else forNeighbourhoods<ONE>(in.far_new, nfar, nfull, ltype, t0, stride, wrapped, set);
   for (int64_t q = t0; q < nfar; q += stride) {
     forSlotAndImages(G, in.far_new[q], [&](int64_t slot) {
-      const int8_t v = fresh(ltype + slot);
+      const int8_t v = typeNow<ONE>(ltype + slot);
       if (!isVacant(v) && !(v & kFar)) typeBitsOr(ltype, slot, kFar);
     });
     in.far_prev[q] = in.far_new[q];
   }
 }
 __global__ __launch_bounds__(kBlock) void kFlag(Geom G, InterDev in, int8_t* ltype, const Ctl* ctl) {
-  flagBody(G, in, ltype, ctl, static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x,
+  flagBody<false>(G, in, ltype, ctl, static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x,
            static_cast<int64_t>(gridDim.x) * kBlock);
 }
 
@@ -742,7 +754,7 @@ __global__ __launch_bounds__(kDT) void kDecideAll(DecideArgs A, int quick) {
   const int tid = threadIdx.x;
   const bool index = A.ctl->n_prev > 0 || A.ctl->n_far_prev > 0;
   const bool stage = quick && A.ctl->n_stage > 0;
-  if (index) unflagBody(A.G, A.in, A.ltype, A.ctl, tid, kDT);
+  if (index) unflagBody<true>(A.G, A.in, A.ltype, A.ctl, tid, kDT);
   if (stage) {
     quickClaim(A.G, A.in, A.ctl, tid, kDT);
     __syncthreads();
@@ -753,7 +765,7 @@ __global__ __launch_bounds__(kDT) void kDecideAll(DecideArgs A, int quick) {
   __syncthreads();
   decideBody(A);
   __syncthreads();
-  flagBody(A.G, A.in, A.ltype, A.ctl, tid, kDT);
+  flagBody<true>(A.G, A.in, A.ltype, A.ctl, tid, kDT);
 }
 
 __global__ void kRescan(Ctl* ctl) { ctl->rescan = 1; }
@@ -1007,12 +1019,12 @@ constexpr int kBatchFlagBlocks = 32;  // of the flag kernels: a hot box has hund
 
 __global__ __launch_bounds__(kBlock) void kUnflagB(const BatchBox* __restrict__ boxes) {
   const BatchBox& B = boxes[blockIdx.x / kBatchFlagBlocks];
-  unflagBody(B.G, B.in, B.type, B.ctl, static_cast<int64_t>(blockIdx.x % kBatchFlagBlocks) * kBlock + threadIdx.x,
+  unflagBody<false>(B.G, B.in, B.type, B.ctl, static_cast<int64_t>(blockIdx.x % kBatchFlagBlocks) * kBlock + threadIdx.x,
              static_cast<int64_t>(kBatchFlagBlocks) * kBlock);
 }
 __global__ __launch_bounds__(kBlock) void kFlagB(const BatchBox* __restrict__ boxes) {
   const BatchBox& B = boxes[blockIdx.x / kBatchFlagBlocks];
-  flagBody(B.G, B.in, B.type, B.ctl, static_cast<int64_t>(blockIdx.x % kBatchFlagBlocks) * kBlock + threadIdx.x,
+  flagBody<false>(B.G, B.in, B.type, B.ctl, static_cast<int64_t>(blockIdx.x % kBatchFlagBlocks) * kBlock + threadIdx.x,
            static_cast<int64_t>(kBatchFlagBlocks) * kBlock);
 }
 // args[2 b + flip]: the decide arguments of box b for either buffer
