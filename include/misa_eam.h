@@ -253,7 +253,7 @@ int misa_get_launch_shape(const misa_handle* h, int32_t* ty, int32_t* gathers_rh
 /* Force passes (mixed and FP64) in persistent blocks that hold the majority
  * species' spline knots in LDS (the mixed pass also the pruned offsets):
  * MISA_LDS_AUTO (default; boxes whose sites fill the persistent launch, some
- * 260,000 atoms), MISA_LDS_ON, MISA_LDS_OFF.  The FP64 density and energy
+ * 260,000 atoms, with few enough solutes: 16 % in FP64, 35 % mixed), MISA_LDS_ON, MISA_LDS_OFF.  The FP64 density and energy
  * passes follow the same choice.  No counterpart in the
  * reference (a tuning switch of this build's kernels); the pairs, their
  * order and their rounding are the same either way, so results are

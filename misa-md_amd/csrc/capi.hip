@@ -747,11 +747,15 @@ int misa_upload_state(misa_handle* h, const void* atoms, const void* inter, int6
     if (t > 2 || t < -1) return false;
     return !(t >= 0 && h->have_pot && !h->species_present[t]);
   };
+  int64_t live = 0, solutes = 0;
   for (int64_t k = 0; k < b.n[2]; k++)
     for (int64_t j = 0; j < b.n[1]; j++)
-      for (int64_t i = 0; i < 2 * b.n[0]; i++)
-        if (!checkType(a[b.refIndex(i + 2 * b.g, j + b.g, k + b.g)].type))
-          return fail(h, MISA_E_ARG, "atom type unknown or missing from the potential file");
+      for (int64_t i = 0; i < 2 * b.n[0]; i++) {
+        const int t = a[b.refIndex(i + 2 * b.g, j + b.g, k + b.g)].type;
+        if (!checkType(t)) return fail(h, MISA_E_ARG, "atom type unknown or missing from the potential file");
+        live += t >= 0;
+        solutes += t > 0;
+      }
   const AtomElement* ia = static_cast<const AtomElement*>(inter);
   for (int64_t i = 0; i < n_inter; i++)
     if (ia[i].type < 0 || !checkType(ia[i].type)) return fail(h, MISA_E_ARG, "bad inter-atom type");
@@ -759,6 +763,7 @@ int misa_upload_state(misa_handle* h, const void* atoms, const void* inter, int6
   if (!h->aos_dev) HIPCHECK(h, hipMalloc(&h->aos_dev, bytes));
   HIPCHECK(h, hipMemcpyAsync(h->aos_dev, atoms, bytes, hipMemcpyHostToDevice, h->stream));
   h->s.cur = 0;
+  h->s.solutes = live > 0 ? static_cast<double>(solutes) / static_cast<double>(live) : 0.0;
   launchUpload(h->s, h->aos_dev, b.sx, b.sy, h->stream);
   launchHaloAll(h->s, h->s.cur, h->stream);
   HIPCHECK(h, hipGetLastError());

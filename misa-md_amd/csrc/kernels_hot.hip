@@ -2067,9 +2067,15 @@ unsigned persistentGrid(const DevState& s) { return static_cast<unsigned>(s.ncu 
 // 4096 wavefronts): at 60^3 cells FP64 156 against 216 us, mixed 83 against
 // 108; at 50^3 148 against 163 and 81 against 80; at 40^3, half the
 // wavefronts idle, 83 against 73 and 46 against 43.
-bool useLds(const DevState& s) {
+// The queued pairs cost more than the masked gathers of the other passes where
+// they are many: 80^3 cells, FP64 with 3 / 10 / 25 / 60 % solutes 507 / 626 / 866
+// / 1262 us a step with LDS against 683 / 720 / 779 / 883, mixed 284 / 327 / 439
+// / 617 against 328 / 371 / 458 / 555.
+constexpr double kSolutesD = 0.16, kSolutesM = 0.35;
+bool useLds(const DevState& s, double most = 1.0) {
   if (s.ncu < 8 || s.lds == kLdsOff) return false;
   if (s.lds == kLdsOn) return true;
+  if (s.solutes > most) return false;
   return static_cast<int64_t>(siteGrid(s.G)) * kBlock >= static_cast<int64_t>(persistentGrid(s)) * kBlockP;
 }
 
@@ -2098,7 +2104,7 @@ void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t
     // against 117 us, 100^3 372 against 483, with 6 % solutes at 900 K 60^3 123
     // against 134, 90^3 344 against 397; where every pass scans all offsets
     // (766 000 atoms) 257 against 238, so those stay with kRhoDf.
-    if (useLds(s) && ldsReady && !scan && s.skin > 0.0)
+    if (useLds(s, kSolutesD) && ldsReady && !scan && s.skin > 0.0)
       kRhoDL<kURhoD><<<persistentGrid(s), kBlockP, lk.bytes, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask,
                                                                    s.smask, rcs * rcs, iv, s.in, r64, lk.mlo, lk.nkn);
     else if (shared)
@@ -2145,7 +2151,7 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
   const XPtr xn = xp(s.x[1 - s.cur]);
   const StageArgs sa = stageOf(s);
   const InterView iv = interView(s, mixed);
-  const bool lds = useLds(s);
+  const bool lds = useLds(s, mixed ? kSolutesM : kSolutesD);
   const LdsKnots lk = ldsKnotsForce(t32.nr);
   const LdsKnots lkd = ldsKnotsForceD(t64.nr);
 #define MISA_FORCE(M)                                                                                         \

@@ -86,6 +86,7 @@ struct DevState {
   // pass) and the choice of that pass (MISA_LDS_AUTO / ON / OFF)
   int ncu = 0;
   int lds = 0;  // kLdsAuto, kLdsOn, kLdsOff
+  double solutes = 0.0;  // share of the uploaded lattice atoms that are not Fe
   // neighbour skin of the mixed density pass (A; 0: every step scans all
   // pruned offsets) and, per wavefront, the pruned offsets within cutoff +
   // skin for some lane at the last full scan (2 words)
