@@ -291,6 +291,10 @@ int misa_set_xcd_slabs(misa_handle* h, const int32_t zlo[9]);
 #define MISA_FORCE_PASS_MIXED_LDS 2
 #define MISA_FORCE_PASS_FP64_LDS 3
 int misa_force_pass_used(const misa_handle* h, int32_t* kind);
+/* The steps of the last misa_step call whose ownership pass (atom::decide) ran
+ * in one workgroup (short lists in a box of few sites) and over a grid.  The
+ * same lists in the same order either way. */
+int misa_decide_forms_used(const misa_handle* h, int64_t out[2]);
 
 /* ---- host mirror of libcomm's domain at one rank ----
  *

@@ -62,6 +62,7 @@ struct misa_handle {
   int force_pass = -1;       // MISA_FORCE_PASS_* of the last force pass launched
   bool range_check = false;  // a density beyond the F(rho) table fails the call
   int64_t flags_seen = 0;    // the device flags at the last check
+  int64_t decides[2] = {0, 0};  // of the last misa_step: in one workgroup, over a grid
   bool few_listed = false;   // at the last look the decide's lists were short (kFewListed)
   // XCD slabs cut by measured work (misa_set_xcd_balance); virtual blocks
   // per parity per XCD the wave-mask and partial-sum arrays are sized for
@@ -1016,6 +1017,7 @@ void enqFirstAndDecide(misa_handle* h, const StepPlan& p, bool lattice, bool vma
   {
     Timer t(h, 2);
     launchDecide(h->s, 0, p.mixed, p.few, h->stream);
+    h->decides[p.few ? 0 : 1]++;
   }
 }
 
@@ -1111,6 +1113,7 @@ int misa_step(misa_handle* h, int64_t nsteps) {
   StepPlan p = planOf(h);
   const bool look = decideInOneGroup(h->s);
   p.few = look && h->few_listed;
+  h->decides[0] = h->decides[1] = 0;
   clearEvents(h);
   hipEvent_t e0, e1;
   HIPCHECK(h, hipEventCreate(&e0));
@@ -1721,6 +1724,12 @@ int misa_defect_counters(misa_handle* h, int64_t out[3]) {
 int misa_force_pass_used(const misa_handle* h, int32_t* kind) {
   if (!h || !kind) return MISA_E_ARG;
   *kind = h->force_pass;
+  return MISA_OK;
+}
+
+int misa_decide_forms_used(const misa_handle* h, int64_t out[2]) {
+  if (!h || !out) return MISA_E_ARG;
+  for (int k = 0; k < 2; k++) out[k] = h->decides[k];
   return MISA_OK;
 }
 

@@ -398,22 +398,25 @@ __device__ __forceinline__ void decideBody(const DecideArgs& A) {
   const Geom& G = A.G;
   InterDev in = A.in;
   const int tid = threadIdx.x;
-  int nl = static_cast<int>(A.ctl->n_inter);
   __shared__ int sFar;   // far lattice atoms for this index (kFarScan's in mode 1)
   __shared__ int sNear;  // refilled atoms within 0.2a of their site
+  // inter atoms, staged atoms, and those of them put back already: read once,
+  // for all wavefronts, since the early end below clears the counters
+  __shared__ int sInter, sStage, sQuick;
   __shared__ uint64_t sKeys[kSortLds];
   if (tid == 0) {
     sFar = static_cast<int>(min(fresh(&A.ctl->n_far), in.cap));
     sNear = 0;
+    sInter = static_cast<int>(A.ctl->n_inter);
+    sStage = A.mode == 0 ? static_cast<int>(min(A.ctl->n_stage, in.cap)) : 0;
+    sQuick = A.mode == 0 ? static_cast<int>(fresh(&A.ctl->n_quick)) : 0;
   }
   __syncthreads();
   unsigned long long* err = reinterpret_cast<unsigned long long*>(&A.ctl->err_flags);
-  int refills = 0, staged = 0;
+  int nl = sInter, refills = 0, staged = 0;
   // no inter atom, and every staged atom put back already: the lists stay empty
-  const int64_t quick = A.mode == 0 ? fresh(&A.ctl->n_quick) : 0;
-  if (nl == 0 && (A.mode != 0 || A.ctl->n_stage == quick)) {
-    const int back = static_cast<int>(quick);
-    if (tid == 0) finishDecide(A, 0, 0, min(sFar, static_cast<int>(in.cap)), back, back, 0);
+  if (nl == 0 && sStage == sQuick) {
+    if (tid == 0) finishDecide(A, 0, 0, min(sFar, static_cast<int>(in.cap)), sQuick, sQuick, 0);
     return;
   }
 
@@ -422,9 +425,9 @@ __device__ __forceinline__ void decideBody(const DecideArgs& A) {
     // (atom.cpp:28-53 walks the sub-box z -> y -> x and appends): sort the
     // staged atoms by the reference linear index of their site.  Entries
     // that quickRefill already put back (key kQuickDone) are left out.
-    const int nsAll = static_cast<int>(min(A.ctl->n_stage, in.cap));
+    const int nsAll = sStage;
     staged = nsAll;
-    refills = static_cast<int>(quick);
+    refills = sQuick;
     int ns = 0;  // the entries still staged, compacted before the sort
     for (int base = 0; base < nsAll; base += kDT) {
       const int i = base + tid;

@@ -141,6 +141,7 @@ _SIGS = {
     "misa_set_launch_shape": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32]),
     "misa_set_lds_tables": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32]),
     "misa_force_pass_used": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int32)]),
+    "misa_decide_forms_used": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int64)]),
     "misa_set_xcd_balance": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32]),
     "misa_xcd_slabs": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int32)]),
     "misa_set_xcd_slabs": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int32)]),
@@ -357,6 +358,12 @@ class EamDevice:
         k = ctypes.c_int32()
         self._check(self.lib.misa_force_pass_used(self.h, ctypes.byref(k)), "misa_force_pass_used")
         return {0: "kForce", 1: "kForceM", 2: "kForceL", 3: "kForceDL"}.get(k.value, "none")
+
+    def decide_forms(self):
+        """Steps of the last step() call with the decide in one workgroup, and over a grid."""
+        out = (ctypes.c_int64 * 2)()
+        self._check(self.lib.misa_decide_forms_used(self.h, out), "misa_decide_forms_used")
+        return out[0], out[1]
 
     def set_xcd_balance(self, on):
         """Cut the XCD z-slabs by the force pass's measured work (default on)."""
