@@ -696,8 +696,10 @@ int misa_get_potential_table(const misa_handle* h, int kind, int idx, double* ou
   return MISA_OK;
 }
 
-// The records of the buffer that the next step writes, as a hook's scratch.
+// The records of the buffers that the next step writes, as a hook's scratch:
+// the FP64 ones, and the mixed ones for the species.
 static site::Rec64 hookRecs(const misa_handle* h) { return site::Rec64{h->s.pxy[1 - h->s.cur], h->s.pzw[1 - h->s.cur]}; }
+static uint8_t* hookSpecies(const misa_handle* h) { return reinterpret_cast<uint8_t*>(h->s.rec[1 - h->s.cur]); }
 
 static int hookCall(misa_handle* h, int which, void* atoms, double rc) {
   if (!h || !atoms) return MISA_E_ARG;
@@ -706,7 +708,7 @@ static int hookCall(misa_handle* h, int which, void* atoms, double rc) {
   const size_t bytes = static_cast<size_t>(h->box.slots()) * sizeof(AtomElement);
   if (!h->aos_dev) HIPCHECK(h, hipMalloc(&h->aos_dev, bytes));
   HIPCHECK(h, hipMemcpyAsync(h->aos_dev, atoms, bytes, hipMemcpyHostToDevice, h->stream));
-  launchHook(which, h->box, rc, h->s.in.full, h->t64, hookRecs(h), h->aos_dev, h->stream);
+  launchHook(which, h->box, rc, h->s.in.full, h->t64, hookRecs(h), hookSpecies(h), h->aos_dev, h->stream);
   HIPCHECK(h, hipGetLastError());
   HIPCHECK(h, copyToHost(atoms, h->aos_dev, bytes, h->stream));
   return MISA_OK;
@@ -726,7 +728,7 @@ int misa_lat_hook_noalloc(misa_handle* h, int which, void* atoms, double rc) {
   AtomElement* a = static_cast<AtomElement*>(stage);
   // the whole array is overwritten by the copy: nothing in it needs clearing
   HIPCHECK(h, hipMemcpyAsync(a, atoms, bytes, hipMemcpyHostToDevice, h->stream));
-  launchHook(which, h->box, rc, h->s.in.full, h->t64, hookRecs(h), a, h->stream);
+  launchHook(which, h->box, rc, h->s.in.full, h->t64, hookRecs(h), hookSpecies(h), a, h->stream);
   HIPCHECK(h, hipGetLastError());
   HIPCHECK(h, hipMemcpyAsync(atoms, a, bytes, hipMemcpyDeviceToHost, h->stream));
   HIPCHECK(h, hipStreamSynchronize(h->stream));

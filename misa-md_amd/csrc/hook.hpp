@@ -10,8 +10,8 @@
 namespace misa {
 
 // which: 0 rho, 1 df, 2 force.  full: the handle's full lists on the device;
-// rec: scratch for a record per slot.
+// rec, sp: scratch for a record and a byte per slot.
 void launchHook(int which, const Box& b, double rc, const FullPlaneOffsets* full, const Tables<double>& tb, site::Rec64 rec,
-                AtomElement* a, hipStream_t st);
+                uint8_t* sp, AtomElement* a, hipStream_t st);
 
 }  // namespace misa

@@ -5,10 +5,11 @@
 //
 // A site's neighbours sit 104 bytes and more apart in that array, so that a
 // wavefront's read of one field touches a cache line a lane.  kHookPack first
-// takes position, species and F' out of it into 16-byte halves {x, y} and
-// {z, w} per parity-plane slot (the FP64 site records of site_common.hpp,
-// handle scratch), and the sums read those: 64 neighbours in two coalesced
-// loads (54 000 cells: density 217 -> 37 us, force 188 -> 52, packing 7 each).
+// takes what a sum needs out of it into 16-byte halves {x, y} and {z, w} per
+// parity-plane slot (handle scratch), and the sums read those: 64 neighbours
+// in two coalesced loads (54 000 cells: density 217 -> 37 us, force 188 -> 54,
+// packing 7 each).  The w holds the species for the density sum; for the force
+// sum it holds the caller's F' whole, and the species come as a byte each.
 // Four wavefronts share 64 sites, each with a quarter of the
 // reference's full offset list (NeighbourIndex even/odd,
 // neighbour_index.inl:13-76), since a hook's boxes have too few sites to hide
@@ -50,7 +51,9 @@ __device__ __forceinline__ int64_t hookPlaneSlot(const HookGeom& G, int64_t r) {
   return (X & 1) * G.plane + row * G.NX + (X >> 1);
 }
 
-__global__ __launch_bounds__(kHookBlock) void kHookPack(HookGeom G, const AtomElement* __restrict__ a, Rec64 rec) {
+template <bool FORCE>
+__global__ __launch_bounds__(kHookBlock) void kHookPack(HookGeom G, const AtomElement* __restrict__ a, Rec64 rec,
+                                                        uint8_t* __restrict__ sp) {
   const int64_t r = static_cast<int64_t>(blockIdx.x) * kHookBlock + threadIdx.x;
   if (r >= G.slots) return;
   const AtomElement& e = a[r];
@@ -58,9 +61,11 @@ __global__ __launch_bounds__(kHookBlock) void kHookPack(HookGeom G, const AtomEl
   if (e.type < 0) {
     rec.xy[s] = make_double2(kVacantPos64, kVacantPos64);
     rec.zw[s] = make_double2(kVacantPos64, 0.0);
+    if (FORCE) sp[s] = 0;
   } else {
     rec.xy[s] = make_double2(e.x[0], e.x[1]);
-    rec.zw[s] = make_double2(e.x[2], packW64(e.df, e.type));
+    rec.zw[s] = make_double2(e.x[2], FORCE ? e.df : packW64(0.0, e.type));
+    if (FORCE) sp[s] = static_cast<uint8_t>(e.type);
   }
 }
 
@@ -149,6 +154,7 @@ __global__ __launch_bounds__(kHookBlock) void kHookDf(HookGeom G, Tables<double>
 
 __global__ __launch_bounds__(kHookBlock) void kHookForce(HookGeom G, const FullPlaneOffsets* __restrict__ full,
                                                          Tables<double> tb, Rec64 rec,
+                                                         const uint8_t* __restrict__ sp,
                                                          AtomElement* __restrict__ a) {
   __shared__ double sums[kHookParts][3][64];
   const int p = blockIdx.y;
@@ -159,15 +165,17 @@ __global__ __launch_bounds__(kHookBlock) void kHookForce(HookGeom G, const FullP
   hookSite(G, p, t < nsub ? t : nsub - 1, r, s);
   double2 xy = rec.xy[s], zw = rec.zw[s];
   if (a[r].type < 0) xy.x = xy.y = zw.x = kNoAtom;  // out of reach of the vacancies' records too
-  const int ei = recSpecies64(zw.y);
+  const int ei = sp[s];
   const double dfi = a[r].df;
   double f0 = 0, f1 = 0, f2 = 0;
   forHookPart<kHookForceGroup>(*full, p, part, [&](const int32_t (&o)[kHookForceGroup], int nv) {
     double2 nxy[kHookForceGroup], nzw[kHookForceGroup];
+    int nsp[kHookForceGroup];
 #pragma unroll
     for (int u = 0; u < kHookForceGroup; ++u) {
       nxy[u] = rec.xy[s + o[u]];
       nzw[u] = rec.zw[s + o[u]];
+      nsp[u] = sp[s + o[u]];
     }
     bool in[kHookForceGroup];
     double q[kHookForceGroup], ri[kHookForceGroup];
@@ -182,7 +190,7 @@ __global__ __launch_bounds__(kHookBlock) void kHookForce(HookGeom G, const FullP
       if (in[u]) {
         ri[u] = rsqrtRefined(r2);
         const int m = knotOf(r2 > 0.0 ? r2 * ri[u] : 0.0, tb.rdr, tb.nr, false, q[u]);
-        const int ej = recSpecies64(nzw[u].y);
+        const int ej = nsp[u];
         const double2* k = reinterpret_cast<const double2*>(
             tb.pairF + (static_cast<int64_t>(ei * 3 + ej) * tb.nr + m) * kPairRec);
 #pragma unroll
@@ -239,7 +247,7 @@ HookGeom hookGeom(const Box& b, double rc) {
 }  // namespace
 
 void launchHook(int which, const Box& b, double rc, const FullPlaneOffsets* o, const Tables<double>& tb, Rec64 rec,
-                AtomElement* a, hipStream_t st) {
+                uint8_t* sp, AtomElement* a, hipStream_t st) {
   const HookGeom G = hookGeom(b, rc);
   const int64_t nsub = b.n[0] * b.n[1] * b.n[2];
   if (which == 1) {
@@ -247,11 +255,14 @@ void launchHook(int which, const Box& b, double rc, const FullPlaneOffsets* o, c
     return;
   }
   const dim3 grid(static_cast<unsigned>((nsub + 63) / 64), 2, 1);
-  kHookPack<<<static_cast<unsigned>((G.slots + kHookBlock - 1) / kHookBlock), kHookBlock, 0, st>>>(G, a, rec);
-  if (which == 0)
+  const unsigned packs = static_cast<unsigned>((G.slots + kHookBlock - 1) / kHookBlock);
+  if (which == 0) {
+    kHookPack<false><<<packs, kHookBlock, 0, st>>>(G, a, rec, sp);
     kHookRho<<<grid, kHookBlock, 0, st>>>(G, o, tb, rec, a);
-  else
-    kHookForce<<<grid, kHookBlock, 0, st>>>(G, o, tb, rec, a);
+  } else {
+    kHookPack<true><<<packs, kHookBlock, 0, st>>>(G, a, rec, sp);
+    kHookForce<<<grid, kHookBlock, 0, st>>>(G, o, tb, rec, sp, a);
+  }
 }
 
 }  // namespace misa
