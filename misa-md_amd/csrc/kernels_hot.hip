@@ -1710,7 +1710,7 @@ __global__ __launch_bounds__(kBlock) void kForceMP(Geom G, LatOffsets O, Tables<
                                                    Ctl* ctl, InterView iv, InterDev in, int mlo) {
   using Term = typename Sum3<ACC>::Term;
   __shared__ Term chunks[kChunks][3][64];
-  __shared__ double others[3][3][64];
+  __shared__ WaveSumsM others[3];
   __shared__ TailHits hits;
   if (blockIdx.x < kFrontBlocks) {
     interForceBody<float, MODE>(G, tb, iv, x, type, reinterpret_cast<const float*>(rec) + 3, 4, in, vp, frontWave(),
@@ -1736,9 +1736,11 @@ __global__ __launch_bounds__(kBlock) void kForceMP(Geom G, LatOffsets O, Tables<
     forceSumM<U>(O, tb, rec, dl, static_cast<float>(G.rc2), mlo, q.s, q.p, ei, me, b0, b1, sums, oth);
   }
   if (q.rg > 0) {
-    others[q.rg - 1][0][lane] = oth.x;
-    others[q.rg - 1][1][lane] = oth.y;
-    others[q.rg - 1][2][lane] = oth.z;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      others[q.rg - 1].hi[c][lane] = oth.hi[c];
+      others[q.rg - 1].lo[c][lane] = oth.lo[c];
+    }
   }
   findTailHits(hits, q.rg, iv, x.c, type, G.rc2, q.p, q.s, q.ti);
   __syncthreads();
@@ -1755,11 +1757,12 @@ __global__ __launch_bounds__(kBlock) void kForceMP(Geom G, LatOffsets O, Tables<
       acc.flush();
     }
 #pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      oth.x += others[r][0][lane];
-      oth.y += others[r][1][lane];
-      oth.z += others[r][2][lane];
-    }
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        oth.hi[c] += others[r].hi[c][lane];
+        oth.lo[c] += others[r].lo[c][lane];
+      }
     addOther3(acc, oth);
     forceTailM<ACC, MODE>(G, q.s, q.p, q.cx, q.cy, q.cz, q.ti, ei, me.w, acc, x, xn, type, rec, recn, v, f, id, vp,
                           st, ctl, tb, iv, vb, db, &hits);
@@ -1800,7 +1803,7 @@ __device__ __forceinline__ void forceVBlockL(const Geom& G, const LatOffsets& O,
                                              const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                              const uint64_t* __restrict__ id, const VerletParams& vp,
                                              const StageArgs& st, Ctl* ctl, const InterView& iv, const float4* dl,
-                                             const float4* offT, const float4* knT, int mlo, WaveQueueM& wq, WaveSums& ws, uint32_t b,
+                                             const float4* offT, const float4* knT, int mlo, WaveQueueM& wq, WaveSumsM& ws, uint32_t b,
                                              uint32_t tl, Shift shift, unsigned long long& vb,
                                              unsigned long long& db) {
   int64_t s = 0;
@@ -1865,7 +1868,10 @@ __device__ __forceinline__ void forceVBlockL(const Geom& G, const LatOffsets& O,
     while (qn >= least) {
       if (!sums) {
         sums = true;
-        for (int c = 0; c < 3; ++c) ws.s[c][threadIdx.x & 63u] = 0.0;
+        for (int c = 0; c < 3; ++c) {
+          ws.hi[c][threadIdx.x & 63u] = 0.0;
+          ws.lo[c][threadIdx.x & 63u] = 0;
+        }
       }
       waveLdsFence();
       const int n = qn < 64 ? qn : 64;
@@ -1886,9 +1892,10 @@ __device__ __forceinline__ void forceVBlockL(const Geom& G, const LatOffsets& O,
   OtherM oth;
   if (sums) {
     waveLdsFence();
-    oth.x = ws.s[0][threadIdx.x & 63u];
-    oth.y = ws.s[1][threadIdx.x & 63u];
-    oth.z = ws.s[2][threadIdx.x & 63u];
+    for (int c = 0; c < 3; ++c) {
+      oth.hi[c] = ws.hi[c][threadIdx.x & 63u];
+      oth.lo[c] = ws.lo[c][threadIdx.x & 63u];
+    }
   }
   if (!live) return;
   addOther3(acc, oth);
@@ -1929,7 +1936,7 @@ __global__ __launch_bounds__(kBlockP) void kForceL(Geom G, LatOffsets O, Tables<
                                                    unsigned long long* zwork) {
   __shared__ float4 offT[2 * kMaxLatOffsets];  // {lattice vector, record shift * 16}
   __shared__ WaveQueueM queues[kBlockP / 64];
-  __shared__ WaveSums sums[kBlockP / 64];
+  __shared__ WaveSumsM sums[kBlockP / 64];
   extern __shared__ float4 knT[];  // Fe-Fe r*phi cubics, Fe density slope cubics (fillKnots)
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   for (int i = threadIdx.x; i < 2 * kMaxLatOffsets; i += kBlockP) offT[i] = dl[2 * kMaxLatOffsets + i];
@@ -1963,7 +1970,7 @@ __global__ __launch_bounds__(kBlockP) void kForceLB(const BatchBox* __restrict__
                                                     int nkn) {
   __shared__ float4 offT[2 * kMaxLatOffsets];
   __shared__ WaveQueueM queues[kBlockP / 64];
-  __shared__ WaveSums sums[kBlockP / 64];
+  __shared__ WaveSumsM sums[kBlockP / 64];
   extern __shared__ float4 knT[];
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   for (int i = threadIdx.x; i < 2 * kMaxLatOffsets; i += kBlockP) offT[i] = dlp[i];
@@ -2005,10 +2012,10 @@ constexpr int kUDouble = 2;
 
 // LDS of the mixed force pass: kKnotsM knots (mixed_site.hpp) beside the
 // kernel's static LDS (the offset table, 4 KB, the queues, 18 KB, and the sums
-// of the pairs set aside, 24 KB) in the 160 KB of a compute unit.
+// of the pairs set aside, 36 KB) in the 160 KB of a compute unit.
 constexpr int kForceLdsBytes = 32 * kKnotsM;
 static_assert(kForceLdsBytes + 2 * kMaxLatOffsets * 16 +
-                      static_cast<int>(kBlockP / 64 * (sizeof(WaveQueueM) + sizeof(WaveSums))) <=
+                      static_cast<int>(kBlockP / 64 * (sizeof(WaveQueueM) + sizeof(WaveSumsM))) <=
                   160 * 1024,
               "the LDS of one block per compute unit");
 struct LdsKnots {

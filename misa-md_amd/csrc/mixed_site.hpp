@@ -97,12 +97,12 @@ __device__ __forceinline__ float pairFpM(float q, float rinv, const float4& z, c
   return -psip * rinv;
 }
 
-// Knots the mixed LDS force pass holds, from the last one down (1.55 A on where
+// Knots the mixed LDS force pass holds, from the last one down (1.94 A on where
 // the table has 5000 over 5.6 A).  The two cubics of a knot sit in arrays of
 // their own, so that the lanes' 16-byte reads spread over all banks (side by
 // side, either read met only every second group of four banks), at a distance
 // that fits the read's immediate offset.
-constexpr int kKnotsM = 3616;
+constexpr int kKnotsM = 3264;
 
 // Whether a pair is one that the LDS force passes hold segments for: two Fe
 // atoms at a knot from mlo on.  The others are summed apart (pair_queue.hpp).
@@ -205,7 +205,7 @@ __device__ __forceinline__ void forceGroupL(const float4& me, float dfi, int ei,
 template <typename Shift>
 __device__ __forceinline__ void drainQueueM(const uint16_t* q, int n, const float4& me, uint32_t o16, Rsrc rr,
                                             Rsrc rtab, Rsrc rtabD, const Tables<float>& tb, const float4* T,
-                                            Shift shift, WaveSums& ws) {
+                                            Shift shift, WaveSumsM& ws) {
 #pragma clang fp contract(off)
   const int lane = static_cast<int>(threadIdx.x & 63u);
   const bool on = lane < n;
@@ -232,9 +232,13 @@ __device__ __forceinline__ void drainQueueM(const uint16_t* q, int n, const floa
   const f32x3 si = ld3(rtabD, (__umul24(ei, nr) + m) * 16u);
   const float fp = pairFpM(pp, ri, zc, sj, si, ej == ei, own.w, nb.w, tb.rdr);
   if (on) {
-    ldsAdd(&ws.s[0][owner], gridTerm(d0, fp));
-    ldsAdd(&ws.s[1][owner], gridTerm(d1, fp));
-    ldsAdd(&ws.s[2][owner], gridTerm(d2, fp));
+    const float dd[3] = {d0, d1, d2};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const Term2 t = splitTerm(dd[c], fp);
+      ldsAdd(&ws.hi[c][owner], t.hi);
+      ldsAdd(&ws.lo[c][owner], t.lo);
+    }
   }
 }
 
@@ -242,18 +246,19 @@ __device__ __forceinline__ void drainQueueM(const uint16_t* q, int n, const floa
 // component (where it is not zero: a site without such pairs keeps its bits).
 template <int ACC>
 __device__ __forceinline__ void addOther3(Sum3<ACC>& acc, const OtherM& o) {
+  const double x = o.sum(0), y = o.sum(1), z = o.sum(2);
   if constexpr (ACC == 0) {
-    acc.f0 += o.x;
-    acc.f1 += o.y;
-    acc.f2 += o.z;
+    acc.f0 += x;
+    acc.f1 += y;
+    acc.f2 += z;
   } else if constexpr (ACC == 1) {
-    if (o.x != 0.0) acc.a.add(static_cast<float>(o.x));
-    if (o.y != 0.0) acc.b.add(static_cast<float>(o.y));
-    if (o.z != 0.0) acc.c.add(static_cast<float>(o.z));
+    if (x != 0.0) acc.a.add(static_cast<float>(x));
+    if (y != 0.0) acc.b.add(static_cast<float>(y));
+    if (z != 0.0) acc.c.add(static_cast<float>(z));
   } else {
-    acc.f0 += static_cast<float>(o.x);
-    acc.f1 += static_cast<float>(o.y);
-    acc.f2 += static_cast<float>(o.z);
+    acc.f0 += static_cast<float>(x);
+    acc.f1 += static_cast<float>(y);
+    acc.f2 += static_cast<float>(z);
   }
 }
 

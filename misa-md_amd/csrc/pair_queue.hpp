@@ -39,27 +39,49 @@ __device__ __forceinline__ void waveLdsFence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
-__device__ __forceinline__ void ldsAdd(double* p, double v) {
+template <typename T>
+__device__ __forceinline__ void ldsAdd(T* p, T v) {
   __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Mixed precision: the terms of the pairs set aside, as FP64 products of the
-// FP32 factors rounded to multiples of 2^-36 eV/A (1.5e-11, far below the
-// FP32 factors' own rounding), so that their FP64 sums are exact (up to
-// 2^17 eV/A) and do not depend on the order they are added in.
-constexpr double kTermGrid = 1.5 * 65536.0;
-__device__ __forceinline__ double gridTerm(float d, float fp) {
+// Mixed precision: the sum of the pairs set aside does not depend on the order
+// they are added in.  A term, the exact FP64 product t of two FP32 factors, is
+// taken apart into a multiple of 2^-32 eV/A and the rest in whole units of
+// 2^-56; an FP64 and an integer sum of those parts over a site's 128 offsets
+// are exact (for |t| below 2^19 eV/A), and the two meet in one rounding at the
+// end.  A term loses at most 2^-57 eV/A, less than FP64 additions in order lose
+// once a partial sum is above 0.1 eV/A, and keeps the bits of its FP32 factor
+// down to 1e-10 eV/A.  (In order instead, each lane over the noted pairs of its
+// site, kForceL took 370 to 410 us at 2M atoms against 300: the 58 pairs of one
+// atom of another species are then a chain that the other lanes wait for.)
+constexpr double kTermHi = 1.5 * 1048576.0;  // 1.5 x 2^20: the last bit of a sum with it is 2^-32
+constexpr double kTermLo = 0.09375;          // 1.5 x 2^-4: 2^-56
+constexpr double kLoUnit = 1.0 / 72057594037927936.0;
+struct Term2 {
+  double hi;
+  int lo;
+};
+__device__ __forceinline__ Term2 splitTerm(float d, float fp) {
 #pragma clang fp contract(off)
   const double t = static_cast<double>(d) * static_cast<double>(fp);
-  return (t + kTermGrid) - kTermGrid;
+  Term2 s;
+  s.hi = (t + kTermHi) - kTermHi;
+  s.lo = __double2loint((t - s.hi) + kTermLo);  // the low word of 1.5 x 2^52 + the units
+  return s;
 }
 struct OtherM {
-  double x = 0, y = 0, z = 0;
+  double hi[3] = {0, 0, 0};
+  int lo[3] = {0, 0, 0};
   __device__ __forceinline__ void add(float d0, float d1, float d2, float fp) {
-    x += gridTerm(d0, fp);
-    y += gridTerm(d1, fp);
-    z += gridTerm(d2, fp);
+    const float d[3] = {d0, d1, d2};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const Term2 t = splitTerm(d[c], fp);
+      hi[c] += t.hi;
+      lo[c] += t.lo;
+    }
   }
+  __device__ __forceinline__ double sum(int c) const { return __fma_rn(static_cast<double>(lo[c]), kLoUnit, hi[c]); }
 };
 
 // The queue of one wavefront: pairs as offset << 6 | lane.  Two groups of four
@@ -68,9 +90,14 @@ constexpr int kQueueM = 576;
 struct WaveQueueM {
   uint16_t q[kQueueM];
 };
-// Sums of the pairs set aside, per component and lane of the wavefront.
+// Sums of the pairs set aside, per component and lane of the wavefront; in
+// mixed precision of either part of their terms.
 struct WaveSums {
   double s[3][64];
+};
+struct WaveSumsM {
+  double hi[3][64];
+  int lo[3][64];
 };
 
 // FP64: the sums of the pairs set aside run over the offsets in order, one
