@@ -251,13 +251,19 @@ int misa_autotune(misa_handle* h, int64_t steps, int32_t* best_ty, double* best_
 int misa_set_launch_shape(misa_handle* h, int32_t ty, int32_t gathers_rho, int32_t gathers_force);
 int misa_get_launch_shape(const misa_handle* h, int32_t* ty, int32_t* gathers_rho, int32_t* gathers_force);
 /* Force passes (mixed and FP64) in persistent blocks that hold the majority
- * species' spline knots in LDS (the mixed pass also the pruned offsets):
- * MISA_LDS_AUTO (default; boxes whose sites fill the persistent launch, some
- * 260,000 atoms, with few enough solutes: 16 % in FP64, 35 % mixed), MISA_LDS_ON, MISA_LDS_OFF.  The FP64 density and energy
- * passes follow the same choice.  No counterpart in the
- * reference (a tuning switch of this build's kernels); the pairs, their
- * order and their rounding are the same either way, so results are
- * bit-identical. */
+ * species' spline knots in LDS (the mixed pass also the pruned offsets).
+ * MISA_LDS_AUTO (default): in boxes whose sites fill the persistent launch,
+ * some 260,000 atoms, and by the share of pairs whose knots LDS does not hold
+ * (a solute on either side, or, with more than some 5,000 knots, a distance
+ * below the first one held): while it is small those pairs go through a
+ * queue, beyond they are gathered under a mask, and where hardly any pair is
+ * held the passes from global memory run.  MISA_LDS_ON: the LDS passes with
+ * the queue, in every box.  MISA_LDS_OFF: none.  The FP64 density pass with
+ * its cubics in LDS goes by a share of its own, and runs with a neighbour skin
+ * only, after the first force evaluation; the energy pass goes by the size.
+ * No counterpart in the reference (a tuning switch of this build's kernels);
+ * the pairs, their order and their rounding are the same either way, so
+ * results are bit-identical. */
 #define MISA_LDS_AUTO 0
 #define MISA_LDS_ON 1
 #define MISA_LDS_OFF 2
@@ -281,15 +287,17 @@ int misa_set_xcd_slabs(misa_handle* h, const int32_t zlo[9]);
 /* The force pass the last force evaluation launched (-1 before any):
  * kForce (FP64) or kForceM (mixed) with spline segments from global memory
  * (kForceP and kForceMP in boxes of few sites count as these),
- * kForceL (mixed, persistent blocks with the majority species' segments in
- * LDS) or kForceDL (FP64, persistent blocks with the majority species'
- * segments in LDS).  The LDS passes run where MISA_LDS_* picks them; the
+ * kForceL (mixed) or kForceDL (FP64) in persistent blocks with the majority
+ * species' segments in LDS and a queue, kForceLG or kForceDG the same with
+ * masked gathers.  The LDS passes run where MISA_LDS_* picks them; the
  * library falls back to kForceM / kForce when the device refuses their LDS
  * size. */
 #define MISA_FORCE_PASS_FP64 0
 #define MISA_FORCE_PASS_MIXED 1
 #define MISA_FORCE_PASS_MIXED_LDS 2
 #define MISA_FORCE_PASS_FP64_LDS 3
+#define MISA_FORCE_PASS_MIXED_LDS_GATHER 4
+#define MISA_FORCE_PASS_FP64_LDS_GATHER 5
 int misa_force_pass_used(const misa_handle* h, int32_t* kind);
 /* The steps of the last misa_step call whose ownership pass (atom::decide) ran
  * in one workgroup (short lists in a box of few sites) and over a grid.  The

@@ -27,6 +27,7 @@ struct misa_handle {
   DevState s{};
   Offsets ref{};
   bool have_offsets = false;
+  std::vector<double> pairLengths;  // ideal lengths of the pruned pairs of one parity
   LatOffsets lat{};
   FullPlaneOffsets fullPlane{};
   float4 dlHost[2 * kMaxLatOffsets]{};  // lattice vectors of the pruned offsets (mixed records)
@@ -103,8 +104,13 @@ VerletParams verletOf(double dt) {  // NewtonMotion::preComputeDtInv2m (newton_m
   return vp;
 }
 
+void setNear(misa_handle* h) {
+  if (h->have_offsets && h->have_pot) setNearShares(h->s, h->pairLengths, h->box.rc, h->setfl.nr, h->setfl.dr);
+}
+
 int buildPlaneOffsets(misa_handle* h) {
   const Box& b = h->box;
+  h->pairLengths.clear();
   const double keep = b.f + 0.41;  // rc/a + 2 * 0.2 (max displacement) + 0.01 margin
   for (int p = 0; p < 2; p++) {
     const std::vector<int64_t>& L = p == 0 ? h->ref.even : h->ref.odd;
@@ -138,6 +144,7 @@ int buildPlaneOffsets(misa_handle* h) {
             make_float4(static_cast<float>((po.dcx + hdp) * b.a), static_cast<float>((po.dy + hdp) * b.a),
                         static_cast<float>((po.dz + hdp) * b.a), packedBits);
         h->lat.off[p][nl++] = static_cast<int32_t>(d);
+        if (p == 0) h->pairLengths.push_back(po.len * b.a);
       }
     }
     h->lat.n[p] = nl;
@@ -198,6 +205,7 @@ int buildPlaneOffsets(misa_handle* h) {
     if (e != hipSuccess) return fail(h, MISA_E_HIP, std::string("hipMemcpy offsets: ") + hipGetErrorString(e));
   }
   h->have_offsets = true;
+  setNear(h);
   h->gen++;
   return MISA_OK;
 }
@@ -684,6 +692,7 @@ int misa_set_potential_file(misa_handle* h, const char* path) {
   a32.rhoD = h->tab32 + oRhoD;
   a32.pairZ = h->tab32 + oPairZ;
   h->have_pot = true;
+  setNear(h);
   return MISA_OK;
 }
 
@@ -766,7 +775,9 @@ int misa_upload_state(misa_handle* h, const void* atoms, const void* inter, int6
   if (!h->aos_dev) HIPCHECK(h, hipMalloc(&h->aos_dev, bytes));
   HIPCHECK(h, hipMemcpyAsync(h->aos_dev, atoms, bytes, hipMemcpyHostToDevice, h->stream));
   h->s.cur = 0;
-  h->s.solutes = live > 0 ? static_cast<double>(solutes) / static_cast<double>(live) : 0.0;
+  const double share = live > 0 ? static_cast<double>(solutes) / static_cast<double>(live) : 0.0;
+  if (share != h->s.solutes) h->gen++;  // a captured step may take another force pass
+  h->s.solutes = share;
   launchUpload(h->s, h->aos_dev, b.sx, b.sy, h->stream);
   launchHaloAll(h->s, h->s.cur, h->stream);
   HIPCHECK(h, hipGetLastError());
@@ -1142,7 +1153,9 @@ int misa_step(misa_handle* h, int64_t nsteps) {
   HIPCHECK(h, hipGetLastError());
   HIPCHECK(h, hipEventRecord(e1, h->stream));
   const int rc = finishSteps(h, nsteps, e0, e1);
-  if (rc != MISA_OK || !measure || h->force_pass != MISA_FORCE_PASS_MIXED_LDS) return rc;
+  if (rc != MISA_OK || !measure ||
+      (h->force_pass != MISA_FORCE_PASS_MIXED_LDS && h->force_pass != MISA_FORCE_PASS_MIXED_LDS_GATHER))
+    return rc;
   return balanceSlabs(h);
 }
 
@@ -1361,33 +1374,7 @@ int buildFused(misa_batch* b) {
   for (int i = 0; i < n; i++) {
     misa_handle* h = b->hs[i];
     const DevState& s = h->s;
-    site::BatchBox& B = hb[i];
-    std::memset(&B, 0, sizeof(B));
-    B.G = s.G;
-    B.O = h->lat;
-    B.t32 = h->t32;
-    B.iv = interView(s, true);
-    B.in = s.in;
-    for (int c = 0; c < 2; c++)
-      for (int k = 0; k < 3; k++) B.x[c][k] = s.x[c][k];
-    for (int k = 0; k < 3; k++) {
-      B.v[k] = s.v[k];
-      B.f[k] = s.f[k];
-    }
-    B.type = s.type;
-    B.id = s.id;
-    B.rec[0] = s.rec[0];
-    B.rec[1] = s.rec[1];
-    B.dl = s.dl;
-    B.wmask = s.wmask;
-    B.smask = s.smask;
-    const double rcs = std::sqrt(s.G.rc2) + s.skin;
-    B.rcs2 = static_cast<float>(rcs * rcs);
-    B.skin = s.skin;
-    B.vp = verletOf(h->dt);
-    B.st = site::stageOf(s);
-    B.ctl = s.ctl;
-    B.cur = s.cur;
+    hb[i] = site::boxOf(s, h->lat, h->t32, interView(s, true), verletOf(h->dt));
     rs[i + 1] = rs[i] + site::siteGrid(s.G);
     vs[i + 1] = vs[i] + static_cast<uint32_t>(2 * s.G.W.bpx);
   }
@@ -1430,12 +1417,21 @@ int captureFused(misa_batch* b) {
   const misa_handle* h0 = b->hs[0];
   const int n = static_cast<int>(b->hs.size());
   BHIP(b, hipStreamBeginCapture(b->origin, hipStreamCaptureModeRelaxed));
+  double solutes = 0.0, sites = 0.0;
+  bool queue = true;  // asked for on every box
+  for (const misa_handle* h : b->hs) {
+    solutes += h->s.solutes * static_cast<double>(h->s.G.nsub);
+    sites += static_cast<double>(h->s.G.nsub);
+    queue = queue && h->s.lds == MISA_LDS_ON;
+  }
+  const LdsForm form = queue ? kLdsQueue : batchForceForm(solutes / sites, h0->s.nearM);
   bool lds = true;
   for (int f = 0; f < 2; f++) {
     launchInterBatch(0, b->boxes, n, f, nullptr, b->origin);
     launchRhoDfBatch(b->boxes, b->rhoStart, n, b->rhoBlocks, h0->acc, f, b->origin);
     launchInterBatch(1, b->boxes, n, f, nullptr, b->origin);
-    lds = lds && launchForceBatch(b->boxes, b->vstart, n, h0->s.dl, h0->t32.nr, h0->s.ncu, h0->acc, f, b->origin);
+    lds = lds && launchForceBatch(b->boxes, b->vstart, n, h0->s.dl, h0->t32.nr, h0->s.ncu, h0->acc, form, f,
+                                  b->origin);
     launchInterBatch(2, b->boxes, n, f ^ 1, b->decideArgs, b->origin);
   }
   const hipError_t e0 = hipGetLastError();

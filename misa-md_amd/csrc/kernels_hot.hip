@@ -40,6 +40,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <vector>
 
 #include "device_common.hpp"
 #include "inter_common.hpp"
@@ -667,10 +668,12 @@ __device__ __forceinline__ ForceSiteD forceSiteOf(const Geom& G, const LatOffset
                     mlo};
 }
 // The pairs of range rg (mask word w) of a site: the held ones into part, the
-// others into opart, in offset order.
-template <int U>
+// others into opart, in offset order.  With LDS the Fe-Fe segments from knot
+// first on come from knD (pairSegD).
+template <int U, bool LDS = false>
 __device__ __forceinline__ void forceRangeD(const ForceSiteD& c, const Tables<double>& tb, uint32_t w, int rg,
-                                            Force3& part, Force3& opart) {
+                                            Force3& part, Force3& opart, const double* knD = nullptr,
+                                            int first = 0) {
   auto group = [&](auto UC, const int* ks) {
     constexpr int V = decltype(UC)::value;
     double d0[V], d1[V], d2[V], wj[V];
@@ -697,7 +700,7 @@ __device__ __forceinline__ void forceRangeD(const ForceSiteD& c, const Tables<do
         const int m = knotM(r2 * ri[u], tb.rdr, tb.nr, pp[u]);
         const int ej = recSpecies64(wj[u]);
         held[u] = heldPair(c.ei, static_cast<uint32_t>(ej), m, c.mlo);
-        pairSegD<false>(c.rtab, c.rtabR, nullptr, 0, c.pairBase, tb.nr, c.ei, ej, m, rec[u], reci[u]);
+        pairSegD<LDS>(c.rtab, c.rtabR, knD, first, c.pairBase, tb.nr, c.ei, ej, m, rec[u], reci[u]);
       }
     }
 #pragma unroll
@@ -720,14 +723,15 @@ __device__ __forceinline__ void forceRangeD(const ForceSiteD& c, const Tables<do
 }
 
 // One site of the FP64 force pass, one wavefront over all its offsets.
-template <int MODE, int U>
+template <int MODE, int U, bool LDS = false>
 __device__ __forceinline__ void forceSiteD(const Geom& G, const LatOffsets& O, const Tables<double>& tb, CXPtr x,
                                            XPtr xn, const int8_t* __restrict__ type, const double* __restrict__ df,
                                            const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
                                            const uint64_t* __restrict__ id, const VerletParams& vp,
                                            const StageArgs& st, Ctl* ctl, const InterView& iv, const Rec64& r64,
                                            const Rec64& rn64, int mlo, uint32_t b, uint32_t tl,
-                                           unsigned long long& vb, unsigned long long& db) {
+                                           unsigned long long& vb, unsigned long long& db,
+                                           const double* knD = nullptr, int first = 0) {
   int64_t s;
   int p, cx, cy, cz;
   if (!siteOfBlock(G, b, tl, s, p, cx, cy, cz)) return;
@@ -743,7 +747,7 @@ __device__ __forceinline__ void forceSiteD(const Geom& G, const LatOffsets& O, c
   const uint64_t m0 = uniform64(wmask[2 * wv]), m1 = uniform64(wmask[2 * wv + 1]);
   for (int rg = 0; rg < 4; ++rg) {
     Force3 part, opart;
-    forceRangeD<U>(c, tb, maskWord(m0, m1, rg), rg, part, opart);
+    forceRangeD<U, LDS>(c, tb, maskWord(m0, m1, rg), rg, part, opart, knD, first);
     tot.add(part);
     otot.add(opart);
   }
@@ -1404,17 +1408,21 @@ __global__ __launch_bounds__(kBlock) void kEnergyD(Geom G, LatOffsets O, const F
                      vals);
   blockSumD<3, kBlock>(vals, partials + 3 * blockIdx.x);
 }
+// The Fe-Fe segments from knot mlo on, 7 doubles a knot (pairSegD).
+__device__ __forceinline__ void fillKnots7(const Tables<double>& tb, double* knD, int mlo, int nkn) {
+  const double* z = tb.pairF + static_cast<size_t>(mlo) * kPairRec;  // row (Fe, Fe) is the first
+  for (int i = threadIdx.x; i < 7 * nkn; i += kBlockP) {
+    const int k = i / 7, q = i - 7 * k;
+    knD[i] = z[static_cast<size_t>(k) * kPairRec + q];
+  }
+}
 __global__ __launch_bounds__(kBlockP) void kEnergyDL(Geom G, LatOffsets O, const FullPlaneOffsets* __restrict__ full,
                                                      Tables<double> tb, CXPtr x, const int8_t* __restrict__ type,
                                                      const double* __restrict__ rho, const double* __restrict__ df,
                                                      const uint64_t* __restrict__ smask, int all, Rec64 r64,
                                                      double* partials, int mlo, int nkn) {
   extern __shared__ double knD[];
-  const double* z = tb.pairF + static_cast<size_t>(mlo) * kPairRec;  // row (Fe, Fe) is the first
-  for (int i = threadIdx.x; i < 7 * nkn; i += kBlockP) {
-    const int k = i / 7, q = i - 7 * k;
-    knD[i] = z[static_cast<size_t>(k) * kPairRec + q];
-  }
+  fillKnots7(tb, knD, mlo, nkn);
   __syncthreads();
   double vals[3] = {0, 0, 0};
   forVirtualBlocks(G, [&](uint32_t b, uint32_t tl) {
@@ -1459,6 +1467,35 @@ __global__ __launch_bounds__(kBlockP) void kForceDL(Geom G, LatOffsets O, Tables
   forVirtualBlocks(G, [&](uint32_t b, uint32_t tl) {
     forceVBlockD<MODE, U>(G, O, tb, x, xn, type, df, wmask, v, f, id, vp, st, ctl, iv, r64, rn64, kn, mlo,
                           queues[wave], sums[wave], b, tl, vb, db);
+  });
+  if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
+  if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
+}
+
+// The FP64 force pass in persistent blocks with the Fe-Fe segments from knot
+// `first` on in LDS (7 doubles a knot) and the other pairs' gathered under a
+// mask, a lane each (forceSiteD): the form where so many pairs are not held
+// that their queue costs more than the load slots of the masked gathers.
+template <int MODE, int U>
+__global__ __launch_bounds__(kBlockP) void kForceDG(Geom G, LatOffsets O, Tables<double> tb, CXPtr x, XPtr xn,
+                                                    const int8_t* __restrict__ type, const double* __restrict__ df,
+                                                    const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
+                                                    const uint64_t* __restrict__ id, VerletParams vp, StageArgs st,
+                                                    Ctl* ctl, InterView iv, InterDev in, Rec64 r64, Rec64 rn64,
+                                                    int mlo, int first, int nkn) {
+  extern __shared__ double knD[];
+  fillKnots7(tb, knD, first, nkn);
+  __syncthreads();
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  interForceBody<double, MODE>(G, tb, iv, x, type, df, 1, in, vp, static_cast<int>(wave * gridDim.x + blockIdx.x),
+                               static_cast<int>(gridDim.x) * (kBlockP / 64));
+  unsigned long long vb = 0, db = 0;
+  forVirtualBlocks(G, [&](uint32_t b, uint32_t tl) {
+    unsigned long long vbs = 0, dbs = 0;
+    forceSiteD<MODE, U, true>(G, O, tb, x, xn, type, df, wmask, v, f, id, vp, st, ctl, iv, r64, rn64, mlo, b, tl, vbs,
+                              dbs, knD, first);
+    vb = vbs > vb ? vbs : vb;
+    db = dbs > db ? dbs : db;
   });
   if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
   if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
@@ -1738,7 +1775,7 @@ __global__ __launch_bounds__(kBlock) void kForceMP(Geom G, LatOffsets O, Tables<
   if (q.rg > 0) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      others[q.rg - 1].hi[c][lane] = oth.hi[c];
+      others[q.rg - 1].hi[c][lane] = oth.hi(c);
       others[q.rg - 1].lo[c][lane] = oth.lo[c];
     }
   }
@@ -1759,10 +1796,7 @@ __global__ __launch_bounds__(kBlock) void kForceMP(Geom G, LatOffsets O, Tables<
 #pragma unroll
     for (int r = 0; r < 3; ++r)
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        oth.hi[c] += others[r].hi[c][lane];
-        oth.lo[c] += others[r].lo[c][lane];
-      }
+      for (int c = 0; c < 3; ++c) oth.join(c, others[r].hi[c][lane], others[r].lo[c][lane]);
     addOther3(acc, oth);
     forceTailM<ACC, MODE>(G, q.s, q.p, q.cx, q.cy, q.cz, q.ti, ei, me.w, acc, x, xn, type, rec, recn, v, f, id, vp,
                           st, ctl, tb, iv, vb, db, &hits);
@@ -1892,10 +1926,7 @@ __device__ __forceinline__ void forceVBlockL(const Geom& G, const LatOffsets& O,
   OtherM oth;
   if (sums) {
     waveLdsFence();
-    for (int c = 0; c < 3; ++c) {
-      oth.hi[c] = ws.hi[c][threadIdx.x & 63u];
-      oth.lo[c] = ws.lo[c][threadIdx.x & 63u];
-    }
+    for (int c = 0; c < 3; ++c) oth.join(c, ws.hi[c][threadIdx.x & 63u], ws.lo[c][threadIdx.x & 63u]);
   }
   if (!live) return;
   addOther3(acc, oth);
@@ -1906,14 +1937,64 @@ __device__ __forceinline__ void forceVBlockL(const Geom& G, const LatOffsets& O,
   db = dbs > db ? dbs : db;
 }
 
+// One virtual block of the gather form of the LDS force pass: per site the same
+// pairs and sums as kForceM, the Fe-Fe segments from knot `first` on from LDS
+// (forceGroupG), as are the offsets' lattice vectors (offT).
+template <int ACC, int MODE, int U, typename Shift>
+__device__ __forceinline__ void forceVBlockG(const Geom& G, const LatOffsets& O, const Tables<float>& tb, CXPtr x,
+                                             XPtr xn, const int8_t* __restrict__ type,
+                                             const float4* __restrict__ rec, float4* __restrict__ recn,
+                                             const uint64_t* __restrict__ wmask, XPtr v, XPtr f,
+                                             const uint64_t* __restrict__ id, const VerletParams& vp,
+                                             const StageArgs& st, Ctl* ctl, const InterView& iv, const float4* offT,
+                                             const float4* knT, int mlo, int first, uint32_t b, uint32_t tl,
+                                             Shift shift, unsigned long long& vb, unsigned long long& db) {
+  int64_t s;
+  int p, cx, cy, cz;
+  if (!siteOfBlock(G, b, tl, s, p, cx, cy, cz)) return;
+  const int8_t ti = type[s];
+  if (isVacant(ti)) {  // vacancy: keeps its stale position (atom.cpp:43-47)
+    vacancyForceM<MODE>(G, s, p, cx, cy, cz, x, xn, recn, f);
+    return;
+  }
+  const Rsrc rr = rsrcBelow(rec, O.lo);
+  const float rc2 = static_cast<float>(G.rc2);
+  const int ei = species(ti);
+  const float4 me = rec[s];
+  const uint32_t o16 = static_cast<uint32_t>(s) * 16u;
+  const uint32_t pairBase = static_cast<uint32_t>(ei * 3) * static_cast<uint32_t>(tb.nr);
+  const float4* T = offT + p * kMaxLatOffsets;
+  Sum3<ACC> acc;
+  OtherM oth;
+  const uint32_t wv = b * (kBlock / 64) + __builtin_amdgcn_readfirstlane(tl >> 6);
+  // a group's entries past the mask's last offset get a lattice vector out
+  // of range: beyond the cutoff, they add nothing
+  forMaskGroupsFull<U>(uniform64(wmask[2 * wv]), uniform64(wmask[2 * wv + 1]), [&](const int* ks, const bool* act) {
+    float4 nb[U], d[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) d[u] = T[act[u] ? ks[u] : kPadOffset];
+#pragma unroll
+    for (int u = 0; u < U; ++u) nb[u] = ldRec4(rr, o16 + shift(d[u].w), 0);
+    forceGroupG(me, ei, pairBase, nb, d, rc2, tb, knT, mlo, first, ks, acc, oth);
+  });
+  flushChunk3(acc);
+  addOther3(acc, oth);
+  unsigned long long vbs = 0, dbs = 0;
+  forceTailM<ACC, MODE>(G, s, p, cx, cy, cz, ti, ei, me.w, acc, x, xn, type, rec, recn, v, f, id, vp, st, ctl, tb,
+                        iv, vbs, dbs);
+  vb = vbs > vb ? vbs : vb;
+  db = dbs > db ? dbs : db;
+}
+
 // The LDS knots of the force pass, the Fe-Fe r*phi cubics from knot mlo on and
-// kKnotsM entries further the Fe density slope cubics (one block fills them).
+// SLOPES entries further the Fe density slope cubics (one block fills them).
+template <int SLOPES = kKnotsM>
 __device__ __forceinline__ void fillKnots(const Tables<float>& tb, float4* knT, int mlo, int nkn) {
   const float4* z4 = reinterpret_cast<const float4*>(tb.pairZ);  // row (Fe, Fe) is the first
   const float4* s4 = reinterpret_cast<const float4*>(tb.rhoD);   // row Fe is the first
   for (int i = threadIdx.x; i < nkn; i += kBlockP) {
     knT[i] = z4[mlo + i];
-    knT[kKnotsM + i] = s4[mlo + i];
+    knT[SLOPES + i] = s4[mlo + i];
   }
 }
 
@@ -1958,6 +2039,82 @@ __global__ __launch_bounds__(kBlockP) void kForceL(Geom G, LatOffsets O, Tables<
   if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
 }
 
+// The box record that is a kernel's first argument, read from the argument
+// segment where it is used.  Arguments by value are loaded at the start and
+// keep scalar registers to their last use; in kForceLG they left too few for
+// the lane masks of the loop over the pairs, which then spilled to lanes (twice
+// the instructions).
+__device__ __forceinline__ const BatchBox& boxArgument() {
+  auto p = (const __attribute__((address_space(4))) BatchBox*)__builtin_amdgcn_kernarg_segment_ptr();
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(p));
+#endif
+  return *(const BatchBox*)p;
+}
+
+// kForceL's gather form, for boxes with many pairs that are not held: the
+// masked gathers of forceGroupG in place of the queue, whose room in LDS holds
+// knots instead (4,988, from 0.01 A on where the table has 5000 over 5.6 A).
+template <int ACC, int MODE, int U>
+__global__ __launch_bounds__(kBlockP) void kForceLG(BatchBox, int mlo, int first, int nkn,
+                                                    unsigned long long* zwork) {
+  __shared__ float4 offT[2 * kMaxLatOffsets];
+  extern __shared__ float4 knT[];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  {
+    const BatchBox& B = boxArgument();
+    const int c = B.cur;
+    for (int i = threadIdx.x; i < 2 * kMaxLatOffsets; i += kBlockP) offT[i] = B.dl[2 * kMaxLatOffsets + i];
+    fillKnots<kKnotsG>(B.t32, knT, first, nkn);
+    interForceBody<float, MODE>(B.G, B.t32, B.iv, cxp(B.x[c]), B.type, reinterpret_cast<const float*>(B.rec[c]) + 3,
+                                4, B.in, B.vp, static_cast<int>(wave * gridDim.x + blockIdx.x),
+                                static_cast<int>(gridDim.x) * (kBlockP / 64));
+  }
+  __syncthreads();
+  unsigned long long vb = 0, db = 0;
+  const RecShift shift;
+  forVirtualBlocks(boxArgument().G, [&](uint32_t b, uint32_t tl) {
+    const long long t0 = zwork ? clock64() : 0;
+    const BatchBox& B = boxArgument();
+    const int c = B.cur;
+    forceVBlockG<ACC, MODE, U>(B.G, B.O, B.t32, cxp(B.x[c]), xp(B.x[1 - c]), B.type, B.rec[c], B.rec[1 - c], B.wmask,
+                               xp(B.v), xp(B.f), B.id, B.vp, B.st, B.ctl, B.iv, offT, knT, mlo, first, b, tl, shift, vb, db);
+    if (zwork) addPlaneWork(B.G, zwork, b, tl, t0);
+  });
+  const BatchBox& B = boxArgument();
+  if (MODE == 0 && B.vp.vmax) waveMaxTo(vb, B.vp.vmax);
+  if (MODE == 1) waveMaxTo(db, &B.ctl->dispmax2);
+}
+
+// Walks the virtual blocks of a batch's persistent launch: on each XCD those of
+// box 0, then box 1, ...  body(box, block of the box, thread, maxima).
+template <int MODE, typename Body>
+__device__ __forceinline__ void forBatchBlocks(const BatchBox* __restrict__ boxes, const uint32_t* vstart, int nbox,
+                                               Body body) {
+  constexpr uint32_t V = kBlockP / kBlock;
+  const uint32_t c = blockIdx.x & 7u, q = blockIdx.x >> 3, Q = gridDim.x >> 3;
+  const uint32_t sub = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlock);
+  const uint32_t tl = threadIdx.x % kBlock;
+  const uint32_t nvb = vstart[nbox];
+  unsigned long long vb = 0, db = 0;
+  int lastBox = -1;
+  const auto close = [&] {  // the maxima go to the box they came from
+    if (lastBox < 0) return;
+    if (MODE == 0 && boxes[lastBox].vp.vmax) waveMaxTo(vb, boxes[lastBox].vp.vmax);
+    if (MODE == 1) waveMaxTo(db, &boxes[lastBox].ctl->dispmax2);
+  };
+  for (uint32_t k = q * V + sub; k < nvb; k += Q * V) {
+    const int bi = boxOfBlock(vstart, nbox, k);
+    if (bi != lastBox) {
+      close();
+      vb = db = 0;
+      lastBox = bi;
+    }
+    body(boxes[bi], c + 8u * (k - vstart[bi]), tl, vb, db);
+  }
+  close();
+}
+
 // The LDS force pass of every box of a batch in one persistent launch: on
 // each XCD the blocks walk the virtual blocks of box 0, then box 1, ...
 // (vstart[b] counts the virtual blocks per XCD before box b).  All boxes
@@ -1976,35 +2133,33 @@ __global__ __launch_bounds__(kBlockP) void kForceLB(const BatchBox* __restrict__
   for (int i = threadIdx.x; i < 2 * kMaxLatOffsets; i += kBlockP) offT[i] = dlp[i];
   fillKnots(boxes[0].t32, knT, mlo, nkn);
   __syncthreads();
-  constexpr uint32_t V = kBlockP / kBlock;
-  const uint32_t c = blockIdx.x & 7u, q = blockIdx.x >> 3, Q = gridDim.x >> 3;
-  const uint32_t sub = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlock);
-  const uint32_t tl = threadIdx.x % kBlock;
-  const uint32_t nvb = vstart[nbox];
-  unsigned long long vb = 0, db = 0;
-  int lastBox = -1;
-  for (uint32_t k = q * V + sub; k < nvb; k += Q * V) {
-    const int bi = boxOfBlock(vstart, nbox, k);
-    const BatchBox& B = boxes[bi];
-    if (bi != lastBox) {  // the maxima go to the box they came from
-      if (lastBox >= 0) {
-        if (MODE == 0 && boxes[lastBox].vp.vmax) waveMaxTo(vb, boxes[lastBox].vp.vmax);
-        if (MODE == 1) waveMaxTo(db, &boxes[lastBox].ctl->dispmax2);
-      }
-      vb = db = 0;
-      lastBox = bi;
-    }
+  forBatchBlocks<MODE>(boxes, vstart, nbox, [&](const BatchBox& B, uint32_t b, uint32_t tl, unsigned long long& vb,
+                                                unsigned long long& db) {
     const int cb = B.cur ^ flip;
-    const int32_t plane = static_cast<int32_t>(B.G.plane), NX = B.G.NX, NY = B.G.NY, lo = B.O.lo;
-    const PackedShift shift{plane, NX, NY, lo};
+    const PackedShift shift{static_cast<int32_t>(B.G.plane), B.G.NX, B.G.NY, B.O.lo};
     forceVBlockL<ACC, MODE, U>(B.G, B.O, B.t32, cxp(B.x[cb]), xp(B.x[1 - cb]), B.type, B.rec[cb], B.rec[1 - cb],
                                B.wmask, xp(B.v), xp(B.f), B.id, B.vp, B.st, B.ctl, B.iv, dlp, offT, knT, mlo,
-                               queues[wave], sums[wave], c + 8u * (k - vstart[bi]), tl, shift, vb, db);
-  }
-  if (lastBox >= 0) {
-    if (MODE == 0 && boxes[lastBox].vp.vmax) waveMaxTo(vb, boxes[lastBox].vp.vmax);
-    if (MODE == 1) waveMaxTo(db, &boxes[lastBox].ctl->dispmax2);
-  }
+                               queues[wave], sums[wave], b, tl, shift, vb, db);
+  });
+}
+// Its gather form (forceVBlockG).
+template <int ACC, int MODE, int U>
+__global__ __launch_bounds__(kBlockP) void kForceLGB(const BatchBox* __restrict__ boxes, const uint32_t* vstart,
+                                                     int nbox, int flip, const float4* __restrict__ dlp, int mlo,
+                                                     int first, int nkn) {
+  __shared__ float4 offT[2 * kMaxLatOffsets];
+  extern __shared__ float4 knT[];
+  for (int i = threadIdx.x; i < 2 * kMaxLatOffsets; i += kBlockP) offT[i] = dlp[i];
+  fillKnots<kKnotsG>(boxes[0].t32, knT, first, nkn);
+  __syncthreads();
+  forBatchBlocks<MODE>(boxes, vstart, nbox, [&](const BatchBox& B, uint32_t b, uint32_t tl, unsigned long long& vb,
+                                                unsigned long long& db) {
+    const int cb = B.cur ^ flip;
+    const PackedShift shift{static_cast<int32_t>(B.G.plane), B.G.NX, B.G.NY, B.O.lo};
+    forceVBlockG<ACC, MODE, U>(B.G, B.O, B.t32, cxp(B.x[cb]), xp(B.x[1 - cb]), B.type, B.rec[cb], B.rec[1 - cb],
+                               B.wmask, xp(B.v), xp(B.f), B.id, B.vp, B.st, B.ctl, B.iv, offT, knT, mlo, first, b, tl,
+                               shift, vb, db);
+  });
 }
 
 // Offsets a group in the FP64 force passes.
@@ -2063,6 +2218,19 @@ LdsKnots ldsKnotsEnergy(int nr) {
   k.bytes = static_cast<size_t>(56) * static_cast<size_t>(k.nkn);
   return k;
 }
+// The FP64 force pass's gather form: the same 7 doubles a knot.
+constexpr int kForceLdsBytesDG = kEnergyLdsBytes;
+LdsKnots ldsKnotsForceDG(int nr) { return ldsKnotsEnergy(nr); }
+// The mixed force pass's gather form: kKnotsG knots beside the offset table.
+constexpr int kForceLdsBytesG = 32 * kKnotsG;
+static_assert(kForceLdsBytesG + 2 * kMaxLatOffsets * 16 <= 160 * 1024, "the LDS of one block per compute unit");
+LdsKnots ldsKnotsForceG(int nr) {
+  LdsKnots k;
+  k.nkn = std::min(nr, kKnotsG);
+  k.mlo = nr - k.nkn;
+  k.bytes = kForceLdsBytesG;
+  return k;
+}
 bool setLdsBytes(const void* fn, int bytes) {
   return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
 }
@@ -2074,16 +2242,51 @@ unsigned persistentGrid(const DevState& s) { return static_cast<unsigned>(s.ncu 
 // 4096 wavefronts): at 60^3 cells FP64 156 against 216 us, mixed 83 against
 // 108; at 50^3 148 against 163 and 81 against 80; at 40^3, half the
 // wavefronts idle, 83 against 73 and 46 against 43.
-// The queued pairs cost more than the masked gathers of the other passes where
-// they are many: 80^3 cells, FP64 with 3 / 10 / 25 / 60 % solutes 507 / 626 / 866
-// / 1262 us a step with LDS against 683 / 720 / 779 / 883, mixed 284 / 327 / 439
-// / 617 against 328 / 371 / 458 / 555.
-constexpr double kSolutesD = 0.16, kSolutesM = 0.35;
-bool useLds(const DevState& s, double most = 1.0) {
+bool useLds(const DevState& s) {
   if (s.ncu < 8 || s.lds == kLdsOff) return false;
   if (s.lds == kLdsOn) return true;
-  if (s.solutes > most) return false;
   return static_cast<int64_t>(siteGrid(s.G)) * kBlock >= static_cast<int64_t>(persistentGrid(s)) * kBlockP;
+}
+// Which form: by the share of pairs whose segments LDS does not hold, those
+// with a solute and, where the knots held begin beyond the nearest neighbours,
+// the like pairs below them.  The queue wins while they are few, masked gathers
+// beyond, and the pass from global memory where next to nothing is held.
+// 108^3 cells (2.5M atoms), 300 K, us with queue / gathers / neither, by
+// solutes and by knots over 5.6 A (80^3 crosses over at the same shares):
+//                      5000             10000             20000
+//   FP64    0 %   505/ 537/ 986    718/ 626/1034   1203/1035/1077
+//         1.5 %   665/ 781/1083    988/ 865/1161   1397/1236/1299
+//           6 %   844/ 814/1131   1153/ 913/1222   1540/1349/1401
+//          15 %  1122/ 857/1197   1389/1008/1314   1735/1591/1590
+//          25 %  1394/ 945/1252   1641/1222/1396   1931/1793/1770
+//          60 %  2000/1474/1403   2137/1721/1555   2333/2149/2055
+//   mixed   0 %   313/ 311/ 435    463/ 358/ 533    743/ 475/ 778
+//         1.5 %   373/ 445/ 498    516/ 459/ 594    796/ 566/ 815
+//           6 %   448/ 467/ 531    585/ 494/ 675    916/ 647/ 903
+//          15 %   572/ 491/ 622    749/ 545/ 834   1099/ 781/1054
+//          60 %  1092/ 761/ 931   1358/ 950/1176   1597/1198/1377
+//         100 %  (80^3)  - / 313/ 284
+// A batch of 15 boxes, mixed, us a step with queue / gathers: 332/354 at 1.5 %,
+// 354/365 at 6, 380/367 at 10, 586/483 at 60; 406/388 on 10000 knots.
+double unheld(double solutes, double near) {
+  const double like = (1.0 - solutes) * (1.0 - solutes);
+  return 1.0 - like * (1.0 - near);
+}
+constexpr double kQueueShareD = 0.08, kGatherShareD = 0.83, kQueueShareM = 0.145, kGatherShareM = 0.985;
+LdsForm forceForm(const DevState& s, bool mixed) {
+  if (!useLds(s)) return kLdsNone;
+  if (s.lds == kLdsOn) return kLdsQueue;
+  if (unheld(s.solutes, mixed ? s.nearM : s.nearD) <= (mixed ? kQueueShareM : kQueueShareD))
+    return kLdsQueue;
+  return unheld(s.solutes, mixed ? 0.0 : s.nearDG) <= (mixed ? kGatherShareM : kGatherShareD) ? kLdsGather : kLdsNone;
+}
+// The FP64 density pass has no gather form: LDS cubics and queue against
+// neither, by solutes, the same boxes: 0 % 380/576, 6 % 506/594, 15 % 594/616,
+// 25 % 717/637; 10000 knots 0 % 564/641, 1.5 % 662/652, 6 % 710/662; 20000
+// knots 755/731.
+constexpr double kQueueShareRho = 0.17;
+bool rhoLdsPays(const DevState& s) {
+  return s.lds == kLdsOn || s.solutes + (1.0 - s.solutes) * 0.5 * s.nearRhoD <= kQueueShareRho;
 }
 
 // Boxes whose sites fill at most this many wavefronts (64 sites each) take the
@@ -2094,6 +2297,23 @@ bool useShared(const DevState& s) {
 }
 
 }  // namespace
+
+void setNearShares(DevState& s, const std::vector<double>& lengths, double rc, int nr, double dr) {
+  // a shell counts in proportion where the first knot lies within 0.15 A of it
+  const auto share = [&](int mlo) {
+    double below = 0.0, all = 0.0;
+    for (const double len : lengths) {
+      if (len >= rc) continue;
+      all += 1.0;
+      below += std::min(1.0, std::max(0.0, (mlo * dr - len) / 0.3 + 0.5));
+    }
+    return all > 0.0 ? below / all : 0.0;
+  };
+  s.nearD = share(ldsKnotsForceD(nr).mlo);
+  s.nearDG = share(ldsKnotsForceDG(nr).mlo);
+  s.nearRhoD = share(ldsKnotsRhoD(nr).mlo);
+  s.nearM = share(ldsKnotsForce(nr).mlo);
+}
 
 void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
                  bool mixed, int acc, bool store_rho, bool scan, hipStream_t st) {
@@ -2111,7 +2331,7 @@ void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t
     // against 117 us, 100^3 372 against 483, with 6 % solutes at 900 K 60^3 123
     // against 134, 90^3 344 against 397; where every pass scans all offsets
     // (766 000 atoms) 257 against 238, so those stay with kRhoDf.
-    if (useLds(s, kSolutesD) && ldsReady && !scan && s.skin > 0.0)
+    if (useLds(s) && rhoLdsPays(s) && ldsReady && !scan && s.skin > 0.0)
       kRhoDL<kURhoD><<<persistentGrid(s), kBlockP, lk.bytes, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask,
                                                                    s.smask, rcs * rcs, iv, s.in, r64, lk.mlo, lk.nkn);
     else if (shared)
@@ -2158,19 +2378,26 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
   const XPtr xn = xp(s.x[1 - s.cur]);
   const StageArgs sa = stageOf(s);
   const InterView iv = interView(s, mixed);
-  const bool lds = useLds(s, mixed ? kSolutesM : kSolutesD);
-  const LdsKnots lk = ldsKnotsForce(t32.nr);
-  const LdsKnots lkd = ldsKnotsForceD(t64.nr);
+  const LdsForm form = forceForm(s, mixed);
+  const LdsKnots lk = ldsKnotsForce(t32.nr), lg = ldsKnotsForceG(t32.nr);
+  const LdsKnots lkd = ldsKnotsForceD(t64.nr), lgd = ldsKnotsForceDG(t64.nr);
 #define MISA_FORCE(M)                                                                                         \
   do {                                                                                                        \
-    static const bool ldsReady =                                                                              \
+    static const bool queueReady =                                                                            \
         setLdsBytes(reinterpret_cast<const void*>(&kForceDL<M, kUDouble>), kForceLdsBytesD);                 \
+    static const bool gatherReady =                                                                           \
+        setLdsBytes(reinterpret_cast<const void*>(&kForceDG<M, kUDouble>), kForceLdsBytesDG);                \
     const Rec64 r64{s.pxy[s.cur], s.pzw[s.cur]}, rn64{s.pxy[1 - s.cur], s.pzw[1 - s.cur]};                   \
-    if (lds && ldsReady) {                                                                                    \
+    if (form == kLdsQueue && queueReady) {                                                                    \
       kind = 3;                                                                                               \
       kForceDL<M, kUDouble><<<persistentGrid(s), kBlockP, lkd.bytes, st>>>(                                   \
           s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv, s.in, r64,   \
           rn64, lkd.mlo, lkd.nkn);                                                                            \
+    } else if (form == kLdsGather && gatherReady) {                                                           \
+      kind = 5;                                                                                               \
+      kForceDG<M, kUDouble><<<persistentGrid(s), kBlockP, lgd.bytes, st>>>(                                   \
+          s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v), xp(s.f), s.id, vp, sa, s.ctl, iv, s.in, r64,   \
+          rn64, lkd.mlo, lgd.mlo, lgd.nkn);                                                                   \
     } else if (shared) {                                                                                      \
       kForceP<M, kUDouble><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, xn, s.type, s.df64, s.wmask, xp(s.v), \
                                                     xp(s.f), s.id, vp, sa, s.ctl, iv, s.in, r64, rn64,    \
@@ -2183,13 +2410,19 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
   } while (0)
 #define MISA_FORCE_MU(A, M, U)                                                                                \
   do {                                                                                                        \
-    static const bool ldsReady =                                                                              \
+    static const bool queueReady =                                                                            \
         setLdsBytes(reinterpret_cast<const void*>(&kForceL<A, M, U>), kForceLdsBytes);                       \
-    if (lds && ldsReady) {                                                                                    \
+    static const bool gatherReady =                                                                           \
+        setLdsBytes(reinterpret_cast<const void*>(&kForceLG<A, M, U>), kForceLdsBytesG);                     \
+    if (form == kLdsQueue && queueReady) {                                                                    \
       kind = 2;                                                                                               \
       kForceL<A, M, U><<<persistentGrid(s), kBlockP, lk.bytes, st>>>(                                         \
           s.G, o, t32, x, xn, s.type, s.rec[s.cur], s.rec[1 - s.cur], s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, \
           sa, s.ctl, iv, s.in, lk.mlo, lk.nkn, s.zmeasure ? s.zwork : nullptr);                                     \
+    } else if (form == kLdsGather && gatherReady) {                                                           \
+      kind = 4;                                                                                               \
+      kForceLG<A, M, U><<<persistentGrid(s), kBlockP, lg.bytes, st>>>(                                        \
+          boxOf(s, o, t32, iv, vp), lk.mlo, lg.mlo, lg.nkn, s.zmeasure ? s.zwork : nullptr);                  \
     } else if (shared) {                                                                                      \
       kForceMP<A, M, U><<<grid, kBlock, 0, st>>>(s.G, o, t32, x, xn, s.type, s.rec[s.cur],                \
                                                      s.rec[1 - s.cur], s.dl, s.wmask, xp(s.v), xp(s.f), s.id, vp, \
@@ -2255,15 +2488,25 @@ void launchRhoDfBatch(const BatchBox* boxes, const uint32_t* rhoStart, int nbox,
   else kRhoDfMB<2, 4><<<blocks, kBlock, 0, st>>>(boxes, rhoStart, nbox, flip);
 }
 
+LdsForm batchForceForm(double solutes, double nearM) {
+  return unheld(solutes, nearM) <= kQueueShareM ? kLdsQueue : kLdsGather;
+}
+
 bool launchForceBatch(const BatchBox* boxes, const uint32_t* vstart, int nbox, const float4* dl, int nr, int ncu,
-                      int acc, int flip, hipStream_t st) {
-  const LdsKnots lk = ldsKnotsForce(nr);
+                      int acc, LdsForm form, int flip, hipStream_t st) {
+  const LdsKnots lk = ldsKnotsForce(nr), lg = ldsKnotsForceG(nr);
   const unsigned grid = static_cast<unsigned>(ncu / 8 * 8);
 #define MISA_FORCE_B(A)                                                                                      \
   do {                                                                                                       \
-    static const bool ready = setLdsBytes(reinterpret_cast<const void*>(&kForceLB<A, 1, 4>), kForceLdsBytes); \
-    if (!ready) return false;                                                                                \
-    kForceLB<A, 1, 4><<<grid, kBlockP, lk.bytes, st>>>(boxes, vstart, nbox, flip, dl, lk.mlo, lk.nkn);        \
+    static const bool queueReady =                                                                           \
+        setLdsBytes(reinterpret_cast<const void*>(&kForceLB<A, 1, 4>), kForceLdsBytes);                      \
+    static const bool gatherReady =                                                                          \
+        setLdsBytes(reinterpret_cast<const void*>(&kForceLGB<A, 1, 4>), kForceLdsBytesG);                    \
+    if (!queueReady || !gatherReady) return false;                                                           \
+    if (form == kLdsQueue)                                                                                   \
+      kForceLB<A, 1, 4><<<grid, kBlockP, lk.bytes, st>>>(boxes, vstart, nbox, flip, dl, lk.mlo, lk.nkn);      \
+    else                                                                                                     \
+      kForceLGB<A, 1, 4><<<grid, kBlockP, lg.bytes, st>>>(boxes, vstart, nbox, flip, dl, lk.mlo, lg.mlo, lg.nkn); \
   } while (0)
   if (acc == 0) MISA_FORCE_B(0);
   else if (acc == 1) MISA_FORCE_B(1);

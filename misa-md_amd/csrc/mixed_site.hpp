@@ -103,6 +103,8 @@ __device__ __forceinline__ float pairFpM(float q, float rinv, const float4& z, c
 // side, either read met only every second group of four banks), at a distance
 // that fits the read's immediate offset.
 constexpr int kKnotsM = 3264;
+// and those of its gather form, which keeps no queue.
+constexpr int kKnotsG = 4988;
 
 // Whether a pair is one that the LDS force passes hold segments for: two Fe
 // atoms at a knot from mlo on.  The others are summed apart (pair_queue.hpp).
@@ -195,6 +197,73 @@ __device__ __forceinline__ void forceGroupL(const float4& me, float dfi, int ei,
         wq.q[qn + laneRank(other[u])] = static_cast<uint16_t>((ks[u] << 6) | (threadIdx.x & 63u));
       qn += __builtin_popcountll(other[u]);
     }
+  addGroup3(acc, ks, d0, d1, d2, fp);
+}
+
+// The entry at a byte offset of a table, by a base in two scalar registers: the
+// four of a buffer descriptor are too many where LDS pointers, cuts and masks
+// fill the rest (spilled to lanes, they cost twice the pass's instructions).
+template <typename T>
+__device__ __forceinline__ T tableAt(const float* base, uint32_t off) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + off);
+}
+
+// forceGroupM with the Fe-Fe r*phi cubics and the Fe density slope cubics from
+// knot `first` on in LDS (kKnotsG entries apart): every lane reads its segments
+// there, at a clamped knot; a lane whose pair involves another species, or lies
+// below that knot, then re-reads what it needs from global memory, in a branch
+// that only a wavefront with such a lane enters (after the LDS reads, so that
+// no global load waits in front of them).
+template <typename Acc, int V>
+__device__ __forceinline__ void forceGroupG(const float4& me, int ei, uint32_t pairBase, const float4 (&nb)[V],
+                                            const float4 (&d)[V], float rc2,
+                                            const Tables<float>& tb, const float4* knT, int mlo, int first,
+                                            const int* ks, Acc& acc, OtherM& oth) {
+#pragma clang fp contract(off)
+  bool in[V], like[V], held[V], re[V];
+  float d0[V], d1[V], d2[V], pp[V], ri[V];
+  int mm[V];
+  uint32_t ejv[V];
+  float4 zc[V];
+  f32x3 sj[V], si[V];
+  bool any = false;
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    const float r2 = dist2M(me, nb[u], d[u], d0[u], d1[u], d2[u]);
+    in[u] = r2 < rc2;
+    ri[u] = __builtin_amdgcn_rsqf(r2);
+    mm[u] = knotM(r2 * ri[u], tb.rdr, tb.nr, pp[u]);
+    ejv[u] = static_cast<uint32_t>(recSpecies(nb[u].x));
+    like[u] = ejv[u] == static_cast<uint32_t>(ei);
+    held[u] = in[u] && heldPair(ei, ejv[u], mm[u], mlo);
+    const float4* kn = knT + (max(mm[u], first) - first);
+    zc[u] = kn[0];
+    const float4 s4 = kn[kKnotsG];
+    sj[u] = f32x3{s4.x, s4.y, s4.z};
+    si[u] = sj[u];
+    re[u] = in[u] && ((static_cast<uint32_t>(ei) | ejv[u]) != 0u || mm[u] < first);
+    any |= re[u];
+  }
+  if (__ballot(any)) {  // the pair needs r*phi from memory; the slopes as their species or knot say
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      if (!re[u]) continue;
+      const bool low = mm[u] < first;
+      const uint32_t rowj = __umul24(ejv[u], static_cast<uint32_t>(tb.nr)) + static_cast<uint32_t>(mm[u]);
+      zc[u] = tableAt<float4>(tb.pairZ, (pairBase + rowj) * 16u);
+      if (ejv[u] != 0u || low) sj[u] = tableAt<f32x3>(tb.rhoD, rowj * 16u);
+      if (!like[u] && (ei != 0 || low))
+        si[u] = tableAt<f32x3>(tb.rhoD, (__umul24(static_cast<uint32_t>(ei), static_cast<uint32_t>(tb.nr)) +
+                                         static_cast<uint32_t>(mm[u])) * 16u);
+    }
+  }
+  float fp[V];
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    const float f = pairFpM(pp[u], ri[u], zc[u], sj[u], si[u], like[u], me.w, nb[u].w, tb.rdr);
+    if (in[u] && !held[u]) oth.add(d0[u], d1[u], d2[u], f);
+    fp[u] = held[u] ? f : 0.0f;
+  }
   addGroup3(acc, ks, d0, d1, d2, fp);
 }
 

@@ -48,7 +48,7 @@ __device__ __forceinline__ void ldsAdd(T* p, T v) {
 // they are added in.  A term, the exact FP64 product t of two FP32 factors, is
 // taken apart into a multiple of 2^-32 eV/A and the rest in whole units of
 // 2^-56; an FP64 and an integer sum of those parts over a site's 128 offsets
-// are exact (for |t| below 2^19 eV/A), and the two meet in one rounding at the
+// are exact (for sums below 2^19 eV/A), and the two meet in one rounding at the
 // end.  A term loses at most 2^-57 eV/A, less than FP64 additions in order lose
 // once a partial sum is above 0.1 eV/A, and keeps the bits of its FP32 factor
 // down to 1e-10 eV/A.  (In order instead, each lane over the noted pairs of its
@@ -63,25 +63,35 @@ struct Term2 {
 };
 __device__ __forceinline__ Term2 splitTerm(float d, float fp) {
 #pragma clang fp contract(off)
-  const double t = static_cast<double>(d) * static_cast<double>(fp);
+  const double x = static_cast<double>(d), f = static_cast<double>(fp);
   Term2 s;
-  s.hi = (t + kTermHi) - kTermHi;
-  s.lo = __double2loint((t - s.hi) + kTermLo);  // the low word of 1.5 x 2^52 + the units
+  s.hi = __fma_rn(x, f, kTermHi) - kTermHi;
+  s.lo = __double2loint(__fma_rn(x, f, kTermLo - s.hi));  // the low word of 1.5 x 2^52 + the units
   return s;
 }
+// A lane's sum.  The FP64 part starts at kTermHi and so rounds every term to
+// the grid as it is added (a tie may go the other way than in splitTerm; the
+// rest makes up for it).
 struct OtherM {
-  double hi[3] = {0, 0, 0};
+  double a[3] = {kTermHi, kTermHi, kTermHi};
   int lo[3] = {0, 0, 0};
   __device__ __forceinline__ void add(float d0, float d1, float d2, float fp) {
+#pragma clang fp contract(off)
     const float d[3] = {d0, d1, d2};
+    const double f = static_cast<double>(fp);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const Term2 t = splitTerm(d[c], fp);
-      hi[c] += t.hi;
-      lo[c] += t.lo;
+      const double x = static_cast<double>(d[c]), v = __fma_rn(x, f, a[c]), h = v - a[c];
+      a[c] = v;
+      lo[c] += __double2loint(__fma_rn(x, f, kTermLo - h));
     }
   }
-  __device__ __forceinline__ double sum(int c) const { return __fma_rn(static_cast<double>(lo[c]), kLoUnit, hi[c]); }
+  __device__ __forceinline__ double hi(int c) const { return a[c] - kTermHi; }
+  __device__ __forceinline__ void join(int c, double h, int l) {
+    a[c] += h;
+    lo[c] += l;
+  }
+  __device__ __forceinline__ double sum(int c) const { return __fma_rn(static_cast<double>(lo[c]), kLoUnit, hi(c)); }
 };
 
 // The queue of one wavefront: pairs as offset << 6 | lane.  Two groups of four

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 #include "device_common.hpp"
 #include "host_setup.hpp"
@@ -54,6 +55,9 @@ struct InterDev {
   FullPlaneOffsets* full = nullptr;
 };
 
+// Force passes without segments in LDS, with the pairs that are not held in a
+// queue, and with masked gathers for them.
+enum LdsForm { kLdsNone, kLdsQueue, kLdsGather };
 // Choice of the LDS-table force pass (the values of MISA_LDS_AUTO / ON / OFF).
 constexpr int kLdsAuto = 0, kLdsOn = 1, kLdsOff = 2;
 
@@ -87,6 +91,9 @@ struct DevState {
   int ncu = 0;
   int lds = 0;  // kLdsAuto, kLdsOn, kLdsOff
   double solutes = 0.0;  // share of the uploaded lattice atoms that are not Fe
+  // share of a site's pairs in the ideal lattice that lie below the first knot
+  // held in LDS, per pass (setNearShares)
+  double nearD = 0.0, nearDG = 0.0, nearRhoD = 0.0, nearM = 0.0;
   // neighbour skin of the mixed density pass (A; 0: every step scans all
   // pruned offsets) and, per wavefront, the pruned offsets within cutoff +
   // skin for some lane at the last full scan (2 words)
@@ -120,6 +127,9 @@ struct VerletParams {
 void launchUpload(const DevState& s, const AtomElement* aos_dev, int64_t sx, int64_t sy, hipStream_t st);
 void launchDownload(const DevState& s, AtomElement* aos_dev, int64_t sx, int64_t sy, bool mixed, hipStream_t st);
 void launchHaloAll(const DevState& s, int buf, hipStream_t st);
+// The shares of near pairs for the choice of the LDS passes, from the ideal
+// lengths of a site's pairs and the potential's grid.
+void setNearShares(DevState& s, const std::vector<double>& lengths, double rc, int nr, double dr);
 // The density pass of the inter atoms and the lattice in one launch, and the
 // force pass of both.  Force modes: 0 f stored, v += c f (secondstep); 1 and
 // the next first half step (for the lattice with the decide's staging); 2 f
@@ -127,8 +137,8 @@ void launchHaloAll(const DevState& s, int buf, hipStream_t st);
 // scan: this density pass goes over all offsets (no skin masks yet).
 void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
                  bool mixed, int acc, bool store_rho, bool scan, hipStream_t st);
-// Returns the force pass launched: 0 kForce (FP64), 1 kForceM, 2 kForceL (the
-// values of MISA_FORCE_PASS_*).
+// Returns the force pass launched: 0 kForce (FP64), 1 kForceM, 2 kForceL, 3
+// kForceDL, 4 kForceLG, 5 kForceDG (the values of MISA_FORCE_PASS_*).
 int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
                 bool mixed, int acc, int mode, const VerletParams& vp, hipStream_t st);
 void launchFirst(const DevState& s, bool mixed, const VerletParams& vp, hipStream_t st);
@@ -197,6 +207,9 @@ void launchInterBatch(int which, const site::BatchBox* boxes, int nbox, int flip
 void launchRhoDfBatch(const site::BatchBox* boxes, const uint32_t* rhoStart, int nbox, unsigned blocks, int acc,
                       int flip, hipStream_t st);
 bool launchForceBatch(const site::BatchBox* boxes, const uint32_t* vstart, int nbox, const float4* dl, int nr,
-                      int ncu, int acc, int flip, hipStream_t st);
+                      int ncu, int acc, LdsForm form, int flip, hipStream_t st);
+// The form that pays for a batch with this share of solutes and of near pairs
+// (DevState::nearM).
+LdsForm batchForceForm(double solutes, double nearM);
 
 }  // namespace misa

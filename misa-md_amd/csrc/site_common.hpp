@@ -604,6 +604,36 @@ inline StageArgs stageOf(const DevState& s) {
   }
   return a;
 }
+// The record of a box for a force pass on its current buffers.
+inline BatchBox boxOf(const DevState& s, const LatOffsets& o, const Tables<float>& t32, const InterView& iv,
+                      const VerletParams& vp) {
+  BatchBox B{};
+  B.G = s.G;
+  B.O = o;
+  B.t32 = t32;
+  B.iv = iv;
+  B.in = s.in;
+  for (int c = 0; c < 2; c++)
+    for (int k = 0; k < 3; k++) B.x[c][k] = s.x[c][k];
+  for (int k = 0; k < 3; k++) {
+    B.v[k] = s.v[k];
+    B.f[k] = s.f[k];
+  }
+  B.type = s.type;
+  B.id = s.id;
+  B.rec[0] = s.rec[0];
+  B.rec[1] = s.rec[1];
+  B.dl = s.dl;
+  B.wmask = s.wmask;
+  B.smask = s.smask;
+  B.rcs2 = static_cast<float>((std::sqrt(s.G.rc2) + s.skin) * (std::sqrt(s.G.rc2) + s.skin));
+  B.skin = s.skin;
+  B.vp = vp;
+  B.st = stageOf(s);
+  B.ctl = s.ctl;
+  B.cur = s.cur;
+  return B;
+}
 
 
 }  // namespace site

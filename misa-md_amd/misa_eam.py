@@ -344,7 +344,8 @@ class EamDevice:
                     "misa_set_launch_shape")
 
     def set_lds_tables(self, mode):
-        """LDS_AUTO, LDS_ON or LDS_OFF: the passes with their majority-species tables in LDS."""
+        """LDS_AUTO, LDS_ON (with a queue for the other pairs) or LDS_OFF: the passes with their
+        majority-species tables in LDS."""
         self._check(self.lib.misa_set_lds_tables(self.h, int(mode)), "misa_set_lds_tables")
 
     def defect_counters(self):
@@ -357,7 +358,8 @@ class EamDevice:
         """Name of the force kernel the last force evaluation launched."""
         k = ctypes.c_int32()
         self._check(self.lib.misa_force_pass_used(self.h, ctypes.byref(k)), "misa_force_pass_used")
-        return {0: "kForce", 1: "kForceM", 2: "kForceL", 3: "kForceDL"}.get(k.value, "none")
+        return {0: "kForce", 1: "kForceM", 2: "kForceL", 3: "kForceDL", 4: "kForceLG",
+                5: "kForceDG"}.get(k.value, "none")
 
     def decide_forms(self):
         """Steps of the last step() call with the decide in one workgroup, and over a grid."""
