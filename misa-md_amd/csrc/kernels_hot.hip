@@ -73,8 +73,12 @@ __device__ __forceinline__ uint32_t waveId(uint32_t b) {
 // The site passes carry the inter atoms' work of the same pass along, in their
 // first kFrontBlocks blocks (a multiple of 8, so that the others keep their
 // XCD): neither part reads what the other writes, and a launch of its own for
-// a list that is mostly empty costs 2 to 5 us.
-constexpr uint32_t kFrontBlocks = 64;
+// a list that is mostly empty costs 2 to 5 us.  With no inter atom 64 blocks
+// and 256 take the same step (2 000 to 93 000 atoms, 36 to 71 us); with many of
+// them 64 are too few wavefronts, a wavefront working one atom off after the
+// other (93 000 atoms FP64: 4 000 inter atoms 766 -> 603 us a step, 12 000 3174 ->
+// 2481; 755 and 2689 in launches of their own).
+constexpr uint32_t kFrontBlocks = 256;
 __device__ __forceinline__ int frontWave() {
   return static_cast<int>(blockIdx.x * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
 }
