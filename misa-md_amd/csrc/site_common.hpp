@@ -430,6 +430,7 @@ struct Sum3;
 template <>
 struct Sum3<0> {
   using Term = double;
+  static constexpr bool kFiniteOnly = false;
   double f0 = 0, f1 = 0, f2 = 0;
   double g0 = 0, g1 = 0, g2 = 0;
   int chunk = 0;
@@ -450,6 +451,7 @@ struct Sum3<0> {
 template <>
 struct Sum3<1> {
   using Term = float;
+  static constexpr bool kFiniteOnly = true;
   Sum1<1> a, b, c;
   float g0 = 0, g1 = 0, g2 = 0;
   int chunk = 0;
@@ -470,6 +472,7 @@ struct Sum3<1> {
 template <>
 struct Sum3<2> {
   using Term = float;
+  static constexpr bool kFiniteOnly = false;
   float f0 = 0, f1 = 0, f2 = 0;
   float g0 = 0, g1 = 0, g2 = 0;
   int chunk = 0;
@@ -491,6 +494,7 @@ constexpr int kChunks = 16;  // chunks of eight offsets of a wavefront's 128-bit
 template <int ACC>
 struct ChunkSums {
   using Term = typename Sum3<ACC>::Term;
+  static constexpr bool kFiniteOnly = Sum3<ACC>::kFiniteOnly;
   Term g0 = 0, g1 = 0, g2 = 0;
   int chunk;
   Term (*out)[3][64];
@@ -504,8 +508,11 @@ struct ChunkSums {
 };
 // The force terms of a group of lattice neighbours (ks[u]: its offset, the
 // same in every lane, ascending over a site's groups).  fp is 0 for a
-// neighbour that does not count and the displacements are finite (a
-// vacancy's too), so such a term adds an exact zero.
+// neighbour that does not count, and its term an exact zero where the
+// displacement is finite (a vacancy's too).  An atom uploaded without a finite
+// FP32 displacement is within no cutoff; with compensated sums (kFiniteOnly)
+// it fails the call all the same, by the products with 0 in its neighbours'
+// sums, in the other modes it counts for none of them.
 template <typename Acc, int V>
 __device__ __forceinline__ void addGroup3(Acc& acc, const int* ks, const float (&d0)[V], const float (&d1)[V],
                                           const float (&d2)[V], const float (&fp)[V]) {
@@ -519,9 +526,10 @@ __device__ __forceinline__ void addGroup3(Acc& acc, const int* ks, const float (
       acc.chunk = t;
     }
     const T f = static_cast<T>(fp[u]);
-    acc.g0 = __builtin_elementwise_fma(static_cast<T>(d0[u]), f, acc.g0);
-    acc.g1 = __builtin_elementwise_fma(static_cast<T>(d1[u]), f, acc.g1);
-    acc.g2 = __builtin_elementwise_fma(static_cast<T>(d2[u]), f, acc.g2);
+    const bool counts = Acc::kFiniteOnly || fp[u] != 0.0f;
+    acc.g0 = __builtin_elementwise_fma(static_cast<T>(counts ? d0[u] : 0.0f), f, acc.g0);
+    acc.g1 = __builtin_elementwise_fma(static_cast<T>(counts ? d1[u] : 0.0f), f, acc.g1);
+    acc.g2 = __builtin_elementwise_fma(static_cast<T>(counts ? d2[u] : 0.0f), f, acc.g2);
   }
 }
 template <typename Acc>
