@@ -434,11 +434,12 @@ def main():
         log("developing the cascade to %.2f ps (FP32-mixed, untimed)" % args.develop_ps)
         dstate, t_dev, dev_steps = develop_cascade(dev, state, site, args.pka_energy, args.develop_ps)
         del state
-        runs, launched = {}, {}
+        runs, launched, launched_rho = {}, {}, {}
         for name, mode in (("fp64", M.PREC_FP64), ("mixed", MIXED)):
             log("%s run, developed cascade" % name)
             runs[name] = run_developed(dev, dstate, mode, args.steps, args.warmup)
             launched[name] = dev.force_pass()
+            launched_rho[name] = dev.density_pass()
         del dstate
         log("force error")
         fmax, frms, f_scale = force_error(dev)
@@ -470,11 +471,13 @@ def main():
 
     kernels = {
         "mixed": {"force_kernel": launched["mixed"], "force_ms": avg_force_ms, "force_GBs": achieved,
-                  "rho_kernel": "kRhoDfM", "rho_ms": avg_rho_ms, "rho_GBs": gbs(RHO_BYTES["mixed"], avg_rho_ms),
+                  "rho_kernel": launched_rho["mixed"], "rho_ms": avg_rho_ms,
+                  "rho_GBs": gbs(RHO_BYTES["mixed"], avg_rho_ms),
                   "other_ms_per_step": t32["other_ms"] / args.steps, "share_of_step": shares(t32, s32)},
         "fp64": {"force_kernel": launched["fp64"], "force_ms": avg_force64,
                  "force_GBs": gbs(FORCE_BYTES["fp64"], avg_force64),
-                 "rho_kernel": "kRhoDL", "rho_ms": avg_rho64, "rho_GBs": gbs(RHO_BYTES["fp64"], avg_rho64),
+                 "rho_kernel": launched_rho["fp64"], "rho_ms": avg_rho64,
+                 "rho_GBs": gbs(RHO_BYTES["fp64"], avg_rho64),
                  "other_ms_per_step": t64["other_ms"] / args.steps, "share_of_step": shares(t64, s64)},
     }
     res = {

@@ -299,6 +299,13 @@ int misa_set_xcd_slabs(misa_handle* h, const int32_t zlo[9]);
 #define MISA_FORCE_PASS_MIXED_LDS_GATHER 4
 #define MISA_FORCE_PASS_FP64_LDS_GATHER 5
 int misa_force_pass_used(const misa_handle* h, int32_t* kind);
+/* The density pass of the last force evaluation (-1 before any): kRhoDf (FP64)
+ * or kRhoDfM (mixed) with the cubics from global memory (kRhoDfP and kRhoDfMP
+ * in boxes of few sites count as these), or kRhoDL (FP64, cubics in LDS). */
+#define MISA_DENSITY_PASS_FP64 0
+#define MISA_DENSITY_PASS_MIXED 1
+#define MISA_DENSITY_PASS_FP64_LDS 2
+int misa_density_pass_used(const misa_handle* h, int32_t* kind);
 /* The steps of the last misa_step call whose ownership pass (atom::decide) ran
  * in one workgroup (short lists in a box of few sites) and over a grid.  The
  * same lists in the same order either way. */

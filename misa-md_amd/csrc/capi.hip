@@ -61,6 +61,7 @@ struct misa_handle {
   double timings[4] = {0, 0, 0, 0};
   int64_t launches[3] = {0, 0, 0};
   int force_pass = -1;       // MISA_FORCE_PASS_* of the last force pass launched
+  int density_pass = -1;     // MISA_DENSITY_PASS_* of the last density pass launched
   bool range_check = false;  // a density beyond the F(rho) table fails the call
   int64_t flags_seen = 0;    // the device flags at the last check
   int64_t decides[2] = {0, 0};  // of the last misa_step: in one workgroup, over a grid
@@ -954,7 +955,7 @@ static void forcePass(misa_handle* h, int mode, bool store_rho, const VerletPara
   const bool mixed = h->precision == MISA_PREC_MIXED;
   {
     Timer t(h, 0);
-    launchRhoDf(h->s, h->lat, h->t64, h->t32, mixed, h->acc, store_rho, mode == 2, h->stream);
+    h->density_pass = launchRhoDf(h->s, h->lat, h->t64, h->t32, mixed, h->acc, store_rho, mode == 2, h->stream);
     h->mask_gen = h->gen;
   }
   {
@@ -1722,6 +1723,12 @@ int misa_defect_counters(misa_handle* h, int64_t out[3]) {
 int misa_force_pass_used(const misa_handle* h, int32_t* kind) {
   if (!h || !kind) return MISA_E_ARG;
   *kind = h->force_pass;
+  return MISA_OK;
+}
+
+int misa_density_pass_used(const misa_handle* h, int32_t* kind) {
+  if (!h || !kind) return MISA_E_ARG;
+  *kind = h->density_pass;
   return MISA_OK;
 }
 

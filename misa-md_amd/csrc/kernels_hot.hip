@@ -2319,8 +2319,8 @@ void setNearShares(DevState& s, const std::vector<double>& lengths, double rc, i
   s.nearM = share(ldsKnotsForce(nr).mlo);
 }
 
-void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
-                 bool mixed, int acc, bool store_rho, bool scan, hipStream_t st) {
+int launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
+                bool mixed, int acc, bool store_rho, bool scan, hipStream_t st) {
   double* rho = store_rho ? s.rho : nullptr;
   const bool shared = useShared(s);
   const unsigned grid = kFrontBlocks + (shared ? 4 : 1) * siteGrid(s.G);
@@ -2335,10 +2335,12 @@ void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t
     // against 117 us, 100^3 372 against 483, with 6 % solutes at 900 K 60^3 123
     // against 134, 90^3 344 against 397; where every pass scans all offsets
     // (766 000 atoms) 257 against 238, so those stay with kRhoDf.
-    if (useLds(s) && rhoLdsPays(s) && ldsReady && !scan && s.skin > 0.0)
+    if (useLds(s) && rhoLdsPays(s) && ldsReady && !scan && s.skin > 0.0) {
       kRhoDL<kURhoD><<<persistentGrid(s), kBlockP, lk.bytes, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask,
                                                                    s.smask, rcs * rcs, iv, s.in, r64, lk.mlo, lk.nkn);
-    else if (shared)
+      return 2;
+    }
+    if (shared)
       kRhoDfP<4><<<grid, kBlock, 0, st>>>(s.G, o, t64, x, s.type, s.df64, rho, s.wmask, s.smask, rcs * rcs, iv, s.in,
                                           r64, lk.mlo);
     else
@@ -2371,6 +2373,7 @@ void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t
     }
 #undef MISA_RHO_M
   }
+  return mixed ? 1 : 0;
 }
 
 int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,

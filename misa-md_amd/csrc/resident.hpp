@@ -134,9 +134,10 @@ void setNearShares(DevState& s, const std::vector<double>& lengths, double rc, i
 // force pass of both.  Force modes: 0 f stored, v += c f (secondstep); 1 and
 // the next first half step (for the lattice with the decide's staging); 2 f
 // stored only.
-// scan: this density pass goes over all offsets (no skin masks yet).
-void launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
-                 bool mixed, int acc, bool store_rho, bool scan, hipStream_t st);
+// scan: this density pass goes over all offsets (no skin masks yet).  Returns
+// the density pass launched: 0 kRhoDf, 1 kRhoDfM, 2 kRhoDL (MISA_DENSITY_PASS_*).
+int launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,
+                bool mixed, int acc, bool store_rho, bool scan, hipStream_t st);
 // Returns the force pass launched: 0 kForce (FP64), 1 kForceM, 2 kForceL, 3
 // kForceDL, 4 kForceLG, 5 kForceDG (the values of MISA_FORCE_PASS_*).
 int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t64, const Tables<float>& t32,

@@ -141,6 +141,7 @@ _SIGS = {
     "misa_set_launch_shape": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32]),
     "misa_set_lds_tables": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32]),
     "misa_force_pass_used": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int32)]),
+    "misa_density_pass_used": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int32)]),
     "misa_decide_forms_used": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int64)]),
     "misa_set_xcd_balance": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32]),
     "misa_xcd_slabs": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int32)]),
@@ -360,6 +361,12 @@ class EamDevice:
         self._check(self.lib.misa_force_pass_used(self.h, ctypes.byref(k)), "misa_force_pass_used")
         return {0: "kForce", 1: "kForceM", 2: "kForceL", 3: "kForceDL", 4: "kForceLG",
                 5: "kForceDG"}.get(k.value, "none")
+
+    def density_pass(self):
+        """Name of the density kernel the last force evaluation launched."""
+        k = ctypes.c_int32()
+        self._check(self.lib.misa_density_pass_used(self.h, ctypes.byref(k)), "misa_density_pass_used")
+        return {0: "kRhoDf", 1: "kRhoDfM", 2: "kRhoDL"}.get(k.value, "none")
 
     def decide_forms(self):
         """Steps of the last step() call with the decide in one workgroup, and over a grid."""
