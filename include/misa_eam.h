@@ -253,7 +253,7 @@ int misa_get_launch_shape(const misa_handle* h, int32_t* ty, int32_t* gathers_rh
 /* Force passes (mixed and FP64) in persistent blocks that hold the majority
  * species' spline knots in LDS (the mixed pass also the pruned offsets).
  * MISA_LDS_AUTO (default): in boxes whose sites fill the persistent launch,
- * some 260,000 atoms, and by the share of pairs whose knots LDS does not hold
+ * some 330,000 atoms, and by the share of pairs whose knots LDS does not hold
  * (a solute on either side, or, with more than some 5,000 knots, a distance
  * below the first one held): while it is small those pairs go through a
  * queue, beyond they are gathered under a mask, and where hardly any pair is

@@ -2241,15 +2241,17 @@ bool setLdsBytes(const void* fn, int bytes) {
 // One persistent block per compute unit, a whole number per XCD.
 unsigned persistentGrid(const DevState& s) { return static_cast<unsigned>(s.ncu / 8 * 8); }
 // The LDS-table passes: on request, or by default where the sites fill the
-// wavefronts of the persistent launch, 16 a compute unit, at least once.
-// Force pass against the one from global memory (its form for few sites up to
-// 4096 wavefronts): at 60^3 cells FP64 156 against 216 us, mixed 83 against
-// 108; at 50^3 148 against 163 and 81 against 80; at 40^3, half the
-// wavefronts idle, 83 against 73 and 46 against 43.
+// persistent launch, 16 wavefronts a compute unit, one and a quarter times.  Just
+// above once, its second round is nearly empty.  Step FP64 / mixed, with LDS
+// against without: 60^3 cells, 1.65 times, 206/304 and 142/174 us, 6 % solutes
+// 277/340 and 165/188; 56^3, 1.34 times, 208/247 and 139/149, 6 % 275/279 and
+// 158/155; 52x51x53, 1.07 times, 205/213 and 131/126, 6 % 277/246 and 151/135.
+bool fillsLaunch(const DevState& s, double times) {
+  return static_cast<double>(siteGrid(s.G)) * kBlock >= times * persistentGrid(s) * kBlockP;
+}
 bool useLds(const DevState& s) {
   if (s.ncu < 8 || s.lds == kLdsOff) return false;
-  if (s.lds == kLdsOn) return true;
-  return static_cast<int64_t>(siteGrid(s.G)) * kBlock >= static_cast<int64_t>(persistentGrid(s)) * kBlockP;
+  return s.lds == kLdsOn || fillsLaunch(s, 1.25);
 }
 // Which form: by the share of pairs whose segments LDS does not hold, those
 // with a solute and, where the knots held begin beyond the nearest neighbours,
@@ -2282,7 +2284,12 @@ LdsForm forceForm(const DevState& s, bool mixed) {
   if (s.lds == kLdsOn) return kLdsQueue;
   if (unheld(s.solutes, mixed ? s.nearM : s.nearD) <= (mixed ? kQueueShareM : kQueueShareD))
     return kLdsQueue;
-  return unheld(s.solutes, mixed ? 0.0 : s.nearDG) <= (mixed ? kGatherShareM : kGatherShareD) ? kLdsGather : kLdsNone;
+  if (mixed) return unheld(s.solutes, 0.0) <= kGatherShareM ? kLdsGather : kLdsNone;
+  // With half of the pairs or more gathered, FP64 gains some 8 %, which a last
+  // round of few blocks takes back: 56^3 cells, 1.3 rounds, 20000 knots 301 us a
+  // step against 281 without LDS.
+  const double share = unheld(s.solutes, s.nearDG);
+  return share <= 0.5 || (share <= kGatherShareD && fillsLaunch(s, 2.0)) ? kLdsGather : kLdsNone;
 }
 // The FP64 density pass has no gather form: LDS cubics and queue against
 // neither, by solutes, the same boxes: 0 % 380/576, 6 % 506/594, 15 % 594/616,

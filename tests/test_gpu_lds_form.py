@@ -77,6 +77,16 @@ def test_automatic_form(potentials, precision, cells, ratio, nr, want):
     b.close()
 
 
+@pytest.mark.parametrize("precision,plain,lds", [(M.PREC_FP64, "kForce", "kForceDL"),
+                                                 (M.PREC_MIXED_KAHAN, "kForceM", "kForceL")])
+def test_boxes_about_as_large_as_the_persistent_launch(potentials, precision, plain, lds):
+    """Sites that fill it a little more than once leave its second round empty."""
+    for cells, want in (((50, 50, 50), plain), ((52, 51, 53), plain), ((56, 56, 56), lds)):
+        dev = _box(potentials[5000], cells, DILUTE, precision, M.LDS_AUTO, 100.0)
+        assert dev.force_pass() == want, cells
+        dev.close()
+
+
 @pytest.mark.parametrize("precision", [M.PREC_MIXED, M.PREC_MIXED_KAHAN, M.PREC_MIXED_F32SUM])
 @pytest.mark.parametrize("ratio,nr", [(DILUTE, 5000), (MOST, 5000), (NONE, 5000), (FE, 20000)])
 def test_batch_forms_end_on_the_bits_of_single_boxes(potentials, precision, ratio, nr):
