@@ -309,8 +309,11 @@ __device__ __forceinline__ void rhoTailD(const Geom& G, int64_t s, int p, int cx
   });
 }
 
+// (Two sums, for the neighbours held in LDS elsewhere and for the others, need
+// more registers than one: bound to seven wavefronts a SIMD it spills, 580 us
+// at 108^3 cells; to five 554, with one sum 538.)
 template <int U>
-__global__ __launch_bounds__(kBlock, 7) void kRhoDf(Geom G, LatOffsets O, Tables<double> tb, CXPtr x,
+__global__ __launch_bounds__(kBlock, 5) void kRhoDf(Geom G, LatOffsets O, Tables<double> tb, CXPtr x,
                                                  const int8_t* __restrict__ type, double* __restrict__ df,
                                                  double* __restrict__ rho_out, uint64_t* __restrict__ wmask,
                                                  uint64_t* __restrict__ smask, double rcs2, InterView iv,
@@ -2292,10 +2295,9 @@ LdsForm forceForm(const DevState& s, bool mixed) {
   return share <= 0.5 || (share <= kGatherShareD && fillsLaunch(s, 2.0)) ? kLdsGather : kLdsNone;
 }
 // The FP64 density pass has no gather form: LDS cubics and queue against
-// neither, by solutes, the same boxes: 0 % 380/576, 6 % 506/594, 15 % 594/616,
-// 25 % 717/637; 10000 knots 0 % 564/641, 1.5 % 662/652, 6 % 710/662; 20000
-// knots 755/731.
-constexpr double kQueueShareRho = 0.17;
+// neither, by solutes, the same boxes: 0 % 380/553 us, 6 % 506/575, 15 %
+// 597/598; 10000 knots 0 % 564/616, 1.5 % 656/629; 20000 knots 744/716.
+constexpr double kQueueShareRho = 0.13;
 bool rhoLdsPays(const DevState& s) {
   return s.lds == kLdsOn || s.solutes + (1.0 - s.solutes) * 0.5 * s.nearRhoD <= kQueueShareRho;
 }
