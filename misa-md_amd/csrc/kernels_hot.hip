@@ -71,18 +71,22 @@ __device__ __forceinline__ uint32_t waveId(uint32_t b) {
 }
 
 // The site passes carry the inter atoms' work of the same pass along, in their
-// first kFrontBlocks blocks (a multiple of 8, so that the others keep their
-// XCD): neither part reads what the other writes, and a launch of its own for
-// a list that is mostly empty costs 2 to 5 us.  With no inter atom 64 blocks
-// and 256 take the same step (2 000 to 93 000 atoms, 36 to 71 us); with many of
-// them 64 are too few wavefronts, a wavefront working one atom off after the
-// other (93 000 atoms FP64: 4 000 inter atoms 766 -> 603 us a step, 12 000 3174 ->
-// 2481; 755 and 2689 in launches of their own).
-constexpr uint32_t kFrontBlocks = 256;
+// first blocks (a multiple of 8, so that the others keep their XCD): neither
+// part reads what the other writes, and a launch of its own for a list that is
+// mostly empty costs 2 to 5 us.  A wavefront works one atom off after the
+// other, and a cascade's inter atoms grow with the box: as many blocks as the
+// site grid has, 64 to 256.  64 everywhere are too few wavefronts for thousands
+// (93 000 atoms FP64: 4 000 inter atoms 766 -> 603 us a step with 256, 12 000 3174
+// -> 2481; 755 and 2689 in launches of their own); 256 everywhere cost 2 000 atoms
+// at rest 0.5 us a pass.
+__host__ __device__ inline uint32_t frontBlocks(const Geom& G) {
+  const uint32_t n = static_cast<uint32_t>(16 * G.W.bpx);
+  return n < 64u ? 64u : n > 256u ? 256u : n;
+}
 __device__ __forceinline__ int frontWave() {
   return static_cast<int>(blockIdx.x * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
 }
-constexpr int kFrontWaves = static_cast<int>(kFrontBlocks) * (kBlock / 64);
+__device__ __forceinline__ int frontWaves(const Geom& G) { return static_cast<int>(frontBlocks(G) * (kBlock / 64)); }
 // A wavefront-uniform 64-bit value moved to scalar registers.
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
@@ -318,11 +322,11 @@ __global__ __launch_bounds__(kBlock, 5) void kRhoDf(Geom G, LatOffsets O, Tables
                                                  double* __restrict__ rho_out, uint64_t* __restrict__ wmask,
                                                  uint64_t* __restrict__ smask, double rcs2, InterView iv,
                                                  InterDev in, Rec64 r64, int mlo) {
-  if (blockIdx.x < kFrontBlocks) {
-    interRhoBody<double>(G, tb, iv, x, type, in, frontWave(), kFrontWaves);
+  if (blockIdx.x < frontBlocks(G)) {
+    interRhoBody<double>(G, tb, iv, x, type, in, frontWave(), frontWaves(G));
     return;
   }
-  const uint32_t b = blockIdx.x - kFrontBlocks;
+  const uint32_t b = blockIdx.x - frontBlocks(G);
   int64_t s;
   int p, cx, cy, cz;
   if (!siteOfBlock(G, b, threadIdx.x, s, p, cx, cy, cz)) return;
@@ -437,11 +441,11 @@ __global__ __launch_bounds__(kBlock) void kRhoDfP(Geom G, LatOffsets O, Tables<d
                                                   InterDev in, Rec64 r64, int mlo) {
   __shared__ RangeParts parts, oparts;
   __shared__ TailHits hits;
-  if (blockIdx.x < kFrontBlocks) {
-    interRhoBody<double>(G, tb, iv, x, type, in, frontWave(), kFrontWaves);
+  if (blockIdx.x < frontBlocks(G)) {
+    interRhoBody<double>(G, tb, iv, x, type, in, frontWave(), frontWaves(G));
     return;
   }
-  const SharedSite q = sharedSite(G, type, blockIdx.x - kFrontBlocks);
+  const SharedSite q = sharedSite(G, type, blockIdx.x - frontBlocks(G));
   const bool live = !isVacant(q.ti);
   const bool skin = __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(live && (q.ti & kWide));
   RangeSum<0> acc, oacc;
@@ -773,11 +777,11 @@ __global__ __launch_bounds__(kBlock) void kForceP(Geom G, LatOffsets O, Tables<d
                                                   int mlo) {
   __shared__ double parts[3][6][64];
   __shared__ TailHits hits;
-  if (blockIdx.x < kFrontBlocks) {
-    interForceBody<double, MODE>(G, tb, iv, x, type, df, 1, in, vp, frontWave(), kFrontWaves);
+  if (blockIdx.x < frontBlocks(G)) {
+    interForceBody<double, MODE>(G, tb, iv, x, type, df, 1, in, vp, frontWave(), frontWaves(G));
     return;
   }
-  const SharedSite q = sharedSite(G, type, blockIdx.x - kFrontBlocks);
+  const SharedSite q = sharedSite(G, type, blockIdx.x - frontBlocks(G));
   const int lane = static_cast<int>(threadIdx.x & 63u);
   ForceSiteD c{};
   Force3 part, opart;
@@ -1042,12 +1046,12 @@ __global__ __launch_bounds__(kBlock) void kForce(Geom G, LatOffsets O, Tables<do
                                                  int mlo) {
   unsigned long long vb = 0;  // |v|^2 bits after the secondstep (MODE 0)
   unsigned long long db = 0;  // |dx|^2 bits of the drift (MODE 1)
-  if (blockIdx.x < kFrontBlocks) {
-    interForceBody<double, MODE>(G, tb, iv, x, type, df, 1, in, vp, frontWave(), kFrontWaves);
+  if (blockIdx.x < frontBlocks(G)) {
+    interForceBody<double, MODE>(G, tb, iv, x, type, df, 1, in, vp, frontWave(), frontWaves(G));
     return;
   }
   forceSiteD<MODE, U>(G, O, tb, x, xn, type, df, wmask, v, f, id, vp, st, ctl, iv, r64, rn64, mlo,
-                      blockIdx.x - kFrontBlocks, threadIdx.x, vb, db);
+                      blockIdx.x - frontBlocks(G), threadIdx.x, vb, db);
   if (MODE == 0 && vp.vmax) waveMaxTo(vb, vp.vmax);
   if (MODE == 1) waveMaxTo(db, &ctl->dispmax2);
 }
@@ -1621,11 +1625,11 @@ __global__ __launch_bounds__(kBlock) void kRhoDfMP(Geom G, LatOffsets O, Tables<
                                                    float rcs2, InterView iv, InterDev in) {
   __shared__ RangeParts parts;
   __shared__ TailHits hits;
-  if (blockIdx.x < kFrontBlocks) {
-    interRhoBody<float>(G, tb, iv, x, type, in, frontWave(), kFrontWaves);
+  if (blockIdx.x < frontBlocks(G)) {
+    interRhoBody<float>(G, tb, iv, x, type, in, frontWave(), frontWaves(G));
     return;
   }
-  const SharedSite q = sharedSite(G, type, blockIdx.x - kFrontBlocks);
+  const SharedSite q = sharedSite(G, type, blockIdx.x - frontBlocks(G));
   const bool live = !isVacant(q.ti);
   const bool skin = __builtin_amdgcn_readfirstlane(iv.ctl->skin_mode) != 0 && !__ballot(live && (q.ti & kWide));
   RangeSum<ACC> acc;
@@ -1653,11 +1657,11 @@ __global__ __launch_bounds__(kBlock, U == 4 ? 8 : 6) void kRhoDfM(Geom G, LatOff
                                                   const float4* __restrict__ dl, double* __restrict__ rho_out,
                                                   uint64_t* __restrict__ wmask, uint64_t* __restrict__ smask,
                                                   float rcs2, InterView iv, InterDev in) {
-  if (blockIdx.x < kFrontBlocks) {
-    interRhoBody<float>(G, tb, iv, x, type, in, frontWave(), kFrontWaves);
+  if (blockIdx.x < frontBlocks(G)) {
+    interRhoBody<float>(G, tb, iv, x, type, in, frontWave(), frontWaves(G));
     return;
   }
-  rhoPassM<ACC, U>(G, O, tb, x, type, rec, dl, rho_out, wmask, smask, rcs2, iv, blockIdx.x - kFrontBlocks);
+  rhoPassM<ACC, U>(G, O, tb, x, type, rec, dl, rho_out, wmask, smask, rcs2, iv, blockIdx.x - frontBlocks(G));
 }
 
 // The density pass of every box of a batch in one launch: the blocks of box
@@ -1711,12 +1715,12 @@ __global__ __launch_bounds__(kBlock) void kForceM(Geom G, LatOffsets O, Tables<f
                                                   Ctl* ctl, InterView iv, InterDev in, int mlo) {
   unsigned long long vb = 0;  // |v|^2 bits after the secondstep (MODE 0)
   unsigned long long db = 0;  // |dx|^2 bits of the drift (MODE 1)
-  if (blockIdx.x < kFrontBlocks) {
+  if (blockIdx.x < frontBlocks(G)) {
     interForceBody<float, MODE>(G, tb, iv, x, type, reinterpret_cast<const float*>(rec) + 3, 4, in, vp, frontWave(),
-                                kFrontWaves);
+                                frontWaves(G));
     return;
   }
-  const uint32_t b = blockIdx.x - kFrontBlocks;
+  const uint32_t b = blockIdx.x - frontBlocks(G);
   [&] {
     int64_t s;
     int p, cx, cy, cz;
@@ -1756,12 +1760,12 @@ __global__ __launch_bounds__(kBlock) void kForceMP(Geom G, LatOffsets O, Tables<
   __shared__ Term chunks[kChunks][3][64];
   __shared__ WaveSumsM others[3];
   __shared__ TailHits hits;
-  if (blockIdx.x < kFrontBlocks) {
+  if (blockIdx.x < frontBlocks(G)) {
     interForceBody<float, MODE>(G, tb, iv, x, type, reinterpret_cast<const float*>(rec) + 3, 4, in, vp, frontWave(),
-                                kFrontWaves);
+                                frontWaves(G));
     return;
   }
-  const SharedSite q = sharedSite(G, type, blockIdx.x - kFrontBlocks);
+  const SharedSite q = sharedSite(G, type, blockIdx.x - frontBlocks(G));
   const int lane = static_cast<int>(threadIdx.x & 63u);
   const int ei = species(q.ti);
   float4 me = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -2332,7 +2336,7 @@ int launchRhoDf(const DevState& s, const LatOffsets& o, const Tables<double>& t6
                 bool mixed, int acc, bool store_rho, bool scan, hipStream_t st) {
   double* rho = store_rho ? s.rho : nullptr;
   const bool shared = useShared(s);
-  const unsigned grid = kFrontBlocks + (shared ? 4 : 1) * siteGrid(s.G);
+  const unsigned grid = frontBlocks(s.G) + (shared ? 4 : 1) * siteGrid(s.G);
   const InterView iv = interView(s, mixed);
   const CXPtr x = cxp(s.x[s.cur]);
   const double rcs = std::sqrt(s.G.rc2) + s.skin;
@@ -2389,7 +2393,7 @@ int launchForce(const DevState& s, const LatOffsets& o, const Tables<double>& t6
                 bool mixed, int acc, int mode, const VerletParams& vp, hipStream_t st) {
   int kind = mixed ? 1 : 0;
   const bool shared = useShared(s);
-  const unsigned grid = kFrontBlocks + (shared ? 4 : 1) * siteGrid(s.G);
+  const unsigned grid = frontBlocks(s.G) + (shared ? 4 : 1) * siteGrid(s.G);
   const CXPtr x = cxp(s.x[s.cur]);
   const XPtr xn = xp(s.x[1 - s.cur]);
   const StageArgs sa = stageOf(s);
