@@ -1445,8 +1445,10 @@ __global__ __launch_bounds__(kBlockP) void kEnergyDL(Geom G, LatOffsets O, const
 // The FP64 force pass in persistent blocks, one per compute unit, with the
 // Fe-Fe segments from knot mlo on in LDS (forceVBlockD).  2M atoms with the
 // fused half steps: 546 us, against 657 with 7 doubles a knot, the other pairs
-// re-read under a mask and one group in flight.  Its four wavefronts per SIMD
-// still wait a third of their time; VALU issue takes 59 % of the slots.
+// re-read under a mask and one group in flight.  At 16M atoms (4.41 ms) the
+// queued neighbours' records come from beyond the L2 a second time, 1189 bytes
+// an atom in all, 4.3 TB/s or 90 % of what a copy reaches; the texture-data
+// units are 90 % busy and VALU issue takes 64 % of the cycles.
 template <int MODE, int U>
 __global__ __launch_bounds__(kBlockP) void kForceDL(Geom G, LatOffsets O, Tables<double> tb, CXPtr x, XPtr xn,
                                                     const int8_t* __restrict__ type, const double* __restrict__ df,
@@ -2014,10 +2016,12 @@ __device__ __forceinline__ void fillKnots(const Tables<float>& tb, float4* knT, 
 // one broadcast per offset), the Fe-Fe r*phi cubics and the Fe density slope
 // cubics from knot mlo on (one block fills them once).  Per site the same
 // pairs, in the same order and with the same rounding, as kForceM.
-// 16M-atom cascade 2.44 -> 2.24 ms against segments re-read under a mask, one
-// group in flight and the two cubics side by side in LDS; 2M atoms with the
-// fused half steps 309 -> 280 us.  Its VALU issue (71 % of the slots, 3,800
-// instructions per 64 sites) and its LDS reads (44 %) bound it.
+// 2M atoms with the fused half steps 308 -> 303 us, 16M-atom cascade 2.44 -> 2.35
+// ms, against segments re-read under a mask, one group in flight and the two
+// cubics side by side in LDS (280 and 2.24 while the terms of the queued pairs
+// were rounded to 2^-36 eV/A on the way).  Its VALU issue (70 % of the cycles,
+// 3,990 instructions per 64 sites), the texture-data units (86 % busy) and its LDS
+// reads (43 %, half of that bank conflicts) bound it together.
 template <int ACC, int MODE, int U>
 __global__ __launch_bounds__(kBlockP) void kForceL(Geom G, LatOffsets O, Tables<float> tb, CXPtr x, XPtr xn,
                                                    const int8_t* __restrict__ type, const float4* __restrict__ rec,
@@ -2208,7 +2212,7 @@ LdsKnots ldsKnotsForceD(int nr) {
   return k;
 }
 // The FP64 density pass's LDS knots, 32 bytes each, beside its queues and
-// sums: 4542 knots, from 0.51 A on where the table has 5000 over 5.6 A.
+// sums: 4670 knots, from 0.37 A on where the table has 5000 over 5.6 A.
 constexpr int kURhoD = 2;
 constexpr int kRhoLdsBytesD =
     160 * 1024 - static_cast<int>(kBlockP / 64 * (sizeof(WaveQueueD<kURhoD>) + sizeof(WaveSum1))) - 64;

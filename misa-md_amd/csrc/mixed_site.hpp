@@ -161,7 +161,7 @@ __device__ __forceinline__ void forceGroupM(const float4& me, float dfi, int ei,
 // from knot mlo on in LDS (knT, kKnotsM entries apart): the held pairs of the
 // group, the same terms in the same order.  The other pairs
 // within the cutoff go to the wavefront's queue; qn counts it.  The pass is
-// bound by its VALU instructions (80 % of the issue slots), so the tests are
+// bound by its VALU instructions first (70 % of the cycles), so the tests are
 // combined as wavefront masks in scalar registers.
 template <int ACC, int V>
 __device__ __forceinline__ void forceGroupL(const float4& me, float dfi, int ei, const float4 (&nb)[V],
